@@ -162,7 +162,8 @@ int micro_write_vtu(const char *name);
  * mesh: the 3-row block of an interior node is fixed by the materials of its
  * 8 elements, so each RVE keeps a dictionary of the 256 possible blocks (the
  * same FP64 sums, rounded) and one pattern byte per node; the matrix then
- * lives in L1/L2 instead of HBM. */
+ * lives in L1/L2 instead of HBM.  An RVE small enough to be swept on chip is
+ * solved from those blocks with either storage. */
 #define MM_ELL_FULL 0
 #define MM_ELL_DICT 1
 
@@ -192,9 +193,13 @@ typedef struct {
   double inner_rtol;     /* per-sweep PCG target */
   int max_inner_its;
   int max_sweeps;
-  int steps_per_launch;  /* PCG iterations per launch / graph replay */
+  int steps_per_launch;  /* PCG iterations per launch / graph replay (whole
+                            sweeps, at most six, while every RVE being solved
+                            is small enough to be swept on chip: up to about
+                            32 x 32 elements across) */
   int use_graph;         /* capture the steps in a hipGraph */
-  int sync_every_step;   /* plain path: host reads the state after every step */
+  int sync_every_step;   /* plain path: host reads the state after every PCG
+                            iteration (no on-chip sweeps) */
   int ell_storage;       /* MM_ELL_FULL or MM_ELL_DICT (default DICT) */
   int initial_guess;     /* MM_GUESS_ZERO or MM_GUESS_AFFINE (default AFFINE) */
   int solver_streams;    /* 1, or 2 (default): resident RVEs stepped in two
@@ -202,7 +207,9 @@ typedef struct {
   int profile_step_kernel; /* 1: no graph, one stream, and every launch of the
                             PCG step kernel (kernel A: SpMV + p/q update)
                             timed with HIP events (mm_engine_step_kernel_times) */
-  int march_planes;      /* kernel A: 0 works slab by slab, gathering every
+  int march_planes;      /* kernel A, which steps the RVEs that are not swept on
+                            chip (and all of them with sync_every_step or
+                            profile_step_kernel): 0 works slab by slab, gathering every
                             neighbour from memory; n > 0 (default 8) marches
                             in-plane chunks of slab_nodes nodes through runs
                             of n z-planes with the neighbour planes staged in

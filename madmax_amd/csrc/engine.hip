@@ -72,6 +72,10 @@ struct RangeAlloc {
   }
 };
 
+// Solver steps per launch where every RVE is solved by resident sweeps: the
+// first residual, up to three sweeps, the averages and the result.
+constexpr int kSweepSteps = 6;
+
 enum SlotState { SL_FREE = 0, SL_ACTIVE = 1, SL_CACHED = 2 };
 
 struct HostSlot {
@@ -217,10 +221,17 @@ struct mm_engine {
   bool act_dirty = true;
   long long act_n[2] = {0, 0}, tile_n[2] = {0, 0};
   int a_lds[2] = {0, 0}, a_slab[2] = {0, 0}, s_big[2] = {0, 0};
+  // resident sweep: per group g the workgroups' (slot, load case * 16 + rank)
+  // at units + g * unit_stride, [0].x their count, staged in st_units, and its
+  // ticket counter (parts of act_list's, st_act's and rves' allocations)
+  int2 *units = nullptr, *st_units = nullptr;
+  unsigned *ticket = nullptr;
+  size_t unit_stride = 0;
+  long long unit_n[2] = {0, 0};
   // one captured graph per set of launch shapes (grids: powers of two >= 64
   // covering each group's slabs and tiles, 0 for an empty group; kernel A's
   // LDS); the kernels read the active count from their list
-  std::map<std::array<int, 10>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
+  std::map<std::array<int, 13>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
   // stats / threading
   std::mutex step_mu;
   long long completed = 0, nsteps = 0;
@@ -263,6 +274,10 @@ struct mm_engine {
     P.a_lds = 0;
     P.a_slab = 0;
     P.s_big = 0;
+    P.units = units;
+    P.ticket = ticket;
+    P.u_grid = 0;
+    P.u_lds = 0;
     P.dict = dict;
     P.dict64 = dict64;
     P.SN = SN;
@@ -417,6 +432,11 @@ extern "C" int mm_engine_create(const mm_engine_config *cfg, mm_engine **out)
   e->elem_cap = e->nslab_cap * e->SN + 64;
   const size_t nrows = (size_t)e->nslab_cap * e->rows_per_slab();
   const size_t slots = nrows * kW;
+  // the active lists, then the resident sweep's units (a resident RVE has K *
+  // scw of them, scw at most kSweepMaxRanks and at most its slabs)
+  const size_t act_ints = 4 * ((size_t)e->nslab_cap + 1);
+  e->unit_stride = 1 + (size_t)e->K * std::min<size_t>((size_t)kSweepMaxRanks * e->rve_cap, (size_t)e->nslab_cap);
+  const size_t lists = act_ints * sizeof(int) + 2 * e->unit_stride * sizeof(int2);
   if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess) {
     delete e;
     return MM_ERR_HIP;
@@ -449,7 +469,8 @@ extern "C" int mm_engine_create(const mm_engine_config *cfg, mm_engine **out)
     else EALLOC(e->dict, (size_t)e->rve_cap * kDictPat * kDictEntry * 4);
   }
   EALLOC(e->npat, (size_t)e->nslab_cap * e->SN);
-  EALLOC(e->act_list, 4 * ((size_t)e->nslab_cap + 1) * 4);
+  EALLOC(e->act_list, lists);
+  e->units = reinterpret_cast<int2 *>(e->act_list + act_ints);
   EALLOC(e->dinv, nrows * e->tsz);
   EALLOC(e->x64, nrows * e->K * 8);
   EALLOC(e->d, nrows * e->K * e->tsz);
@@ -459,7 +480,8 @@ extern "C" int mm_engine_create(const mm_engine_config *cfg, mm_engine **out)
   EALLOC(e->part, (size_t)e->nslab_cap * kPartDoubles * 8);
   EALLOC(e->slab_rve, (size_t)e->nslab_cap * 4);
   EALLOC(e->slab_node0, (size_t)e->nslab_cap * 4);
-  EALLOC(e->rves, (size_t)e->rve_cap * sizeof(RveDev));
+  EALLOC(e->rves, (size_t)e->rve_cap * sizeof(RveDev) + 2 * sizeof(unsigned));  // and the two tickets
+  e->ticket = reinterpret_cast<unsigned *>(e->rves + e->rve_cap);
   EALLOC(e->elem_mat, (size_t)e->elem_cap);
   EALLOC(e->ke_tab, (size_t)e->rve_cap * kNmat * kKe * 8);
   EALLOC(e->c_tab, (size_t)e->rve_cap * kNmat * 36 * 8);
@@ -471,17 +493,17 @@ extern "C" int mm_engine_create(const mm_engine_config *cfg, mm_engine **out)
     goto fail;
   }
   memset(e->out_host, 0, (size_t)e->rve_cap * sizeof(RveOut));
-  if (hipHostMalloc((void **)&e->st_act, 4 * ((size_t)e->nslab_cap + 1) * 4, hipHostMallocDefault) !=
-      hipSuccess) {
+  if (hipHostMalloc((void **)&e->st_act, lists, hipHostMallocDefault) != hipSuccess) {
     rc = MM_ERR_HIP;
     goto fail;
   }
+  e->st_units = reinterpret_cast<int2 *>(e->st_act + act_ints);
   if (hipHostGetDevicePointer((void **)&e->out_dev, e->out_host, 0) != hipSuccess) {
     rc = MM_ERR_HIP;
     goto fail;
   }
   if (hipMemsetAsync(e->slab_rve, 0xff, (size_t)e->nslab_cap * 4, e->stream) != hipSuccess ||
-      hipMemsetAsync(e->rves, 0, (size_t)e->rve_cap * sizeof(RveDev), e->stream) != hipSuccess) {
+      hipMemsetAsync(e->rves, 0, (size_t)e->rve_cap * sizeof(RveDev) + 2 * sizeof(unsigned), e->stream) != hipSuccess) {
     rc = MM_ERR_HIP;
     goto fail;
   }
@@ -742,6 +764,53 @@ static int march_lds_need(const mm_engine *e, const HostSlot &h)
                      : 0;
 }
 
+// Resident sweep of an RVE of nx x ny x nz nodes (RveDev::scw ..): the fewest
+// workgroups per load case whose share of the interior z-planes fits the lanes'
+// items and the LDS, cut into items of few enough planes that small RVEs still
+// occupy the lanes.  cw = 0 (kernels A and B) without an interior, where the
+// planes are too wide or too many, and for the engines whose steps are single
+// PCG iterations by request: sync_every_step reads the state after each,
+// profile_step_kernel times each one's kernel A.  Fixed by the RVE and the
+// engine configuration alone.
+struct SweepTiling {
+  int cw = 0, lp = 0, nch = 0;
+};
+static SweepTiling sweep_tiling(const mm_engine *e, const mm_rve_spec &s, long long nslab)
+{
+  SweepTiling t;
+  if (e->cfg.sync_every_step || e->cfg.profile_step_kernel) return t;
+  const long long nix = s.nex - 1, niy = s.ney - 1, niz = s.nez - 1;
+  const int tsz = (int)e->tsz, waves = kSweepLanes / 64, most = waves * kSweepItems;
+  if (nix < 1 || niy < 1 || niz < 1 || nix > 4096 || niy > 4096) return t;
+  const long long ns = sweep_strips(s.nex + 1, s.ney + 1);
+  const long long plane = (long long)sweep_plane(s.nex + 1, s.ney + 1) * 3 * tsz;
+  const long long room = (kSweepMaxLds - sweep_dict_bytes(tsz)) / plane;  // planes that fit
+  double best = 0.0;
+  for (int cw = 1; cw <= kSweepMaxRanks && cw <= niz && cw <= nslab; cw++) {
+    const long long L = (niz + cw - 1) / cw;
+    for (long long nch = 1; nch <= L && nch * ns <= most; nch++) {
+      const long long lp = (L + nch - 1) / nch;
+      if (lp > sweep_max_planes(tsz) || sweep_lds_planes((int)lp, (int)nch) > room) continue;
+      // an iteration's time in planes of a strip: the longest wave's items, each
+      // with its latency, or the fullest SIMD's, and the barriers and sums;
+      // times the CUs it holds
+      const double S = (double)(ns * nch), u = sweep_unroll((int)lp);
+      const double cost =
+          cw * (std::max(std::ceil(S / waves) * (u + 4.0), std::ceil(S / 4.0) * (u + 1.0)) + (cw > 1 ? 12.0 : 4.0));
+      if (t.cw && cost >= best) continue;
+      best = cost;
+      t.cw = cw;
+      t.lp = (int)lp;
+      t.nch = (int)nch;
+    }
+  }
+  if (t.cw > 1) {  // the exchanged words must fit the RVE's part of p, q and d
+    const long long part = nslab * e->rows_per_slab() * (long long)tsz;
+    if (8LL * (t.cw - 1) * sweep_words(sweep_positions(s.nex + 1, s.ney + 1), tsz) > part || 8LL * kSweepSumWords > part) t = SweepTiling();
+  }
+  return t;
+}
+
 static void fill_state(const mm_engine *e, const HostSlot &h, RveDev *st, int warm)
 {
   memset(st, 0, sizeof(*st));
@@ -782,7 +851,11 @@ static void fill_state(const mm_engine *e, const HostSlot &h, RveDev *st, int wa
   st->mnzc = mt.mnzc;
   st->mnt = mt.mnt;
   st->mncg = mt.mncg;
-  st->big = h.nslab >= e->cfg.big_slabs ? 1 : 0;
+  const SweepTiling sw = sweep_tiling(e, s, h.nslab);
+  st->scw = sw.cw;
+  st->slp = sw.lp;
+  st->snch = sw.nch;
+  st->big = (sw.cw == 0 && h.nslab >= e->cfg.big_slabs) ? 1 : 0;
   for (int k = 0; k < h.req.nload; k++)
     for (int i = 0; i < MM_NVOI; i++) st->load[k][i] = h.req.strain[k][i];
   if (warm)
@@ -959,11 +1032,17 @@ static int update_active(mm_engine *e)
   const bool march = e->cfg.march_planes > 0;
   long long n[2] = {0, 0}, nt[2] = {0, 0};
   int lds[2] = {0, 0}, slab_mode[2] = {0, 0}, big[2] = {0, 0};
+  std::vector<std::pair<long long, int2>> res[2];  // (nodes, (slot, ranks)) of the resident sweeps
   int g = 0;
   for (auto &r : runs) {
     const HostSlot &h = e->slots[r.second];
     if (g == 0 && ngroup == 2 && n[0] > 0 && 2 * n[0] >= total) g = 1;
     for (long long b = 0; b < h.nslab; b++) e->st_act[g * stride + 1 + n[g]++] = (int)(r.first + b);
+    const SweepTiling sw = sweep_tiling(e, h.req.rve, h.nslab);
+    if (sw.cw > 0) {
+      res[g].push_back({h.nrow / 3, make_int2(r.second, sw.cw)});
+      continue;
+    }
     if (h.nslab >= e->cfg.big_slabs) big[g] = 1;
     const MarchTiling m = march_tiling(e, h.req.rve, h.nslab);
     if (march && m.mcpp > 0) {
@@ -983,6 +1062,19 @@ static int update_active(mm_engine *e)
         MM_HIP(hipMemcpyAsync(e->act_list + (2 + q) * stride, e->st_act + (2 + q) * stride,
                               (size_t)(nt[q] + 1) * 4, hipMemcpyHostToDevice, e->stream));
     }
+    // the largest RVEs first, so that the last workgroups to finish are short
+    std::stable_sort(res[q].begin(), res[q].end(),
+                     [](const auto &a, const auto &b) { return a.first > b.first; });
+    int2 *un = e->st_units + q * e->unit_stride;
+    long long nu = 0;
+    for (auto &r : res[q])
+      for (int k = 0; k < e->slots[r.second.x].req.nload; k++)
+        for (int c = 0; c < r.second.y; c++) un[1 + nu++] = make_int2(r.second.x, k * kSweepMaxRanks + c);
+    un[0] = make_int2((int)nu, 0);
+    if (q < ngroup)
+      MM_HIP(hipMemcpyAsync(e->units + q * e->unit_stride, un, (size_t)(nu + 1) * sizeof(int2),
+                            hipMemcpyHostToDevice, e->stream));
+    e->unit_n[q] = nu;
     e->act_n[q] = n[q];
     e->tile_n[q] = nt[q];
     e->a_lds[q] = (march && nt[q] > 0) ? march_lds_class(lds[q]) : 0;
@@ -1007,7 +1099,7 @@ static int launch_grid(long long n)
 // work.  The second chain fills the first one's launch gaps and kernel tails
 // (A's register use leaves no room for B's waves beside it, so the two do not
 // otherwise overlap).
-static int queue_steps(mm_engine *e, int grid0, int grid1)
+static int queue_steps(mm_engine *e, int grid0, int grid1, int nsteps)
 {
   EngPtrs P0 = e->ptrs(), P1 = P0;
   P1.act_list = e->act_list + ((size_t)e->nslab_cap + 1);
@@ -1020,12 +1112,17 @@ static int queue_steps(mm_engine *e, int grid0, int grid1)
   P1.a_slab = e->a_slab[1];
   P0.s_big = e->s_big[0];
   P1.s_big = e->s_big[1];
+  P1.units = e->units + e->unit_stride;
+  P1.ticket = e->ticket + 1;
+  P0.u_grid = launch_grid(e->unit_n[0]);
+  P1.u_grid = launch_grid(e->unit_n[1]);
+  P0.u_lds = P1.u_lds = kSweepMaxLds;
   const SolveParams sp = e->params();
-  const int nk = 3 * e->cfg.steps_per_launch;
+  const int nk = 3 * nsteps;
   const bool f64 = e->fp64, dm = e->dict_mode;
   int rc = 0;
   if (e->cfg.profile_step_kernel && grid1 == 0) {
-    const int ns = e->cfg.steps_per_launch;
+    const int ns = nsteps;
     while ((int)e->prof_ev.size() < 2 * ns) {
       hipEvent_t ev;
       MM_HIP(hipEventCreate(&ev));
@@ -1042,7 +1139,7 @@ static int queue_steps(mm_engine *e, int grid0, int grid1)
   }
   if (grid1 == 0) return eng_launch_steps(f64, e->K, dm, P0, sp, grid0, 0, nk, e->stream);
   int first = 0;
-  if (grid0 > 0) {
+  if (grid0 > 0 && P0.u_grid == 0) {  // a resident sweep is too long a kernel to wait for
     if ((rc = eng_launch_steps(f64, e->K, dm, P0, sp, grid0, 0, 1, e->stream))) return rc;
     first = 1;
   }
@@ -1061,14 +1158,18 @@ static int run_steps(mm_engine *e)
   if (rc) return rc;
   const int grid0 = launch_grid(e->act_n[0]), grid1 = launch_grid(e->act_n[1]);
   if (grid0 == 0 && grid1 == 0) return 0;
-  if (!e->cfg.use_graph) return queue_steps(e, grid0, grid1);
-  const std::array<int, 10> key = {grid0, grid1, launch_grid(e->tile_n[0]), launch_grid(e->tile_n[1]),
+  // where every RVE is resident a step is a whole sweep: kSweepSteps of them
+  // finish a solve of up to three sweeps
+  int nsteps = e->cfg.steps_per_launch;
+  if (e->tile_n[0] + e->tile_n[1] == 0 && !e->a_slab[0] && !e->a_slab[1]) nsteps = std::min(nsteps, kSweepSteps);
+  if (!e->cfg.use_graph) return queue_steps(e, grid0, grid1, nsteps);
+  const std::array<int, 13> key = {grid0, grid1, launch_grid(e->tile_n[0]), launch_grid(e->tile_n[1]),
                                    e->a_lds[0], e->a_lds[1], e->a_slab[0], e->a_slab[1], e->s_big[0],
-                                   e->s_big[1]};
+                                   e->s_big[1], launch_grid(e->unit_n[0]), launch_grid(e->unit_n[1]), nsteps};
   auto it = e->graphs.find(key);
   if (it == e->graphs.end()) {
     MM_HIP(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-    rc = queue_steps(e, grid0, grid1);
+    rc = queue_steps(e, grid0, grid1, nsteps);
     hipGraph_t g = nullptr;
     hipError_t ce = hipStreamEndCapture(e->stream, &g);
     if (rc) {

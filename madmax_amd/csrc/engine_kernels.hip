@@ -30,6 +30,7 @@
 // (an agent-scope release in every workgroup costs an L2 write-back each).
 #include <hip/hip_runtime.h>
 
+#include "engine_device.h"
 #include "mm_device.h"
 #include "mm_internal.h"
 
@@ -792,144 +793,6 @@ struct Pair<double> {
   using type = double2;
 };
 
-// Per-slab partial sums of the launch that produced them, summed over the
-// RVE's slabs in slab order (group_sum_cols): every workgroup of the consuming
-// launch forms the same totals.  A slab has kPart partial values, value i
-// at part[i * part_stride + slab] (value-major, so that a sum over an RVE's
-// slabs reads contiguous memory).  Values:
-//   [0, K)      p.q            (A -> B)
-//   [K, 3K)     r.r, r.z       (B -> A)
-//   [3K, 7K)    residual norms (R -> A)
-//   [0, 12K)    averages       (R -> A), never pending with the others
-struct SlabPart {
-  double *p;
-  long long s;
-  __device__ __forceinline__ double &operator[](int i) const { return p[(size_t)i * s]; }
-};
-__device__ __forceinline__ SlabPart slab_part(const EngPtrs &P, int slab)
-{
-  return SlabPart{P.part + slab, P.part_stride};
-}
-
-// Start of a refinement sweep from the reduced residual norms s4 =
-// {||r64||^2, ||r||^2, r.z, ||r_cold||^2} per load case (FP64 residual r64,
-// its rounding r, cold-start right-hand side r_cold).
-template <int K>
-__device__ void start_sweep(SolveState &N, const double (&s4)[4 * K], const RveDev *R,
-                            const SolveParams &sp)
-{
-  const bool need_cold = (R->warm || R->affine) && N.sweep == 0;
-  unsigned done_out = 0;
-  for (int k = 0; k < K; k++) {
-    const double rn = sqrt(s4[k]);
-    N.rnorm[k] = rn;
-    if (N.sweep == 0) N.r0[k] = need_cold ? sqrt(s4[3 * K + k]) : rn;
-    const bool conv = (k >= R->nload) || N.r0[k] == 0.0 || rn <= sp.rtol * N.r0[k] ||
-                      rn < sp.abs_tol || N.sweep >= sp.max_sweeps;
-    if (conv) done_out |= 1u << k;
-    // absolute target of this sweep: inner_rtol of the sweep's right-hand
-    // side, but no tighter than what the outer tolerance still needs
-    const double cap = (N.r0[k] > 0.0 && rn > 0.0) ? 0.5 * sp.rtol * N.r0[k] / rn : 0.0;
-    N.bnorm_in[k] = fmax(sp.inner_rtol, cap) * sqrt(s4[K + k]);
-    N.beta[k] = 0.0;
-    N.rz[k] = s4[2 * K + k];
-  }
-  const unsigned all = (1u << K) - 1u;
-  N.done_out = done_out;
-  if ((done_out & all) == all) {
-    N.phase = PH_AVG;
-  } else {
-    N.done_in = done_out;
-    N.its = 0;
-    N.phase = PH_INNER;
-  }
-}
-
-// End of a PCG iteration from the reduced s2 = {r.r, r.z}: each load case
-// stops at its own sweep target; the sweep ends (x += d, then a new FP64
-// residual) when all have, or at max_inner_its.  Returns true at sweep end.
-template <int K>
-__device__ bool inner_check(SolveState &N, const double (&s2)[2 * K], const SolveParams &sp)
-{
-  N.its += 1;
-  unsigned done = N.done_in;
-  const unsigned all = (1u << K) - 1u;
-  for (int k = 0; k < K; k++) {
-    const double rr = s2[k], rz = s2[K + k];
-    if ((done >> k) & 1u) {
-      N.beta[k] = 0.0;
-      continue;
-    }
-    if (sqrt(rr) <= N.bnorm_in[k] || N.rz[k] == 0.0) {
-      done |= 1u << k;
-      N.beta[k] = 0.0;
-    } else {
-      N.beta[k] = rz / N.rz[k];
-      N.rz[k] = rz;
-    }
-  }
-  N.done_in = done;
-  if ((done & all) == all || N.its >= sp.max_inner_its) {
-    N.its_total += N.its;
-    N.sweep += 1;
-    N.phase = PH_RES;
-    return true;
-  }
-  return false;
-}
-
-// Volume averages and tangent of a finished RVE (micro/src/homogenize.c:
-// 344-368, :80) from the averaging partials; run by one workgroup.
-template <int K, int L>
-__device__ void finish_rve(const EngPtrs &P, int slot, const RveDev *R, SolveState &N,
-                           const SolveParams &sp, double (&lds)[L])
-{
-  __shared__ double tot[MM_MAX_RHS][12];
-  const double *p0 = slab_part(P, R->first_slab).p;
-#pragma unroll 1
-  for (int k = 0; k < K; k++) group_sum_cols_lds<12>(p0, R->nslab, P.part_stride, k * 12, &tot[k][0], lds);
-  __shared__ double sig[MM_MAX_RHS][6];
-  if (threadIdx.x != 0) return;
-  RveOut *o = P.out + slot;
-  double rel = 0.0;
-  bool ok = true;
-#pragma unroll 1
-  for (int k = 0; k < K; k++) {
-#pragma unroll 1
-    for (int i = 0; i < 12; i++) {
-      const double s = tot[k][i] / R->vol;
-      if (i < 6) o->strain[k][i] = s;
-      else {
-        o->stress[k][i - 6] = s;
-        sig[k][i - 6] = s;
-      }
-    }
-    if (k < R->nload) {
-      const double r0 = N.r0[k], rn = N.rnorm[k];
-      rel = fmax(rel, (r0 > 0.0) ? rn / r0 : 0.0);
-      if (!(r0 == 0.0 || rn <= sp.rtol * r0 || rn < sp.abs_tol)) ok = false;
-    }
-  }
-  for (int i = 0; i < 36; i++) o->c[i] = 0.0;
-  if (R->tangent_mode == MM_TANGENT_UNIT && K >= 6) {
-    for (int i = 0; i < 6; i++)
-      for (int j = 0; j < 6; j++) o->c[j * 6 + i] = sig[i][j] / R->load[i][i];
-  } else if (R->tangent_mode == MM_TANGENT_FD && K >= 7) {
-    for (int i = 0; i < 6; i++)
-      for (int j = 0; j < 6; j++)
-        o->c[j * 6 + i] = (sig[i + 1][j] - sig[0][j]) / (R->load[i + 1][i] - R->load[0][i]);
-  }
-  o->residual_rel = rel;
-  o->its_total = N.its_total;
-  o->sweeps = N.sweep;
-  o->status = ok ? MM_OK : MM_NOT_CONVERGED;
-  N.status = o->status;
-  N.phase = PH_DONE;
-  __threadfence_system();
-  o->phase = PH_DONE;
-  __threadfence_system();
-}
-
 // The INNER work of kernel A for one slab: w = A z (one lane per node), then
 // on the node's own rows p = z + beta p, q = w + beta q (so q = A p without
 // gathering p) and the partial p.q.  Every load case is gathered (a per-case
@@ -1023,10 +886,10 @@ __global__ __launch_bounds__(256) void k_step_a(EngPtrs P, SolveParams sp)
   const int slot = P.slab_rve[slab];
   if (slot < 0) return;
   RveDev *R = P.rves + slot;
-  if (P.a_lds > 0 && R->mcpp > 0) return;  // k_step_a_march's
-  const bool writer = slab == R->first_slab;
-  const int nslab = R->nslab;
-  const int phase0 = R->st[2].phase;
+  // read together: a branch between them would make each a round trip
+  const int mcpp = R->mcpp, scw = R->scw, nslab = R->nslab, first = R->first_slab, phase0 = R->st[2].phase;
+  if ((P.a_lds > 0 && mcpp > 0) || scw > 0) return;  // k_step_a_march's or k_sweep's
+  const bool writer = slab == first;
   const double *p0 = slab_part(P, R->first_slab).p;
   if (phase0 == PH_AVGRED) {
     if (!writer) return;
@@ -1612,8 +1475,27 @@ __global__ __launch_bounds__(256) void k_step_b(EngPtrs P, SolveParams sp)
   if (slot < 0) return;
   RveDev *R = P.rves + slot;
   const SolveState *S = &R->st[0];
+  const int scw = R->scw, phase = S->phase;  // read together
+  if (scw > 0) {
+    // a resident sweep has run to its end: the count is the largest of the
+    // load cases' (as inner_check counts), and the residual comes next
+    if (slab == R->first_slab && tid == 0) {
+      SolveState N = *S;
+      if (N.phase == PH_INNER) {
+        N.its = 0;
+        for (int k = 0; k < K; k++)
+          if (!((N.done_in >> k) & 1u)) N.its = max(N.its, R->lits[k]);
+        N.its_total += N.its;
+        N.sweep += 1;
+        N.phase = PH_RES;
+      }
+      R->st[1] = N;
+      *P.ticket = 0u;  // for the next resident sweep
+    }
+    return;
+  }
   if (slab == R->first_slab && tid == 0) R->st[1] = *S;
-  if (S->phase != PH_INNER) return;
+  if (phase != PH_INNER) return;
   const unsigned skip = S->done_in;
   const int nslab = R->nslab;
   double s1[K];
@@ -1716,6 +1598,28 @@ __global__ __launch_bounds__(256) void k_step_b(EngPtrs P, SolveParams sp)
 // or warm-started measures it at sweep 0 from the boundary neighbours alone.
 // PH_AVG: per-slab partial volume averages of strain and stress in FP64,
 // sum_gp (.) w_gp per element through sum_gp B w, one load case at a time.
+// Zeroes the slab's share of the words that the ranks of a resident sweep
+// exchange (tag 0 is no iteration's).
+template <typename TS, int K>
+__device__ void sweep_words_zero(const EngPtrs &P, const RveDev *R, int slab)
+{
+  typedef unsigned long long u64;
+  const int ls = slab - R->first_slab;
+  const int nw = (R->scw - 1) * sweep_words(sweep_positions(R->nx, R->ny), (int)sizeof(TS));
+#pragma unroll 1
+  for (int k = 0; k < K; k++) {
+    const long long b0 = sweep_region(R->nslab, P.SN, K, (int)sizeof(TS), R->first_slab, k);
+    u64 *up = reinterpret_cast<u64 *>((char *)P.p + b0), *down = reinterpret_cast<u64 *>((char *)P.q + b0);
+    for (int i = ls * (int)blockDim.x + (int)threadIdx.x; i < nw; i += R->nslab * (int)blockDim.x) {
+      up[i] = 0;
+      down[i] = 0;
+    }
+    if (ls == 0)
+      for (int i = threadIdx.x; i < kSweepSumWords; i += blockDim.x)
+        reinterpret_cast<u64 *>((char *)P.d + b0)[i] = 0;
+  }
+}
+
 template <typename TS, int K>
 __device__ void res_slab(const EngPtrs &P, int slab, int slot, const RveDev *R, bool need_cold,
                          double (&lds)[RedLds<K>::size])
@@ -1771,7 +1675,7 @@ __device__ void res_slab(const EngPtrs &P, int slab, int slot, const RveDev *R, 
     }
     const long long nb = node_vec(P, R->first_slab, n, K);
     const TS *dinv = (const TS *)P.dinv + (long long)slab * RS + 3 * tid;
-    TS ri[3][K], zi[3][K], zero[3][K];
+    TS ri[3][K], zi[3][K];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
       const TS dg = dinv[d];
@@ -1780,7 +1684,6 @@ __device__ void res_slab(const EngPtrs &P, int slab, int slot, const RveDev *R, 
         const double rk = -r64[d][k];
         ri[d][k] = (TS)rk;
         zi[d][k] = dg * ri[d][k];
-        zero[d][k] = (TS)0;
         v[k] = fma(rk, rk, v[k]);
         v[K + k] = fma((double)ri[d][k], (double)ri[d][k], v[K + k]);
         v[2 * K + k] = fma((double)ri[d][k], (double)zi[d][k], v[2 * K + k]);
@@ -1789,10 +1692,18 @@ __device__ void res_slab(const EngPtrs &P, int slab, int slot, const RveDev *R, 
     }
 
     scatter_node<TS, K>((TS *)P.z, nb, RS, zi);
-    scatter_node<TS, K>((TS *)P.d, nb, RS, zero);
-    scatter_node<TS, K>((TS *)P.p, nb, RS, zero);
-    scatter_node<TS, K>((TS *)P.q, nb, RS, zero);
+    if (R->scw == 0) {  // a resident sweep starts d, p and q itself
+      TS zero[3][K];
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int k = 0; k < K; k++) zero[d][k] = (TS)0;
+      scatter_node<TS, K>((TS *)P.d, nb, RS, zero);
+      scatter_node<TS, K>((TS *)P.p, nb, RS, zero);
+      scatter_node<TS, K>((TS *)P.q, nb, RS, zero);
+    }
   }
+  if (R->scw > 1) sweep_words_zero<TS, K>(P, R, slab);
   block_sum<4 * K>(v, lds);
   if (tid == 0) {
     const SlabPart part = slab_part(P, slab);
@@ -2018,13 +1929,17 @@ static int launch_steps(const EngPtrs &P, const SolveParams &sp, int grid, int f
   for (int i = first; i < first + nkern; i++) {
     switch (i % 3) {
       case 0:
-        // with the march on (a_lds > 0), its tiles and, if any RVE is
-        // processed slab by slab (a_slab), k_step_a for those
+        // the resident RVEs' sweeps (u_grid > 0), the march's tiles (a_lds >
+        // 0) and, if any RVE is processed slab by slab (a_slab), k_step_a
+        if (P.u_grid > 0) {
+          const int rc = eng_launch_sweep(sizeof(TS) == 8, K, P, sp, s);
+          if (rc) return rc;
+        }
         if (P.a_lds > 0 && P.a_grid > 0) {
           if (DICT) k_step_a_march_dict<TS, K><<<P.a_grid, P.SN, P.a_lds, s>>>(P, sp);
           else k_step_a_march_full<TS, K><<<P.a_grid, P.SN, P.a_lds, s>>>(P, sp);
         }
-        if (P.a_lds == 0 || P.a_slab) k_step_a<TS, K, DICT><<<grid, P.SN, 0, s>>>(P, sp);
+        if (P.a_slab) k_step_a<TS, K, DICT><<<grid, P.SN, 0, s>>>(P, sp);
         if (P.s_big) k_step_s<TS, K><<<grid < kRGrid ? grid : kRGrid, P.SN, 0, s>>>(P);
         break;
       case 1: k_step_b<TS, K><<<grid, P.SN, 0, s>>>(P, sp); break;

@@ -1,0 +1,667 @@
+// engine_sweep.hip -- a whole PCG sweep of an RVE load case on chip.
+//
+// One workgroup, or a cluster of scw workgroups that split the RVE's interior
+// z-planes, runs every PCG iteration of one sweep of one load case in a single
+// launch: z in LDS (its own planes and one halo plane either side), p, q and d
+// in registers, the dictionary blocks in LDS.  See RveDev::scw for which RVEs.
+//
+// Why: kernels A and B move eleven vector passes per iteration through HBM and
+// are two to four launches; here an iteration moves only the planes between
+// ranks and the partial sums.  What bounds it: vector issue (the 243 multiply-
+// adds of a node's rows, 61% of all vector instructions; 80% of the issue slots
+// of a full SIMD while w = A z runs) and, for clusters, two exchanges of 2.5 us.
+// One 30^3 load case (4 ranks of 8 planes, FP32) takes 27.8 us per iteration
+// alone and 30.7 with 64 of them on the GPU; kernels A, B and R took 640 us for
+// 768 of them, 53 per 64.  Measured on the way there, same case:
+//   z neighbours read from LDS, one per key: 38 us; x-neighbours through DPP: 31
+//   (LDS reads per node 81 -> 27 dwords);
+//   1,024 lanes at 128 VGPRs, items of 4 planes: 32 us (spills, dictionary reads
+//   shared by half as many nodes);
+//   two workgroups per CU, items of 3 planes: 67 us per 60 load cases (bound by
+//   the dictionary's LDS reads);
+//   waiting for r.r / r.z before w = A z instead of behind it: 31 us.
+// Whole solves (rtol 1e-10): 128 x 30^3 tangents 187 -> 75 ms, 64 uneven cells
+// 8^3 .. 32^3 50 -> 14 ms, 24 x 20^3 in FP64 25.5 -> 7.1 ms, one 10^3 4.7 -> 1.2.
+#include <hip/hip_runtime.h>
+
+#include "engine_device.h"
+#include "mm_device.h"
+#include "mm_internal.h"
+
+namespace mm {
+
+namespace {
+
+typedef unsigned long long u64;
+
+// The tile of one workgroup: rank rk of the RVE's scw owns the interior planes
+// zs .. ze-1.  LDS plane s holds plane zs - 1 + s; inside a plane interior node
+// (ix, iy) (both counted from 0) sits at pos = 1 + (iy + 1) (nix + 1) + ix, so
+// that a zero column between the rows and a zero row before and after them
+// stand for the boundary nodes, whose z is zero in every correction solve.
+struct SweepGeo {
+  int nix, ncol, rsx, pw;  // interior columns per row, per plane; row and plane strides
+  int npos, nstrip;        // positions of a plane's rows with their zero column; strips of them
+  int zs, ze, np, rk, cw;
+  int lp, nch;             // planes per item; items per column
+  int nx, nxy, fs;
+};
+
+// The RVE's fields are the same in every lane but read through vector memory;
+// readfirstlane keeps them, and every address formed from them, scalar.
+__device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+__device__ __forceinline__ SweepGeo sweep_geo(const RveDev *R, int rk)
+{
+  SweepGeo g;
+  g.nx = scalar(R->nx);
+  const int ny = scalar(R->ny), niz = scalar(R->nz) - 2;
+  g.nix = g.nx - 2;
+  g.ncol = g.nix * (ny - 2);
+  g.rsx = g.nix + 1;
+  g.pw = sweep_plane(g.nx, ny);
+  g.npos = g.rsx * (ny - 2);
+  g.nstrip = sweep_strips(g.nx, ny);
+  g.rk = rk;
+  g.cw = scalar(R->scw);
+  g.zs = 1 + rk * niz / g.cw;
+  g.ze = 1 + (rk + 1) * niz / g.cw;
+  g.np = g.ze - g.zs;
+  g.lp = scalar(R->slp);
+  g.nch = scalar(R->snch);
+  g.nxy = g.nx * ny;
+  g.fs = scalar(R->first_slab);
+  return g;
+}
+
+// Three consecutive values: one 96-bit LDS read in FP32.
+typedef float lds_f3 __attribute__((ext_vector_type(3), aligned(4)));
+__device__ __forceinline__ void lds_read3(const float *p, float (&v)[3])
+{
+  const lds_f3 t = *(const __attribute__((address_space(3))) lds_f3 *)p;
+  v[0] = t.x;
+  v[1] = t.y;
+  v[2] = t.z;
+}
+__device__ __forceinline__ void lds_read3(const double *p, double (&v)[3])
+{
+#pragma unroll
+  for (int d = 0; d < 3; d++) v[d] = ((const __attribute__((address_space(3))) double *)p)[d];
+}
+
+// w[d] += a[e][d] * (x[e] of the lane before, DX = 0, or after, DX = 2), e = 0,
+// 1, 2 in turn: the shift rides on the multiply-add.  (x may come straight from
+// a vector instruction, which a DPP read must not follow within two cycles.)
+template <int DX>
+__device__ __forceinline__ void fma_lane_x(const float (&a)[3][3], const float (&x)[3], float (&w)[3])
+{
+#define MM_FMAC_DPP(SHIFT)                                                             \
+  asm("s_nop 1\n\t"                                                                    \
+      "v_fmac_f32_dpp %0, %3, %6 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %1, %3, %7 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %2, %3, %8 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %0, %4, %9 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %1, %4, %10 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %2, %4, %11 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %0, %5, %12 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %1, %5, %13 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %2, %5, %14 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1"     \
+      : "+v"(w[0]), "+v"(w[1]), "+v"(w[2])                                               \
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(a[0][0]), "v"(a[0][1]), "v"(a[0][2]), "v"(a[1][0]), "v"(a[1][1]), \
+        "v"(a[1][2]), "v"(a[2][0]), "v"(a[2][1]), "v"(a[2][2]))
+  if constexpr (DX == 0) MM_FMAC_DPP("wave_shr:1");
+  else MM_FMAC_DPP("wave_shl:1");
+#undef MM_FMAC_DPP
+}
+template <int DX>
+__device__ __forceinline__ void fma_lane_x(const double (&a)[3][3], const double (&x)[3], double (&w)[3])
+{
+  constexpr int shift = DX == 0 ? 0x138 : 0x130;  // wave_shr:1, wave_shl:1
+#pragma unroll
+  for (int e = 0; e < 3; e++) {
+    const int2 b = __builtin_bit_cast(int2, x[e]);
+    const double xe = __builtin_bit_cast(double, make_int2(__builtin_amdgcn_update_dpp(0, b.x, shift, 0xf, 0xf, true),
+                                                           __builtin_amdgcn_update_dpp(0, b.y, shift, 0xf, 0xf, true)));
+#pragma unroll
+    for (int d = 0; d < 3; d++) w[d] = fma(a[e][d], xe, w[d]);
+  }
+}
+
+// w += block DX of the three x-neighbours (dictionary row Db) times z, for LP
+// nodes of the lane's column whose own z rows in that strip are x.
+template <typename TS, int LP, int DX>
+__device__ __forceinline__ void sweep_key(const TS *Db, const TS (&x)[LP][3], TS (&w)[LP][3])
+{
+  constexpr int blk = sweep_dict_block((int)sizeof(TS));
+  TS a[3][3];  // [d'][d]
+#pragma unroll
+  for (int e = 0; e < 3; e++) lds_read3(Db + DX * blk + e * (blk / 3), a[e]);
+#pragma unroll
+  for (int l = 0; l < LP; l++) {
+    if constexpr (DX != 1) {
+      fma_lane_x<DX>(a, x[l], w[l]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 3; e++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) w[l][d] = fma(a[e][d], x[l][e], w[l][d]);
+    }
+  }
+}
+
+// Words that the workgroups of a cluster pass to each other: 32 bits of
+// payload under the tag of the iteration that wrote them, one 64-bit relaxed
+// atomic access at agent scope each way.  A reader polls the word until it
+// carries the tag it waits for, so payload and readiness arrive together and
+// no fence (an L2 write-back or invalidate) is needed.  A word is rewritten
+// only after a sum over the cluster that its reader joined after reading it.
+__device__ __forceinline__ void put_word(u64 *p, unsigned tag, unsigned bits)
+{
+  __hip_atomic_store(p, ((u64)tag << 32) | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ u64 get_word(const u64 *p)
+{
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// Bound on a wait in polls (half a minute or more).  A rank waits for the
+// slowest of its cluster to run one phase, or, before its first exchange, for a
+// rank that has no CU yet: until a running sweep ends.  A wait that reaches the
+// bound ends the sweep without an update.
+constexpr int kSweepPolls = 1 << 25;
+
+struct SweepExch {
+  u64 *up, *down, *sum;  // top planes to the next rank, bottom planes to the previous, partial sums
+};
+
+// A double moved between lanes (0 where no lane supplies one).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_get(double v)
+{
+  const int2 b = __builtin_bit_cast(int2, v);
+  return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_update_dpp(0, b.x, CTRL, ROWS, 0xf, true),
+                                              __builtin_amdgcn_update_dpp(0, b.y, CTRL, ROWS, 0xf, true)));
+}
+
+// Sums NV values over the workgroup: valid in every lane, one barrier.  buf
+// (NV * 8 doubles) must not be rewritten before the next barrier.
+template <int NV>
+__device__ __forceinline__ void lanes_sum(double (&v)[NV], double *buf)
+{
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    v[i] += dpp_get<0x111, 0xf>(v[i]);  // row_shr:1, 2, 4, 8: lane 15 of each row has its sum
+    v[i] += dpp_get<0x112, 0xf>(v[i]);
+    v[i] += dpp_get<0x114, 0xf>(v[i]);
+    v[i] += dpp_get<0x118, 0xf>(v[i]);
+    v[i] += dpp_get<0x142, 0xa>(v[i]);  // row_bcast:15 into rows 1 and 3
+    v[i] += dpp_get<0x143, 0xc>(v[i]);  // row_bcast:31 into rows 2 and 3: lane 63 has the total
+  }
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (lane == 63)
+#pragma unroll
+    for (int i = 0; i < NV; i++) buf[i * (kSweepLanes / 64) + wid] = v[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    double s = 0.0;
+#pragma unroll
+    for (int w = 0; w < kSweepLanes / 64; w++) s += buf[i * (kSweepLanes / 64) + w];
+    v[i] = s;
+  }
+}
+
+// Sums NV values over the workgroups of a cluster: lane 0 posts the workgroup's
+// own, every wave then collects all of them and adds them in rank order, so
+// that every lane of every rank has the same bits.  Collecting returns false
+// when the wait ran out.
+template <int NV>
+__device__ __forceinline__ void cluster_post(const double (&v)[NV], u64 *sum, int rk, unsigned tag)
+{
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int i = 0; i < NV; i++) {
+      const u64 b = __builtin_bit_cast(u64, v[i]);
+      put_word(sum + rk * 8 + 2 * i, tag, (unsigned)b);
+      put_word(sum + rk * 8 + 2 * i + 1, tag, (unsigned)(b >> 32));
+    }
+}
+template <int NV>
+__device__ __forceinline__ bool cluster_collect(double (&v)[NV], const u64 *sum, int cw, unsigned tag)
+{
+  const int lane = threadIdx.x & 63;
+  const bool mine = lane < cw * 2 * NV;
+  const u64 *src = sum + (mine ? (lane / (2 * NV)) * 8 + lane % (2 * NV) : 0);
+  u64 w = 0;
+  int n = 0;
+  for (;;) {
+    if (mine) w = get_word(src);
+    if (__all(!mine || (unsigned)(w >> 32) == tag)) break;
+    if (++n > kSweepPolls) return false;
+  }
+  const unsigned bits = (unsigned)w;
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    double s = 0.0;
+    for (int r = 0; r < cw; r++) {
+      const unsigned lo = __builtin_amdgcn_readlane(bits, r * 2 * NV + 2 * i);
+      const unsigned hi = __builtin_amdgcn_readlane(bits, r * 2 * NV + 2 * i + 1);
+      s += __builtin_bit_cast(double, ((u64)hi << 32) | lo);
+    }
+    v[i] = s;
+  }
+  return true;
+}
+
+// Publishes a node's three rows as the words of position pos of a plane.
+__device__ __forceinline__ void put_node(u64 *dst, int npos, int pos, unsigned tag, const float (&x)[3])
+{
+#pragma unroll
+  for (int d = 0; d < 3; d++) put_word(dst + d * npos + pos, tag, __builtin_bit_cast(unsigned, x[d]));
+}
+__device__ __forceinline__ void put_node(u64 *dst, int npos, int pos, unsigned tag, const double (&x)[3])
+{
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    const u64 b = __builtin_bit_cast(u64, x[d]);
+    put_word(dst + (2 * d) * npos + pos, tag, (unsigned)b);
+    put_word(dst + (2 * d + 1) * npos + pos, tag, (unsigned)(b >> 32));
+  }
+}
+__device__ __forceinline__ void word_node(const u64 *w, float *dst)
+{
+#pragma unroll
+  for (int d = 0; d < 3; d++) dst[d] = __builtin_bit_cast(float, (unsigned)w[d]);
+}
+__device__ __forceinline__ void word_node(const u64 *w, double *dst)
+{
+#pragma unroll
+  for (int d = 0; d < 3; d++) dst[d] = __builtin_bit_cast(double, (w[2 * d + 1] << 32) | (w[2 * d] & 0xffffffffull));
+}
+
+// LDS planes 0 and np + 1 <- the words that the neighbouring ranks published
+// under `tag` (lo, hi: null at the tile's ends).  All words of a position are
+// asked for together, again until each carries the tag.
+template <typename TS>
+__device__ __forceinline__ bool get_planes(const SweepGeo &g, TS *zl, const u64 *lo, const u64 *hi, unsigned tag)
+{
+  constexpr int W = 3 * (int)(sizeof(TS) / 4);
+  bool ok = true;
+  for (int c = threadIdx.x; c < g.npos; c += kSweepLanes) {
+    if (c % g.rsx == g.nix) continue;  // the zero column
+    u64 a[W], b[W];
+    int n = 0;
+    for (;;) {
+      bool all = true;
+#pragma unroll
+      for (int i = 0; i < W; i++) {
+        a[i] = lo ? get_word(lo + i * g.npos + c) : (u64)tag << 32;
+        b[i] = hi ? get_word(hi + i * g.npos + c) : (u64)tag << 32;
+      }
+#pragma unroll
+      for (int i = 0; i < W; i++) all = all && (unsigned)(a[i] >> 32) == tag && (unsigned)(b[i] >> 32) == tag;
+      if (all) break;
+      if (++n > kSweepPolls) {
+        ok = false;
+        break;
+      }
+    }
+    if (lo) word_node(a, zl + (c + g.rsx + 1) * 3);
+    if (hi) word_node(b, zl + ((g.np + 1) * g.pw + c + g.rsx + 1) * 3);
+  }
+  return ok;
+}
+
+// Item j of lane tid: the LDS position of its column in the plane below its
+// first node, that node, the planes of the wave's strip (0: none), and whether
+// the lane has a node there (if not it only supplies z to its neighbours).  Strip st of the tile is nstrip
+// strips per run of planes; lanes 1 .. 62 of its wave work.
+struct SweepItem {
+  int lds, node, cnt, h;
+  bool on;
+};
+__device__ __forceinline__ SweepItem sweep_item(const SweepGeo &g, int tid, int j)
+{
+  const int st = scalar((tid >> 6) + j * (kSweepLanes / 64)), ln = tid & 63;
+  const int h = st / g.nstrip, pos = (st - h * g.nstrip) * kSweepStrip + ln - 1;
+  const int iy = pos < 0 ? 0 : pos / g.rsx, ix = pos < 0 ? g.nix : pos - iy * g.rsx;
+  const int zf = g.zs + h * g.lp;
+  SweepItem it;
+  it.cnt = h < g.nch ? max(min(g.lp, g.ze - zf), 0) : 0;
+  it.on = it.cnt > 0 && ix < g.nix && pos < g.npos && ln >= 1 && ln <= kSweepStrip;
+  it.h = h;
+  it.lds = (h < g.nch ? h * g.lp : 0) * g.pw + min(pos, g.npos - 1) + g.rsx + 1;
+  it.node = it.on ? (ix + 1) + (iy + 1) * g.nx + zf * g.nxy : 1 + g.nx + g.nxy;  // any interior one if off
+  return it;
+}
+
+// Position of an item's column from its LDS offset.
+__device__ __forceinline__ int item_pos(const SweepGeo &g, int z0, int h)
+{
+  return z0 / 3 - h * g.lp * g.pw - g.rsx - 1;
+}
+
+// The sweep of one load case on this workgroup's tile; zl holds z = dinv r of
+// the sweep's right-hand side.  An item is one interior column times lp planes,
+// LP >= lp of its nodes' rows in registers, one lane each; a wave takes strips
+// of kSweepStrip consecutive positions, so that the x-neighbours of a node are
+// the lanes beside it and come from them (DPP) instead of LDS.  The arithmetic of a node is kernel A's and kernel B's (the
+// row product in neighbour-key order, r = z / dinv formed for the dots); only
+// the grouping of the dot products differs.  Returns the iterations taken.
+template <typename TS, int LP>
+__device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, int K, int k, TS *zl,
+                                          const TS *dict, double *red, int *s_fail, const SweepExch &X, double rz,
+                                          double tgt, int max_its)
+{
+  constexpr int NI = kSweepItems;
+  const int tid = threadIdx.x, fs = g.fs, SN = P.SN, RS = 3 * SN;
+  TS p[NI][LP][3], q[NI][LP][3], dd[NI][LP][3];
+  int z0[NI], d0[NI], cnt[NI], hc[NI];
+  bool on[NI];
+#pragma unroll
+  for (int j = 0; j < NI; j++) {
+    const SweepItem it = sweep_item(g, tid, j);
+    cnt[j] = scalar(it.cnt);
+    hc[j] = scalar(it.h);
+    on[j] = it.on;
+    z0[j] = it.lds * 3;
+    // the phases do not vary along z: one pattern per column; lanes without a
+    // node take the zero entry, so that their q, r and dot products are zero
+    const int pat = P.npat[(long long)(fs + (it.node >> P.sn_shift)) * SN + (it.node & (SN - 1))] & 15;
+    d0[j] = (it.on ? pat : 16) * sweep_dict_stride((int)sizeof(TS));
+#pragma unroll
+    for (int l = 0; l < LP; l++)
+#pragma unroll
+      for (int d = 0; d < 3; d++) p[j][l][d] = q[j][l][d] = dd[j][l][d] = (TS)0;
+  }
+  const int ps0 = g.pw * 3, words = sweep_words(g.npos, (int)sizeof(TS));
+  const u64 *lo = g.rk > 0 ? X.up + (long long)(g.rk - 1) * words : nullptr;
+  const u64 *hi = g.rk + 1 < g.cw ? X.down + (long long)g.rk * words : nullptr;
+  double v2[2] = {0.0, 0.0};
+  int n = 0;
+#pragma unroll 1
+  for (;;) {
+    double v1[1] = {0.0}, beta = 0.0;
+    TS b;
+    bool done = false;
+    // opaque per iteration: the addresses that follow from these are formed
+    // where they are used and not kept in registers
+    int ps = ps0;
+    asm volatile("" : "+s"(ps));
+#pragma unroll
+    for (int j = 0; j < NI; j++) asm volatile("" : "+v"(z0[j]));
+#pragma unroll
+    for (int j = 0; j < NI; j++) {
+      if (j > 0 && cnt[j] == 0) continue;
+      TS w[LP][3];
+#pragma unroll
+      for (int l = 0; l < LP; l++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) w[l][d] = (TS)0;
+#pragma unroll 1
+      for (int dz = 0; dz < 3; dz++)
+#pragma unroll 1
+        for (int dy = 0; dy < 3; dy++) {
+          const TS *zr = zl + z0[j] + dz * ps + (dy - 1) * g.rsx * 3;
+          const TS *Db = dict + d0[j] + (3 * dy + 9 * dz) * sweep_dict_block((int)sizeof(TS));
+          TS x[LP][3];
+#pragma unroll
+          for (int l = 0; l < LP; l++) lds_read3(zr + l * ps, x[l]);
+          sweep_key<TS, LP, 0>(Db, x, w);
+          sweep_key<TS, LP, 1>(Db, x, w);
+          sweep_key<TS, LP, 2>(Db, x, w);
+        }
+      if (j == 0) {
+        // w = A z needs neither r.r nor r.z of the last update: their sums over
+        // the cluster, posted before it, have arrived by now
+        if (n > 0) {
+          if (g.cw > 1 && !cluster_collect<2>(v2, X.sum + kSweepMaxRanks * 8, g.cw, (unsigned)n)) *s_fail = 1;
+          done = scalar(sqrt(v2[0]) <= tgt || rz == 0.0 || n >= max_its) != 0;
+          if (done) break;
+          beta = v2[1] / rz;
+          rz = v2[1];
+        }
+        b = (TS)beta;
+      }
+      TS x[LP][3];
+#pragma unroll
+      for (int l = 0; l < LP; l++) lds_read3(zl + z0[j] + (l + 1) * ps, x[l]);
+#pragma unroll
+      for (int l = 0; l < LP; l++) {
+        if (l >= cnt[j]) break;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          p[j][l][d] = fma(b, p[j][l][d], x[l][d]);
+          q[j][l][d] = fma(b, q[j][l][d], w[l][d]);
+          v1[0] = fma((double)p[j][l][d], (double)q[j][l][d], v1[0]);
+        }
+      }
+    }
+    if (done) break;
+    const unsigned tag = (unsigned)n + 1u;
+    lanes_sum<1>(v1, red);
+    if (g.cw > 1) {
+      cluster_post<1>(v1, X.sum, g.rk, tag);
+      if (!cluster_collect<1>(v1, X.sum, g.cw, tag)) *s_fail = 1;
+    }
+    const TS al = (TS)((v1[0] == 0.0) ? 0.0 : rz / v1[0]);
+    v2[0] = v2[1] = 0.0;
+#pragma unroll
+    for (int j = 0; j < NI; j++) {
+      if (j > 0 && cnt[j] == 0) continue;
+      TS dg[3], yg[3];  // the column's dinv and its reciprocal, after its blocks
+      lds_read3(dict + d0[j] + 27 * sweep_dict_block((int)sizeof(TS)), dg);
+      lds_read3(dict + d0[j] + 27 * sweep_dict_block((int)sizeof(TS)) + sweep_dict_block((int)sizeof(TS)) / 3, yg);
+      TS x[LP][3];
+#pragma unroll
+      for (int l = 0; l < LP; l++) lds_read3(zl + z0[j] + (l + 1) * ps, x[l]);
+#pragma unroll
+      for (int l = 0; l < LP; l++) {
+        if (l >= cnt[j]) break;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          dd[j][l][d] = fma(al, p[j][l][d], dd[j][l][d]);
+          const TS zi = fma(-al, dg[d] * q[j][l][d], x[l][d]);
+          x[l][d] = zi;
+          // r = z / dinv: the quotient from the reciprocal and its exact
+          // remainder, correctly rounded (Markstein)
+          TS r = zi * yg[d];
+          r = fma(fma(-r, dg[d], zi), yg[d], r);
+          v2[0] = fma((double)r, (double)r, v2[0]);
+          v2[1] = fma((double)r, (double)zi, v2[1]);
+        }
+        if (on[j]) {
+#pragma unroll
+          for (int d = 0; d < 3; d++) zl[z0[j] + (l + 1) * ps + d] = x[l][d];
+          if (l == 0 && lo && hc[j] == 0)
+            put_node(X.down + (long long)(g.rk - 1) * words, g.npos, item_pos(g, z0[j], hc[j]), tag, x[l]);
+          if (hi && l == cnt[j] - 1 && hc[j] == g.nch - 1)
+            put_node(X.up + (long long)g.rk * words, g.npos, item_pos(g, z0[j], hc[j]), tag, x[l]);
+        }
+      }
+    }
+    lanes_sum<2>(v2, red + kSweepLanes / 64);  // its barrier also ends the writes of z
+    n++;
+    if (g.cw > 1) {
+      cluster_post<2>(v2, X.sum + kSweepMaxRanks * 8, g.rk, tag);
+      if (!get_planes<TS>(g, zl, lo, hi, tag)) *s_fail = 1;
+      __syncthreads();
+      if (scalar(*s_fail)) return n;  // a wait ran out: no update; the residual shows it
+    }
+  }
+  if (g.cw > 1) {
+    __syncthreads();
+    if (scalar(*s_fail)) return n;
+  }
+  int t2 = tid;
+  asm volatile("" : "+v"(t2));  // the items' nodes are formed again, not kept
+#pragma unroll
+  for (int j = 0; j < NI; j++) {
+    const SweepItem it = sweep_item(g, t2, j);
+#pragma unroll
+    for (int l = 0; l < LP; l++)
+      if (it.on && l < it.cnt) {
+        const int m = it.node + l * g.nxy;
+        double *xo = P.x64 + ((long long)(fs + (m >> P.sn_shift)) * K + k) * RS + 3 * (m & (SN - 1));
+#pragma unroll
+        for (int d = 0; d < 3; d++) xo[d] += (double)dd[j][l][d];
+      }
+  }
+  return n;
+}
+
+// sweep_case for the tile's item length.
+template <typename TS>
+struct SweepRun {
+  const EngPtrs &P;
+  const SweepGeo &g;
+  int K, k;
+  TS *zl;
+  const TS *dict;
+  double *red;
+  int *fail;
+  const SweepExch &X;
+  double rz, tgt;
+  int max_its;
+  template <int LP>
+  __device__ __forceinline__ int go() const
+  {
+    if constexpr (LP > 2)
+      if (g.lp <= LP - 2) return go<LP - 2>();
+    return sweep_case<TS, LP>(P, g, K, k, zl, dict, red, fail, X, rz, tgt, max_its);
+  }
+};
+
+extern __shared__ __attribute__((aligned(16))) double sweep_dyn[];
+
+}  // namespace
+
+// The resident RVEs' kernel A (reads st[2], writes st[0]).  Workgroups take the
+// entries of the unit list (RVE slot, load case * 16 + rank) by ticket, in list
+// order: the ranks of a cluster are consecutive entries, so the started
+// workgroups form whole clusters but for the last one, the whole ones finish
+// without waiting for anyone else, and their places go to the missing ranks
+// (also beside other such launches: each leaves at most one cluster of at most
+// 16 workgroups waiting, and the GPU has more places than the queues' launches
+// can fill with those).
+// A sweep's end (its iteration count is the largest of the load cases') is
+// entered into the state by kernel B.
+template <typename TS, int K>
+__global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp)
+{
+  __shared__ double lds[64];
+  __shared__ double red[3 * (kSweepLanes / 64)];
+  __shared__ double tot[4 * K];
+  __shared__ SolveState N;
+  __shared__ int s_unit, s_fail;
+  const int tid = threadIdx.x;
+  if (tid == 0) {
+    s_unit = (int)__hip_atomic_fetch_add(P.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_fail = 0;
+  }
+  __syncthreads();
+  const int u = scalar(s_unit);
+  if (u >= P.units[0].x) return;
+  const int slot = scalar(P.units[1 + u].x);
+  const int case_rank = scalar(P.units[1 + u].y);
+  const int k = case_rank / kSweepMaxRanks, rk = case_rank % kSweepMaxRanks;
+  RveDev *R = P.rves + slot;
+  const int phase0 = R->st[2].phase;
+  const bool writer = k == 0 && rk == 0;
+  if (phase0 == PH_AVGRED) {
+    if (!writer) return;
+    if (tid == 0) N = R->st[2];
+    __syncthreads();
+    finish_rve<K>(P, slot, R, N, sp, lds);
+    if (tid == 0) R->st[0] = N;
+    return;
+  }
+  if (tid == 0) N = R->st[2];
+  if (phase0 == PH_RESRED) {
+    group_sum_cols_lds<4 * K>(slab_part(P, R->first_slab).p, R->nslab, P.part_stride, 3 * K, tot, lds);
+    if (tid == 0) start_sweep<K>(N, *reinterpret_cast<const double(*)[4 * K]>(tot), R, sp);
+  }
+  __syncthreads();
+  if (writer && tid == 0) R->st[0] = N;
+  if (N.phase != PH_INNER || ((N.done_in >> k) & 1u)) return;
+
+  const SweepGeo g = sweep_geo(R, rk);
+  const int SN = P.SN, RS = 3 * SN, fs = g.fs, tsz = (int)sizeof(TS);
+  TS *dict = reinterpret_cast<TS *>(sweep_dyn);
+  TS *zl = reinterpret_cast<TS *>(reinterpret_cast<unsigned char *>(sweep_dyn) + sweep_dict_bytes(tsz));
+  // the 16 blocks of patterns that repeat along z, rounded from the FP64
+  // dictionary (the values of the solver dictionary)
+  const double *D = P.dict64 + (size_t)slot * kDictPat * kDictEntry;
+  for (int i = tid; i < sweep_dict_stride(tsz); i += kSweepLanes) dict[16 * sweep_dict_stride(tsz) + i] = (TS)0;
+  for (int i = tid; i < 16 * 27 * 9; i += kSweepLanes) {
+    const int e = i / (27 * 9), o = i - e * (27 * 9), key = o / 9, j = o - key * 9;
+    dict[e * sweep_dict_stride(tsz) + key * sweep_dict_block(tsz) + (j / 3) * (sweep_dict_block(tsz) / 3) + j % 3] =
+        (TS)D[(size_t)(e * 17) * kDictEntry + key * kDictBlk + (j / 3) * 4 + j % 3];
+  }
+  for (int i = tid; i < 16 * 3; i += kSweepLanes) {
+    const int e = i / 3, d = i - e * 3;
+    // the solver's dinv of a node of that pattern, and its reciprocal
+    const TS dg = (TS)(1.0 / D[(size_t)(e * 17) * kDictEntry + 13 * kDictBlk + d * 4 + d]);
+    TS *o = dict + e * sweep_dict_stride(tsz) + 27 * sweep_dict_block(tsz) + d;
+    o[0] = dg;
+    o[sweep_dict_block(tsz) / 3] = (TS)1 / dg;
+  }
+  const int zlen = sweep_lds_planes(g.lp, g.nch) * g.pw * 3;
+  for (int i = tid; i < zlen; i += kSweepLanes) zl[i] = (TS)0;
+  __syncthreads();
+  for (int s = 0; s < g.np + 2; s++) {
+    const int z = g.zs - 1 + s;
+    if (z == 0 || z == R->nz - 1) continue;
+    for (int c = tid; c < g.ncol; c += kSweepLanes) {
+      const int iy = c / g.nix, m = (c - iy * g.nix + 1) + (iy + 1) * g.nx + z * g.nxy;
+      const TS *src = (const TS *)P.z + ((long long)(fs + (m >> P.sn_shift)) * K + k) * RS + 3 * (m & (SN - 1));
+      TS *dst = zl + (s * g.pw + 1 + (iy + 1) * g.rsx + c - iy * g.nix) * 3;
+#pragma unroll
+      for (int d = 0; d < 3; d++) dst[d] = src[d];
+    }
+  }
+  __syncthreads();
+  SweepExch X;
+  const long long b0 = sweep_region(scalar(R->nslab), SN, K, tsz, fs, k);
+  X.up = reinterpret_cast<u64 *>((char *)P.p + b0);
+  X.down = reinterpret_cast<u64 *>((char *)P.q + b0);
+  X.sum = reinterpret_cast<u64 *>((char *)P.d + b0);
+  const double rz = N.rz[k], tgt = N.bnorm_in[k];
+  int n;
+  const SweepRun<TS> run{P, g, K, k, zl, dict, red, &s_fail, X, rz, tgt, sp.max_inner_its};
+  n = run.template go<sweep_max_planes((int)sizeof(TS))>();
+  if (rk == 0 && tid == 0) R->lits[k] = n;
+}
+
+template <typename TS, int K>
+static int launch_sweep(const EngPtrs &P, const SolveParams &sp, hipStream_t s)
+{
+  if (P.u_grid <= 0 || P.u_lds <= 0 || P.u_lds > kSweepMaxLds) return MM_ERR_ARG;
+  k_sweep<TS, K><<<P.u_grid, kSweepLanes, P.u_lds, s>>>(P, sp);
+  MM_HIP(hipGetLastError());
+  return 0;
+}
+
+#define MM_SWEEP_DISPATCH(FP64, K, F, ...)       \
+  do {                                           \
+    if (FP64) {                                  \
+      switch (K) {                               \
+        case 1: return F<double, 1>(__VA_ARGS__); \
+        case 6: return F<double, 6>(__VA_ARGS__); \
+        case 7: return F<double, 7>(__VA_ARGS__); \
+        default: return MM_ERR_ARG;              \
+      }                                          \
+    }                                            \
+    switch (K) {                                 \
+      case 1: return F<float, 1>(__VA_ARGS__);   \
+      case 6: return F<float, 6>(__VA_ARGS__);   \
+      case 7: return F<float, 7>(__VA_ARGS__);   \
+      default: return MM_ERR_ARG;                \
+    }                                            \
+  } while (0)
+
+int eng_launch_sweep(bool fp64, int K, const EngPtrs &P, const SolveParams &sp, hipStream_t s)
+{
+  MM_SWEEP_DISPATCH(fp64, K, launch_sweep, P, sp, s);
+}
+
+}  // namespace mm

@@ -124,6 +124,12 @@ struct RveDev {
   // workgroup of the consuming kernel would use), and kernels A and B read
   // the totals instead of each workgroup re-summing nslab partials.
   int big;
+  // resident sweep (engine_sweep.hip): scw > 0 workgroups per load case hold
+  // the PCG state of a whole sweep on chip, each slp * snch or fewer of the
+  // interior z-planes in items of slp planes of one column; lits[k] is the
+  // iteration count of load case k in the sweep.  scw == 0: kernels A and B.
+  int scw, slp, snch;
+  int lits[MM_MAX_RHS];
   double rr_rz[2 * MM_MAX_RHS];
   double pq[MM_MAX_RHS];
   double fx[MM_MAX_FIBERS], fy[MM_MAX_FIBERS], fr[MM_MAX_FIBERS];
@@ -177,6 +183,9 @@ struct EngPtrs {
   int a_lds;     // dynamic LDS bytes of the plane march; 0: march off
   int a_slab;    // march on: some RVEs (mcpp == 0) need k_step_a as well
   int s_big;     // the group holds an RVE with big != 0: kernel S runs after A
+  const int2 *units;  // [0].x: resident-sweep workgroups, [1..]: (slot, load case * 16 + rank)
+  unsigned *ticket;   // next unit to take; kernel B zeroes it (resident RVEs' first slabs)
+  int u_grid, u_lds;  // launch of the resident sweep (0: none in the group)
 };
 
 
@@ -218,6 +227,53 @@ inline int march_lds_bytes(int SN, int nx, int ny, int K, int tsz, bool dict)
 }
 constexpr int kMarchMaxLds = 64 * 1024;
 
+// ---------------------------------------------------------------------------
+// Resident sweep (engine_sweep.hip): sizes shared by the host's tiling and the
+// kernel.
+constexpr int kSweepLanes = 512;  // two waves per SIMD, 256 VGPRs each
+constexpr int kSweepItems = 2;    // items (a column times slp planes) per lane
+constexpr int kSweepMaxRanks = 16;
+constexpr int kSweepMaxLds = 160 * 1024 - 2816;  // dynamic; the static part is below 2.75 KB
+__host__ __device__ constexpr int sweep_max_planes(int tsz) { return tsz == 8 ? 4 : 8; }
+// The unrolled item lengths: a sweep of lp planes per item runs the next one.
+__host__ __device__ constexpr int sweep_unroll(int lp)
+{
+  return lp <= 2 ? 2 : (lp + 1) / 2 * 2;
+}
+// Positions per wave: lanes 0 and 63 supply the x-neighbours of lanes 1 and 62.
+constexpr int kSweepStrip = 62;
+__host__ __device__ constexpr int sweep_positions(int nx, int ny) { return (nx - 1) * (ny - 2); }
+__host__ __device__ constexpr int sweep_strips(int nx, int ny)
+{
+  return (sweep_positions(nx, ny) + kSweepStrip - 1) / kSweepStrip;
+}
+// LDS planes of a tile: every plane that the unrolled items read.
+__host__ __device__ constexpr int sweep_lds_planes(int lp, int nch)
+{
+  return (nch - 1) * lp + sweep_unroll(lp) + 2;
+}
+// Values per LDS plane: interior nodes, a zero column between rows, a zero row
+// before and after them and one value in front.
+__host__ __device__ constexpr int sweep_plane(int nx, int ny) { return 1 + ny * (nx - 1); }
+// LDS dictionary: the 16 patterns that are the same in both z-layers of
+// elements (the phases do not vary along z), each its 27 blocks, then dinv and
+// 1 / dinv of such a node, and an entry of zeros.  FP32 rows of 3 padded to 16 bytes (one 96-bit read
+// each); the entries' strides spread them over the banks.
+__host__ __device__ constexpr int sweep_dict_block(int tsz) { return tsz == 8 ? 9 : 12; }
+__host__ __device__ constexpr int sweep_dict_stride(int tsz) { return tsz == 8 ? 250 : 332; }
+__host__ __device__ constexpr int sweep_dict_bytes(int tsz) { return 17 * sweep_dict_stride(tsz) * tsz; }
+// The words a cluster exchanges live in the RVE's runs of p (top planes), q
+// (bottom planes) and d (partial sums), which a resident sweep does not use
+// otherwise: load case k has the k-th part of the run.  Kernel R zeroes them
+// before each sweep.
+__host__ __device__ inline long long sweep_region(int nslab, int SN, int K, int tsz, int first_slab, int k)
+{
+  return ((long long)first_slab * K + (long long)k * nslab) * 3 * SN * tsz;  // first byte
+}
+// 64-bit words of one plane: 32 bits of the three rows of every position.
+__host__ __device__ constexpr int sweep_words(int npos, int tsz) { return 3 * npos * (tsz / 4); }
+constexpr int kSweepSumWords = 2 * kSweepMaxRanks * 8;  // two sums, 64 bytes per rank
+
 // assembly modes
 enum AsmMode : int { ASM_FULL = 0, ASM_X_ONLY = 1, ASM_DICT = 2 };
 
@@ -227,6 +283,8 @@ bool eng_supported_rhs(int K);
 // nkern solver launches of the cycle A (0) -> B (1) -> R (2), from `first`
 int eng_launch_steps(bool fp64, int K, bool dict, const EngPtrs &P, const SolveParams &sp, int grid,
                      int first, int nkern, hipStream_t s);
+// the resident sweep of the RVEs in P.units
+int eng_launch_sweep(bool fp64, int K, const EngPtrs &P, const SolveParams &sp, hipStream_t s);
 int eng_launch_dict(bool fp64, int n, const int *slots, const double *ke_tab, void *dict, hipStream_t s);
 int eng_launch_assemble(bool fp64, int K, const EngPtrs &P, int nblk, const int *slab_list, int mode,
                         hipStream_t s);
