@@ -115,32 +115,34 @@ __global__ void k_admit(int n, const int *__restrict__ slots, const RveDev *__re
   }
 }
 
-// Element stiffness per (RVE, material), one wavefront each.  B at the 8
-// gauss points is built in LDS from the hex8 tables of src/fem.c:309-405
-// with dN/dx_d = ds * 2 / h_d; C is the isotropic tangent in the form of
-// src/material.c:16-22; Ke follows micro/src/assembly.c:97-107 term by term
-// (terms with an exactly zero factor are skipped, which leaves every sum
-// bit-identical).  Also stores C and sum_gp B w for the averaging phase.
+// Element stiffness per (RVE, material), one wavefront each.  The derivatives
+// at the 8 gauss points are built in LDS from the hex8 tables of
+// src/fem.c:309-405 with dN/dx_d = ds * 2 / h_d; C is the isotropic tangent in
+// the form of src/material.c:16-22; Ke follows micro/src/assembly.c:97-107 term
+// by term, lane 8 a + b the 3 x 3 block of nodes a and b (terms with an exactly
+// zero factor are skipped, which leaves every sum bit-identical).  Also stores C
+// and sum_gp B w for the averaging phase.  A chain of FP64 adds on one
+// wavefront: testing all 288 terms of nine entries per lane took 98 us whatever
+// the batch, this 26.
 __global__ __launch_bounds__(64) void k_ke(int n, const int *__restrict__ work,
                                            const RveDev *__restrict__ rves,
                                            double *__restrict__ ke_tab, double *__restrict__ c_tab_out,
                                            double *__restrict__ bw_tab)
 {
 #pragma clang fp contract(off)
-  __shared__ double B[6][24][8];
+  __shared__ double ds[8][8][3];  // [gauss point][node][axis]
   __shared__ double C[36];
-  __shared__ double wp[8];
   if ((int)blockIdx.x >= n) return;
   const int slot = work[2 * blockIdx.x], mat = work[2 * blockIdx.x + 1];
   const RveDev &R = rves[slot];
   const int tid = threadIdx.x;
   const double h[3] = {R.hx, R.hy, R.hz};
-  for (int i = tid; i < 6 * 24 * 8; i += 64) (&B[0][0][0])[i] = 0.0;
-  __syncthreads();
+  const double vol = h[0] * h[1] * h[2];
+  const double w = vol / 8;
   const double ga = 0.577350269189626;
-  // sign pattern of nodes / gauss points: 0(-,-,-) 1(+,-,-) 2(+,+,-) 3(-,+,-) 4..7 with z = +
-  for (int i = tid; i < 8 * 8; i += 64) {
-    const int a = i >> 3, g = i & 7;
+  {
+    // sign pattern of nodes / gauss points: 0(-,-,-) 1(+,-,-) 2(+,+,-) 3(-,+,-) 4..7 with z = +
+    const int a = tid >> 3, g = tid & 7;
     const double sa[3] = {(a == 1 || a == 2 || a == 5 || a == 6) ? 1.0 : -1.0,
                           (a == 2 || a == 3 || a == 6 || a == 7) ? 1.0 : -1.0, (a >= 4) ? 1.0 : -1.0};
     const double sg[3] = {(g == 1 || g == 2 || g == 5 || g == 6) ? 1.0 : -1.0,
@@ -150,16 +152,9 @@ __global__ __launch_bounds__(64) void k_ke(int n, const int *__restrict__ work,
     const double ds0 = sa[0] * f[1] * f[2] * 0.125;
     const double ds1 = sa[1] * f[0] * f[2] * 0.125;
     const double ds2 = sa[2] * f[0] * f[1] * 0.125;
-    const double dx = ds0 * 2 / h[0], dy = ds1 * 2 / h[1], dz = ds2 * 2 / h[2];
-    B[0][3 * a + 0][g] = dx;
-    B[1][3 * a + 1][g] = dy;
-    B[2][3 * a + 2][g] = dz;
-    B[3][3 * a + 0][g] = dy;
-    B[3][3 * a + 1][g] = dx;
-    B[4][3 * a + 1][g] = dz;
-    B[4][3 * a + 2][g] = dy;
-    B[5][3 * a + 0][g] = dz;
-    B[5][3 * a + 2][g] = dx;
+    ds[g][a][0] = ds0 * 2 / h[0];
+    ds[g][a][1] = ds1 * 2 / h[1];
+    ds[g][a][2] = ds2 * 2 / h[2];
   }
   if (tid < 36) {
     const int i = tid / 6, j = tid % 6;
@@ -169,32 +164,52 @@ __global__ __launch_bounds__(64) void k_ke(int n, const int *__restrict__ work,
     else if (i == j) base = (1 - 2 * nu) / 2;
     C[tid] = base * (E / ((1 + nu) * (1 - 2 * nu)));
   }
-  if (tid < 8) {
-    const double vol = h[0] * h[1] * h[2];
-    wp[tid] = vol / 8;
-  }
   __syncthreads();
-  double *ke = ke_tab + ((size_t)slot * kNmat + mat) * kKe;
-  for (int e = tid; e < kKe; e += 64) {
-    const int i = e / 24, j = e % 24;
-    double acc = 0.0;
-    for (int g = 0; g < 8; g++)
-      for (int k = 0; k < 6; k++)
-        for (int hh = 0; hh < 6; hh++) {
-          const double bh = B[hh][i][g];
-          const double c = C[hh * 6 + k];
-          const double bk = B[k][j][g];
-          if (bh == 0.0 || c == 0.0 || bk == 0.0) continue;
-          acc = acc + bh * c * bk * wp[g];
-        }
-    ke[e] = acc;
+  // rows of B with a value in column d of a node, and the derivative there
+  constexpr int row[3][3] = {{0, 3, 5}, {1, 3, 4}, {2, 4, 5}}, der[3][3] = {{0, 1, 2}, {1, 0, 2}, {2, 1, 0}};
+  const int a = tid >> 3, b = tid & 7;
+  double acc[3][3];
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+#pragma unroll
+    for (int dd = 0; dd < 3; dd++) acc[d][dd] = 0.0;
+#pragma unroll 1
+  for (int g = 0; g < 8; g++) {
+    double ba[3], bb[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      ba[d] = ds[g][a][d];
+      bb[d] = ds[g][b][d];
+    }
+#pragma unroll
+    for (int dd = 0; dd < 3; dd++)
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int ik = 0; ik < 3; ik++)
+#pragma unroll
+          for (int ih = 0; ih < 3; ih++) {
+            const double c = C[row[d][ih] * 6 + row[dd][ik]];
+            if (__builtin_amdgcn_readfirstlane(c == 0.0)) continue;  // the same in every lane
+            const double bh = ba[der[d][ih]], bk = bb[der[dd][ik]];
+            const double t = acc[d][dd] + bh * c * bk * w;
+            acc[d][dd] = (bh == 0.0 || bk == 0.0) ? acc[d][dd] : t;
+          }
   }
+  double *ke = ke_tab + ((size_t)slot * kNmat + mat) * kKe + 3 * a * kNd + 3 * b;
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+#pragma unroll
+    for (int dd = 0; dd < 3; dd++) ke[d * kNd + dd] = acc[d][dd];
   if (tid < 36) c_tab_out[((size_t)slot * kNmat + mat) * 36 + tid] = C[tid];
   if (mat == 0)
     for (int e = tid; e < 6 * 24; e += 64) {
-      const int v = e / 24, i = e % 24;
+      const int v = e / 24, i = e % 24, node = i / 3, d = i % 3;
+      int k = -1;  // the derivative at B[v][i], if any
+      for (int t = 0; t < 3; t++)
+        if (row[d][t] == v) k = der[d][t];
       double s = 0.0;
-      for (int g = 0; g < 8; g++) s += B[v][i][g] * wp[g];
+      for (int g = 0; g < 8; g++) s += (k < 0 ? 0.0 : ds[g][node][k]) * w;
       bw_tab[(size_t)slot * 144 + e] = s;
     }
 }

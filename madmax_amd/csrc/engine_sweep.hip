@@ -149,6 +149,19 @@ __device__ __forceinline__ void sweep_key(const TS *Db, const TS (&x)[LP][3], TS
   }
 }
 
+// w += the three blocks of strip (dz, dy), whose rows start at zr.
+template <typename TS, int LP>
+__device__ __forceinline__ void sweep_strip(const TS *zr, int ps, const TS *dict, int dz, int dy, TS (&w)[LP][3])
+{
+  const TS *Db = dict + (3 * dy + 9 * dz) * sweep_dict_block((int)sizeof(TS));
+  TS x[LP][3];
+#pragma unroll
+  for (int l = 0; l < LP; l++) lds_read3(zr + l * ps, x[l]);
+  sweep_key<TS, LP, 0>(Db, x, w);
+  sweep_key<TS, LP, 1>(Db, x, w);
+  sweep_key<TS, LP, 2>(Db, x, w);
+}
+
 // Words that the workgroups of a cluster pass to each other: 32 bits of
 // payload under the tag of the iteration that wrote them, one 64-bit relaxed
 // atomic access at agent scope each way.  A reader polls the word until it
@@ -397,19 +410,11 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
       for (int l = 0; l < LP; l++)
 #pragma unroll
         for (int d = 0; d < 3; d++) w[l][d] = (TS)0;
+      const TS *zr = zl + z0[j] - g.rsx * 3, *Db = dict + d0[j];
 #pragma unroll 1
       for (int dz = 0; dz < 3; dz++)
 #pragma unroll 1
-        for (int dy = 0; dy < 3; dy++) {
-          const TS *zr = zl + z0[j] + dz * ps + (dy - 1) * g.rsx * 3;
-          const TS *Db = dict + d0[j] + (3 * dy + 9 * dz) * sweep_dict_block((int)sizeof(TS));
-          TS x[LP][3];
-#pragma unroll
-          for (int l = 0; l < LP; l++) lds_read3(zr + l * ps, x[l]);
-          sweep_key<TS, LP, 0>(Db, x, w);
-          sweep_key<TS, LP, 1>(Db, x, w);
-          sweep_key<TS, LP, 2>(Db, x, w);
-        }
+        for (int dy = 0; dy < 3; dy++) sweep_strip<TS, LP>(zr + dz * ps + dy * g.rsx * 3, ps, Db, dz, dy, w);
       if (j == 0) {
         // w = A z needs neither r.r nor r.z of the last update: their sums over
         // the cluster, posted before it, have arrived by now

@@ -23,7 +23,7 @@ namespace mm {
 namespace {
 
 constexpr int kNnz = 81;  // ELL width of the 3D hex8 Jacobian (micro/src/alloc.c:6)
-constexpr int kEB = 8;    // elements per wavefront in the stiffness kernel
+constexpr int kEB = 8;    // elements per wavefront in the residual kernel
 constexpr double kGauss = 0.577350269189626;  // src/fem.c:324
 
 // Device view of the mesh.
@@ -85,38 +85,37 @@ __device__ __forceinline__ void node_coord(const FeDev &F, int ix, int iy, int i
   }
 }
 
-// Physical derivatives dsh[a][i] and weight at gauss point g of element e:
-// structured (ds * 2 / h, w = vol_e / 8; src/fem.c:42-54 extended to 3D) or
-// isoparametric (J = sum_n ds X, cofactor inverse, dsh = J^-1 ds, w = |det J|
-// times the unit hex8 weight; src/fem.c:411-471, macro/src/assembly.c:115).
-__device__ void gp_dsh(const FeDev &F, int e, int g, double (&dsh)[8][3], double &w)
+// Gauss point g of element e: what its nodes' physical derivatives are formed
+// from, and the weight.  Structured: ds * 2 / h, w = vol_e / 8
+// (src/fem.c:42-54 extended to 3D).  Isoparametric: J = sum_n ds X, its cofactor
+// inverse, dsh = J^-1 ds, w = |det J| times the unit hex8 weight
+// (src/fem.c:411-471, macro/src/assembly.c:115).
+struct GpGeo {
+  double iJ[3][3], w;
+};
+__device__ void gp_geo(const FeDev &F, int e, int g, GpGeo &G)
 {
 #pragma clang fp contract(off)
   if (!F.iso) {
-    const double h[3] = {F.hx, F.hy, F.hz};
-    for (int a = 0; a < 8; a++) {
-      double ds[3];
-      master_ds(a, g, ds);
-      for (int d = 0; d < 3; d++) dsh[a][d] = ds[d] * 2 / h[d];
-    }
-    const double vol = h[0] * h[1] * h[2];
-    w = vol / 8;
+    const double vol = F.hx * F.hy * F.hz;
+    G.w = vol / 8;
     return;
-  }
-  double X[8][3], ds[8][3];
-  for (int a = 0; a < 8; a++) {
-    int ix, iy, iz;
-    elem_node(F, e, a, ix, iy, iz);
-    node_coord(F, ix, iy, iz, X[a]);
-    master_ds(a, g, ds[a]);
   }
   double J[3][3];
   for (int i = 0; i < 3; i++)
-    for (int j = 0; j < 3; j++) {
-      double s = 0.0;
-      for (int n = 0; n < 8; n++) s += ds[n][i] * X[n][j];
-      J[i][j] = s;
-    }
+    for (int j = 0; j < 3; j++) J[i][j] = 0.0;
+#pragma unroll
+  for (int n = 0; n < 8; n++) {
+    int ix, iy, iz;
+    double X[3], ds[3];
+    elem_node(F, e, n, ix, iy, iz);
+    node_coord(F, ix, iy, iz, X);
+    master_ds(n, g, ds);
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+      for (int j = 0; j < 3; j++) J[i][j] += ds[i] * X[j];
+  }
   const double c00 = +J[1][1] * J[2][2] - J[2][1] * J[1][2], c01 = -J[1][0] * J[2][2] + J[2][0] * J[1][2],
                c02 = +J[1][0] * J[2][1] - J[2][0] * J[1][1];
   const double c10 = -J[0][1] * J[2][2] + J[2][1] * J[0][2], c11 = +J[0][0] * J[2][2] - J[2][0] * J[0][2],
@@ -126,13 +125,34 @@ __device__ void gp_dsh(const FeDev &F, int e, int g, double (&dsh)[8][3], double
   const double det = J[0][0] * c00 + J[0][1] * c01 + J[0][2] * c02;
   const double iJ[3][3] = {{c00 / det, c10 / det, c20 / det}, {c01 / det, c11 / det, c21 / det},
                            {c02 / det, c12 / det, c22 / det}};
-  for (int a = 0; a < 8; a++)
-    for (int i = 0; i < 3; i++) {
-      double s = 0.0;
-      for (int j = 0; j < 3; j++) s += iJ[i][j] * ds[a][j];
-      dsh[a][i] = s;
-    }
-  w = fabs(det) * 1.0;
+  for (int i = 0; i < 3; i++)
+    for (int j = 0; j < 3; j++) G.iJ[i][j] = iJ[i][j];
+  G.w = fabs(det) * 1.0;
+}
+__device__ __forceinline__ void gp_node_dsh(const FeDev &F, const GpGeo &G, int a, int g, double (&dsh)[3])
+{
+#pragma clang fp contract(off)
+  double ds[3];
+  master_ds(a, g, ds);
+  if (!F.iso) {
+    dsh[0] = ds[0] * 2 / F.hx;
+    dsh[1] = ds[1] * 2 / F.hy;
+    dsh[2] = ds[2] * 2 / F.hz;
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 3; i++) {
+    double s = 0.0;
+#pragma unroll
+    for (int j = 0; j < 3; j++) s += G.iJ[i][j] * ds[j];
+    dsh[i] = s;
+  }
+}
+
+// Reads an address that is the same in every lane through the scalar unit.
+__device__ __forceinline__ double wave_load(const double *p)
+{
+  return *(const __attribute__((address_space(4))) double *)p;
 }
 
 // B[v][3a + d] from dsh[a][.] (Voigt xx, yy, zz, xy, yz, xz; engineering
@@ -149,52 +169,79 @@ __device__ __forceinline__ double bval(const double (&dsh)[3], int v, int d)
   }
 }
 
+// Rows of B with a value in column d of a node, ascending, and which of the
+// node's derivatives stands there (bval).
+__device__ constexpr int kBRow[3][3] = {{0, 3, 5}, {1, 3, 4}, {2, 4, 5}};
+__device__ constexpr int kBDer[3][3] = {{0, 1, 2}, {1, 0, 2}, {2, 1, 0}};
+
 // Element stiffness k[i][j] = sum_gp sum_k sum_h B[h][i] C[h][k] B[k][j] w
 // (micro/src/assembly.c:97-107, macro/src/assembly.c:173-181), one wavefront
-// per block of kEB elements: lane 8 el + g computes the derivatives of its
-// element's gauss point g into LDS, then the lanes share the 576 entries of
-// each element.  Terms with a zero factor are skipped (adding an exact zero
-// leaves every sum unchanged).
-__global__ __launch_bounds__(64) void k_fe_ke(FeDev F, double *__restrict__ ke_out)
+// per element: lane 8 g + a forms the derivatives of node a at gauss point g,
+// then lane 8 a + b sums the 3 x 3 block of nodes a and b.  Terms with a zero
+// factor are skipped (adding an exact zero leaves every sum unchanged): B's
+// structural zeros by construction, a zero of C for the whole wavefront.
+// Bound by FP64 issue (3 multiplies and an add per term, no contraction).  With
+// one entry per lane and all 36 (k, h) pairs tested in turn it took 1.44 ms for
+// 4,096 elements with full tangents and 1.37 for 720 with isotropic ones (a
+// chain of branches per lane); this 0.075 and 0.025.
+__global__ __launch_bounds__(256) void k_fe_ke(FeDev F, double *__restrict__ ke_out)
 {
 #pragma clang fp contract(off)
-  __shared__ double s_dsh[kEB][8][8][3];
-  __shared__ double s_w[kEB][8];
-  __shared__ double s_c[kEB][8][36];
-  const int e0 = blockIdx.x * kEB, l = threadIdx.x;
-  {
-    const int el = l / 8, g = l % 8, e = e0 + el;
-    if (e < F.nelm) {
-      double dsh[8][3], w;
-      gp_dsh(F, e, g, dsh, w);
-      for (int a = 0; a < 8; a++)
-        for (int d = 0; d < 3; d++) s_dsh[el][g][a][d] = dsh[a][d];
-      s_w[el][g] = w;
-      const double *c = F.c_gp ? F.c_gp + ((long long)e * 8 + g) * 36 : F.cmat + (size_t)F.elem_mat[e] * 36;
-      for (int i = 0; i < 36; i++) s_c[el][g][i] = c[i];
-    }
+  __shared__ double s_dsh[4][8][8][3];
+  __shared__ double s_w[4][8];
+  const int wv = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const int e = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + wv);
+  const bool on = e < F.nelm;
+  if (on) {
+    GpGeo G;
+    gp_geo(F, e, l >> 3, G);
+    double dsh[3];
+    gp_node_dsh(F, G, l & 7, l >> 3, dsh);
+#pragma unroll
+    for (int d = 0; d < 3; d++) s_dsh[wv][l >> 3][l & 7][d] = dsh[d];
+    if ((l & 7) == 0) s_w[wv][l >> 3] = G.w;
   }
   __syncthreads();
-  for (int idx = l; idx < kEB * 576; idx += 64) {
-    const int el = idx / 576, ent = idx % 576, e = e0 + el;
-    if (e >= F.nelm) break;
-    const int i = ent / 24, j = ent % 24, a = i / 3, d = i % 3, b = j / 3, dd = j % 3;
-    double acc = 0.0;
-    for (int g = 0; g < 8; g++) {
-      const double w = s_w[el][g];
-      for (int k = 0; k < 6; k++) {
-        const double bk = bval(s_dsh[el][g][b], k, dd);
-        if (bk == 0.0) continue;
-        for (int h = 0; h < 6; h++) {
-          const double bh = bval(s_dsh[el][g][a], h, d);
-          const double c = s_c[el][g][h * 6 + k];
-          if (bh == 0.0 || c == 0.0) continue;
-          acc = acc + bh * c * bk * w;
-        }
-      }
+  if (!on) return;
+  const int a = l >> 3, b = l & 7;
+  const double *cg = F.c_gp ? F.c_gp + (long long)e * 8 * 36
+                            : F.cmat + (size_t)__builtin_amdgcn_readfirstlane((int)F.elem_mat[e]) * 36;
+  const int cstep = F.c_gp ? 36 : 0;
+  double acc[3][3];
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+#pragma unroll
+    for (int dd = 0; dd < 3; dd++) acc[d][dd] = 0.0;
+#pragma unroll 1
+  for (int g = 0; g < 8; g++) {
+    const double w = s_w[wv][g];
+    double ba[3], bb[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      ba[d] = s_dsh[wv][g][a][d];
+      bb[d] = s_dsh[wv][g][b][d];
     }
-    ke_out[(long long)e * 576 + ent] = acc;
+    const double *C = cg + g * cstep;
+#pragma unroll
+    for (int dd = 0; dd < 3; dd++)
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int ik = 0; ik < 3; ik++)
+#pragma unroll
+          for (int ih = 0; ih < 3; ih++) {
+            const double c = wave_load(C + kBRow[d][ih] * 6 + kBRow[dd][ik]);
+            if (c == 0.0) continue;
+            const double bh = ba[kBDer[d][ih]], bk = bb[kBDer[dd][ik]];
+            const double t = acc[d][dd] + bh * c * bk * w;
+            acc[d][dd] = (bh == 0.0 || bk == 0.0) ? acc[d][dd] : t;
+          }
   }
+  double *out = ke_out + (long long)e * 576 + 72 * a + 3 * b;
+#pragma unroll
+  for (int d = 0; d < 3; d++)
+#pragma unroll
+    for (int dd = 0; dd < 3; dd++) out[24 * d + dd] = acc[d][dd];
 }
 
 // Affine displacement u = E X of Voigt strain s (micro/src/homogenize.c:335-342).
@@ -206,136 +253,130 @@ __device__ __forceinline__ double affine(const double *s, const double (&X)[3], 
   return s[5] / 2 * X[0] + s[4] / 2 * X[1] + s[2] * X[2];
 }
 
-// Element displacement: x at the element's unknowns, plus E X (true
-// coordinates) for the periodic fluctuation.
-__device__ void elem_disp(const FeDev &F, int e, const double *x, const double *strain, double (&ue)[24])
+// Element residual res_e[i] = sum_gp sum_j B[j][i] sigma_j w
+// (micro/src/assembly.c:45-56, macro/src/assembly.c:29-41), kEB elements per
+// wavefront: lane 8 el + n loads the displacement of the element's node n (x at
+// its unknown, plus E X at its true coordinates for the periodic fluctuation),
+// lane 8 el + g forms the strain (all 24 terms, src order) and the stress (C
+// strain, or given) of gauss point g, and the lanes then share the elements'
+// rows and averages, each summed over the gauss points in order.  Optional
+// outputs: the residual, the strains, and the averages' sums and weight.
+// Latency-bound at the sizes in use (a handful of wavefronts); one lane per
+// element took 37 us for 4,096 elements, this 13.
+__global__ __launch_bounds__(64) void k_fe_res(FeDev F, const double *__restrict__ x, const double *strain,
+                                              const double *__restrict__ stress_gp, double *__restrict__ res_out,
+                                              double *__restrict__ eps_out, double *__restrict__ avg_out)
 {
 #pragma clang fp contract(off)
-  for (int a = 0; a < 8; a++) {
+  __shared__ double s_u[kEB][24];
+  __shared__ double s_dsh[kEB][8][24];
+  __shared__ double s_es[kEB][8][12];  // strain, stress
+  __shared__ double s_w[kEB][8];
+  const int l = threadIdx.x, el = l >> 3, g = l & 7, e0 = blockIdx.x * kEB, e = e0 + el;
+  const bool on = e < F.nelm;
+  if (on) {
     int ix, iy, iz;
-    elem_node(F, e, a, ix, iy, iz);
+    elem_node(F, e, g, ix, iy, iz);
     const long long u = unknown_of(F, ix, iy, iz);
     double X[3];
     if (F.periodic) node_coord(F, ix, iy, iz, X);
-    for (int d = 0; d < 3; d++) ue[3 * a + d] = F.periodic ? x[3 * u + d] + affine(strain, X, d) : x[3 * u + d];
+    for (int d = 0; d < 3; d++)
+      s_u[el][3 * g + d] = F.periodic ? x[3 * u + d] + affine(strain, X, d) : x[3 * u + d];
   }
-}
-
-// Gauss-point strain (all 24 terms, src order) and stress (C strain or given).
-__device__ void gp_strain_stress(const FeDev &F, int e, int g, const double (&dsh)[8][3], const double (&ue)[24],
-                                 const double *stress_gp, double (&eps)[6], double (&sig)[6])
-{
-#pragma clang fp contract(off)
-  for (int v = 0; v < 6; v++) {
-    double s = 0.0;
-    for (int a = 0; a < 8; a++)
-      for (int d = 0; d < 3; d++) s += bval(dsh[a], v, d) * ue[3 * a + d];
-    eps[v] = (F.flush && fabs(s) < 1.0e-6) ? 0.0 : s;
-  }
-  if (stress_gp) {
-    for (int v = 0; v < 6; v++) sig[v] = stress_gp[((long long)e * 8 + g) * 6 + v];
-    return;
-  }
-  const double *c = F.c_gp ? F.c_gp + ((long long)e * 8 + g) * 36 : F.cmat + (size_t)F.elem_mat[e] * 36;
-  for (int i = 0; i < 6; i++) {
-    double s = 0.0;
-    for (int j = 0; j < 6; j++) s += c[i * 6 + j] * eps[j];
-    sig[i] = s;
-  }
-}
-
-// Element residual res_e[i] = sum_gp sum_j B[j][i] sigma_j w
-// (micro/src/assembly.c:45-56, macro/src/assembly.c:29-41); one lane per
-// element.  With out_eps, the gauss-point strains are stored instead.
-__global__ __launch_bounds__(256) void k_fe_res(FeDev F, const double *__restrict__ x, const double *strain,
-                                               const double *__restrict__ stress_gp, double *__restrict__ res_out,
-                                               double *__restrict__ eps_out, double *__restrict__ avg_out)
-{
-#pragma clang fp contract(off)
-  const int e = blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= F.nelm) return;
-  double ue[24], re[24], se[6], ss[6], wsum = 0.0;
-  elem_disp(F, e, x, strain, ue);
-  for (int i = 0; i < 24; i++) re[i] = 0.0;
-  for (int v = 0; v < 6; v++) {
-    se[v] = 0.0;
-    ss[v] = 0.0;
-  }
-  for (int g = 0; g < 8; g++) {
-    double dsh[8][3], w, eps[6], sig[6];
-    gp_dsh(F, e, g, dsh, w);
-    gp_strain_stress(F, e, g, dsh, ue, stress_gp, eps, sig);
+  __syncthreads();
+  if (on) {
+    GpGeo G;
+    gp_geo(F, e, g, G);
+    double eps[6];
+#pragma unroll
+    for (int v = 0; v < 6; v++) eps[v] = 0.0;
+#pragma unroll
+    for (int a = 0; a < 8; a++) {
+      double dsh[3];
+      gp_node_dsh(F, G, a, g, dsh);
+#pragma unroll
+      for (int d = 0; d < 3; d++) s_dsh[el][g][3 * a + d] = dsh[d];
+#pragma unroll
+      for (int v = 0; v < 6; v++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) eps[v] += bval(dsh, v, d) * s_u[el][3 * a + d];
+    }
+#pragma unroll
+    for (int v = 0; v < 6; v++) {
+      if (F.flush && fabs(eps[v]) < 1.0e-6) eps[v] = 0.0;
+      s_es[el][g][v] = eps[v];
+    }
     if (eps_out)
       for (int v = 0; v < 6; v++) eps_out[((long long)e * 8 + g) * 6 + v] = eps[v];
-    if (res_out)
-      for (int a = 0; a < 8; a++)
-        for (int d = 0; d < 3; d++)
-          for (int j = 0; j < 6; j++) re[3 * a + d] = re[3 * a + d] + bval(dsh[a], j, d) * sig[j] * w;
-    for (int v = 0; v < 6; v++) {  // micro/src/homogenize.c:344-368
-      ss[v] += sig[v] * w;
-      se[v] += eps[v] * w;
+    const double *c = F.c_gp ? F.c_gp + ((long long)e * 8 + g) * 36 : F.cmat + (size_t)F.elem_mat[e] * 36;
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+      double s = 0.0;
+      if (stress_gp) {
+        s = stress_gp[((long long)e * 8 + g) * 6 + i];
+      } else {
+#pragma unroll
+        for (int j = 0; j < 6; j++) s += c[i * 6 + j] * eps[j];
+      }
+      s_es[el][g][6 + i] = s;
     }
-    wsum += w;
+    s_w[el][g] = G.w;
   }
+  __syncthreads();
+  const int ne = min(kEB, F.nelm - e0);
   if (res_out)
-    for (int i = 0; i < 24; i++) res_out[(long long)e * 24 + i] = re[i];
-  if (avg_out) {  // element sums (for the volume average) and the element's weight
-    double *o = avg_out + (long long)e * 13;
-    for (int v = 0; v < 6; v++) {
-      o[v] = se[v];
-      o[6 + v] = ss[v];
+    for (int i = l; i < ne * 24; i += 64) {
+      const int q = i / 24, r = i - q * 24, a = r / 3, d = r - a * 3;
+      double s = 0.0;
+      for (int k = 0; k < 8; k++) {
+        const double w = s_w[q][k];
+        const double dsh[3] = {s_dsh[q][k][3 * a], s_dsh[q][k][3 * a + 1], s_dsh[q][k][3 * a + 2]};
+#pragma unroll
+        for (int j = 0; j < 6; j++) s = s + bval(dsh, j, d) * s_es[q][k][6 + j] * w;
+      }
+      res_out[(long long)e0 * 24 + i] = s;
     }
-    o[12] = wsum;
-  }
+  if (avg_out)  // element sums (for the volume average) and the element's weight (micro/src/homogenize.c:344-368)
+    for (int i = l; i < ne * 13; i += 64) {
+      const int q = i / 13, v = i - q * 13;
+      double s = 0.0;
+      for (int k = 0; k < 8; k++) s += (v == 12) ? s_w[q][k] : s_es[q][k][v] * s_w[q][k];
+      avg_out[(long long)e0 * 13 + i] = s;
+    }
 }
 
-// The (element, local node) pairs of unknown node u in ascending element id
-// (and local index), the order in which the reference's element loop
-// reaches the node.
-__device__ int node_elems(const FeDev &F, int u, int (&pe)[8], int (&pa)[8])
+// Unknown node u's place on the grid (or the torus).
+__device__ __forceinline__ void unknown_place(const FeDev &F, int u, int &ux, int &uy, int &uz)
 {
-  int ux, uy, uz;
+  const int sx = F.periodic ? F.nex : F.nx, sy = F.periodic ? F.ney : F.ny;
+  ux = u % sx;
+  uy = (u / sx) % sy;
+  uz = u / (sx * sy);
+}
+// The c-th of the up to 8 elements around an unknown node in ascending element
+// id, the order in which the reference's element loop reaches the node, and the
+// node's corner a there; false if there is none (c counts absent ones too).
+// Along each axis the element before the node comes first, on the torus the
+// element after it at place 0 (the one before is the last).
+__device__ __forceinline__ bool node_elem(const FeDev &F, int ux, int uy, int uz, int c, int &e, int &a)
+{
+  int lx = 1 - (c & 1), ly = 1 - ((c >> 1) & 1), lz = 1 - (c >> 2);
   if (F.periodic) {
-    ux = u % F.nex;
-    uy = (u / F.nex) % F.ney;
-    uz = u / (F.nex * F.ney);
-  } else {
-    ux = u % F.nx;
-    uy = (u / F.nx) % F.ny;
-    uz = u / (F.nx * F.ny);
+    if (ux == 0) lx = 1 - lx;
+    if (uy == 0) ly = 1 - ly;
+    if (uz == 0) lz = 1 - lz;
   }
-  int n = 0;
-  for (int a = 0; a < 8; a++) {
-    int lx, ly, lz;
-    local_coords(a, &lx, &ly, &lz);
-    int ex = ux - lx, ey = uy - ly, ez = uz - lz;
-    if (F.periodic) {
-      ex = (ex + F.nex) % F.nex;
-      ey = (ey + F.ney) % F.ney;
-      ez = (ez + F.nez) % F.nez;
-    } else if (ex < 0 || ey < 0 || ez < 0 || ex >= F.nex || ey >= F.ney || ez >= F.nez) {
-      continue;
-    }
-    pe[n] = ex + ey * F.nex + ez * F.nex * F.ney;
-    pa[n] = a;
-    n++;
+  int ex = ux - lx, ey = uy - ly, ez = uz - lz;
+  if (F.periodic) {
+    if (ex < 0) ex += F.nex;
+    if (ey < 0) ey += F.ney;
+    if (ez < 0) ez += F.nez;
+  } else if (ex < 0 || ey < 0 || ez < 0 || ex >= F.nex || ey >= F.ney || ez >= F.nez) {
+    return false;
   }
-  for (int i = 1; i < n; i++)  // insertion sort by (element, local node)
-    for (int j = i; j > 0 && (pe[j] < pe[j - 1] || (pe[j] == pe[j - 1] && pa[j] < pa[j - 1])); j--) {
-      const int te = pe[j], ta = pa[j];
-      pe[j] = pe[j - 1];
-      pa[j] = pa[j - 1];
-      pe[j - 1] = te;
-      pa[j - 1] = ta;
-    }
-  return n;
-}
-
-__device__ __forceinline__ int elem_unknown(const FeDev &F, int e, int b)
-{
-  int ix, iy, iz;
-  elem_node(F, e, b, ix, iy, iz);
-  return unknown_of(F, ix, iy, iz);
+  e = ex + ey * F.nex + ez * F.nex * F.ney;
+  a = local_node(lx, ly, lz);
+  return true;
 }
 
 // Residual of unknown node u: res[3u+d] = sum over its (element, a) pairs in
@@ -349,89 +390,132 @@ __global__ __launch_bounds__(256) void k_fe_node_res(FeDev F, const double *__re
   const int u = blockIdx.x * blockDim.x + threadIdx.x;
   double v[1] = {0.0};
   if (u < F.nunk) {
-    int pe[8], pa[8];
-    const int n = node_elems(F, u, pe, pa);
+    int ux, uy, uz;
+    unknown_place(F, u, ux, uy, uz);
+    double r[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      int e, a;
+      if (!node_elem(F, ux, uy, uz, c, e, a)) continue;
+#pragma unroll
+      for (int d = 0; d < 3; d++) r[d] = r[d] + res_e[(long long)e * 24 + 3 * a + d];
+    }
+#pragma unroll
     for (int d = 0; d < 3; d++) {
-      double r = 0.0;
-      for (int c = 0; c < n; c++) r = r + res_e[(long long)pe[c] * 24 + 3 * pa[c] + d];
-      if (F.dir[3 * (long long)u + d]) r = 0.0;
-      res[3 * (long long)u + d] = r;
-      v[0] += r * r;
+      if (F.dir[3 * (long long)u + d]) r[d] = 0.0;
+      res[3 * (long long)u + d] = r[d];
+      v[0] += r[d] * r[d];
     }
   }
   block_sum<1>(v, lds);
   if (threadIdx.x == 0) part[blockIdx.x] = v[0];
 }
 
-// One workgroup sums n partial values of width w (value i of item k at
-// p[k * w + i]) in item order; out[i] receives the totals.
+// Workgroup i sums the n partial values i of width w (value i of item k at
+// p[k * w + i]) in item order; out[i] receives the total.
 __global__ __launch_bounds__(256) void k_fe_sum(const double *__restrict__ p, int n, int w, double *__restrict__ out)
 {
-  __shared__ double lds[16 * 13];
-  double s[13];
-  for (int i = 0; i < 13; i++) s[i] = 0.0;
-  for (int k = threadIdx.x; k < n; k += blockDim.x)
-    for (int i = 0; i < w; i++) s[i] += p[(long long)k * w + i];
-  block_sum<13>(s, lds);
-  if (threadIdx.x == 0)
-    for (int i = 0; i < w; i++) out[i] = s[i];
+  __shared__ double lds[16];
+  double s[1] = {0.0};
+  for (int k = threadIdx.x; k < n; k += blockDim.x) s[0] += p[(long long)k * w + blockIdx.x];
+  block_sum<1>(s, lds);
+  if (threadIdx.x == 0) out[blockIdx.x] = s[0];
 }
 
-// ELL rows of unknown node u in the reference's layout: the neighbours in
-// first-touch order (elements ascending, then their local nodes), each
+// ELL rows of the unknown nodes in the reference's layout: a node's neighbours
+// in first-touch order (elements ascending, then their local nodes), each
 // slot the sum of the contributing element entries in ascending element
 // order (src/ell.c:46-84 over micro/src/assembly.c:93-110).  Dirichlet rows
 // become identity rows with their columns kept (src/ell.c:86-101); with
 // zero_cols, Dirichlet columns are zeroed in the other rows.  Output in the
 // slab layout of the device ELL (S rows per slab, column-major slots), and
 // dinv = 1 / diagonal.
-__global__ __launch_bounds__(256) void k_fe_node_ell(FeDev F, const double *__restrict__ ke, int S,
-                                                    int *__restrict__ cols, double *__restrict__ vals,
-                                                    double *__restrict__ dinv)
+//
+// 32 lanes per node, lane k for the neighbour at offset key k = (dx + 1) + 3 (dy
+// + 1) + 9 (dz + 1): of the node's elements in order, those with a corner there
+// contribute (at most one corner each, also on the torus, whose sides have three
+// or more elements), and the slot is the number of neighbours touched before the
+// key's first (element, corner).  The rows are collected in LDS and written as
+// runs of kNodes * 3 rows per slot.  Bound by the write (974 bytes a row) from
+// some 10^5 nodes on, by latency below.  One lane per node searching all
+// (element, corner) pairs for every entry took 1.62 ms for the 4,913 nodes of a
+// 16^3 block and 1.59 for the 990 of 9 x 8 x 10; this 0.024 and 0.017.
+constexpr int kNodes = 16;
+__global__ __launch_bounds__(32 * kNodes) void k_fe_node_ell(FeDev F, const double *__restrict__ ke, int S,
+                                                            int *__restrict__ cols, double *__restrict__ vals,
+                                                            double *__restrict__ dinv)
 {
 #pragma clang fp contract(off)
-  const int u = blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= F.nunk) return;
-  int pe[8], pa[8];
-  const int np = node_elems(F, u, pe, pa);
-  int nb[27], nnb = 0;
-  for (int c = 0; c < np; c++) {
-    if (c > 0 && pe[c] == pe[c - 1]) continue;  // same element again: no new columns
-    for (int b = 0; b < 8; b++) {
-      const int m = elem_unknown(F, pe[c], b);
-      bool seen = false;
-      for (int t = 0; t < nnb; t++) seen = seen || nb[t] == m;
-      if (!seen && nnb < 27) nb[nnb++] = m;
+  __shared__ double s_val[kNnz][3 * kNodes];
+  __shared__ int s_col[kNnz][3 * kNodes];
+  const int u0 = blockIdx.x * kNodes, nd = threadIdx.x >> 5, key = threadIdx.x & 31, u = u0 + nd;
+  const int nrows = 3 * min(kNodes, F.nunk - u0);
+  for (int i = threadIdx.x; i < kNnz * 3 * kNodes; i += blockDim.x) {
+    (&s_val[0][0])[i] = 0.0;
+    (&s_col[0][0])[i] = -1;
+  }
+  __syncthreads();
+  const bool on = u < F.nunk && key < 27;
+  int pos = 64, ux, uy, uz;
+  unknown_place(F, u, ux, uy, uz);
+  double v[3][3];
+  if (on) {
+    const int dx = key % 3 - 1, dy = (key / 3) % 3 - 1, dz = key / 9 - 1;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      int e, a, lx, ly, lz;
+      if (!node_elem(F, ux, uy, uz, c, e, a)) continue;
+      local_coords(a, &lx, &ly, &lz);
+      lx += dx;
+      ly += dy;
+      lz += dz;
+      if (((lx | ly | lz) & ~1) != 0) continue;  // not a corner of this element
+      const int b = local_node(lx, ly, lz);
+      const double *k = ke + (long long)e * 576 + 72 * a + 3 * b;
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int dd = 0; dd < 3; dd++) v[d][dd] = (pos == 64) ? k[24 * d + dd] : v[d][dd] + k[24 * d + dd];
+      if (pos == 64) pos = 8 * c + b;
     }
   }
-  for (int d = 0; d < 3; d++) {
-    const long long row = 3LL * u + d;
-    const long long base = (row / S) * (long long)S * kNnz + row % S;
-    const bool drow = F.dir[row];
-    double diag = 0.0;
-    for (int t = 0; t < 27; t++)
+  // the neighbours touched before this one
+  unsigned long long touched = (pos < 64) ? 1ull << pos : 0ull;
+#pragma unroll
+  for (int off = 16; off > 0; off >>= 1) touched |= __shfl_xor(touched, off, 32);
+  if (pos < 64) {
+    const int slot = __popcll(touched & ((1ull << pos) - 1ull));
+    int nb;
+    if (F.periodic) {
+      const int mx = ux + key % 3 - 1 + F.nex, my = uy + (key / 3) % 3 - 1 + F.ney, mz = uz + key / 9 - 1 + F.nez;
+      nb = mx % F.nex + (my % F.ney) * F.nex + (mz % F.nez) * F.nex * F.ney;
+    } else {
+      nb = u + key % 3 - 1 + ((key / 3) % 3 - 1) * F.nx + (key / 9 - 1) * F.nx * F.ny;
+    }
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+      const long long row = 3LL * u + d;
+      const bool drow = F.dir[row];
+#pragma unroll
       for (int dd = 0; dd < 3; dd++) {
-        const int j = 3 * t + dd;
-        int col = -1;
-        double v = 0.0;
-        if (t < nnb) {
-          col = 3 * nb[t] + dd;
-          bool first = true;
-          for (int c = 0; c < np; c++)
-            for (int b = 0; b < 8; b++) {
-              if (elem_unknown(F, pe[c], b) != nb[t]) continue;
-              const double kv = ke[(long long)pe[c] * 576 + (3 * pa[c] + d) * 24 + 3 * b + dd];
-              v = first ? kv : v + kv;
-              first = false;
-            }
-          if (drow) v = (col == row) ? 1.0 : 0.0;
-          else if (F.zero_cols && F.dir[col]) v = 0.0;
-          if (col == row) diag = v;
-        }
-        cols[base + (long long)j * S] = col;
-        vals[base + (long long)j * S] = v;
+        const int col = 3 * nb + dd;
+        double t = v[d][dd];
+        if (drow) t = (col == row) ? 1.0 : 0.0;
+        else if (F.zero_cols && F.dir[col]) t = 0.0;
+        if (col == row) dinv[row] = 1 / t;
+        s_val[3 * slot + dd][3 * nd + d] = t;
+        s_col[3 * slot + dd][3 * nd + d] = col;
       }
-    dinv[row] = 1 / diag;
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < kNnz * 3 * kNodes; i += blockDim.x) {
+    const int j = i / (3 * kNodes), r = i - j * (3 * kNodes);
+    if (r >= nrows) continue;
+    const long long row = 3LL * u0 + r;
+    const long long at = (row / S) * (long long)S * kNnz + (long long)j * S + row % S;
+    cols[at] = s_col[j][r];
+    vals[at] = s_val[j][r];
   }
 }
 
@@ -712,7 +796,7 @@ int fe_residual(Fe *f, const double *strain, const double *stress_gp, double *no
   const double *sg = nullptr;
   if ((rc = upload_stress(f, stress_gp, &sg))) return rc;
   const FeDev &F = f->F;
-  k_fe_res<<<grid_of(F.nelm, 256), 256, 0, f->s>>>(F, f->x, f->strain, sg, f->res_e, nullptr, nullptr);
+  k_fe_res<<<grid_of(F.nelm, kEB), 64, 0, f->s>>>(F, f->x, f->strain, sg, f->res_e, nullptr, nullptr);
   const int g = grid_of(F.nunk, 256);
   k_fe_node_res<<<g, 256, 0, f->s>>>(F, f->res_e, f->res, f->part);
   k_fe_sum<<<1, 256, 0, f->s>>>(f->part, g, 1, f->tot);
@@ -741,7 +825,7 @@ int fe_gp_strain(Fe *f, const double *strain, double *out)
     return MM_ERR_ALLOC;
   // the stress of the gauss points is computed and discarded: with a
   // stress input absent the tangent supplies it
-  k_fe_res<<<grid_of(f->F.nelm, 256), 256, 0, f->s>>>(f->F, f->x, f->strain, nullptr, nullptr, f->gp_buf, nullptr);
+  k_fe_res<<<grid_of(f->F.nelm, kEB), 64, 0, f->s>>>(f->F, f->x, f->strain, nullptr, nullptr, f->gp_buf, nullptr);
   MM_HIP(hipGetLastError());
   MM_HIP(hipMemcpyAsync(out, f->gp_buf, (size_t)f->F.nelm * 8 * 6 * 8, hipMemcpyDeviceToHost, f->s));
   MM_HIP(hipStreamSynchronize(f->s));
@@ -752,8 +836,8 @@ int fe_assemble(Fe *f)
 {
   if (!f) return MM_ERR_ARG;
   const FeDev &F = f->F;
-  k_fe_ke<<<grid_of(F.nelm, kEB), 64, 0, f->s>>>(F, f->ke);
-  k_fe_node_ell<<<grid_of(F.nunk, 256), 256, 0, f->s>>>(F, f->ke, f->S, f->ell_cols, f->ell_vals, f->ell_dinv);
+  k_fe_ke<<<grid_of(F.nelm, 4), 256, 0, f->s>>>(F, f->ke);
+  k_fe_node_ell<<<grid_of(F.nunk, kNodes), 32 * kNodes, 0, f->s>>>(F, f->ke, f->S, f->ell_cols, f->ell_vals, f->ell_dinv);
   MM_HIP(hipGetLastError());
   MM_HIP(hipStreamSynchronize(f->s));
   return 0;
@@ -807,8 +891,8 @@ int fe_averages(Fe *f, const double *strain, double *strain_ave, double *stress_
   int rc = upload_strain(f, strain);
   if (rc) return rc;
   const FeDev &F = f->F;
-  k_fe_res<<<grid_of(F.nelm, 256), 256, 0, f->s>>>(F, f->x, f->strain, nullptr, nullptr, nullptr, f->avg);
-  k_fe_sum<<<1, 256, 0, f->s>>>(f->avg, F.nelm, 13, f->tot);
+  k_fe_res<<<grid_of(F.nelm, kEB), 64, 0, f->s>>>(F, f->x, f->strain, nullptr, nullptr, nullptr, f->avg);
+  k_fe_sum<<<13, 256, 0, f->s>>>(f->avg, F.nelm, 13, f->tot);
   MM_HIP(hipGetLastError());
   double t[16];
   MM_HIP(hipMemcpyAsync(t, f->tot, 13 * 8, hipMemcpyDeviceToHost, f->s));
