@@ -106,12 +106,14 @@ int ell_device_solve_pcg(ell_device *d, ell_solver *solver, const double *b, dou
 int ell_device_solve_jacobi(ell_device *d, ell_solver *solver, const double *b, double *x);
 int ell_device_destroy(ell_device *d);
 /* How ell_device_solve_pcg (and the _noalloc variant) runs its iterations on
- * this mirror.  0 (the default): two launches per iteration, q = A p and the
- * vector update, each of whose workgroups first sums the other's slab
- * partials itself.  n > 0: one cooperative persistent kernel that runs up to
+ * this mirror.  0 (the default): small matrices with slabs of 256 rows (up to
+ * 384 slabs of at most 81 slots, the columns that one slab spans within the LDS)
+ * in one launch per solve with the matrix on chip; others in two launches per
+ * iteration, q = A p and the vector update, each of whose workgroups first sums
+ * the other's slab partials itself.  n > 0: one cooperative persistent kernel that runs up to
  * n whole iterations per launch, its workgroups meeting at two grid barriers
- * per iteration.  In both, the host checks for convergence between launches.
- * With 256-row slabs both give the same bits.  Returns 1 for n < 0, or for
+ * per iteration.  The host checks for convergence between launches.
+ * With 256-row slabs all of them give the same bits.  Returns 1 for n < 0, or for
  * n > 0 on a mirror whose slabs are not 256 rows or on a device without
  * cooperative launch.  No counterpart in the reference: it selects how the
  * PCG loop is mapped onto kernels. */

@@ -17,6 +17,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <condition_variable>
 #include <mutex>
 #include <vector>
 
@@ -75,6 +76,13 @@ constexpr int kU = 8;
 // k_reduce launches (four).  On one MI355X: 350 slabs (30^3 RVE) 0.042 ms
 // against 0.045 ms per iteration; 12,070 slabs (100^3) 0.89 against 0.73.
 constexpr int kSelfSumSlabs = 1024;
+// Slots that k_pcg_spmv fetches ahead on matrices of up to kAheadSlabs slabs,
+// where a row's chain of memory round trips is what the kernel waits for, and
+// where the chip is full of waves (kU) beyond.  us per iteration with kU, 14, 21
+// and 27: 46,875 rows 27.7, 25.0, 25.2, 27.4; 89,373 rows (350 slabs) 36.2, 32.5,
+// 33.7, 46.
+constexpr int kAhead = 14;
+constexpr int kAheadSlabs = 1024;
 __device__ inline double row_dot_exact(const int *__restrict__ cols, const double *__restrict__ vals,
                                        long long slab_base, int S, int nnz, int lane,
                                        const double *__restrict__ x)
@@ -230,60 +238,87 @@ __global__ void k_pcg_init(const int *__restrict__ cols, const double *__restric
 // buffer's pairs (one 16-byte gather per column) and writes the new p into
 // the other buffer, whose z the update then writes.
 
+// Slots j0 .. j0 + U - 1 of one row: column ids and values, fetched together.
+template <int U>
+struct PcgSlots {
+  int c[U];
+  double v[U];
+};
+template <int U>
+__device__ __forceinline__ void pcg_fetch(const int *__restrict__ cols, const double *__restrict__ vals, int nnz, int S,
+                                          long long base, int lane, int j0, PcgSlots<U> &s)
+{
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const bool in = j0 + u < nnz;
+    const long long e = base + (long long)(j0 + u) * S + lane;
+    s.c[u] = in ? __builtin_nontemporal_load(&cols[e]) : -1;
+    s.v[u] = in ? __builtin_nontemporal_load(&vals[e]) : 0.0;
+  }
+}
+
 // Row `row` (lane `lane` of slab `slab`) of q = A p with p = z + beta p_old
 // formed on the fly from the current pairs zc, both for the own row, whose p
 // is stored in zn, and for every gathered column; returns q_row * p_row.
-// Shared by the per-step kernels and the fused kernel, so both do the same
-// arithmetic.
-__device__ inline double pcg_q_row(const int *__restrict__ cols, const double *__restrict__ vals, int nnz, int S,
-                                   int slab, int lane, long long row, const double2 *__restrict__ zc, double beta,
-                                   double2 *__restrict__ zn, double *__restrict__ q)
+// `cur` holds the row's first U slots; accumulated in slot order whatever U is.
+// Shared by the per-step kernels and the fused kernel, so all do the same
+// arithmetic.  With AHEAD the next U slots are fetched before the pairs of the
+// current ones are used, so a trip costs one memory round trip, not two.
+template <int U, bool AHEAD>
+__device__ __forceinline__ double pcg_q_row(const int *__restrict__ cols, const double *__restrict__ vals, int nnz,
+                                            int S, int slab, int lane, long long row,
+                                            const double2 *__restrict__ zc, double beta, double2 *__restrict__ zn,
+                                            double *__restrict__ q, PcgSlots<U> cur)
 {
   const long long base = (long long)slab * S * nnz;
+  const double2 own = zc[row];
   double acc = 0.0;
-  // kU slots per round trip, as in row_dot_exact; accumulated in slot order
-  for (int j0 = 0; j0 < nnz; j0 += kU) {
-    int c[kU];
-    double v[kU], t[kU];
+  for (int j0 = 0; j0 < nnz; j0 += U) {
+    double2 w[U];
 #pragma unroll
-    for (int u = 0; u < kU; u++) {
-      const bool in = j0 + u < nnz;
-      const long long e = base + (long long)(j0 + u) * S + lane;
-      c[u] = in ? __builtin_nontemporal_load(&cols[e]) : -1;
-      v[u] = in ? __builtin_nontemporal_load(&vals[e]) : 0.0;
-    }
-#pragma unroll
-    for (int u = 0; u < kU; u++) {
-      const double2 w = (c[u] >= 0) ? zc[c[u]] : make_double2(0.0, 0.0);
-      t[u] = w.x + beta * w.y;
-    }
+    for (int u = 0; u < U; u++) w[u] = (cur.c[u] >= 0) ? zc[cur.c[u]] : make_double2(0.0, 0.0);
+    PcgSlots<U> next;
+    if (AHEAD && j0 + U < nnz) pcg_fetch<U>(cols, vals, nnz, S, base, lane, j0 + U, next);
     bool stop = false;
 #pragma unroll
-    for (int u = 0; u < kU; u++) {
-      if (c[u] == -1) {
+    for (int u = 0; u < U; u++) {
+      if (cur.c[u] == -1) {
         stop = true;
         break;
       }
-      acc += v[u] * t[u];
+      acc += cur.v[u] * (w[u].x + beta * w[u].y);
     }
     if (stop) break;
+    if (!AHEAD && j0 + U < nnz) pcg_fetch<U>(cols, vals, nnz, S, base, lane, j0 + U, next);
+    cur = next;
   }
-  const double2 w = zc[row];
-  const double pi = w.x + beta * w.y;
+  const double pi = own.x + beta * own.y;
   zn[row].y = pi;
   q[row] = acc;
   return pi * acc;
 }
 
-// Row `row` of x += alpha p, r -= alpha q, z = dinv r, with p and the new z
-// in the pairs zp; v = {r.r, r.z} terms.
-__device__ inline void pcg_update_row(long long row, double alpha, const double *__restrict__ dinv,
-                                      double2 *__restrict__ zp, const double *__restrict__ q,
-                                      double *__restrict__ x, double *__restrict__ r, double (&v)[2])
+// Row `row` of x += alpha p, r -= alpha q, z = dinv r, the new z into the pairs
+// zp; v = {r.r, r.z} terms.
+struct PcgRow {
+  double dinv, q, x, r, p;
+};
+__device__ __forceinline__ void pcg_row_load(long long row, const double *__restrict__ dinv,
+                                             const double *__restrict__ q, const double *__restrict__ x,
+                                             const double *__restrict__ r, PcgRow &w)
 {
-  const double xi = x[row] + alpha * zp[row].y;
-  const double ri = r[row] - alpha * q[row];
-  const double zi = dinv[row] * ri;
+  w.dinv = dinv[row];
+  w.q = q[row];
+  w.x = x[row];
+  w.r = r[row];
+}
+__device__ __forceinline__ void pcg_update_row(long long row, double alpha, const PcgRow &w,
+                                               double2 *__restrict__ zp, double *__restrict__ x,
+                                               double *__restrict__ r, double (&v)[2])
+{
+  const double xi = w.x + alpha * w.p;
+  const double ri = w.r - alpha * w.q;
+  const double zi = w.dinv * ri;
   x[row] = xi;
   r[row] = ri;
   zp[row].x = zi;
@@ -304,16 +339,19 @@ __device__ inline void pcg_update_row(long long row, double alpha, const double 
 
 // First the update's r.r / r.z (part[.][1..2]) give the iteration count, the
 // convergence test and beta (nothing to sum right after the start); then
-// q = A p (pcg_q_row) with partial p.q (part[.][0]).
-__global__ void k_pcg_spmv(const int *__restrict__ cols, const double *__restrict__ vals,
-                                                  int nrow, int nnz, int S, int nslab, double2 *__restrict__ zpA,
-                                                  double2 *__restrict__ zpB, double *__restrict__ q,
-                                                  double *__restrict__ part, const IterState *st_in,
-                                                  IterState *st_out, int self_sum)
+// q = A p (pcg_q_row) with partial p.q (part[.][0]).  The row's first slots are
+// asked for before the scalars are formed.
+template <int U, bool AHEAD>
+__global__ __launch_bounds__(AHEAD ? 256 : 1024) void k_pcg_spmv(const int *__restrict__ cols, const double *__restrict__ vals, int nrow, int nnz, int S,
+                           int nslab, double2 *__restrict__ zpA, double2 *__restrict__ zpB, double *__restrict__ q,
+                           double *__restrict__ part, const IterState *st_in, IterState *st_out, int self_sum)
 {
   __shared__ double lds[48];
   __shared__ IterState N;
   const int lane = threadIdx.x;
+  const long long row = (long long)blockIdx.x * S + lane;
+  PcgSlots<U> first;
+  pcg_fetch<U>(cols, vals, nnz, S, (long long)blockIdx.x * S * nnz, lane, 0, first);  // padding rows hold -1
   if (lane == 0) N = *st_in;
   __syncthreads();
   if (self_sum && !N.done && !N.fresh) {
@@ -331,15 +369,16 @@ __global__ void k_pcg_spmv(const int *__restrict__ cols, const double *__restric
   const double beta = N.beta;
   const double2 *zc = N.pbuf ? zpB : zpA;
   double2 *zn = N.pbuf ? zpA : zpB;
-  const long long row = (long long)blockIdx.x * S + lane;
   double v[1] = {0.0};
-  if (row < nrow) v[0] = pcg_q_row(cols, vals, nnz, S, blockIdx.x, lane, row, zc, beta, zn, q);
+  if (row < nrow) v[0] = pcg_q_row<U, AHEAD>(cols, vals, nnz, S, blockIdx.x, lane, row, zc, beta, zn, q, first);
   block_sum<1>(v, lds);
   if (lane == 0) part[blockIdx.x * 4] = v[0];
 }
 
 // alpha from the p.q partials; x += alpha p, r -= alpha q, z = dinv r
-// (pcg_update_row); partials r.r, r.z (part[.][1..2]).
+// (pcg_update_row); partials r.r, r.z (part[.][1..2]).  The row's vectors are
+// asked for before the scalars are formed, both buffers' p because the state
+// says which is the new one.
 __global__ void k_pcg_update(int nrow, int S, int nslab, const double *__restrict__ dinv,
                              double2 *__restrict__ zpA, double2 *__restrict__ zpB, const double *__restrict__ q,
                              double *__restrict__ x, double *__restrict__ r, double *__restrict__ part,
@@ -348,6 +387,15 @@ __global__ void k_pcg_update(int nrow, int S, int nslab, const double *__restric
   __shared__ double lds[32];
   __shared__ IterState N;
   const int lane = threadIdx.x;
+  const long long row = (long long)blockIdx.x * S + lane;
+  const bool on = row < nrow;
+  PcgRow w = {0.0, 0.0, 0.0, 0.0, 0.0};
+  double pA = 0.0, pB = 0.0;
+  if (on) {
+    pcg_row_load(row, dinv, q, x, r, w);
+    pA = zpA[row].y;
+    pB = zpB[row].y;
+  }
   if (lane == 0) N = *st_in;
   __syncthreads();
   if (self_sum && !N.done) {
@@ -361,11 +409,10 @@ __global__ void k_pcg_update(int nrow, int S, int nslab, const double *__restric
   }
   if (blockIdx.x == 0 && lane == 0) *st_out = N;
   if (N.done) return;
-  const double alpha = N.alpha;
-  double2 *zp = N.pbuf ? zpB : zpA;  // the pairs whose p k_pcg_spmv wrote
-  const long long row = (long long)blockIdx.x * S + lane;
+  w.p = N.pbuf ? pB : pA;                // the pairs whose p k_pcg_spmv wrote
+  double2 *zp = N.pbuf ? zpB : zpA;
   double v[2] = {0.0, 0.0};
-  if (row < nrow) pcg_update_row(row, alpha, dinv, zp, q, x, r, v);
+  if (on) pcg_update_row(row, N.alpha, w, zp, x, r, v);
   block_sum<2>(v, lds);
   if (lane == 0) {
     part[blockIdx.x * 4 + 1] = v[0];
@@ -477,7 +524,9 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
     for (int slab = blockIdx.x; slab < nslab; slab += G) {
       const long long row = (long long)slab * S + lane;
       double v[1] = {0.0};
-      if (row < nrow) v[0] = pcg_q_row(cols, vals, nnz, S, slab, lane, row, zc, beta, zn, q);
+      PcgSlots<kU> first;
+      pcg_fetch<kU>(cols, vals, nnz, S, (long long)slab * S * nnz, lane, 0, first);
+      if (row < nrow) v[0] = pcg_q_row<kU, false>(cols, vals, nnz, S, slab, lane, row, zc, beta, zn, q, first);
       block_sum<1>(v, lds);
       if (lane == 0) part[slab * 4] = v[0];
     }
@@ -492,7 +541,12 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
     for (int slab = blockIdx.x; slab < nslab; slab += G) {
       const long long row = (long long)slab * S + lane;
       double v[2] = {0.0, 0.0};
-      if (row < nrow) pcg_update_row(row, alpha, dinv, zp, q, x, r, v);
+      if (row < nrow) {
+        PcgRow w;
+        pcg_row_load(row, dinv, q, x, r, w);
+        w.p = zp[row].y;
+        pcg_update_row(row, alpha, w, zp, x, r, v);
+      }
       block_sum<2>(v, lds);
       if (lane == 0) {
         part[slab * 4 + 1] = v[0];
@@ -521,6 +575,270 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
     st->done = done;
     st->fresh = 0;
   }
+}
+
+// ---- the same iteration with the matrix on chip ------------------------------
+// k_pcg_resident runs a whole solve in one launch, one workgroup per slab of 256
+// rows.  Each lane holds its row: the values and the LDS places of its columns
+// (two to a register) for the whole solve, x, r, z and p too.  p of every column
+// between the slab's lowest and highest lives in LDS: after an update the owners
+// publish z as tagged words, and every workgroup forms p = z + beta p for its
+// columns, the same bits as the owner.  p.q and {r.r, r.z} go round as tagged
+// words too and are summed by every workgroup in the order of the other mappings
+// (group_sum_rows: slab-strided, then block_sum).  With the same row arithmetic
+// and scalar steps all mappings give the same bits.
+//
+// Bound by the two exchanges of an iteration and the columns' z between them;
+// the two launches per iteration that it replaces were bound by the host's
+// launches for small matrices and by reading 12 bytes per entry for larger ones.
+// Elasticity systems of N^3 elements with 81 slots, us per iteration, two launches
+// against this: 2,970 rows 22.7 and 8.6, 14,739 rows 23.6 and 9.6, 46,875 rows
+// 25.0 and 12.4, 89,373 rows 32.5 and 17.2.
+//
+// All workgroups have to run at the same time.  They are at most 384, two to a CU
+// (one, 192, where the LDS of two does not fit): 192 CUs, which leaves 64 for
+// kernels of other streams that wait for workgroups of their own, as the engine's
+// sweeps do (at most 15 CUs each).  Solves of one process share the 192 CUs
+// (ResShare).  Every wait is bounded all the same, and a solve whose wait ran out,
+// for instance beside another process's, is done again in the two-launch form.
+constexpr int kResSlots = 81;  // rows of 27 nodes' 3 dofs; five registers for two slots, 203 of 256
+constexpr int kResMaxSlabs = 384;
+constexpr int kResOneCuLds = 78 * 1024;  // up to this, two workgroups per CU
+constexpr int kResMaxLds = 156 * 1024;
+constexpr int kResPolls = 1 << 18;  // about 0.2 s
+constexpr int kResMaxDevices = 64;
+
+// Sums NV values over all slabs, valid in every lane: lane 0 of each workgroup
+// has posted its own (NV doubles at sums + slab * 8).  False, in every lane, when
+// a wait of this workgroup ran out since the solve began (`fail`, LDS).
+template <int NV>
+__device__ __forceinline__ bool res_collect(const word_t *sums, int nslab, unsigned tag, double (&out)[NV],
+                                            double (&lds)[48], double *bc, int *fail)
+{
+#pragma unroll
+  for (int i = 0; i < NV; i++) out[i] = 0.0;
+  for (int b = threadIdx.x; b < nslab; b += blockDim.x) {
+    word_t w[2 * NV];
+    int n = 0;
+    for (;;) {
+      bool all = true;
+#pragma unroll
+      for (int i = 0; i < 2 * NV; i++) w[i] = get_word(sums + (long long)b * 8 + i);
+#pragma unroll
+      for (int i = 0; i < 2 * NV; i++) all = all && (unsigned)(w[i] >> 32) == tag;
+      if (all) break;
+      if (++n > kResPolls) {
+        *fail = 1;
+        break;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NV; i++) out[i] += word_double(w[2 * i], w[2 * i + 1]);
+  }
+  block_sum<NV>(out, lds);
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int i = 0; i < NV; i++) bc[i] = out[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < NV; i++) out[i] = bc[i];
+  return __builtin_amdgcn_readfirstlane(*fail) == 0;
+}
+
+extern __shared__ __attribute__((aligned(16))) double res_p[];
+
+// A product that is rounded before it is summed (not contracted into the sum).
+__device__ __forceinline__ double rounded(double v)
+{
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// zw: two words per row (z of the last update), sums: 16 words per slab, all
+// zero on entry (no iteration's tag); zp[row].x is the first z, .y receives x.
+__global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__ cols, const double *__restrict__ vals,
+                                                         int nrow, int nnz, int nslab, int lds_rows,
+                                                         const double *__restrict__ dinv, const double *__restrict__ x0,
+                                                         const double *__restrict__ r0, double2 *__restrict__ zp,
+                                                         word_t *zw, word_t *sums, IterState *st)
+{
+  __shared__ double lds[48];
+  __shared__ double bc[2];
+  __shared__ int s_lo, s_hi, s_fail;
+  if (st->done) return;
+  const int lane = threadIdx.x, slab = blockIdx.x;
+  const long long row = (long long)slab * 256 + lane, base = (long long)slab * 256 * nnz;
+  const bool on = row < nrow;
+  if (lane == 0) {
+    s_lo = nrow;
+    s_hi = -1;
+    s_fail = 0;
+  }
+  __syncthreads();
+  // the row up to its first -1, column places two to a register; the slots
+  // after it add -0.0 * res_p[lds_rows] = -0.0, which changes no sum
+  double v[kResSlots];
+  unsigned o[(kResSlots + 1) / 2];
+  const int *rc = cols + base + lane;
+  const double *rv = vals + base + lane;
+  int cnt = 0, lo = nrow, hi = -1;
+  bool more = on;
+#pragma unroll 1
+  for (int u0 = 0; u0 < nnz; u0 += 9) {
+    int c[9];
+#pragma unroll
+    for (int u = 0; u < 9; u++) c[u] = (on && u0 + u < nnz) ? rc[(u0 + u) * 256] : -1;
+#pragma unroll
+    for (int u = 0; u < 9; u++) {
+      more = more && c[u] != -1;
+      lo = more ? min(lo, c[u]) : lo;
+      hi = more ? max(hi, c[u]) : hi;
+      cnt += more ? 1 : 0;
+    }
+  }
+  if (cnt > 0) {
+    atomicMin(&s_lo, lo);
+    atomicMax(&s_hi, hi);
+  }
+  __syncthreads();
+  lo = __builtin_amdgcn_readfirstlane(s_lo);
+  hi = __builtin_amdgcn_readfirstlane(s_hi);
+  if (hi - lo >= lds_rows) {  // (the host sized the LDS by the widest slab)
+    if (lane == 0) st->pad0 = 1;
+    return;
+  }
+#pragma unroll
+  for (int u0 = 0; u0 < kResSlots; u0 += 9) {
+#pragma unroll
+    for (int u = u0; u < u0 + 9; u++) {
+      unsigned c = lds_rows;
+      v[u] = -0.0;
+      if (u < cnt) {
+        c = rc[u * 256] - lo;
+        v[u] = rv[u * 256];
+      }
+      if (u & 1) o[u / 2] |= c << 16;
+      else o[u / 2] = c;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  int most = cnt;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) most = max(most, __shfl_xor(most, off, 64));
+  most = __builtin_amdgcn_readfirstlane(most);
+  double xi = on ? x0[row] : 0.0, ri = on ? r0[row] : 0.0, zi = on ? zp[row].x : 0.0, pi = 0.0;
+  const double di = on ? dinv[row] : 0.0;
+  for (int e = lo + lane; e <= hi; e += 256) res_p[e - lo] = 0.0;
+  if (lane == 0) res_p[lds_rows] = 0.0;
+  __syncthreads();
+  const double bnorm = st->bnorm, rtol = st->rtol;
+  const int max_its = st->max_its;
+  double rz = st->rz, beta = 0.0, alpha = 0.0, rnorm = st->rnorm;
+  int n = 0, done = 0;
+#pragma unroll 1
+  for (;;) {
+    if (n > 0) {
+      double s[2];
+      if (!res_collect<2>(sums + (long long)nslab * 8, nslab, (unsigned)n, s, lds, bc, &s_fail)) break;
+      int its = n - 1;
+      pcg_after_update(s[0], s[1], rtol, bnorm, max_its, its, rnorm, rz, beta, done);
+      if (__builtin_amdgcn_readfirstlane(done)) break;
+    }
+    // p = z + beta p for the slab's columns, four per trip
+    for (int e0 = lo + lane; e0 <= hi; e0 += 4 * 256) {
+      double z[4];
+      if (n == 0) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) z[i] = (e0 + 256 * i <= hi) ? zp[e0 + 256 * i].x : 0.0;
+      } else {
+        word_t a[4], b[4];
+        int m = 0;
+        for (;;) {
+          bool all = true;
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int e = min(e0 + 256 * i, hi);
+            a[i] = get_word(zw + 2LL * e);
+            b[i] = get_word(zw + 2LL * e + 1);
+          }
+#pragma unroll
+          for (int i = 0; i < 4; i++)
+            all = all && (unsigned)(a[i] >> 32) == (unsigned)n && (unsigned)(b[i] >> 32) == (unsigned)n;
+          if (all) break;
+          if (++m > kResPolls) {
+            s_fail = 1;
+            break;
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) z[i] = word_double(a[i], b[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        if (e0 + 256 * i <= hi) res_p[e0 + 256 * i - lo] = fma(beta, res_p[e0 + 256 * i - lo], z[i]);
+    }
+    pi = fma(beta, pi, zi);
+    __syncthreads();
+    // (o is taken apart anew each time: the places would not fit the registers)
+#pragma unroll
+    for (int u = 0; u < (kResSlots + 1) / 2; u++) asm volatile("" : "+v"(o[u]));
+    double qi = 0.0;
+#pragma unroll
+    for (int u0 = 0; u0 < kResSlots; u0 += 9) {
+      if (u0 < most) {
+        double t[9];
+#pragma unroll
+        for (int u = 0; u < 9; u++) t[u] = res_p[((u0 + u) & 1) ? o[(u0 + u) / 2] >> 16 : o[(u0 + u) / 2] & 0xffffu];
+#pragma unroll
+        for (int u = 0; u < 9; u++) qi = fma(v[u0 + u], t[u], qi);
+      }
+    }
+    const unsigned tag = (unsigned)n + 1u;
+    double s1[1] = {rounded(pi * qi)};
+    block_sum<1>(s1, lds);
+    if (lane == 0) put_double(sums + (long long)slab * 8, tag, s1[0]);
+    if (!res_collect<1>(sums, nslab, tag, s1, lds, bc, &s_fail)) break;
+    alpha = pcg_alpha(rz, s1[0]);
+    xi = fma(alpha, pi, xi);
+    ri = fma(-alpha, qi, ri);
+    zi = di * ri;
+    if (on) put_double(zw + 2 * row, tag, zi);
+    double s2[2] = {rounded(ri * ri), rounded(ri * zi)};  // (zero beyond the last row)
+    block_sum<2>(s2, lds);
+    if (lane == 0) {
+      put_double(sums + (long long)(nslab + slab) * 8, tag, s2[0]);
+      put_double(sums + (long long)(nslab + slab) * 8 + 2, tag, s2[1]);
+    }
+    n++;
+  }
+  if (s_fail) {
+    if (lane == 0) st->pad0 = 1;  // (any of them may; the host reads it after the kernel)
+    return;
+  }
+  if (on) zp[row].y = xi;
+  if (slab == 0 && lane == 0) {
+    st->its = n;
+    st->rnorm = rnorm;
+    st->rz = rz;
+    st->alpha = alpha;
+    st->beta = beta;
+    st->done = done;
+    st->fresh = 0;
+  }
+}
+
+// The exchange sums of k_pcg_resident (its z words are zeroed by k_pcg_init).
+__global__ void k_res_zero(word_t *sums, int n)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) sums[i] = 0;
+}
+
+// x after a resident solve that succeeded.
+__global__ void k_res_take(const IterState *st, const double2 *__restrict__ zp, double *__restrict__ x, int n)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n && !st->fresh && !st->pad0) x[i] = zp[i].y;
 }
 
 // Zeroes the barrier words of k_pcg_fused (a kernel, not a memset node).
@@ -556,6 +874,7 @@ struct ell_device_ {
   double2 *zpA, *zpB;  // PCG {z, p} pairs
   IterState *st;
   unsigned *bar;
+  int band;        // most columns that a slab's rows span (0: not known)
   int fused_its;   // 0: two launches per PCG iteration; n > 0: k_pcg_fused, n iterations per launch
   int fused_grid;  // co-resident workgroups of k_pcg_fused (set with fused_its)
   hipStream_t stream;
@@ -606,6 +925,18 @@ static int upload(ell_device *d, const ell_matrix *m)
       hc[sb + (size_t)j * d->S + lane] = m->cols[(size_t)i * m->nnz + j];
       hv[sb + (size_t)j * d->S + lane] = m->vals[(size_t)i * m->nnz + j];
     }
+  }
+  d->band = 1;
+  for (int s = 0; s < d->nslab; s++) {
+    int lo = m->ncol, hi = -1;
+    const int end = (s + 1) * d->S < m->nrow ? (s + 1) * d->S : m->nrow;
+    for (size_t e = (size_t)s * d->S * m->nnz; e < (size_t)end * m->nnz; e++) {
+      const int c = m->cols[e];
+      if (c < 0) continue;
+      if (c < lo) lo = c;
+      if (c > hi) hi = c;
+    }
+    if (hi - lo + 1 > d->band) d->band = hi - lo + 1;
   }
   std::vector<double> dinv;
   host_diag_inv(m, dinv);
@@ -788,12 +1119,55 @@ extern "C" int ell_device_solve_jacobi(ell_device *d, ell_solver *solver, const 
   return 0;
 }
 
+// The part of a device that resident solves of this process hold together, in
+// halves of a CU; a solve waits here until its workgroups fit beside the others.
+class ResShare {
+ public:
+  ResShare(int device, int halves) : g_(gate(device)), halves_(halves)
+  {
+    std::unique_lock<std::mutex> lk(g_.mu);
+    g_.cv.wait(lk, [&] { return g_.used + halves_ <= kResMaxSlabs; });
+    g_.used += halves_;
+  }
+  ~ResShare()
+  {
+    {
+      std::lock_guard<std::mutex> lk(g_.mu);
+      g_.used -= halves_;
+    }
+    g_.cv.notify_all();
+  }
+  ResShare(const ResShare &) = delete;
+  ResShare &operator=(const ResShare &) = delete;
+
+ private:
+  struct Gate {
+    std::mutex mu;
+    std::condition_variable cv;
+    int used = 0;
+  };
+  static Gate &gate(int device)
+  {
+    static Gate g[kResMaxDevices];
+    return g[device];
+  }
+  Gate &g_;
+  const int halves_;
+};
+
 // Jacobi-PCG on the device mirror with b and x (initial guess in, solution
 // out) in device memory and the work vectors V; the host polls the
 // iteration state every 32 iterations.  Returns 0 when converged, 5 when
 // max_its was reached.
-static int pcg_run(ell_device *d, const PcgVecs &V, ell_solver *solver, const double *b, double *x)
+static int pcg_run(ell_device *d, const PcgVecs &V, ell_solver *solver, const double *b, double *x,
+                   bool may_stay = true)
 {
+  // the matrix on chip (k_pcg_resident) where the columns that a slab spans fit
+  // the LDS and the workgroups the GPU; it was the faster at every size it takes
+  const int res_rows = d->band > 0 ? d->band : d->nrow;
+  const bool resident = may_stay && d->fused_its == 0 && d->S == 256 && d->nnz <= kResSlots &&
+                        d->device < kResMaxDevices && res_rows <= kResMaxLds / 8 &&
+                        d->nslab <= (res_rows * 8 <= kResOneCuLds ? kResMaxSlabs : kResMaxSlabs / 2);
   const int max_its = (solver && solver->max_its > 0) ? solver->max_its : MAX_ITS;
   const double rtol = (solver && solver->min_err > 0) ? solver->min_err : MIN_ERR;
   int rc = set_state(d, V.st, max_its, rtol, 0.0);
@@ -803,8 +1177,21 @@ static int pcg_run(ell_device *d, const PcgVecs &V, ell_solver *solver, const do
   k_reduce<<<1, 256, 0, d->stream>>>(V.part, d->nslab, RED_INIT, V.st);
   MM_HIP(hipGetLastError());
   IterState h;
-  rc = get_state(d, V.st, &h);
-  if (rc) return rc;
+  if (resident) {
+    ResShare share(d->device, res_rows * 8 <= kResOneCuLds ? d->nslab : 2 * d->nslab);
+    word_t *zw = reinterpret_cast<word_t *>(V.zpB), *sums = reinterpret_cast<word_t *>(V.q);
+    k_res_zero<<<(16 * d->nslab + 255) / 256, 256, 0, d->stream>>>(sums, 16 * d->nslab);
+    k_pcg_resident<<<d->nslab, 256, (size_t)(res_rows + 1) * sizeof(double), d->stream>>>(
+        d->cols, d->vals, d->nrow, d->nnz, d->nslab, res_rows, d->dinv, x, V.r, V.zpA, zw, sums, V.st);
+    k_res_take<<<(d->nrow + 255) / 256, 256, 0, d->stream>>>(V.st, V.zpA, x, d->nrow);
+    MM_HIP(hipGetLastError());
+    rc = get_state(d, V.st, &h);
+    if (rc) return rc;
+    if (h.pad0) return pcg_run(d, V, solver, b, x, false);  // a wait ran out: x is as it was
+  } else {
+    rc = get_state(d, V.st, &h);
+    if (rc) return rc;
+  }
   if (h.bnorm == 0.0) {  // zero right-hand side: the solution is zero
     k_zero<<<(d->nrow + 255) / 256, 256, 0, d->stream>>>(x, d->nrow);
     MM_HIP(hipGetLastError());
@@ -834,10 +1221,11 @@ static int pcg_run(ell_device *d, const PcgVecs &V, ell_solver *solver, const do
   // the state passes st[0] -> st[1] -> st[0]; up to kSelfSumSlabs slabs two
   // launches per iteration, beyond that a one-workgroup k_reduce before each
   const int self_sum = d->nslab <= kSelfSumSlabs ? 1 : 0;
+  const auto spmv = d->nslab <= kAheadSlabs && d->S <= 256 ? k_pcg_spmv<kAhead, true> : k_pcg_spmv<kU, false>;
   while (!h.done) {
     for (int k = 0; k < 32; k++) {
-      k_pcg_spmv<<<d->nslab, d->S, 0, d->stream>>>(d->cols, d->vals, d->nrow, d->nnz, d->S, d->nslab, V.zpA,
-                                                   V.zpB, V.q, V.part, V.st, V.st + 1, self_sum);
+      spmv<<<d->nslab, d->S, 0, d->stream>>>(d->cols, d->vals, d->nrow, d->nnz, d->S, d->nslab, V.zpA, V.zpB, V.q,
+                                             V.part, V.st, V.st + 1, self_sum);
       if (!self_sum) k_reduce<<<1, 256, 0, d->stream>>>(V.part, d->nslab, RED_PQ, V.st + 1);
       k_pcg_update<<<d->nslab, d->S, 0, d->stream>>>(d->nrow, d->S, d->nslab, d->dinv, V.zpA, V.zpB, V.q, x,
                                                      V.r, V.part, V.st + 1, V.st, self_sum);
@@ -958,6 +1346,8 @@ void mm::ell_device_arrays(ell_device *d, int **cols, double **vals, double **di
   *S = d->S;
   *s = d->stream;
 }
+
+void mm::ell_device_set_band(ell_device *d, long long band) { d->band = band < d->nrow ? (int)band : 0; }
 
 int mm::ell_device_pcg_device(ell_device *d, ell_solver *solver, const double *b, double *x)
 {

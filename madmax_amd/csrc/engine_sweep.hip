@@ -32,8 +32,6 @@ namespace mm {
 
 namespace {
 
-typedef unsigned long long u64;
-
 // The tile of one workgroup: rank rk of the RVE's scw owns the interior planes
 // zs .. ze-1.  LDS plane s holds plane zs - 1 + s; inside a plane interior node
 // (ix, iy) (both counted from 0) sits at pos = 1 + (iy + 1) (nix + 1) + ix, so
@@ -162,20 +160,6 @@ __device__ __forceinline__ void sweep_strip(const TS *zr, int ps, const TS *dict
   sweep_key<TS, LP, 2>(Db, x, w);
 }
 
-// Words that the workgroups of a cluster pass to each other: 32 bits of
-// payload under the tag of the iteration that wrote them, one 64-bit relaxed
-// atomic access at agent scope each way.  A reader polls the word until it
-// carries the tag it waits for, so payload and readiness arrive together and
-// no fence (an L2 write-back or invalidate) is needed.  A word is rewritten
-// only after a sum over the cluster that its reader joined after reading it.
-__device__ __forceinline__ void put_word(u64 *p, unsigned tag, unsigned bits)
-{
-  __hip_atomic_store(p, ((u64)tag << 32) | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ u64 get_word(const u64 *p)
-{
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 // Bound on a wait in polls (half a minute or more).  A rank waits for the
 // slowest of its cluster to run one phase, or, before its first exchange, for a
 // rank that has no CU yet: until a running sweep ends.  A wait that reaches the
@@ -183,7 +167,7 @@ __device__ __forceinline__ u64 get_word(const u64 *p)
 constexpr int kSweepPolls = 1 << 25;
 
 struct SweepExch {
-  u64 *up, *down, *sum;  // top planes to the next rank, bottom planes to the previous, partial sums
+  word_t *up, *down, *sum;  // top planes to the next rank, bottom planes to the previous, partial sums
 };
 
 // A double moved between lanes (0 where no lane supplies one).
@@ -223,28 +207,27 @@ __device__ __forceinline__ void lanes_sum(double (&v)[NV], double *buf)
   }
 }
 
+// (A word that the ranks of a cluster exchange is rewritten only after a sum
+// over the cluster that its reader joined after reading it.)
+
 // Sums NV values over the workgroups of a cluster: lane 0 posts the workgroup's
 // own, every wave then collects all of them and adds them in rank order, so
 // that every lane of every rank has the same bits.  Collecting returns false
 // when the wait ran out.
 template <int NV>
-__device__ __forceinline__ void cluster_post(const double (&v)[NV], u64 *sum, int rk, unsigned tag)
+__device__ __forceinline__ void cluster_post(const double (&v)[NV], word_t *sum, int rk, unsigned tag)
 {
   if (threadIdx.x == 0)
 #pragma unroll
-    for (int i = 0; i < NV; i++) {
-      const u64 b = __builtin_bit_cast(u64, v[i]);
-      put_word(sum + rk * 8 + 2 * i, tag, (unsigned)b);
-      put_word(sum + rk * 8 + 2 * i + 1, tag, (unsigned)(b >> 32));
-    }
+    for (int i = 0; i < NV; i++) put_double(sum + rk * 8 + 2 * i, tag, v[i]);
 }
 template <int NV>
-__device__ __forceinline__ bool cluster_collect(double (&v)[NV], const u64 *sum, int cw, unsigned tag)
+__device__ __forceinline__ bool cluster_collect(double (&v)[NV], const word_t *sum, int cw, unsigned tag)
 {
   const int lane = threadIdx.x & 63;
   const bool mine = lane < cw * 2 * NV;
-  const u64 *src = sum + (mine ? (lane / (2 * NV)) * 8 + lane % (2 * NV) : 0);
-  u64 w = 0;
+  const word_t *src = sum + (mine ? (lane / (2 * NV)) * 8 + lane % (2 * NV) : 0);
+  word_t w = 0;
   int n = 0;
   for (;;) {
     if (mine) w = get_word(src);
@@ -258,7 +241,7 @@ __device__ __forceinline__ bool cluster_collect(double (&v)[NV], const u64 *sum,
     for (int r = 0; r < cw; r++) {
       const unsigned lo = __builtin_amdgcn_readlane(bits, r * 2 * NV + 2 * i);
       const unsigned hi = __builtin_amdgcn_readlane(bits, r * 2 * NV + 2 * i + 1);
-      s += __builtin_bit_cast(double, ((u64)hi << 32) | lo);
+      s += __builtin_bit_cast(double, ((word_t)hi << 32) | lo);
     }
     v[i] = s;
   }
@@ -266,49 +249,49 @@ __device__ __forceinline__ bool cluster_collect(double (&v)[NV], const u64 *sum,
 }
 
 // Publishes a node's three rows as the words of position pos of a plane.
-__device__ __forceinline__ void put_node(u64 *dst, int npos, int pos, unsigned tag, const float (&x)[3])
+__device__ __forceinline__ void put_node(word_t *dst, int npos, int pos, unsigned tag, const float (&x)[3])
 {
 #pragma unroll
   for (int d = 0; d < 3; d++) put_word(dst + d * npos + pos, tag, __builtin_bit_cast(unsigned, x[d]));
 }
-__device__ __forceinline__ void put_node(u64 *dst, int npos, int pos, unsigned tag, const double (&x)[3])
+__device__ __forceinline__ void put_node(word_t *dst, int npos, int pos, unsigned tag, const double (&x)[3])
 {
 #pragma unroll
   for (int d = 0; d < 3; d++) {
-    const u64 b = __builtin_bit_cast(u64, x[d]);
+    const word_t b = __builtin_bit_cast(word_t, x[d]);
     put_word(dst + (2 * d) * npos + pos, tag, (unsigned)b);
     put_word(dst + (2 * d + 1) * npos + pos, tag, (unsigned)(b >> 32));
   }
 }
-__device__ __forceinline__ void word_node(const u64 *w, float *dst)
+__device__ __forceinline__ void word_node(const word_t *w, float *dst)
 {
 #pragma unroll
   for (int d = 0; d < 3; d++) dst[d] = __builtin_bit_cast(float, (unsigned)w[d]);
 }
-__device__ __forceinline__ void word_node(const u64 *w, double *dst)
+__device__ __forceinline__ void word_node(const word_t *w, double *dst)
 {
 #pragma unroll
-  for (int d = 0; d < 3; d++) dst[d] = __builtin_bit_cast(double, (w[2 * d + 1] << 32) | (w[2 * d] & 0xffffffffull));
+  for (int d = 0; d < 3; d++) dst[d] = word_double(w[2 * d], w[2 * d + 1]);
 }
 
 // LDS planes 0 and np + 1 <- the words that the neighbouring ranks published
 // under `tag` (lo, hi: null at the tile's ends).  All words of a position are
 // asked for together, again until each carries the tag.
 template <typename TS>
-__device__ __forceinline__ bool get_planes(const SweepGeo &g, TS *zl, const u64 *lo, const u64 *hi, unsigned tag)
+__device__ __forceinline__ bool get_planes(const SweepGeo &g, TS *zl, const word_t *lo, const word_t *hi, unsigned tag)
 {
   constexpr int W = 3 * (int)(sizeof(TS) / 4);
   bool ok = true;
   for (int c = threadIdx.x; c < g.npos; c += kSweepLanes) {
     if (c % g.rsx == g.nix) continue;  // the zero column
-    u64 a[W], b[W];
+    word_t a[W], b[W];
     int n = 0;
     for (;;) {
       bool all = true;
 #pragma unroll
       for (int i = 0; i < W; i++) {
-        a[i] = lo ? get_word(lo + i * g.npos + c) : (u64)tag << 32;
-        b[i] = hi ? get_word(hi + i * g.npos + c) : (u64)tag << 32;
+        a[i] = lo ? get_word(lo + i * g.npos + c) : (word_t)tag << 32;
+        b[i] = hi ? get_word(hi + i * g.npos + c) : (word_t)tag << 32;
       }
 #pragma unroll
       for (int i = 0; i < W; i++) all = all && (unsigned)(a[i] >> 32) == tag && (unsigned)(b[i] >> 32) == tag;
@@ -387,8 +370,8 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
       for (int d = 0; d < 3; d++) p[j][l][d] = q[j][l][d] = dd[j][l][d] = (TS)0;
   }
   const int ps0 = g.pw * 3, words = sweep_words(g.npos, (int)sizeof(TS));
-  const u64 *lo = g.rk > 0 ? X.up + (long long)(g.rk - 1) * words : nullptr;
-  const u64 *hi = g.rk + 1 < g.cw ? X.down + (long long)g.rk * words : nullptr;
+  const word_t *lo = g.rk > 0 ? X.up + (long long)(g.rk - 1) * words : nullptr;
+  const word_t *hi = g.rk + 1 < g.cw ? X.down + (long long)g.rk * words : nullptr;
   double v2[2] = {0.0, 0.0};
   int n = 0;
 #pragma unroll 1
@@ -627,9 +610,9 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   __syncthreads();
   SweepExch X;
   const long long b0 = sweep_region(scalar(R->nslab), SN, K, tsz, fs, k);
-  X.up = reinterpret_cast<u64 *>((char *)P.p + b0);
-  X.down = reinterpret_cast<u64 *>((char *)P.q + b0);
-  X.sum = reinterpret_cast<u64 *>((char *)P.d + b0);
+  X.up = reinterpret_cast<word_t *>((char *)P.p + b0);
+  X.down = reinterpret_cast<word_t *>((char *)P.q + b0);
+  X.sum = reinterpret_cast<word_t *>((char *)P.d + b0);
   const double rz = N.rz[k], tgt = N.bnorm_in[k];
   int n;
   const SweepRun<TS> run{P, g, K, k, zl, dict, red, &s_fail, X, rz, tgt, sp.max_inner_its};

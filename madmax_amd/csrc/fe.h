@@ -78,6 +78,8 @@ int fe_get_phase(Fe *f, int *elem_type);
 // host matrix, its arrays, and the Jacobi-PCG on device vectors.
 int ell_device_alloc(int nrow, int nnz, int S, ell_device **out);
 void ell_device_arrays(ell_device *d, int **cols, double **vals, double **dinv, int *S, hipStream_t *s);
+// States that the rows of a slab span at most `band` columns.
+void ell_device_set_band(ell_device *d, long long band);
 int ell_device_pcg_device(ell_device *d, ell_solver *solver, const double *b, double *x);
 
 }  // namespace mm

@@ -652,6 +652,9 @@ int fe_create(const FeMeshDesc &d, Fe **out)
   {
     hipStream_t as;
     ell_device_arrays(f->A, &f->ell_cols, &f->ell_vals, &f->ell_dinv, &f->S, &as);
+    // the nodes of a slab's 256 rows (at most 87), and one node and its corner
+    // neighbours to either side; on the torus any column
+    if (!F.periodic) ell_device_set_band(f->A, 3LL * (87 + 2LL * (1 + F.nx + (long long)F.nx * F.ny)));
   }
   F.coords = f->coords;
   F.elem_mat = f->elem_mat;

@@ -90,4 +90,31 @@ __device__ inline void group_sum_rows(const double *p0, int nslab, int stride, d
   block_sum<NV>(out, lds);
 }
 
+// Words that workgroups of a running kernel pass to each other: 32 bits of
+// payload under a 32-bit tag, one 64-bit relaxed atomic access at agent scope
+// each way.  A reader polls the word until it carries the tag it waits for, so
+// payload and readiness arrive together and no fence (an L2 write-back or
+// invalidate) is needed.  A word may be rewritten once its reader is known to
+// have read it.
+typedef unsigned long long word_t;
+__device__ __forceinline__ void put_word(word_t *p, unsigned tag, unsigned bits)
+{
+  __hip_atomic_store(p, ((word_t)tag << 32) | bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ word_t get_word(const word_t *p)
+{
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A double as two words, and back.
+__device__ __forceinline__ void put_double(word_t *p, unsigned tag, double v)
+{
+  const word_t b = __builtin_bit_cast(word_t, v);
+  put_word(p, tag, (unsigned)b);
+  put_word(p + 1, tag, (unsigned)(b >> 32));
+}
+__device__ __forceinline__ double word_double(word_t lo, word_t hi)
+{
+  return __builtin_bit_cast(double, (hi << 32) | (lo & 0xffffffffull));
+}
+
 }  // namespace mm
