@@ -592,8 +592,8 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
 // the two launches per iteration that it replaces were bound by the host's
 // launches for small matrices and by reading 12 bytes per entry for larger ones.
 // Elasticity systems of N^3 elements with 81 slots, us per iteration, two launches
-// against this: 2,970 rows 22.7 and 8.6, 14,739 rows 23.6 and 9.6, 46,875 rows
-// 25.0 and 12.4, 89,373 rows 32.5 and 17.2.
+// against this: 2,970 rows 22.7 and 7.0, 14,739 rows 23.6 and 8.4, 46,875 rows
+// 25.0 and 11.4, 89,373 rows 32.5 and 17.1.
 //
 // All workgroups have to run at the same time.  They are at most 384, two to a CU
 // (one, 192, where the LDS of two does not fit): 192 CUs, which leaves 64 for

@@ -1477,8 +1477,11 @@ __global__ __launch_bounds__(256) void k_step_a_march_full(EngPtrs P, SolveParam
 // z -= alpha dinv q and the partial r.r, r.z, for the load cases that are
 // still iterating.  The residual itself is not stored: z = dinv r carries it
 // and r = z / dinv is formed in registers for the dot products.
+//
+// Bound by its six streams, so waves in flight count: unbounded the allocator
+// takes up to 190 VGPRs, two waves per SIMD; each bound is the most without spills.
 template <typename TS, int K>
-__global__ __launch_bounds__(256) void k_step_b(EngPtrs P, SolveParams sp)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TS) == 4 || K == 1 ? 8 : K < 7 ? 6 : 5))) void k_step_b(EngPtrs P, SolveParams sp)
 {
   using T2 = typename Pair<TS>::type;
   __shared__ double lds[2 * K * 16];
@@ -1513,15 +1516,13 @@ __global__ __launch_bounds__(256) void k_step_b(EngPtrs P, SolveParams sp)
   if (phase != PH_INNER) return;
   const unsigned skip = S->done_in;
   const int nslab = R->nslab;
-  double s1[K];
+  double s1 = 0.0;  // thread k: load case k
   if (R->big) {
-    for (int k = 0; k < K; k++) s1[k] = R->pq[k];  // summed by kernel S
+    if (tid < K) s1 = R->pq[tid];  // summed by kernel S
   } else {
-    group_sum_cols<K>(slab_part(P, R->first_slab).p, nslab, P.part_stride, 0, s1, lds);
+    s1 = group_sum_cols_lane<K>(slab_part(P, R->first_slab).p, nslab, P.part_stride, 0, lds);
   }
-  if (tid == 0)
-    for (int k = 0; k < K; k++)
-      s_alpha[k] = (((skip >> k) & 1u) || s1[k] == 0.0) ? 0.0 : S->rz[k] / s1[k];
+  if (tid < K) s_alpha[tid] = (((skip >> tid) & 1u) || s1 == 0.0) ? 0.0 : S->rz[tid] / s1;
   __syncthreads();
   const int n0 = P.slab_node0[slab];
   const int rows = min(RS, R->nrow - 3 * n0);
@@ -1594,10 +1595,10 @@ __global__ __launch_bounds__(256) void k_step_b(EngPtrs P, SolveParams sp)
       vu[K + k] = fma((double)ri, (double)zi, vu[K + k]);
     }
   }
-  block_sum<2 * K>(vu, lds);
-  if (tid == 0) {
+  const double sum = block_sum_lane<2 * K>(vu, lds);
+  if (tid < 2 * K) {
     const SlabPart part = slab_part(P, slab);
-    for (int i = 0; i < 2 * K; i++) part[K + i] = vu[i];
+    part[K + tid] = sum;
   }
 }
 

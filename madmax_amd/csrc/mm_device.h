@@ -6,31 +6,93 @@
 
 namespace mm {
 
-// Sums NV values over the block in a fixed order; the result is valid in
-// thread 0.  lds holds 16 doubles per value (blockDim.x <= 1024); its size
-// is checked at compile time.
-template <int NV, int L>
-__device__ inline void block_sum(double (&v)[NV], double (&lds)[L])
+// Two 32-bit halves of a double moved together.
+typedef unsigned halves_t __attribute__((ext_vector_type(2)));
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v)
 {
-  static_assert(L >= NV * 16, "block_sum: LDS scratch too small");
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-    for (int i = 0; i < NV; i++) v[i] += __shfl_down(v[i], off, 64);
+  const halves_t b = __builtin_bit_cast(halves_t, v);
+  halves_t m;
+  m.x = __builtin_amdgcn_update_dpp(0, b.x, CTRL, 0xf, 0xf, true);
+  m.y = __builtin_amdgcn_update_dpp(0, b.y, CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, m);
+}
+// a with its upper half of lanes replaced by b's lower half, plus b with its
+// lower half replaced by a's upper half (OFF 32; of each 32 lanes for OFF 16):
+// lane l < OFF has a[l] + a[l + OFF], lane l + OFF the same of b.
+template <int OFF>
+__device__ __forceinline__ double halve(double a, double b)
+{
+  const halves_t x = __builtin_bit_cast(halves_t, a), y = __builtin_bit_cast(halves_t, b);
+  halves_t lo, hi, p, q;
+  if constexpr (OFF == 32) {
+    lo = __builtin_amdgcn_permlane32_swap(x.x, y.x, false, false);
+    hi = __builtin_amdgcn_permlane32_swap(x.y, y.y, false, false);
+  } else {
+    lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+    hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+  }
+  p.x = lo.x;
+  p.y = hi.x;
+  q.x = lo.y;
+  q.y = hi.y;
+  return __builtin_bit_cast(double, p) + __builtin_bit_cast(double, q);
+}
+
+// Sums NV values over the block in a fixed order; returns the sum of value i in
+// thread i < NV.  lds holds 16 doubles per value (blockDim.x <= 1024); its size
+// is checked at compile time.  Each wave adds lanes 32, 16, 8, 4, 2 and 1 apart,
+// then lane i of wave 0 the waves' value i in order.  The first two steps put two and four values
+// beside each other in one register, so NV values take about 1.5 NV + 4 adds, and
+// the moves between lanes are DPP and permlane swaps in the vector unit: through
+// the LDS (ds_bpermute) a step's round trip is some 100 cycles.  An iteration of
+// k_pcg_resident, with four such sums in a row, took 8.6 us for 2,970 rows with
+// shuffles and a serial sum of the waves, and takes 7.0.
+template <int NV, int L>
+__device__ inline double block_sum_lane(const double (&v)[NV], double (&lds)[L])
+{
+  static_assert(L >= NV * 16 && NV <= 64, "block_sum: LDS scratch too small");
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
-  if (lane == 0)
 #pragma unroll
-    for (int i = 0; i < NV; i++) lds[i * 16 + wid] = v[i];
+  for (int i = 0; i < NV; i += 4) {
+    const double a = halve<32>(v[i], i + 1 < NV ? v[i + 1] : v[i]);
+    const double b = i + 2 < NV ? halve<32>(v[i + 2], i + 3 < NV ? v[i + 3] : v[i + 2]) : a;
+    double t = halve<16>(a, b);
+    t += dpp_move<0x108>(t);  // row_shl:8, 4, 2, 1: lane l takes lane l + 8 ... of its 16
+    t += dpp_move<0x104>(t);
+    t += dpp_move<0x102>(t);
+    t += dpp_move<0x101>(t);
+    // lanes 0, 32, 16 and 48: values i, i + 1, i + 2 and i + 3
+    const int k = i + (lane >> 5) + 2 * ((lane >> 4) & 1);
+    if ((lane & 15) == 0 && k < NV) lds[k * 16 + wid] = t;
+    __builtin_amdgcn_sched_barrier(0);  // (NV sums at a time would take many registers)
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
+  double s = 0.0;
+  if (threadIdx.x < 64) {
+    const double *p = lds + min(lane, NV - 1) * 16;
+    for (int w = 0; w < nw; w += 4) {  // (all 16 places of a value exist)
+      const double t[4] = {p[w], p[w + 1], p[w + 2], p[w + 3]};
 #pragma unroll
-    for (int i = 0; i < NV; i++) {
-      double s = 0.0;
-      for (int w = 0; w < nw; w++) s += lds[i * 16 + w];
-      v[i] = s;
+      for (int k = 0; k < 4; k++)
+        if (w + k < nw) s += t[k];
     }
   }
   __syncthreads();
+  return s;
+}
+// The same with all sums in v, valid in the first wave.
+template <int NV, int L>
+__device__ inline void block_sum(double (&v)[NV], double (&lds)[L])
+{
+  const halves_t b = __builtin_bit_cast(halves_t, block_sum_lane<NV>(v, lds));
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    halves_t r;
+    r.x = __builtin_amdgcn_readlane(b.x, i);
+    r.y = __builtin_amdgcn_readlane(b.y, i);
+    v[i] = __builtin_bit_cast(double, r);
+  }
 }
 
 // Run by every thread of a workgroup: sums partial values off .. off+NV-1
@@ -50,6 +112,19 @@ __device__ inline void group_sum_cols(const double *p0, int nslab, long long vst
 #pragma unroll
     for (int i = 0; i < NV; i++) out[i] += p0[(size_t)(off + i) * vstride + b];
   block_sum<NV>(out, lds);
+}
+// The sum of value i in thread i < NV.
+template <int NV, int L>
+__device__ inline double group_sum_cols_lane(const double *p0, int nslab, long long vstride, int off,
+                                             double (&lds)[L])
+{
+  double v[NV];
+#pragma unroll
+  for (int i = 0; i < NV; i++) v[i] = 0.0;
+  for (int b = threadIdx.x; b < nslab; b += blockDim.x)
+#pragma unroll
+    for (int i = 0; i < NV; i++) v[i] += p0[(size_t)(off + i) * vstride + b];
+  return block_sum_lane<NV>(v, lds);
 }
 
 // group_sum_cols four values at a time, the totals written to out[] (LDS,
