@@ -92,7 +92,8 @@ int ell_solve_pcg(ell_solver *solver, ell_matrix *m, double *b, double *x);
  * otherwise, since the GPU would read x at that index. */
 typedef struct ell_device_ ell_device;
 int ell_device_create(const ell_matrix *m, int slab_rows, ell_device **d);
-/* Re-uploads cols/vals of a matrix with the same shape. */
+/* Re-uploads cols/vals of a matrix with the same shape (row-major entries go
+ * through up to 64 MiB of device memory that the mirror keeps). */
 int ell_device_update(ell_device *d, const ell_matrix *m);
 /* Copies the device matrix back in the reference's row-major layout. */
 int ell_device_download(const ell_device *d, int *cols, double *vals);

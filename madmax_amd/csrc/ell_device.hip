@@ -19,7 +19,6 @@
 #include <cstring>
 #include <condition_variable>
 #include <mutex>
-#include <vector>
 
 #include "ell.h"
 #include "fe.h"
@@ -863,6 +862,97 @@ struct PcgVecs {
   unsigned *bar;   // grid-barrier words of k_pcg_fused
 };
 
+// ---- between the host's row-major layout and the slabs ----------------------
+// PLACE: rows of `rm` (row-major) into the slabs at `sl`, whose rows beyond `rows`
+// get `pad`; else the reverse.  64 rows by 16 slots per trip through the LDS, so
+// that both sides are read and written in runs of 64 to 512 bytes.  Bound by the
+// host's copies (28 GB/s in, 17 out), which move 12 bytes per entry as the loops
+// on the host did that this replaces: 14,688 rows of 81 slots up 6.5 ms before
+// and 0.55 now, down 3.3 and 0.87.
+constexpr int kPlaceSlots = 16;
+template <typename T, bool PLACE>
+__global__ __launch_bounds__(256) void k_ell_place(T *__restrict__ rm, int rows, int nnz, int S, T pad,
+                                                   T *__restrict__ sl)
+{
+  __shared__ T tile[64][kPlaceSlots + 1];
+  const int tid = threadIdx.x, per = S / 64;
+  const int r0 = blockIdx.x * 64;  // first row of the tile, S a multiple of 64
+  T *slab = sl + (long long)(blockIdx.x / per) * S * nnz + (blockIdx.x % per) * 64;
+  T *row = rm + (long long)r0 * nnz;
+  for (int j0 = blockIdx.y * kPlaceSlots; j0 < nnz; j0 += gridDim.y * kPlaceSlots) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int jr = tid % kPlaceSlots, rr = tid / kPlaceSlots + 16 * i;  // along a row
+      const int js = tid / 64 + 4 * i, rs = tid % 64;                    // along a slot
+      if (PLACE) {
+        tile[rr][jr] = (r0 + rr < rows && j0 + jr < nnz) ? row[(long long)rr * nnz + j0 + jr] : pad;
+      } else {
+        tile[rs][js] = (j0 + js < nnz) ? slab[(long long)(j0 + js) * S + rs] : pad;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int jr = tid % kPlaceSlots, rr = tid / kPlaceSlots + 16 * i;
+      const int js = tid / 64 + 4 * i, rs = tid % 64;
+      if (PLACE) {
+        if (j0 + js < nnz) slab[(long long)(j0 + js) * S + rs] = tile[rs][js];
+      } else {
+        if (r0 + rr < rows && j0 + jr < nnz) row[(long long)rr * nnz + j0 + jr] = tile[rr][jr];
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Of each row up to its first -1: the inverse of the diagonal (1 / 0 = inf where
+// there is none, like the reference), and the most columns that the rows of one
+// slab span into *band.
+__global__ void k_ell_scan(const int *__restrict__ cols, const double *__restrict__ vals, int nrow, int ncol, int nnz,
+                           int S, double *__restrict__ dinv, int *band)
+{
+  __shared__ int s_lo, s_hi;
+  const int lane = threadIdx.x;
+  const long long row = (long long)blockIdx.x * S + lane, base = (long long)blockIdx.x * S * nnz + lane;
+  if (lane == 0) {
+    s_lo = ncol;
+    s_hi = -1;
+  }
+  __syncthreads();
+  if (row < nrow) {
+    double d = 0.0;
+    int lo = ncol, hi = -1;
+    bool found = false, more = true;
+    for (int j0 = 0; j0 < nnz && more; j0 += 9) {
+      int c[9];
+#pragma unroll
+      for (int u = 0; u < 9; u++) c[u] = j0 + u < nnz ? cols[base + (long long)(j0 + u) * S] : -1;
+#pragma unroll
+      for (int u = 0; u < 9; u++) {
+        more = more && c[u] != -1;
+        if (!more) continue;
+        lo = min(lo, c[u]);
+        hi = max(hi, c[u]);
+        if (!found && c[u] == row) {
+          found = true;
+          d = vals[base + (long long)(j0 + u) * S];
+        }
+      }
+    }
+    dinv[row] = 1 / d;
+    atomicMin(&s_lo, lo);
+    atomicMax(&s_hi, hi);
+  }
+  __syncthreads();
+  if (lane == 0 && band) atomicMax(band, max(s_hi - s_lo + 1, 1));
+}
+
+__global__ void k_zero_int(int *p, int n)
+{
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i] = 0;
+}
+
 }  // namespace
 
 struct ell_device_ {
@@ -874,77 +964,76 @@ struct ell_device_ {
   double2 *zpA, *zpB;  // PCG {z, p} pairs
   IterState *st;
   unsigned *bar;
+  char *stage;     // row-major entries on their way in (null until the first upload)
   int band;        // most columns that a slab's rows span (0: not known)
   int fused_its;   // 0: two launches per PCG iteration; n > 0: k_pcg_fused, n iterations per launch
   int fused_grid;  // co-resident workgroups of k_pcg_fused (set with fused_its)
   hipStream_t stream;
 };
 
-static void host_diag_inv(const ell_matrix *m, std::vector<double> &dinv)
-{
-  dinv.resize(m->nrow);
-  for (int i = 0; i < m->nrow; i++) {
-    double d = 0.0;
-    if (i < m->ncol) {
-      const int *c = m->cols + (size_t)i * m->nnz;
-      for (int j = 0; j < m->nnz; j++) {
-        if (c[j] == -1) break;
-        if (c[j] == i) {
-          d = m->vals[(size_t)i * m->nnz + j];
-          break;
-        }
-      }
-    }
-    dinv[i] = 1 / d;  // like the reference, a missing diagonal gives inf
-  }
-}
-
 // The kernels read x[col] for every column id, so each must be -1 or a
 // column of the matrix (ell_add_val never stores anything else).
 static int check_cols(const ell_matrix *m)
 {
   const size_t n = (size_t)m->nrow * m->nnz;
-  for (size_t e = 0; e < n; e++) {
-    const int c = m->cols[e];
-    if (c < -1 || c >= m->ncol) {
-      fprintf(stderr, "madmax_amd: ell column id %d at slot %zu outside [-1, %d)\n", c, e, m->ncol);
-      return 1;
+  const int *c = m->cols;
+  const unsigned top = (unsigned)m->ncol;  // c + 1 as unsigned: 0 for -1, past top for what is out of range
+  unsigned bad = 0;
+  for (size_t e = 0; e < n; e++) bad |= (unsigned)c[e] + 1u > top;
+  if (!bad) return 0;
+  for (size_t e = 0; e < n; e++)
+    if ((unsigned)c[e] + 1u > top) {
+      fprintf(stderr, "madmax_amd: ell column id %d at slot %zu outside [-1, %d)\n", c[e], e, m->ncol);
+      break;
     }
-  }
-  return 0;
+  return 1;
+}
+
+// Slabs whose row-major entries (cols and vals, 12 bytes) are staged on the
+// device at a time: up to 64 MiB, at least one slab.
+static int stage_slabs(const ell_device *d)
+{
+  const size_t slab = (size_t)d->S * d->nnz * 12, most = ((size_t)64 << 20) / (slab ? slab : 1);
+  return most < 1 ? 1 : most < (size_t)d->nslab ? (int)most : d->nslab;
+}
+
+static dim3 place_grid(const ell_device *d, int slabs)
+{
+  const int strips = (d->nnz + kPlaceSlots - 1) / kPlaceSlots;
+  return dim3(slabs * (d->S / 64), strips < 1024 ? strips : 1024);
 }
 
 static int upload(ell_device *d, const ell_matrix *m)
 {
-  const size_t slots = (size_t)d->nslab * d->S * d->nnz;
-  std::vector<int> hc(slots, -1);
-  std::vector<double> hv(slots, 0.0);
-  for (int i = 0; i < m->nrow; i++) {
-    const size_t sb = (size_t)(i / d->S) * d->S * d->nnz, lane = i % d->S;
-    for (int j = 0; j < m->nnz; j++) {
-      hc[sb + (size_t)j * d->S + lane] = m->cols[(size_t)i * m->nnz + j];
-      hv[sb + (size_t)j * d->S + lane] = m->vals[(size_t)i * m->nnz + j];
+  if (d->nrow == 0 || d->nnz == 0) {
+    if (d->nrow) {
+      k_ell_scan<<<d->nslab, d->S, 0, d->stream>>>(d->cols, d->vals, d->nrow, d->ncol, 0, d->S, d->dinv, nullptr);
+      MM_HIP(hipGetLastError());
+      MM_HIP(hipStreamSynchronize(d->stream));
     }
+    return 0;
   }
-  d->band = 1;
-  for (int s = 0; s < d->nslab; s++) {
-    int lo = m->ncol, hi = -1;
-    const int end = (s + 1) * d->S < m->nrow ? (s + 1) * d->S : m->nrow;
-    for (size_t e = (size_t)s * d->S * m->nnz; e < (size_t)end * m->nnz; e++) {
-      const int c = m->cols[e];
-      if (c < 0) continue;
-      if (c < lo) lo = c;
-      if (c > hi) hi = c;
-    }
-    if (hi - lo + 1 > d->band) d->band = hi - lo + 1;
+  const int cs = stage_slabs(d);
+  const size_t chunk = (size_t)cs * d->S * d->nnz;
+  if (!d->stage) MM_HIP(hipMalloc((void **)&d->stage, chunk * 12 + 8));
+  double *sv = reinterpret_cast<double *>(d->stage);
+  int *sc = reinterpret_cast<int *>(sv + chunk), *band = sc + chunk;
+  k_zero_int<<<1, 64, 0, d->stream>>>(band, 1);
+  for (int s = 0; s < d->nslab; s += cs) {
+    const int slabs = d->nslab - s < cs ? d->nslab - s : cs;
+    const size_t r0 = (size_t)s * d->S, left = (size_t)d->nrow - r0;
+    const size_t rows = left < (size_t)slabs * d->S ? left : (size_t)slabs * d->S;
+    const size_t n = rows * d->nnz, at = r0 * d->nnz;
+    MM_HIP(hipMemcpyAsync(sc, m->cols + at, n * sizeof(int), hipMemcpyHostToDevice, d->stream));
+    MM_HIP(hipMemcpyAsync(sv, m->vals + at, n * sizeof(double), hipMemcpyHostToDevice, d->stream));
+    k_ell_place<int, true><<<place_grid(d, slabs), 256, 0, d->stream>>>(sc, (int)rows, d->nnz, d->S, -1, d->cols + at);
+    k_ell_place<double, true>
+        <<<place_grid(d, slabs), 256, 0, d->stream>>>(sv, (int)rows, d->nnz, d->S, 0.0, d->vals + at);
+    MM_HIP(hipGetLastError());
   }
-  std::vector<double> dinv;
-  host_diag_inv(m, dinv);
-  MM_HIP(hipMemcpyAsync(d->cols, hc.data(), slots * sizeof(int), hipMemcpyHostToDevice, d->stream));
-  MM_HIP(hipMemcpyAsync(d->vals, hv.data(), slots * sizeof(double), hipMemcpyHostToDevice, d->stream));
-  if (m->nrow)
-    MM_HIP(hipMemcpyAsync(d->dinv, dinv.data(), m->nrow * sizeof(double), hipMemcpyHostToDevice,
-                          d->stream));
+  k_ell_scan<<<d->nslab, d->S, 0, d->stream>>>(d->cols, d->vals, d->nrow, d->ncol, d->nnz, d->S, d->dinv, band);
+  MM_HIP(hipGetLastError());
+  MM_HIP(hipMemcpyAsync(&d->band, band, sizeof(int), hipMemcpyDeviceToHost, d->stream));
   MM_HIP(hipStreamSynchronize(d->stream));
   return 0;
 }
@@ -1016,19 +1105,29 @@ extern "C" int ell_device_update(ell_device *d, const ell_matrix *m)
 extern "C" int ell_device_download(const ell_device *d, int *cols, double *vals)
 {
   if (!d || !cols || !vals) return 1;
-  const size_t slots = (size_t)d->nslab * d->S * d->nnz;
-  std::vector<int> hc(slots);
-  std::vector<double> hv(slots);
-  MM_HIP(hipMemcpyAsync(hc.data(), d->cols, slots * sizeof(int), hipMemcpyDeviceToHost, d->stream));
-  MM_HIP(hipMemcpyAsync(hv.data(), d->vals, slots * sizeof(double), hipMemcpyDeviceToHost, d->stream));
-  MM_HIP(hipStreamSynchronize(d->stream));
-  for (int i = 0; i < d->nrow; i++) {
-    const size_t sb = (size_t)(i / d->S) * d->S * d->nnz, lane = i % d->S;
-    for (int j = 0; j < d->nnz; j++) {
-      cols[(size_t)i * d->nnz + j] = hc[sb + (size_t)j * d->S + lane];
-      vals[(size_t)i * d->nnz + j] = hv[sb + (size_t)j * d->S + lane];
-    }
+  if (d->nrow == 0 || d->nnz == 0) return 0;
+  const int cs = stage_slabs(d);
+  const size_t chunk = (size_t)cs * d->S * d->nnz;
+  char *stage = nullptr;  // of this call: downloads of one mirror may overlap
+  MM_HIP(hipMalloc((void **)&stage, chunk * 12));
+  double *sv = reinterpret_cast<double *>(stage);
+  int *sc = reinterpret_cast<int *>(sv + chunk);
+  hipError_t e = hipSuccess;
+  for (int s = 0; s < d->nslab && e == hipSuccess; s += cs) {
+    const int slabs = d->nslab - s < cs ? d->nslab - s : cs;
+    const size_t r0 = (size_t)s * d->S, left = (size_t)d->nrow - r0;
+    const size_t rows = left < (size_t)slabs * d->S ? left : (size_t)slabs * d->S;
+    const size_t n = rows * d->nnz, at = r0 * d->nnz;
+    k_ell_place<int, false><<<place_grid(d, slabs), 256, 0, d->stream>>>(sc, (int)rows, d->nnz, d->S, -1, d->cols + at);
+    k_ell_place<double, false>
+        <<<place_grid(d, slabs), 256, 0, d->stream>>>(sv, (int)rows, d->nnz, d->S, 0.0, d->vals + at);
+    e = hipGetLastError();
+    if (e == hipSuccess) e = hipMemcpyAsync(cols + at, sc, n * sizeof(int), hipMemcpyDeviceToHost, d->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(vals + at, sv, n * sizeof(double), hipMemcpyDeviceToHost, d->stream);
   }
+  if (e == hipSuccess) e = hipStreamSynchronize(d->stream);
+  (void)hipFree(stage);
+  MM_HIP(e);
   return 0;
 }
 
@@ -1439,6 +1538,7 @@ extern "C" int ell_device_destroy(ell_device *d)
   (void)hipFree(d->part);
   (void)hipFree(d->st);
   (void)hipFree(d->bar);
+  (void)hipFree(d->stage);
   if (d->stream) (void)hipStreamDestroy(d->stream);
   free(d);
   return 0;
