@@ -183,7 +183,8 @@ int micro_write_vtu(const char *name);
 typedef struct {
   int device;
   size_t hbm_budget;     /* bytes for the RVE arena (0 = 80% of free memory) */
-  int max_rves;          /* resident RVE slots (0 = 4096) */
+  int max_rves;          /* resident RVE slots (0 = 4096); on-chip sweeps of an
+                            engine of few slots spread over more of the GPU */
   int slab_nodes;        /* nodes per ELL slab = lanes per workgroup: 64, 128 or 256
                             (0 = 128); a slab holds 3 * slab_nodes rows */
   int nrhs;              /* load cases per RVE, 1..MM_MAX_RHS */
@@ -196,7 +197,7 @@ typedef struct {
   int steps_per_launch;  /* PCG iterations per launch / graph replay (whole
                             sweeps, at most six, while every RVE being solved
                             is small enough to be swept on chip: up to about
-                            32 x 32 elements across) */
+                            100^3 elements in FP32 and 85^3 in FP64) */
   int use_graph;         /* capture the steps in a hipGraph */
   int sync_every_step;   /* plain path: host reads the state after every PCG
                             iteration (no on-chip sweeps) */

@@ -221,7 +221,7 @@ struct mm_engine {
   bool act_dirty = true;
   long long act_n[2] = {0, 0}, tile_n[2] = {0, 0};
   int a_lds[2] = {0, 0}, a_slab[2] = {0, 0}, s_big[2] = {0, 0};
-  // resident sweep: per group g the workgroups' (slot, load case * 16 + rank)
+  // resident sweep: per group g the workgroups' (slot, load case * 256 + rank)
   // at units + g * unit_stride, [0].x their count, staged in st_units, and its
   // ticket counter (parts of act_list's, st_act's and rves' allocations)
   int2 *units = nullptr, *st_units = nullptr;
@@ -433,9 +433,9 @@ extern "C" int mm_engine_create(const mm_engine_config *cfg, mm_engine **out)
   const size_t nrows = (size_t)e->nslab_cap * e->rows_per_slab();
   const size_t slots = nrows * kW;
   // the active lists, then the resident sweep's units (a resident RVE has K *
-  // scw of them, scw at most kSweepMaxRanks and at most its slabs)
+  // scw of them, scw at most its slabs, and past kSweepFreeRanks an eighth)
   const size_t act_ints = 4 * ((size_t)e->nslab_cap + 1);
-  e->unit_stride = 1 + (size_t)e->K * std::min<size_t>((size_t)kSweepMaxRanks * e->rve_cap, (size_t)e->nslab_cap);
+  e->unit_stride = 1 + (size_t)e->K * std::min<size_t>((size_t)kSweepFreeRanks * e->rve_cap + (size_t)e->nslab_cap / 8, (size_t)e->nslab_cap);
   const size_t lists = act_ints * sizeof(int) + 2 * e->unit_stride * sizeof(int2);
   if (hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) != hipSuccess) {
     delete e;
@@ -764,49 +764,80 @@ static int march_lds_need(const mm_engine *e, const HostSlot &h)
                      : 0;
 }
 
-// Resident sweep of an RVE of nx x ny x nz nodes (RveDev::scw ..): the fewest
-// workgroups per load case whose share of the interior z-planes fits the lanes'
-// items and the LDS, cut into items of few enough planes that small RVEs still
-// occupy the lanes.  cw = 0 (kernels A and B) without an interior, where the
-// planes are too wide or too many, and for the engines whose steps are single
-// PCG iterations by request: sync_every_step reads the state after each,
-// profile_step_kernel times each one's kernel A.  Fixed by the RVE and the
+// Resident sweep of an RVE of nx x ny x nz nodes (RveDev::scw ..): the cheapest
+// split of the interior z-planes, and, if whole rows of planes are too many, of
+// the rows, whose shares fit the lanes' items and the LDS, cut into items of few
+// enough planes that small RVEs still occupy the lanes.  cw = 0 (kernels A and
+// B) without an interior, where nothing fits, and for the engines whose steps
+// are single PCG iterations by request: sync_every_step reads the state after
+// each, profile_step_kernel times each one's kernel A.  Fixed by the RVE and the
 // engine configuration alone.
 struct SweepTiling {
-  int cw = 0, lp = 0, nch = 0;
+  int cw = 0, ty = 1, lp = 0, nch = 0;
 };
+
+// Enters ty shares of the rows times cz of the planes into t if they fit and cost
+// less than its `best`; cost(workgroups, time).
+template <typename Cost>
+static void sweep_split(const mm_rve_spec &s, int tsz, int ty, int cz, const Cost &cost_of, double &best,
+                        SweepTiling &t)
+{
+  const int waves = kSweepLanes / 64, items = waves * kSweepItems;
+  const long long rows = (s.ney - 1 + ty - 1) / ty, L = (s.nez - 1 + cz - 1) / cz, cw = (long long)ty * cz;
+  const long long ns = sweep_strips(s.nex + 1, (int)rows + 2);
+  const long long plane = (long long)sweep_plane(s.nex + 1, (int)rows + 2) * 3 * tsz;
+  const long long fit = (kSweepMaxLds - sweep_dict_bytes(tsz)) / plane;  // planes
+  for (long long nch = 1; nch <= L && nch * ns <= items; nch++) {
+    const long long lp = (L + nch - 1) / nch;
+    if (lp > sweep_max_planes(tsz) || sweep_lds_planes((int)lp, (int)nch) > fit) continue;
+    // an iteration's time in planes of a strip: the longest wave's items, each
+    // with its latency, or the fullest SIMD's, and the barriers and sums
+    const double S = (double)(ns * nch), u = sweep_unroll((int)lp);
+    const double time = std::max(std::ceil(S / waves) * (u + 4.0), std::ceil(S / 4.0) * (u + 1.0)) +
+                        (cw > kSweepFreeRanks ? 18.0 : cw > 1 ? 12.0 : 4.0);
+    const double cost = cost_of((double)cw, time);
+    if (t.cw && cost >= best) continue;
+    best = cost;
+    t.cw = (int)cw;
+    t.ty = ty;
+    t.lp = (int)lp;
+    t.nch = (int)nch;
+  }
+}
+
 static SweepTiling sweep_tiling(const mm_engine *e, const mm_rve_spec &s, long long nslab)
 {
   SweepTiling t;
   if (e->cfg.sync_every_step || e->cfg.profile_step_kernel) return t;
-  const long long nix = s.nex - 1, niy = s.ney - 1, niz = s.nez - 1;
-  const int tsz = (int)e->tsz, waves = kSweepLanes / 64, most = waves * kSweepItems;
+  const int nix = s.nex - 1, niy = s.ney - 1, niz = s.nez - 1, tsz = (int)e->tsz;
   if (nix < 1 || niy < 1 || niz < 1 || nix > 4096 || niy > 4096) return t;
-  const long long ns = sweep_strips(s.nex + 1, s.ney + 1);
-  const long long plane = (long long)sweep_plane(s.nex + 1, s.ney + 1) * 3 * tsz;
-  const long long room = (kSweepMaxLds - sweep_dict_bytes(tsz)) / plane;  // planes that fit
-  double best = 0.0;
-  for (int cw = 1; cw <= kSweepMaxRanks && cw <= niz && cw <= nslab; cw++) {
-    const long long L = (niz + cw - 1) / cw;
-    for (long long nch = 1; nch <= L && nch * ns <= most; nch++) {
-      const long long lp = (L + nch - 1) / nch;
-      if (lp > sweep_max_planes(tsz) || sweep_lds_planes((int)lp, (int)nch) > room) continue;
-      // an iteration's time in planes of a strip: the longest wave's items, each
-      // with its latency, or the fullest SIMD's, and the barriers and sums;
-      // times the CUs it holds
-      const double S = (double)(ns * nch), u = sweep_unroll((int)lp);
-      const double cost =
-          cw * (std::max(std::ceil(S / waves) * (u + 4.0), std::ceil(S / 4.0) * (u + 1.0)) + (cw > 1 ? 12.0 : 4.0));
-      if (t.cw && cost >= best) continue;
-      best = cost;
-      t.cw = cw;
-      t.lp = (int)lp;
-      t.nch = (int)nch;
-    }
+  // (past kSweepFreeRanks, workgroups are bounded by the slabs for the unit lists' sake)
+  const int few = (int)std::min<long long>(kSweepFreeRanks, nslab);
+  const int many = (int)std::max<long long>(few, std::min<long long>(kSweepMaxRanks, nslab / 8));
+  const auto search = [&](int most, int ty0, int ty1, const auto &cost) {
+    double best = 0.0;
+    for (int ty = ty0; ty <= ty1 && ty <= most && ty <= niy; ty++)
+      for (int cz = 1; ty * cz <= most && cz <= niz; cz++) sweep_split(s, tsz, ty, cz, cost, best, t);
+  };
+  const double room = 256.0 / ((double)e->K * e->rve_cap);
+  if (room >= 2.0) {
+    // An engine of few RVEs leaves CUs idle: time counts, and, past the CUs that
+    // each cluster has when all of them are active, a little of their cost.  One
+    // load case, ms by kernels A and B, the cheapest split and this one: 30^3 4.7,
+    // 5.8 and 3.0; 48^3 7.9, 10.1 and 4.9; 60 x 52 x 50 11.3, 12.5 and 6.5.
+    search(many, 1, niy, [&](double cw, double time) { return time * std::sqrt(std::sqrt(std::max(1.0, cw / room))); });
+  } else if (e->K == 1) {
+    // Otherwise the CUs' time, but a lone cell must not lose against the launches
+    // of kernels A and B, 23 us an iteration, 40 of this unit.
+    search(many, 1, niy, [](double cw, double time) { return cw * time + std::max(0.0, time - 38.0) * 1e6; });
+  } else {
+    const auto cus = [](double cw, double time) { return cw * time; };
+    for (int ty = 1; ty <= few && !t.cw; ty++) search(few, ty, ty, cus);
+    if (!t.cw) search(many, 1, niy, cus);
   }
-  if (t.cw > 1) {  // the exchanged words must fit the RVE's part of p, q and d
+  if (t.cw > 1) {  // the exchanged words must fit the RVE's part of d
     const long long part = nslab * e->rows_per_slab() * (long long)tsz;
-    if (8LL * (t.cw - 1) * sweep_words(sweep_positions(s.nex + 1, s.ney + 1), tsz) > part || 8LL * kSweepSumWords > part) t = SweepTiling();
+    if (8LL * ((long long)nix * niy * niz * (tsz / 4) + sweep_sum_words(t.cw)) > part) t = SweepTiling();
   }
   return t;
 }
@@ -853,6 +884,7 @@ static void fill_state(const mm_engine *e, const HostSlot &h, RveDev *st, int wa
   st->mncg = mt.mncg;
   const SweepTiling sw = sweep_tiling(e, s, h.nslab);
   st->scw = sw.cw;
+  st->sty = sw.ty;
   st->slp = sw.lp;
   st->snch = sw.nch;
   st->big = (sw.cw == 0 && h.nslab >= e->cfg.big_slabs) ? 1 : 0;
@@ -1033,12 +1065,14 @@ static int update_active(mm_engine *e)
   long long n[2] = {0, 0}, nt[2] = {0, 0};
   int lds[2] = {0, 0}, slab_mode[2] = {0, 0}, big[2] = {0, 0};
   std::vector<std::pair<long long, int2>> res[2];  // (nodes, (slot, ranks)) of the resident sweeps
-  int g = 0;
+  int half = 0;
   for (auto &r : runs) {
     const HostSlot &h = e->slots[r.second];
-    if (g == 0 && ngroup == 2 && n[0] > 0 && 2 * n[0] >= total) g = 1;
-    for (long long b = 0; b < h.nslab; b++) e->st_act[g * stride + 1 + n[g]++] = (int)(r.first + b);
+    if (half == 0 && ngroup == 2 && n[0] > 0 && 2 * n[0] >= total) half = 1;
     const SweepTiling sw = sweep_tiling(e, h.req.rve, h.nslab);
+    // clusters that need most of the CUs at once stay in one chain of launches
+    const int g = sw.cw > kSweepFreeRanks ? 0 : half;
+    for (long long b = 0; b < h.nslab; b++) e->st_act[g * stride + 1 + n[g]++] = (int)(r.first + b);
     if (sw.cw > 0) {
       res[g].push_back({h.nrow / 3, make_int2(r.second, sw.cw)});
       continue;
@@ -1069,7 +1103,7 @@ static int update_active(mm_engine *e)
     long long nu = 0;
     for (auto &r : res[q])
       for (int k = 0; k < e->slots[r.second.x].req.nload; k++)
-        for (int c = 0; c < r.second.y; c++) un[1 + nu++] = make_int2(r.second.x, k * kSweepMaxRanks + c);
+        for (int c = 0; c < r.second.y; c++) un[1 + nu++] = make_int2(r.second.x, k * kSweepUnitRanks + c);
     un[0] = make_int2((int)nu, 0);
     if (q < ngroup)
       MM_HIP(hipMemcpyAsync(e->units + q * e->unit_stride, un, (size_t)(nu + 1) * sizeof(int2),

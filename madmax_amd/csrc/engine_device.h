@@ -29,6 +29,23 @@ __device__ __forceinline__ SlabPart slab_part(const EngPtrs &P, int slab)
   return SlabPart{P.part + slab, P.part_stride};
 }
 
+// The words of load case k of a resident sweep (sweep_region), ni interior nodes.
+struct SweepWords {
+  word_t *w[3], *sum;
+};
+template <typename TS>
+__device__ __forceinline__ SweepWords sweep_words(const EngPtrs &P, int nslab, int K, int first_slab, int k,
+                                                  long long ni)
+{
+  const long long b0 = sweep_region(nslab, P.SN, K, (int)sizeof(TS), first_slab, k);
+  SweepWords X;
+  X.w[0] = reinterpret_cast<word_t *>((char *)P.q + b0);
+  X.w[1] = reinterpret_cast<word_t *>((char *)P.p + b0);
+  X.w[2] = reinterpret_cast<word_t *>((char *)P.d + b0);
+  X.sum = X.w[2] + ni * (long long)(sizeof(TS) / 4);
+  return X;
+}
+
 // Start of a refinement sweep from the reduced residual norms s4 =
 // {||r64||^2, ||r||^2, r.z, ||r_cold||^2} per load case (FP64 residual r64,
 // its rounding r, cold-start right-hand side r_cold).

@@ -1496,16 +1496,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TS) 
   const int scw = R->scw, phase = S->phase;  // read together
   if (scw > 0) {
     // a resident sweep has run to its end: the count is the largest of the
-    // load cases' (as inner_check counts), and the residual comes next
+    // load cases' (as inner_check counts), and the residual comes next.  Load
+    // cases whose cluster did not meet are left for the next launch.
     if (slab == R->first_slab && tid == 0) {
       SolveState N = *S;
       if (N.phase == PH_INNER) {
-        N.its = 0;
-        for (int k = 0; k < K; k++)
-          if (!((N.done_in >> k) & 1u)) N.its = max(N.its, R->lits[k]);
-        N.its_total += N.its;
-        N.sweep += 1;
-        N.phase = PH_RES;
+        bool left = false;
+        for (int k = 0; k < K; k++) {
+          if ((N.done_in >> k) & 1u) continue;
+          if (scw > kSweepFreeRanks) {
+            const long long ni = (long long)(R->nx - 2) * (R->ny - 2) * (R->nz - 2);
+            word_t *meet = sweep_words<TS>(P, R->nslab, K, R->first_slab, k, ni).sum + 16 * scw;
+            const bool ran = meet[1] == kMeetGo;
+            meet[0] = meet[1] = 0;
+            if (!ran) {
+              left = true;
+              continue;
+            }
+            N.done_in |= 1u << k;
+          }
+          N.its = max(N.its, R->lits[k]);
+        }
+        if (!left) {
+          N.its_total += N.its;
+          N.sweep += 1;
+          N.phase = PH_RES;
+        }
       }
       R->st[1] = N;
       *P.ticket = 0u;  // for the next resident sweep
@@ -1619,20 +1635,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TS) 
 template <typename TS, int K>
 __device__ void sweep_words_zero(const EngPtrs &P, const RveDev *R, int slab)
 {
-  typedef unsigned long long u64;
-  const int ls = slab - R->first_slab;
-  const int nw = (R->scw - 1) * sweep_words(sweep_positions(R->nx, R->ny), (int)sizeof(TS));
+  const int ls = slab - R->first_slab, bd = (int)blockDim.x, cw = R->scw, cz = cw / R->sty;
+  const int nixy = (R->nx - 2) * (R->ny - 2), niz = R->nz - 2, ni = nixy * niz;
+  // the planes that ranks exchange: the first and last of each share, or, where
+  // the rows are shared too, all
+  const int nw = R->sty > 1 ? ni : 2 * cz * nixy;
 #pragma unroll 1
   for (int k = 0; k < K; k++) {
-    const long long b0 = sweep_region(R->nslab, P.SN, K, (int)sizeof(TS), R->first_slab, k);
-    u64 *up = reinterpret_cast<u64 *>((char *)P.p + b0), *down = reinterpret_cast<u64 *>((char *)P.q + b0);
-    for (int i = ls * (int)blockDim.x + (int)threadIdx.x; i < nw; i += R->nslab * (int)blockDim.x) {
-      up[i] = 0;
-      down[i] = 0;
+    const SweepWords X = sweep_words<TS>(P, R->nslab, K, R->first_slab, k, ni);
+    for (int i = ls * bd + (int)threadIdx.x; i < nw; i += R->nslab * bd) {
+      int at = i;
+      if (R->sty == 1) {
+        const int pl = i / nixy, r = pl >> 1;
+        at = ((pl & 1) ? (r + 1) * niz / cz - 1 : r * niz / cz) * nixy + i - pl * nixy;
+      }
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int h = 0; h < (int)(sizeof(TS) / 4); h++) X.w[d][(long long)h * ni + at] = 0;
     }
     if (ls == 0)
-      for (int i = threadIdx.x; i < kSweepSumWords; i += blockDim.x)
-        reinterpret_cast<u64 *>((char *)P.d + b0)[i] = 0;
+      for (int i = threadIdx.x; i < sweep_sum_words(cw); i += bd) X.sum[i] = 0;
   }
 }
 

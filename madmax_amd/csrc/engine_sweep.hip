@@ -1,9 +1,10 @@
 // engine_sweep.hip -- a whole PCG sweep of an RVE load case on chip.
 //
 // One workgroup, or a cluster of scw workgroups that split the RVE's interior
-// z-planes, runs every PCG iteration of one sweep of one load case in a single
-// launch: z in LDS (its own planes and one halo plane either side), p, q and d
-// in registers, the dictionary blocks in LDS.  See RveDev::scw for which RVEs.
+// z-planes and, where whole planes are too much, their rows, runs every PCG
+// iteration of one sweep of one load case in a single launch: z in LDS (the
+// tile's own and the nodes around it), p, q and d in registers, the dictionary
+// blocks in LDS.  See RveDev::scw for which RVEs.
 //
 // Why: kernels A and B move eleven vector passes per iteration through HBM and
 // are two to four launches; here an iteration moves only the planes between
@@ -21,7 +22,10 @@
 //   the dictionary's LDS reads);
 //   waiting for r.r / r.z before w = A z instead of behind it: 31 us.
 // Whole solves (rtol 1e-10): 128 x 30^3 tangents 187 -> 75 ms, 64 uneven cells
-// 8^3 .. 32^3 50 -> 14 ms, 24 x 20^3 in FP64 25.5 -> 7.1 ms, one 10^3 4.7 -> 1.2.
+// 8^3 .. 32^3 50 -> 14 ms, 24 x 20^3 in FP64 25.5 -> 7.1 ms, one 10^3 4.7 -> 1.1.
+// Sharing the rows: 32 x 33 x 36 x 40 tangents 122 -> 47 ms, 4 x 60^3 93 -> 38; one
+// load case of 48^3 7.9 -> 4.9 ms, of 100^3 (195 workgroups) 50 -> 18, 74 us an
+// iteration by kernels A, S, B and R and 26 here.
 #include <hip/hip_runtime.h>
 
 #include "engine_device.h"
@@ -32,17 +36,20 @@ namespace mm {
 
 namespace {
 
-// The tile of one workgroup: rank rk of the RVE's scw owns the interior planes
-// zs .. ze-1.  LDS plane s holds plane zs - 1 + s; inside a plane interior node
-// (ix, iy) (both counted from 0) sits at pos = 1 + (iy + 1) (nix + 1) + ix, so
-// that a zero column between the rows and a zero row before and after them
-// stand for the boundary nodes, whose z is zero in every correction solve.
+// The tile of one workgroup: rank rk = rz sty + ry of the RVE's scw owns the
+// interior planes zs .. ze-1 and of each the nr interior rows from ys (counted
+// from 0).  LDS plane s holds plane zs - 1 + s; inside a plane, node (ix, iy) of
+// the tile (both counted from 0) sits at pos = 1 + (iy + 1) (nix + 1) + ix, so
+// that a zero column lies between the rows, and a row before and after them
+// holds the neighbouring tiles' or is zero.  Zeros stand for the boundary nodes,
+// whose z is zero in every correction solve.
 struct SweepGeo {
-  int nix, ncol, rsx, pw;  // interior columns per row, per plane; row and plane strides
-  int npos, nstrip;        // positions of a plane's rows with their zero column; strips of them
-  int zs, ze, np, rk, cw;
-  int lp, nch;             // planes per item; items per column
-  int nx, nxy, fs;
+  int nix, rsx, pw;  // interior columns per row; row and plane strides
+  int npos, nstrip;  // positions of a plane's rows with their zero column; strips of them
+  int zs, ze, np, ys, nr, rk, cw;
+  bool zlo, zhi, ylo, yhi;  // neighbouring ranks
+  int lp, nch;              // planes per item; items per column
+  int nx, nxy, nixy, ni, fs;
 };
 
 // The RVE's fields are the same in every lane but read through vector memory;
@@ -53,18 +60,26 @@ __device__ __forceinline__ SweepGeo sweep_geo(const RveDev *R, int rk)
 {
   SweepGeo g;
   g.nx = scalar(R->nx);
-  const int ny = scalar(R->ny), niz = scalar(R->nz) - 2;
+  const int ny = scalar(R->ny), niz = scalar(R->nz) - 2, ty = scalar(R->sty);
   g.nix = g.nx - 2;
-  g.ncol = g.nix * (ny - 2);
   g.rsx = g.nix + 1;
-  g.pw = sweep_plane(g.nx, ny);
-  g.npos = g.rsx * (ny - 2);
-  g.nstrip = sweep_strips(g.nx, ny);
   g.rk = rk;
   g.cw = scalar(R->scw);
-  g.zs = 1 + rk * niz / g.cw;
-  g.ze = 1 + (rk + 1) * niz / g.cw;
+  const int cz = g.cw / ty, rz = rk / ty, ry = rk - rz * ty;
+  g.zs = 1 + rz * niz / cz;
+  g.ze = 1 + (rz + 1) * niz / cz;
   g.np = g.ze - g.zs;
+  g.ys = ry * (ny - 2) / ty;
+  g.nr = (ry + 1) * (ny - 2) / ty - g.ys;
+  g.zlo = rz > 0;
+  g.zhi = rz + 1 < cz;
+  g.ylo = ry > 0;
+  g.yhi = ry + 1 < ty;
+  g.pw = sweep_plane(g.nx, g.nr + 2);
+  g.npos = g.rsx * g.nr;
+  g.nstrip = sweep_strips(g.nx, g.nr + 2);
+  g.nixy = g.nix * (ny - 2);
+  g.ni = g.nixy * niz;
   g.lp = scalar(R->slp);
   g.nch = scalar(R->snch);
   g.nxy = g.nx * ny;
@@ -166,10 +181,6 @@ __device__ __forceinline__ void sweep_strip(const TS *zr, int ps, const TS *dict
 // bound ends the sweep without an update.
 constexpr int kSweepPolls = 1 << 25;
 
-struct SweepExch {
-  word_t *up, *down, *sum;  // top planes to the next rank, bottom planes to the previous, partial sums
-};
-
 // A double moved between lanes (0 where no lane supplies one).
 template <int CTRL, int ROWS>
 __device__ __forceinline__ double dpp_get(double v)
@@ -248,19 +259,81 @@ __device__ __forceinline__ bool cluster_collect(double (&v)[NV], const word_t *s
   return true;
 }
 
-// Publishes a node's three rows as the words of position pos of a plane.
-__device__ __forceinline__ void put_node(word_t *dst, int npos, int pos, unsigned tag, const float (&x)[3])
+// The same for clusters of more ranks than fit a wave's lanes: lane r collects
+// rank r's and the workgroup adds them (lanes_sum, a barrier).
+template <int NV>
+__device__ __forceinline__ bool cluster_collect_many(double (&v)[NV], const word_t *sum, int cw, unsigned tag,
+                                                     double *buf)
+{
+  const bool mine = (int)threadIdx.x < cw;
+  const word_t *src = sum + (mine ? (int)threadIdx.x * 8 : 0);
+  word_t w[2 * NV];
+  bool ok = true;
+  int n = 0;
+  for (;;) {
+    bool all = true;
+#pragma unroll
+    for (int i = 0; i < 2 * NV; i++) w[i] = get_word(src + i);
+#pragma unroll
+    for (int i = 0; i < 2 * NV; i++) all = all && (unsigned)(w[i] >> 32) == tag;
+    if (!mine || all) break;
+    if (++n > kSweepPolls) {
+      ok = false;
+      break;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NV; i++) v[i] = mine ? word_double(w[2 * i], w[2 * i + 1]) : 0.0;
+  lanes_sum<NV>(v, buf);
+  return ok;
+}
+template <int NV>
+__device__ __forceinline__ bool cluster_sum(double (&v)[NV], const word_t *sum, int cw, unsigned tag, double *buf)
+{
+  if (cw > kSweepFreeRanks) return cluster_collect_many<NV>(v, sum, cw, tag, buf);
+  return cluster_collect<NV>(v, sum, cw, tag);
+}
+
+// A cluster of many ranks meets before its first exchange: the last to arrive
+// lets it go; the first calls it off when ranks stay away for long, in which
+// case all leave and the sweep is tried again by the next launch.  The wait
+// covers the clusters before it in this launch that still run; it differs from
+// one attempt to the next, so that two clusters on different streams that keep
+// each other from the CUs do not go on doing so.  Run by one lane.
+constexpr int kMeetPolls = 1 << 14;  // some 10 ms, plus as much at random
+__device__ __forceinline__ bool cluster_meet(word_t *meet, int cw)
+{
+  const word_t n = __hip_atomic_fetch_add(&meet[0], (word_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  word_t none = 0;
+  if (n + 1 == (word_t)cw)
+    __hip_atomic_compare_exchange_strong(&meet[1], &none, kMeetGo, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_AGENT);
+  const int most = n == 0 ? kMeetPolls + (int)(clock64() & (kMeetPolls - 1)) : 4 * kMeetPolls;
+  for (int i = 0;; i++) {
+    const word_t m = get_word(&meet[1]);
+    if (m != 0) return m == kMeetGo;
+    if (i >= most) {
+      none = 0;
+      __hip_atomic_compare_exchange_strong(&meet[1], &none, kMeetOff, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __builtin_amdgcn_s_sleep(8);
+  }
+}
+
+// Publishes a node's three rows as the words of interior node at.
+__device__ __forceinline__ void put_node(const SweepWords &X, int ni, int at, unsigned tag, const float (&x)[3])
 {
 #pragma unroll
-  for (int d = 0; d < 3; d++) put_word(dst + d * npos + pos, tag, __builtin_bit_cast(unsigned, x[d]));
+  for (int d = 0; d < 3; d++) put_word(X.w[d] + at, tag, __builtin_bit_cast(unsigned, x[d]));
 }
-__device__ __forceinline__ void put_node(word_t *dst, int npos, int pos, unsigned tag, const double (&x)[3])
+__device__ __forceinline__ void put_node(const SweepWords &X, int ni, int at, unsigned tag, const double (&x)[3])
 {
 #pragma unroll
   for (int d = 0; d < 3; d++) {
     const word_t b = __builtin_bit_cast(word_t, x[d]);
-    put_word(dst + (2 * d) * npos + pos, tag, (unsigned)b);
-    put_word(dst + (2 * d + 1) * npos + pos, tag, (unsigned)(b >> 32));
+    put_word(X.w[d] + at, tag, (unsigned)b);
+    put_word(X.w[d] + ni + at, tag, (unsigned)(b >> 32));
   }
 }
 __device__ __forceinline__ void word_node(const word_t *w, float *dst)
@@ -274,35 +347,71 @@ __device__ __forceinline__ void word_node(const word_t *w, double *dst)
   for (int d = 0; d < 3; d++) dst[d] = word_double(w[2 * d], w[2 * d + 1]);
 }
 
-// LDS planes 0 and np + 1 <- the words that the neighbouring ranks published
-// under `tag` (lo, hi: null at the tile's ends).  All words of a position are
-// asked for together, again until each carries the tag.
+// The nodes beside the tile <- the words that the neighbouring ranks published
+// under `tag`: the planes below and above with the rows beside the tile, then of
+// the tile's own planes the rows before and after it.  U nodes of either side
+// per trip, all their words asked for together, again until each carries the tag.
 template <typename TS>
-__device__ __forceinline__ bool get_planes(const SweepGeo &g, TS *zl, const word_t *lo, const word_t *hi, unsigned tag)
+__device__ __forceinline__ bool get_halo(const SweepGeo &g, TS *zl, const SweepWords &X, unsigned tag)
 {
-  constexpr int W = 3 * (int)(sizeof(TS) / 4);
+  constexpr int H = (int)(sizeof(TS) / 4), W = 3 * H, U = H == 1 ? 2 : 1;
+  const int r0 = g.ylo ? 0 : 1, n1 = (g.zlo || g.zhi) ? (g.nr + (g.ylo ? 1 : 0) + (g.yhi ? 1 : 0)) * g.nix : 0;
+  const int n = n1 + ((g.ylo || g.yhi) ? g.np * g.nix : 0);
+  const word_t none = (word_t)tag << 32;
   bool ok = true;
-  for (int c = threadIdx.x; c < g.npos; c += kSweepLanes) {
-    if (c % g.rsx == g.nix) continue;  // the zero column
-    word_t a[W], b[W];
-    int n = 0;
+  int c0 = threadIdx.x;
+  asm volatile("" : "+v"(c0));  // the places are formed here, not kept from one iteration to the next
+  for (; c0 < n; c0 += U * kSweepLanes) {
+    int at[U], dst[U], dat[U], ddst[U];  // the lower side's word and place, the upper side's distance from them
+    bool lo[U], hi[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      int c = c0 + u * kSweepLanes;
+      const bool in = c < n, plane = c < n1;
+      if (!plane) c -= n1;
+      const int r = c / g.nix, ix = c - r * g.nix;
+      if (plane) {  // row r0 + r of planes 0 and np + 1
+        at[u] = ix + g.nix * (g.ys + r0 + r - 1) + g.nixy * (g.zs - 2);
+        dst[u] = 1 + (r0 + r) * g.rsx + ix;
+        dat[u] = (g.np + 1) * g.nixy;
+        ddst[u] = (g.np + 1) * g.pw;
+      } else {  // rows 0 and nr + 1 of plane r + 1
+        at[u] = ix + g.nix * (g.ys - 1) + g.nixy * (g.zs - 1 + r);
+        dst[u] = 1 + ix + (r + 1) * g.pw;
+        dat[u] = (g.nr + 1) * g.nix;
+        ddst[u] = (g.nr + 1) * g.rsx;
+      }
+      lo[u] = in && (plane ? g.zlo : g.ylo);
+      hi[u] = in && (plane ? g.zhi : g.yhi);
+    }
+    word_t a[U][W], b[U][W];
+    int m = 0;
     for (;;) {
       bool all = true;
 #pragma unroll
-      for (int i = 0; i < W; i++) {
-        a[i] = lo ? get_word(lo + i * g.npos + c) : (word_t)tag << 32;
-        b[i] = hi ? get_word(hi + i * g.npos + c) : (word_t)tag << 32;
-      }
+      for (int u = 0; u < U; u++)
 #pragma unroll
-      for (int i = 0; i < W; i++) all = all && (unsigned)(a[i] >> 32) == tag && (unsigned)(b[i] >> 32) == tag;
+        for (int i = 0; i < W; i++) {
+          const word_t *w = X.w[i / H] + (long long)(i % H) * g.ni + at[u];
+          a[u][i] = lo[u] ? get_word(w) : none;
+          b[u][i] = hi[u] ? get_word(w + dat[u]) : none;
+        }
+#pragma unroll
+      for (int u = 0; u < U; u++)
+#pragma unroll
+        for (int i = 0; i < W; i++)
+          all = all && (unsigned)(a[u][i] >> 32) == tag && (unsigned)(b[u][i] >> 32) == tag;
       if (all) break;
-      if (++n > kSweepPolls) {
+      if (++m > kSweepPolls) {
         ok = false;
         break;
       }
     }
-    if (lo) word_node(a, zl + (c + g.rsx + 1) * 3);
-    if (hi) word_node(b, zl + ((g.np + 1) * g.pw + c + g.rsx + 1) * 3);
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (lo[u]) word_node(a[u], zl + dst[u] * 3);
+      if (hi[u]) word_node(b[u], zl + (dst[u] + ddst[u]) * 3);
+    }
   }
   return ok;
 }
@@ -312,8 +421,8 @@ __device__ __forceinline__ bool get_planes(const SweepGeo &g, TS *zl, const word
 // the lane has a node there (if not it only supplies z to its neighbours).  Strip st of the tile is nstrip
 // strips per run of planes; lanes 1 .. 62 of its wave work.
 struct SweepItem {
-  int lds, node, cnt, h;
-  bool on;
+  int lds, node, cnt, h, word;  // word: the first node's among the interior nodes
+  bool on, edge;                // edge: in a row that a neighbouring rank reads
 };
 __device__ __forceinline__ SweepItem sweep_item(const SweepGeo &g, int tid, int j)
 {
@@ -326,14 +435,10 @@ __device__ __forceinline__ SweepItem sweep_item(const SweepGeo &g, int tid, int 
   it.on = it.cnt > 0 && ix < g.nix && pos < g.npos && ln >= 1 && ln <= kSweepStrip;
   it.h = h;
   it.lds = (h < g.nch ? h * g.lp : 0) * g.pw + min(pos, g.npos - 1) + g.rsx + 1;
-  it.node = it.on ? (ix + 1) + (iy + 1) * g.nx + zf * g.nxy : 1 + g.nx + g.nxy;  // any interior one if off
+  it.node = it.on ? (ix + 1) + (g.ys + iy + 1) * g.nx + zf * g.nxy : 1 + g.nx + g.nxy;  // any interior one if off
+  it.word = ix + g.nix * (g.ys + iy) + g.nixy * (zf - 1);
+  it.edge = (g.ylo && iy == 0) || (g.yhi && iy == g.nr - 1);
   return it;
-}
-
-// Position of an item's column from its LDS offset.
-__device__ __forceinline__ int item_pos(const SweepGeo &g, int z0, int h)
-{
-  return z0 / 3 - h * g.lp * g.pw - g.rsx - 1;
 }
 
 // The sweep of one load case on this workgroup's tile; zl holds z = dinv r of
@@ -345,20 +450,22 @@ __device__ __forceinline__ int item_pos(const SweepGeo &g, int z0, int h)
 // the grouping of the dot products differs.  Returns the iterations taken.
 template <typename TS, int LP>
 __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, int K, int k, TS *zl,
-                                          const TS *dict, double *red, int *s_fail, const SweepExch &X, double rz,
+                                          const TS *dict, double *red, int *s_fail, const SweepWords &X, double rz,
                                           double tgt, int max_its)
 {
   constexpr int NI = kSweepItems;
   const int tid = threadIdx.x, fs = g.fs, SN = P.SN, RS = 3 * SN;
   TS p[NI][LP][3], q[NI][LP][3], dd[NI][LP][3];
-  int z0[NI], d0[NI], cnt[NI], hc[NI];
-  bool on[NI];
+  int z0[NI], d0[NI], cnt[NI], hc[NI], wd[NI];
+  bool on[NI], edge[NI];
 #pragma unroll
   for (int j = 0; j < NI; j++) {
     const SweepItem it = sweep_item(g, tid, j);
     cnt[j] = scalar(it.cnt);
     hc[j] = scalar(it.h);
     on[j] = it.on;
+    edge[j] = it.edge;
+    wd[j] = it.word;
     z0[j] = it.lds * 3;
     // the phases do not vary along z: one pattern per column; lanes without a
     // node take the zero entry, so that their q, r and dot products are zero
@@ -369,9 +476,8 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
 #pragma unroll
       for (int d = 0; d < 3; d++) p[j][l][d] = q[j][l][d] = dd[j][l][d] = (TS)0;
   }
-  const int ps0 = g.pw * 3, words = sweep_words(g.npos, (int)sizeof(TS));
-  const word_t *lo = g.rk > 0 ? X.up + (long long)(g.rk - 1) * words : nullptr;
-  const word_t *hi = g.rk + 1 < g.cw ? X.down + (long long)g.rk * words : nullptr;
+  const int ps0 = g.pw * 3;
+  const word_t *sum2 = X.sum + 8 * g.cw;
   double v2[2] = {0.0, 0.0};
   int n = 0;
 #pragma unroll 1
@@ -384,7 +490,7 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
     int ps = ps0;
     asm volatile("" : "+s"(ps));
 #pragma unroll
-    for (int j = 0; j < NI; j++) asm volatile("" : "+v"(z0[j]));
+    for (int j = 0; j < NI; j++) asm volatile("" : "+v"(z0[j]), "+v"(wd[j]));
 #pragma unroll
     for (int j = 0; j < NI; j++) {
       if (j > 0 && cnt[j] == 0) continue;
@@ -402,7 +508,7 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
         // w = A z needs neither r.r nor r.z of the last update: their sums over
         // the cluster, posted before it, have arrived by now
         if (n > 0) {
-          if (g.cw > 1 && !cluster_collect<2>(v2, X.sum + kSweepMaxRanks * 8, g.cw, (unsigned)n)) *s_fail = 1;
+          if (g.cw > 1 && !cluster_sum<2>(v2, sum2, g.cw, (unsigned)n, red + 4 * (kSweepLanes / 64))) *s_fail = 1;
           done = scalar(sqrt(v2[0]) <= tgt || rz == 0.0 || n >= max_its) != 0;
           if (done) break;
           beta = v2[1] / rz;
@@ -429,7 +535,7 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
     lanes_sum<1>(v1, red);
     if (g.cw > 1) {
       cluster_post<1>(v1, X.sum, g.rk, tag);
-      if (!cluster_collect<1>(v1, X.sum, g.cw, tag)) *s_fail = 1;
+      if (!cluster_sum<1>(v1, X.sum, g.cw, tag, red + 3 * (kSweepLanes / 64))) *s_fail = 1;
     }
     const TS al = (TS)((v1[0] == 0.0) ? 0.0 : rz / v1[0]);
     v2[0] = v2[1] = 0.0;
@@ -460,18 +566,16 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
         if (on[j]) {
 #pragma unroll
           for (int d = 0; d < 3; d++) zl[z0[j] + (l + 1) * ps + d] = x[l][d];
-          if (l == 0 && lo && hc[j] == 0)
-            put_node(X.down + (long long)(g.rk - 1) * words, g.npos, item_pos(g, z0[j], hc[j]), tag, x[l]);
-          if (hi && l == cnt[j] - 1 && hc[j] == g.nch - 1)
-            put_node(X.up + (long long)g.rk * words, g.npos, item_pos(g, z0[j], hc[j]), tag, x[l]);
+          if (edge[j] || (l == 0 && g.zlo && hc[j] == 0) || (l == cnt[j] - 1 && g.zhi && hc[j] == g.nch - 1))
+            put_node(X, g.ni, wd[j] + l * g.nixy, tag, x[l]);
         }
       }
     }
     lanes_sum<2>(v2, red + kSweepLanes / 64);  // its barrier also ends the writes of z
     n++;
     if (g.cw > 1) {
-      cluster_post<2>(v2, X.sum + kSweepMaxRanks * 8, g.rk, tag);
-      if (!get_planes<TS>(g, zl, lo, hi, tag)) *s_fail = 1;
+      cluster_post<2>(v2, X.sum + 8 * g.cw, g.rk, tag);
+      if (!get_halo<TS>(g, zl, X, tag)) *s_fail = 1;
       __syncthreads();
       if (scalar(*s_fail)) return n;  // a wait ran out: no update; the residual shows it
     }
@@ -507,7 +611,7 @@ struct SweepRun {
   const TS *dict;
   double *red;
   int *fail;
-  const SweepExch &X;
+  const SweepWords &X;
   double rz, tgt;
   int max_its;
   template <int LP>
@@ -524,20 +628,21 @@ extern __shared__ __attribute__((aligned(16))) double sweep_dyn[];
 }  // namespace
 
 // The resident RVEs' kernel A (reads st[2], writes st[0]).  Workgroups take the
-// entries of the unit list (RVE slot, load case * 16 + rank) by ticket, in list
+// entries of the unit list (RVE slot, load case * 256 + rank) by ticket, in list
 // order: the ranks of a cluster are consecutive entries, so the started
 // workgroups form whole clusters but for the last one, the whole ones finish
 // without waiting for anyone else, and their places go to the missing ranks
 // (also beside other such launches: each leaves at most one cluster of at most
-// 16 workgroups waiting, and the GPU has more places than the queues' launches
-// can fill with those).
+// kSweepFreeRanks workgroups waiting, and the GPU has more places than the
+// queues' launches can fill with those; a larger cluster waits only before it has
+// started, and not for long: cluster_meet).
 // A sweep's end (its iteration count is the largest of the load cases') is
 // entered into the state by kernel B.
 template <typename TS, int K>
 __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp)
 {
   __shared__ double lds[64];
-  __shared__ double red[3 * (kSweepLanes / 64)];
+  __shared__ double red[6 * (kSweepLanes / 64)];
   __shared__ double tot[4 * K];
   __shared__ SolveState N;
   __shared__ int s_unit, s_fail;
@@ -551,7 +656,7 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   if (u >= P.units[0].x) return;
   const int slot = scalar(P.units[1 + u].x);
   const int case_rank = scalar(P.units[1 + u].y);
-  const int k = case_rank / kSweepMaxRanks, rk = case_rank % kSweepMaxRanks;
+  const int k = case_rank / kSweepUnitRanks, rk = case_rank % kSweepUnitRanks;
   RveDev *R = P.rves + slot;
   const int phase0 = R->st[2].phase;
   const bool writer = k == 0 && rk == 0;
@@ -574,6 +679,12 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
 
   const SweepGeo g = sweep_geo(R, rk);
   const int SN = P.SN, RS = 3 * SN, fs = g.fs, tsz = (int)sizeof(TS);
+  const SweepWords X = sweep_words<TS>(P, scalar(R->nslab), K, fs, k, g.ni);
+  if (g.cw > kSweepFreeRanks) {
+    if (tid == 0) s_unit = cluster_meet(X.sum + 16 * g.cw, g.cw) ? 1 : 0;
+    __syncthreads();
+    if (scalar(s_unit) == 0) return;
+  }
   TS *dict = reinterpret_cast<TS *>(sweep_dyn);
   TS *zl = reinterpret_cast<TS *>(reinterpret_cast<unsigned char *>(sweep_dyn) + sweep_dict_bytes(tsz));
   // the 16 blocks of patterns that repeat along z, rounded from the FP64
@@ -599,20 +710,17 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   for (int s = 0; s < g.np + 2; s++) {
     const int z = g.zs - 1 + s;
     if (z == 0 || z == R->nz - 1) continue;
-    for (int c = tid; c < g.ncol; c += kSweepLanes) {
-      const int iy = c / g.nix, m = (c - iy * g.nix + 1) + (iy + 1) * g.nx + z * g.nxy;
+    for (int c = tid; c < (g.nr + 2) * g.nix; c += kSweepLanes) {
+      const int r = c / g.nix, ix = c - r * g.nix;
+      if ((r == 0 && !g.ylo) || (r == g.nr + 1 && !g.yhi)) continue;
+      const int m = (ix + 1) + (g.ys + r) * g.nx + z * g.nxy;
       const TS *src = (const TS *)P.z + ((long long)(fs + (m >> P.sn_shift)) * K + k) * RS + 3 * (m & (SN - 1));
-      TS *dst = zl + (s * g.pw + 1 + (iy + 1) * g.rsx + c - iy * g.nix) * 3;
+      TS *dst = zl + (s * g.pw + 1 + r * g.rsx + ix) * 3;
 #pragma unroll
       for (int d = 0; d < 3; d++) dst[d] = src[d];
     }
   }
   __syncthreads();
-  SweepExch X;
-  const long long b0 = sweep_region(scalar(R->nslab), SN, K, tsz, fs, k);
-  X.up = reinterpret_cast<word_t *>((char *)P.p + b0);
-  X.down = reinterpret_cast<word_t *>((char *)P.q + b0);
-  X.sum = reinterpret_cast<word_t *>((char *)P.d + b0);
   const double rz = N.rz[k], tgt = N.bnorm_in[k];
   int n;
   const SweepRun<TS> run{P, g, K, k, zl, dict, red, &s_fail, X, rz, tgt, sp.max_inner_its};

@@ -125,10 +125,11 @@ struct RveDev {
   // the totals instead of each workgroup re-summing nslab partials.
   int big;
   // resident sweep (engine_sweep.hip): scw > 0 workgroups per load case hold
-  // the PCG state of a whole sweep on chip, each slp * snch or fewer of the
-  // interior z-planes in items of slp planes of one column; lits[k] is the
-  // iteration count of load case k in the sweep.  scw == 0: kernels A and B.
-  int scw, slp, snch;
+  // the PCG state of a whole sweep on chip, sty shares of the interior rows
+  // times scw / sty of the interior z-planes, each slp * snch or fewer planes in
+  // items of slp planes of one column; lits[k] is the iteration count of load
+  // case k in the sweep.  scw == 0: kernels A and B.
+  int scw, sty, slp, snch;
   int lits[MM_MAX_RHS];
   double rr_rz[2 * MM_MAX_RHS];
   double pq[MM_MAX_RHS];
@@ -183,7 +184,7 @@ struct EngPtrs {
   int a_lds;     // dynamic LDS bytes of the plane march; 0: march off
   int a_slab;    // march on: some RVEs (mcpp == 0) need k_step_a as well
   int s_big;     // the group holds an RVE with big != 0: kernel S runs after A
-  const int2 *units;  // [0].x: resident-sweep workgroups, [1..]: (slot, load case * 16 + rank)
+  const int2 *units;  // [0].x: resident-sweep workgroups, [1..]: (slot, load case * 256 + rank)
   unsigned *ticket;   // next unit to take; kernel B zeroes it (resident RVEs' first slabs)
   int u_grid, u_lds;  // launch of the resident sweep (0: none in the group)
 };
@@ -232,7 +233,13 @@ constexpr int kMarchMaxLds = 64 * 1024;
 // kernel.
 constexpr int kSweepLanes = 512;  // two waves per SIMD, 256 VGPRs each
 constexpr int kSweepItems = 2;    // items (a column times slp planes) per lane
-constexpr int kSweepMaxRanks = 16;
+// Workgroups per load case.  A cluster that waits for ranks without a CU holds
+// the CUs of the others; with up to kSweepFreeRanks, four queues of waiting
+// clusters leave room for any missing rank, and larger clusters first meet.
+constexpr int kSweepFreeRanks = 16;
+constexpr int kSweepMaxRanks = 240;  // of 256 CUs
+constexpr unsigned long long kMeetGo = 1, kMeetOff = 2;
+constexpr int kSweepUnitRanks = 256;  // a unit is (slot, load case * this + rank)
 constexpr int kSweepMaxLds = 160 * 1024 - 2816;  // dynamic; the static part is below 2.75 KB
 __host__ __device__ constexpr int sweep_max_planes(int tsz) { return tsz == 8 ? 4 : 8; }
 // The unrolled item lengths: a sweep of lp planes per item runs the next one.
@@ -262,17 +269,17 @@ __host__ __device__ constexpr int sweep_plane(int nx, int ny) { return 1 + ny * 
 __host__ __device__ constexpr int sweep_dict_block(int tsz) { return tsz == 8 ? 9 : 12; }
 __host__ __device__ constexpr int sweep_dict_stride(int tsz) { return tsz == 8 ? 250 : 332; }
 __host__ __device__ constexpr int sweep_dict_bytes(int tsz) { return 17 * sweep_dict_stride(tsz) * tsz; }
-// The words a cluster exchanges live in the RVE's runs of p (top planes), q
-// (bottom planes) and d (partial sums), which a resident sweep does not use
-// otherwise: load case k has the k-th part of the run.  Kernel R zeroes them
-// before each sweep.
+// The words a cluster exchanges live in the RVE's runs of q, p and d, which a
+// resident sweep does not use otherwise: load case k has the k-th part of each.
+// Row d of interior node i of the RVE is word i of run d (FP64: low halves, then
+// the high halves); the partial sums and two words for the meeting of a large
+// cluster follow in d's run.  Kernel R zeroes what the sweep uses before it.
 __host__ __device__ inline long long sweep_region(int nslab, int SN, int K, int tsz, int first_slab, int k)
 {
   return ((long long)first_slab * K + (long long)k * nslab) * 3 * SN * tsz;  // first byte
 }
-// 64-bit words of one plane: 32 bits of the three rows of every position.
-__host__ __device__ constexpr int sweep_words(int npos, int tsz) { return 3 * npos * (tsz / 4); }
-constexpr int kSweepSumWords = 2 * kSweepMaxRanks * 8;  // two sums, 64 bytes per rank
+// Words of the partial sums: two sums, 64 bytes per rank, and the meeting.
+__host__ __device__ constexpr int sweep_sum_words(int cw) { return 16 * cw + 2; }
 
 // assembly modes
 enum AsmMode : int { ASM_FULL = 0, ASM_X_ONLY = 1, ASM_DICT = 2 };

@@ -28,7 +28,7 @@ SIZES = [(2, 2, 2), (2, 3, 9), (1, 4, 5),  # one interior node; a thin column; n
          (10, 9, 6),   # 80 positions: two strips
          (9, 8, 40),   # many planes over few columns
          (20, 17, 11), (31, 32, 6), (32, 32, 3),  # several strips per wave; the widest planes
-         (34, 33, 3)]  # wider: kernels A and B
+         (34, 33, 3)]  # wider: the rows shared too
 
 
 def _solve(eng, specs, loads=None, mode=MM_TANGENT_UNIT):
@@ -82,8 +82,8 @@ def test_step_kernels_agree(precision):
 
 @pytest.mark.parametrize("precision", [MM_PREC_MIXED, MM_PREC_FP64])
 def test_resident_and_other_rves_in_one_batch(precision):
-    """Cells on every path (resident, too wide for it) share the launches, in
-    one and two stream groups, full and dictionary storage, each with the bits
+    """Cells of several splits (planes, planes and rows, one workgroup) share the
+    launches, in one and two stream groups, full and dictionary storage, each with the bits
     it has alone."""
     specs = [rve_spec((24, 23, 12), [(0.5, 0.45, 0.3)]), rve_spec((40, 36, 3), [(0.5, 0.5, 0.3)]),
              rve_spec(7, [(0.4, 0.5, 0.25)])]
