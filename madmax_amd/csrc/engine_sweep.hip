@@ -7,25 +7,26 @@
 // blocks in LDS.  See RveDev::scw for which RVEs.
 //
 // Why: kernels A and B move eleven vector passes per iteration through HBM and
-// are two to four launches; here an iteration moves only the planes between
-// ranks and the partial sums.  What bounds it: vector issue (the 243 multiply-
-// adds of a node's rows, 61% of all vector instructions; 80% of the issue slots
-// of a full SIMD while w = A z runs) and, for clusters, two exchanges of 2.5 us.
-// One 30^3 load case (4 ranks of 8 planes, FP32) takes 27.8 us per iteration
-// alone and 30.7 with 64 of them on the GPU; kernels A, B and R took 640 us for
-// 768 of them, 53 per 64.  Measured on the way there, same case:
+// are two to four launches; here an iteration moves only the nodes between ranks
+// and the partial sums.  What bounds it: vector issue (of some 250 instructions
+// per node and iteration 162 are the multiply-adds of its rows) and, for
+// clusters, two exchanges of 2.5 us.  One 30^3 load case (4 ranks of 8 planes,
+// FP32) takes 25 us per iteration; kernels A, B and R took 640 us for 768 of
+// them, 53 per 64.  Measured on the way there, same case:
 //   z neighbours read from LDS, one per key: 38 us; x-neighbours through DPP: 31
 //   (LDS reads per node 81 -> 27 dwords);
 //   1,024 lanes at 128 VGPRs, items of 4 planes: 32 us (spills, dictionary reads
 //   shared by half as many nodes);
 //   two workgroups per CU, items of 3 planes: 67 us per 60 load cases (bound by
 //   the dictionary's LDS reads);
-//   waiting for r.r / r.z before w = A z instead of behind it: 31 us.
-// Whole solves (rtol 1e-10): 128 x 30^3 tangents 187 -> 75 ms, 64 uneven cells
-// 8^3 .. 32^3 50 -> 14 ms, 24 x 20^3 in FP64 25.5 -> 7.1 ms, one 10^3 4.7 -> 1.1.
-// Sharing the rows: 32 x 33 x 36 x 40 tangents 122 -> 47 ms, 4 x 60^3 93 -> 38; one
-// load case of 48^3 7.9 -> 4.9 ms, of 100^3 (195 workgroups) 50 -> 18, 74 us an
-// iteration by kernels A, S, B and R and 26 here.
+//   waiting for r.r / r.z before w = A z instead of behind it: 31 us;
+//   the planes above and below one by one: 243 multiply-adds, 27.8 to 30.7 us.
+// Whole solves (rtol 1e-10), kernels A and B and this: 128 x 30^3 tangents 187 and
+// 62 ms, 64 uneven cells 8^3 .. 32^3 50 and 13.8 ms, 24 x 20^3 in FP64 25.5 and 6.0
+// ms, one 10^3 4.7 and 0.87.
+// Sharing the rows: 32 x 33 x 36 x 40 tangents 122 and 44 ms, 4 x 60^3 93 and 32;
+// one load case of 48^3 7.9 and 4.1 ms, of 100^3 (195 workgroups) 50 and 17, 74 us
+// an iteration by kernels A, S, B and R and 25 here.
 #include <hip/hip_runtime.h>
 
 #include "engine_device.h"
@@ -102,48 +103,58 @@ __device__ __forceinline__ void lds_read3(const double *p, double (&v)[3])
   for (int d = 0; d < 3; d++) v[d] = ((const __attribute__((address_space(3))) double *)p)[d];
 }
 
-// w[d] += a[e][d] * (x[e] of the lane before, DX = 0, or after, DX = 2), e = 0,
+// w[d] += a[e][d] * (x[e][d] of the lane before, DX = 0, or after, DX = 2), e = 0,
 // 1, 2 in turn: the shift rides on the multiply-add.  (x may come straight from
 // a vector instruction, which a DPP read must not follow within two cycles.)
 template <int DX>
-__device__ __forceinline__ void fma_lane_x(const float (&a)[3][3], const float (&x)[3], float (&w)[3])
+__device__ __forceinline__ void fma_lane_x(const float (&a)[3][3], const float *const (&x)[3][3], float (&w)[3])
 {
 #define MM_FMAC_DPP(SHIFT)                                                             \
   asm("s_nop 1\n\t"                                                                    \
-      "v_fmac_f32_dpp %0, %3, %6 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
-      "v_fmac_f32_dpp %1, %3, %7 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
-      "v_fmac_f32_dpp %2, %3, %8 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
-      "v_fmac_f32_dpp %0, %4, %9 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
-      "v_fmac_f32_dpp %1, %4, %10 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
-      "v_fmac_f32_dpp %2, %4, %11 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
-      "v_fmac_f32_dpp %0, %5, %12 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
-      "v_fmac_f32_dpp %1, %5, %13 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
-      "v_fmac_f32_dpp %2, %5, %14 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1"     \
+      "v_fmac_f32_dpp %0, %3, %12 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %1, %4, %13 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %2, %5, %14 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %0, %6, %15 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %1, %7, %16 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %2, %8, %17 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %0, %9, %18 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %1, %10, %19 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t" \
+      "v_fmac_f32_dpp %2, %11, %20 " SHIFT " row_mask:0xf bank_mask:0xf bound_ctrl:1"     \
       : "+v"(w[0]), "+v"(w[1]), "+v"(w[2])                                               \
-      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(a[0][0]), "v"(a[0][1]), "v"(a[0][2]), "v"(a[1][0]), "v"(a[1][1]), \
+      : "v"(*x[0][0]), "v"(*x[0][1]), "v"(*x[0][2]), "v"(*x[1][0]), "v"(*x[1][1]), "v"(*x[1][2]), "v"(*x[2][0]), \
+        "v"(*x[2][1]), "v"(*x[2][2]), "v"(a[0][0]), "v"(a[0][1]), "v"(a[0][2]), "v"(a[1][0]), "v"(a[1][1]),      \
         "v"(a[1][2]), "v"(a[2][0]), "v"(a[2][1]), "v"(a[2][2]))
   if constexpr (DX == 0) MM_FMAC_DPP("wave_shr:1");
   else MM_FMAC_DPP("wave_shl:1");
 #undef MM_FMAC_DPP
 }
 template <int DX>
-__device__ __forceinline__ void fma_lane_x(const double (&a)[3][3], const double (&x)[3], double (&w)[3])
+__device__ __forceinline__ double lane_x(double v)
 {
   constexpr int shift = DX == 0 ? 0x138 : 0x130;  // wave_shr:1, wave_shl:1
+  const int2 b = __builtin_bit_cast(int2, v);
+  return __builtin_bit_cast(double, make_int2(__builtin_amdgcn_update_dpp(0, b.x, shift, 0xf, 0xf, true),
+                                              __builtin_amdgcn_update_dpp(0, b.y, shift, 0xf, 0xf, true)));
+}
+template <int DX>
+__device__ __forceinline__ void fma_lane_x(const double (&a)[3][3], const double *const (&x)[3][3], double (&w)[3])
+{
 #pragma unroll
   for (int e = 0; e < 3; e++) {
-    const int2 b = __builtin_bit_cast(int2, x[e]);
-    const double xe = __builtin_bit_cast(double, make_int2(__builtin_amdgcn_update_dpp(0, b.x, shift, 0xf, 0xf, true),
-                                                           __builtin_amdgcn_update_dpp(0, b.y, shift, 0xf, 0xf, true)));
-#pragma unroll
-    for (int d = 0; d < 3; d++) w[d] = fma(a[e][d], xe, w[d]);
+    // (x[e] names one or two values)
+    const double x0 = lane_x<DX>(*x[e][0]);
+    const double x1 = x[e][1] == x[e][0] ? x0 : lane_x<DX>(*x[e][1]);
+    const double x2 = x[e][2] == x[e][0] ? x0 : x[e][2] == x[e][1] ? x1 : lane_x<DX>(*x[e][2]);
+    w[0] = fma(a[e][0], x0, w[0]);
+    w[1] = fma(a[e][1], x1, w[1]);
+    w[2] = fma(a[e][2], x2, w[2]);
   }
 }
 
-// w += block DX of the three x-neighbours (dictionary row Db) times z, for LP
-// nodes of the lane's column whose own z rows in that strip are x.
-template <typename TS, int LP, int DX>
-__device__ __forceinline__ void sweep_key(const TS *Db, const TS (&x)[LP][3], TS (&w)[LP][3])
+// w += the block Db times x of the x-neighbour DX (1: the column itself), for LP
+// nodes of the lane's column; x(l, e, d): the value that row e, column d multiplies.
+template <typename TS, int LP, int DX, typename X>
+__device__ __forceinline__ void sweep_key(const TS *Db, const X &x, TS (&w)[LP][3])
 {
   constexpr int blk = sweep_dict_block((int)sizeof(TS));
   TS a[3][3];  // [d'][d]
@@ -151,28 +162,56 @@ __device__ __forceinline__ void sweep_key(const TS *Db, const TS (&x)[LP][3], TS
   for (int e = 0; e < 3; e++) lds_read3(Db + DX * blk + e * (blk / 3), a[e]);
 #pragma unroll
   for (int l = 0; l < LP; l++) {
+    const TS *v[3][3];
+#pragma unroll
+    for (int e = 0; e < 3; e++)
+#pragma unroll
+      for (int d = 0; d < 3; d++) v[e][d] = &x(l, e, d);
     if constexpr (DX != 1) {
-      fma_lane_x<DX>(a, x[l], w[l]);
+      fma_lane_x<DX>(a, v, w[l]);
     } else {
 #pragma unroll
       for (int e = 0; e < 3; e++)
 #pragma unroll
-        for (int d = 0; d < 3; d++) w[l][d] = fma(a[e][d], x[l][e], w[l][d]);
+        for (int d = 0; d < 3; d++) w[l][d] = fma(a[e][d], *v[e][d], w[l][d]);
     }
   }
 }
 
-// w += the three blocks of strip (dz, dy), whose rows start at zr.
+// w += the nine blocks of the columns at dy, whose rows start at zr: those of the
+// node's own plane, then the planes below and above together.  The cell is the
+// same mirrored in z (the phases do not vary along z), so the block below is the
+// block above with the signs of its xz, yz, zx and zy entries changed: of z above
+// and below, the sum goes with the others and the difference with these.  That
+// takes 162 multiply-adds and 18 adds per node in place of 243, two thirds of the
+// dictionary's reads, and reads a column's z once.
 template <typename TS, int LP>
-__device__ __forceinline__ void sweep_strip(const TS *zr, int ps, const TS *dict, int dz, int dy, TS (&w)[LP][3])
+__device__ __forceinline__ void sweep_strip(const TS *zr, int ps, const TS *dict, int dy, TS (&w)[LP][3])
 {
-  const TS *Db = dict + (3 * dy + 9 * dz) * sweep_dict_block((int)sizeof(TS));
-  TS x[LP][3];
+  constexpr int blk = sweep_dict_block((int)sizeof(TS));
+  TS x[LP + 2][3];
 #pragma unroll
-  for (int l = 0; l < LP; l++) lds_read3(zr + l * ps, x[l]);
-  sweep_key<TS, LP, 0>(Db, x, w);
-  sweep_key<TS, LP, 1>(Db, x, w);
-  sweep_key<TS, LP, 2>(Db, x, w);
+  for (int l = 0; l < LP + 2; l++) lds_read3(zr + l * ps, x[l]);
+  {
+    const TS *Db = dict + (3 * dy + 9) * blk;
+    const auto own = [&](int l, int e, int) -> const TS & { return x[l + 1][e]; };
+    sweep_key<TS, LP, 0>(Db, own, w);
+    sweep_key<TS, LP, 1>(Db, own, w);
+    sweep_key<TS, LP, 2>(Db, own, w);
+  }
+  TS s[LP][3], t[LP][3];
+#pragma unroll
+  for (int l = 0; l < LP; l++)
+#pragma unroll
+    for (int e = 0; e < 3; e++) {
+      s[l][e] = x[l + 2][e] + x[l][e];
+      t[l][e] = x[l + 2][e] - x[l][e];
+    }
+  const TS *Db = dict + (3 * dy + 18) * blk;
+  const auto pair = [&](int l, int e, int d) -> const TS & { return (e == 2) == (d == 2) ? s[l][e] : t[l][e]; };
+  sweep_key<TS, LP, 0>(Db, pair, w);
+  sweep_key<TS, LP, 1>(Db, pair, w);
+  sweep_key<TS, LP, 2>(Db, pair, w);
 }
 
 // Bound on a wait in polls (half a minute or more).  A rank waits for the
@@ -445,9 +484,10 @@ __device__ __forceinline__ SweepItem sweep_item(const SweepGeo &g, int tid, int 
 // the sweep's right-hand side.  An item is one interior column times lp planes,
 // LP >= lp of its nodes' rows in registers, one lane each; a wave takes strips
 // of kSweepStrip consecutive positions, so that the x-neighbours of a node are
-// the lanes beside it and come from them (DPP) instead of LDS.  The arithmetic of a node is kernel A's and kernel B's (the
-// row product in neighbour-key order, r = z / dinv formed for the dots); only
-// the grouping of the dot products differs.  Returns the iterations taken.
+// the lanes beside it and come from them (DPP) instead of LDS.  The recurrences
+// are kernel A's and kernel B's (r = z / dinv formed for the dots); the row sums
+// (sweep_strip) and the dot products are grouped differently.  Returns the
+// iterations taken.
 template <typename TS, int LP>
 __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, int K, int k, TS *zl,
                                           const TS *dict, double *red, int *s_fail, const SweepWords &X, double rz,
@@ -501,9 +541,7 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
         for (int d = 0; d < 3; d++) w[l][d] = (TS)0;
       const TS *zr = zl + z0[j] - g.rsx * 3, *Db = dict + d0[j];
 #pragma unroll 1
-      for (int dz = 0; dz < 3; dz++)
-#pragma unroll 1
-        for (int dy = 0; dy < 3; dy++) sweep_strip<TS, LP>(zr + dz * ps + dy * g.rsx * 3, ps, Db, dz, dy, w);
+      for (int dy = 0; dy < 3; dy++) sweep_strip<TS, LP>(zr + dy * g.rsx * 3, ps, Db, dy, w);
       if (j == 0) {
         // w = A z needs neither r.r nor r.z of the last update: their sums over
         // the cluster, posted before it, have arrived by now

