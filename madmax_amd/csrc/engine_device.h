@@ -46,6 +46,119 @@ __device__ __forceinline__ SweepWords sweep_words(const EngPtrs &P, int nslab, i
   return X;
 }
 
+// MI355X dispatches workgroup i to XCD i % 8.  The solver grids are a
+// multiple of 8 and workgroup i processes slab (i % 8) * (grid / 8) + i / 8,
+// so each XCD walks one contiguous run of slabs and the z rows that
+// neighbouring slabs of an RVE share stay in that XCD's L2.
+constexpr int kXcd = 8;
+// Largest grid of kernel R (a multiple of 8; k_step_r loops over the slabs).
+constexpr int kRGrid = 2048;
+__device__ __forceinline__ int xcd_slab()
+{
+  const int per = gridDim.x / kXcd;
+  return (blockIdx.x % kXcd) * per + blockIdx.x / kXcd;
+}
+
+// Solver launches run over the list of slabs being solved (act_list[0] of
+// them, ascending from act_list[1]); the grid is a power of two >= 64 that
+// covers the list.  The list is split in 8 contiguous parts, one per XCD, so
+// neighbouring slabs of an RVE share an L2.  Returns false for workgroups
+// beyond the list.
+__device__ __forceinline__ bool active_in(const int *list, int &slab)
+{
+  const int n = list[0];
+  const int per = (n + kXcd - 1) / kXcd;
+  const int j = blockIdx.x / kXcd;
+  const int i = (blockIdx.x % kXcd) * per + j;
+  if (j >= per || i >= n) return false;
+  slab = list[1 + i];
+  return true;
+}
+__device__ __forceinline__ bool active_slab(const EngPtrs &P, int &slab) { return active_in(P.act_list, slab); }
+
+// Zeroes the slab's share of the words that the ranks of a resident sweep
+// exchange (tag 0 is no iteration's).
+template <typename TS, int K>
+__device__ void sweep_words_zero(const EngPtrs &P, const RveDev *R, int slab)
+{
+  const int ls = slab - R->first_slab, bd = (int)blockDim.x, cw = R->scw, cz = cw / R->sty;
+  const int nixy = (R->nx - 2) * (R->ny - 2), niz = R->nz - 2, ni = nixy * niz;
+  // the planes that ranks exchange: the first and last of each share, or, where
+  // the rows are shared too, all
+  const int nw = R->sty > 1 ? ni : 2 * cz * nixy;
+#pragma unroll 1
+  for (int k = 0; k < K; k++) {
+    const SweepWords X = sweep_words<TS>(P, R->nslab, K, R->first_slab, k, ni);
+    for (int i = ls * bd + (int)threadIdx.x; i < nw; i += R->nslab * bd) {
+      int at = i;
+      if (R->sty == 1) {
+        const int pl = i / nixy, r = pl >> 1;
+        at = ((pl & 1) ? (r + 1) * niz / cz - 1 : r * niz / cz) * nixy + i - pl * nixy;
+      }
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int h = 0; h < (int)(sizeof(TS) / 4); h++) X.w[d][(long long)h * ni + at] = 0;
+    }
+    if (ls == 0)
+      for (int i = threadIdx.x; i < 16 * cw; i += bd) X.sum[i] = 0;  // (the meeting's words: sweep_end)
+  }
+}
+
+// Whether a resident RVE's state st[0] is ready for the residual: it wants its
+// first one, or the sweep has run for every load case that needed it.
+template <typename TS, int K>
+__device__ __forceinline__ bool sweep_ran(const EngPtrs &P, const RveDev *R)
+{
+  const SolveState *S = &R->st[0];
+  if (S->phase != PH_INNER) return S->phase == PH_RES;
+  const int cw = R->scw;
+  if (cw <= kSweepFreeRanks) return true;
+  const long long ni = (long long)(R->nx - 2) * (R->ny - 2) * (R->nz - 2);
+  bool ran = true;
+  for (int k = 0; k < K; k++)
+    if (!((S->done_in >> k) & 1u))
+      ran = ran && sweep_words<TS>(P, R->nslab, K, R->first_slab, k, ni).sum[16 * cw + 1] == kMeetGo;
+  return ran;
+}
+
+// A resident RVE's state between launches, by one lane, after the residual (if
+// any).  The end of a sweep: its iteration count is the largest of the load cases'
+// (as inner_check counts).  Load cases whose cluster did not meet are left for the
+// next launch.
+template <typename TS, int K>
+__device__ void sweep_end(const EngPtrs &P, const RveDev *R, SolveState &N)
+{
+  const int cw = R->scw, phase = N.phase;
+  const long long ni = (long long)(R->nx - 2) * (R->ny - 2) * (R->nz - 2);
+  bool left = false;
+  if (phase == PH_INNER || phase == PH_RES) {
+    for (int k = 0; k < K; k++) {
+      const bool run = phase == PH_INNER && !((N.done_in >> k) & 1u);
+      if (cw > kSweepFreeRanks) {
+        word_t *meet = sweep_words<TS>(P, R->nslab, K, R->first_slab, k, ni).sum + 16 * cw;
+        const bool ran = meet[1] == kMeetGo;
+        meet[0] = meet[1] = 0;
+        if (run && !ran) {
+          left = true;
+          continue;
+        }
+        if (run) N.done_in |= 1u << k;
+      }
+      if (run) N.its = max(N.its, R->lits[k]);
+    }
+  }
+  if (phase == PH_INNER && !left) {
+    N.its_total += N.its;
+    N.sweep += 1;
+    N.phase = PH_RESRED;
+  } else if (phase == PH_RES) {
+    N.phase = PH_RESRED;
+  } else if (phase == PH_AVG) {
+    N.phase = PH_AVGRED;
+  }
+}
+
 // Start of a refinement sweep from the reduced residual norms s4 =
 // {||r64||^2, ||r||^2, r.z, ||r_cold||^2} per load case (FP64 residual r64,
 // its rounding r, cold-start right-hand side r_cold).
@@ -114,45 +227,55 @@ __device__ bool inner_check(SolveState &N, const double (&s2)[2 * K], const Solv
 }
 
 // Volume averages and tangent of a finished RVE (micro/src/homogenize.c:
-// 344-368, :80) from the averaging partials; run by one workgroup.
-template <int K, int L>
-__device__ void finish_rve(const EngPtrs &P, int slot, const RveDev *R, SolveState &N,
-                           const SolveParams &sp, double (&lds)[L])
+// 344-368, :80) from the averaging partials; run by one workgroup.  Bound by its
+// chain of memory round trips: each wave sums every so many of the 12 K values, a
+// lane per slab, and a lane forms each output.  Four values at a time over the
+// workgroup and one lane for the outputs took 38 us for one 10^3
+// cell and 110 for 24 cells up to 30^3; this takes 10 and 20.
+template <int K>
+__device__ void finish_rve(const EngPtrs &P, int slot, const RveDev *R, SolveState &N, const SolveParams &sp)
 {
-  __shared__ double tot[MM_MAX_RHS][12];
+  __shared__ double avg[MM_MAX_RHS][12];
   const double *p0 = slab_part(P, R->first_slab).p;
+  const int tid = threadIdx.x, ln = tid & 63, nslab = R->nslab;
+  const double vol = R->vol;
 #pragma unroll 1
-  for (int k = 0; k < K; k++) group_sum_cols_lds<12>(p0, R->nslab, P.part_stride, k * 12, &tot[k][0], lds);
-  __shared__ double sig[MM_MAX_RHS][6];
-  if (threadIdx.x != 0) return;
+  for (int i0 = 4 * (tid >> 6); i0 < 12 * K; i0 += 4 * ((int)blockDim.x >> 6)) {
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+    for (int b = ln; b < nslab; b += 64)
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i] += p0[(size_t)(i0 + i) * P.part_stride + b];
+    int q;
+    const double s = wave_sum4(v, q);
+    if ((ln & 15) == 0) avg[(i0 + q) / 12][(i0 + q) % 12] = s / vol;
+  }
+  __syncthreads();
   RveOut *o = P.out + slot;
+  const int mode = R->tangent_mode;
+  for (int t = tid; t < 12 * K; t += blockDim.x) {
+    const int k = t / 12, i = t - 12 * k;
+    if (i < 6) o->strain[k][i] = avg[k][i];
+    else o->stress[k][i - 6] = avg[k][i];
+  }
+  for (int t = tid; t < 36; t += blockDim.x) {
+    const int j = t / 6, i = t - 6 * j;  // c[j * 6 + i]: d stress j / d strain i
+    double c = 0.0;
+    if (mode == MM_TANGENT_UNIT && K >= 6) {
+      c = avg[i][6 + j] / R->load[i][i];
+    } else if (mode == MM_TANGENT_FD && K >= 7) {
+      c = (avg[i + 1][6 + j] - avg[0][6 + j]) / (R->load[i + 1][i] - R->load[0][i]);
+    }
+    o->c[t] = c;
+  }
+  __threadfence_system();  // each lane's outputs, before lane 0 says that they are there
+  __syncthreads();
+  if (tid != 0) return;
   double rel = 0.0;
   bool ok = true;
-#pragma unroll 1
-  for (int k = 0; k < K; k++) {
-#pragma unroll 1
-    for (int i = 0; i < 12; i++) {
-      const double s = tot[k][i] / R->vol;
-      if (i < 6) o->strain[k][i] = s;
-      else {
-        o->stress[k][i - 6] = s;
-        sig[k][i - 6] = s;
-      }
-    }
-    if (k < R->nload) {
-      const double r0 = N.r0[k], rn = N.rnorm[k];
-      rel = fmax(rel, (r0 > 0.0) ? rn / r0 : 0.0);
-      if (!(r0 == 0.0 || rn <= sp.rtol * r0 || rn < sp.abs_tol)) ok = false;
-    }
-  }
-  for (int i = 0; i < 36; i++) o->c[i] = 0.0;
-  if (R->tangent_mode == MM_TANGENT_UNIT && K >= 6) {
-    for (int i = 0; i < 6; i++)
-      for (int j = 0; j < 6; j++) o->c[j * 6 + i] = sig[i][j] / R->load[i][i];
-  } else if (R->tangent_mode == MM_TANGENT_FD && K >= 7) {
-    for (int i = 0; i < 6; i++)
-      for (int j = 0; j < 6; j++)
-        o->c[j * 6 + i] = (sig[i + 1][j] - sig[0][j]) / (R->load[i + 1][i] - R->load[0][i]);
+  for (int k = 0; k < K && k < R->nload; k++) {
+    const double r0 = N.r0[k], rn = N.rnorm[k];
+    rel = fmax(rel, (r0 > 0.0) ? rn / r0 : 0.0);
+    if (!(r0 == 0.0 || rn <= sp.rtol * r0 || rn < sp.abs_tol)) ok = false;
   }
   o->residual_rel = rel;
   o->its_total = N.its_total;

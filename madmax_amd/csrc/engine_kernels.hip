@@ -60,36 +60,6 @@ struct MarchLds {
 };
 
 
-// MI355X dispatches workgroup i to XCD i % 8.  The solver grids are a
-// multiple of 8 and workgroup i processes slab (i % 8) * (grid / 8) + i / 8,
-// so each XCD walks one contiguous run of slabs and the z rows that
-// neighbouring slabs of an RVE share stay in that XCD's L2.
-constexpr int kXcd = 8;
-// Largest grid of kernel R (a multiple of 8; k_step_r loops over the slabs).
-constexpr int kRGrid = 2048;
-__device__ __forceinline__ int xcd_slab()
-{
-  const int per = gridDim.x / kXcd;
-  return (blockIdx.x % kXcd) * per + blockIdx.x / kXcd;
-}
-
-// Solver launches run over the list of slabs being solved (act_list[0] of
-// them, ascending from act_list[1]); the grid is a power of two >= 64 that
-// covers the list.  The list is split in 8 contiguous parts, one per XCD, so
-// neighbouring slabs of an RVE share an L2.  Returns false for workgroups
-// beyond the list.
-__device__ __forceinline__ bool active_in(const int *list, int &slab)
-{
-  const int n = list[0];
-  const int per = (n + kXcd - 1) / kXcd;
-  const int j = blockIdx.x / kXcd;
-  const int i = (blockIdx.x % kXcd) * per + j;
-  if (j >= per || i >= n) return false;
-  slab = list[1 + i];
-  return true;
-}
-__device__ __forceinline__ bool active_slab(const EngPtrs &P, int &slab) { return active_in(P.act_list, slab); }
-
 __device__ __forceinline__ int node_class(int ix, int iy, int iz, int nx, int ny, int nz)
 {
   const int cx = (ix == 0) ? 0 : ((ix == nx - 1) ? 2 : 1);
@@ -910,7 +880,7 @@ __global__ __launch_bounds__(256) void k_step_a(EngPtrs P, SolveParams sp)
     if (!writer) return;
     if (tid == 0) N = R->st[2];
     __syncthreads();
-    finish_rve<K>(P, slot, R, N, sp, lds);
+    finish_rve<K>(P, slot, R, N, sp);
     if (tid == 0) R->st[0] = N;
     return;
   }
@@ -1407,7 +1377,7 @@ __device__ __forceinline__ void step_a_march(const EngPtrs &P, const SolveParams
     if (!writer) return;
     if (tid == 0) N = R->st[2];
     __syncthreads();
-    finish_rve<K>(P, slot, R, N, sp, lds);
+    finish_rve<K>(P, slot, R, N, sp);
     if (tid == 0) R->st[0] = N;
     return;
   }
@@ -1494,40 +1464,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TS) 
   RveDev *R = P.rves + slot;
   const SolveState *S = &R->st[0];
   const int scw = R->scw, phase = S->phase;  // read together
-  if (scw > 0) {
-    // a resident sweep has run to its end: the count is the largest of the
-    // load cases' (as inner_check counts), and the residual comes next.  Load
-    // cases whose cluster did not meet are left for the next launch.
-    if (slab == R->first_slab && tid == 0) {
-      SolveState N = *S;
-      if (N.phase == PH_INNER) {
-        bool left = false;
-        for (int k = 0; k < K; k++) {
-          if ((N.done_in >> k) & 1u) continue;
-          if (scw > kSweepFreeRanks) {
-            const long long ni = (long long)(R->nx - 2) * (R->ny - 2) * (R->nz - 2);
-            word_t *meet = sweep_words<TS>(P, R->nslab, K, R->first_slab, k, ni).sum + 16 * scw;
-            const bool ran = meet[1] == kMeetGo;
-            meet[0] = meet[1] = 0;
-            if (!ran) {
-              left = true;
-              continue;
-            }
-            N.done_in |= 1u << k;
-          }
-          N.its = max(N.its, R->lits[k]);
-        }
-        if (!left) {
-          N.its_total += N.its;
-          N.sweep += 1;
-          N.phase = PH_RES;
-        }
-      }
-      R->st[1] = N;
-      *P.ticket = 0u;  // for the next resident sweep
-    }
-    return;
-  }
+  if (scw > 0) return;  // kernel R's
   if (slab == R->first_slab && tid == 0) R->st[1] = *S;
   if (phase != PH_INNER) return;
   const unsigned skip = S->done_in;
@@ -1630,35 +1567,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sizeof(TS) 
 // or warm-started measures it at sweep 0 from the boundary neighbours alone.
 // PH_AVG: per-slab partial volume averages of strain and stress in FP64,
 // sum_gp (.) w_gp per element through sum_gp B w, one load case at a time.
-// Zeroes the slab's share of the words that the ranks of a resident sweep
-// exchange (tag 0 is no iteration's).
-template <typename TS, int K>
-__device__ void sweep_words_zero(const EngPtrs &P, const RveDev *R, int slab)
-{
-  const int ls = slab - R->first_slab, bd = (int)blockDim.x, cw = R->scw, cz = cw / R->sty;
-  const int nixy = (R->nx - 2) * (R->ny - 2), niz = R->nz - 2, ni = nixy * niz;
-  // the planes that ranks exchange: the first and last of each share, or, where
-  // the rows are shared too, all
-  const int nw = R->sty > 1 ? ni : 2 * cz * nixy;
-#pragma unroll 1
-  for (int k = 0; k < K; k++) {
-    const SweepWords X = sweep_words<TS>(P, R->nslab, K, R->first_slab, k, ni);
-    for (int i = ls * bd + (int)threadIdx.x; i < nw; i += R->nslab * bd) {
-      int at = i;
-      if (R->sty == 1) {
-        const int pl = i / nixy, r = pl >> 1;
-        at = ((pl & 1) ? (r + 1) * niz / cz - 1 : r * niz / cz) * nixy + i - pl * nixy;
-      }
-#pragma unroll
-      for (int d = 0; d < 3; d++)
-#pragma unroll
-        for (int h = 0; h < (int)(sizeof(TS) / 4); h++) X.w[d][(long long)h * ni + at] = 0;
-    }
-    if (ls == 0)
-      for (int i = threadIdx.x; i < sweep_sum_words(cw); i += bd) X.sum[i] = 0;
-  }
-}
-
 template <typename TS, int K>
 __device__ void res_slab(const EngPtrs &P, int slab, int slot, const RveDev *R, bool need_cold,
                          double (&lds)[RedLds<K>::size])
@@ -1731,7 +1639,7 @@ __device__ void res_slab(const EngPtrs &P, int slab, int slot, const RveDev *R, 
     }
 
     scatter_node<TS, K>((TS *)P.z, nb, RS, zi);
-    if (R->scw == 0) {  // a resident sweep starts d, p and q itself
+    {
       TS zero[3][K];
 #pragma unroll
       for (int d = 0; d < 3; d++)
@@ -1742,7 +1650,6 @@ __device__ void res_slab(const EngPtrs &P, int slab, int slot, const RveDev *R, 
       scatter_node<TS, K>((TS *)P.q, nb, RS, zero);
     }
   }
-  if (R->scw > 1) sweep_words_zero<TS, K>(P, R, slab);
   block_sum<4 * K>(v, lds);
   if (tid == 0) {
     const SlabPart part = slab_part(P, slab);
@@ -1760,7 +1667,7 @@ __device__ void avg_slab(const EngPtrs &P, int slab, int slot, const RveDev *R,
   const int nslab = R->nslab;
   const SlabPart part = slab_part(P, slab);
   const int ls = slab - R->first_slab;
-  const int nelm = R->nelm;
+  const int nelm = R->nelm, nex = R->nex, ney = R->ney, nx = R->nx, ny = R->ny, first = R->first_slab;
   const int epb = (nelm + nslab - 1) / nslab;
   const int e_end = min(nelm, (ls + 1) * epb);
   for (int i = tid; i < 144; i += blockDim.x) bw[i] = P.bw_tab[(size_t)slot * 144 + i];
@@ -1772,21 +1679,31 @@ __device__ void avg_slab(const EngPtrs &P, int slab, int slot, const RveDev *R,
 #pragma unroll
     for (int i = 0; i < 12; i++) acc[i] = 0.0;
     for (int e = ls * epb + tid; e < e_end; e += blockDim.x) {
-      const int ex = e % R->nex, ey = (e / R->nex) % R->ney, ez = e / (R->nex * R->ney);
-      const int n0 = ex + ey * R->nx + ez * R->nx * R->ny;
+      const int ex = e % nex, ey = (e / nex) % ney, ez = e / (nex * ney);
+      const int n0 = ex + ey * nx + ez * nx * ny;
       const int mat = P.elem_mat[R->elem_base + e];
       const double *C = cm + mat * 36;
       double eps[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-#pragma unroll 1
+      // the eight nodes' loads together: one round trip in place of eight
+      double xv[8][3];
+#pragma unroll
       for (int a = 0; a < 8; a++) {
         int lx, ly, lz;
         local_coords(a, &lx, &ly, &lz);
-        const int node = n0 + lx + ly * R->nx + lz * R->nx * R->ny;
-        for (int dd = 0; dd < 3; dd++) {
-          const double xv = P.x64[node_vec(P, R->first_slab, node, K) + (long long)k * 3 * P.SN + dd];
+        const int node = n0 + lx + ly * nx + lz * nx * ny;
 #pragma unroll
-          for (int vv = 0; vv < 6; vv++) eps[vv] += bw[vv * 24 + 3 * a + dd] * xv;
-        }
+        for (int dd = 0; dd < 3; dd++)
+          xv[a][dd] = P.x64[node_vec(P, first, node, K) + (long long)k * 3 * P.SN + dd];
+      }
+      int at = 0;
+      asm volatile("" : "+s"(at));  // B w is read again from the LDS, not kept in registers
+#pragma unroll
+      for (int a = 0; a < 8; a++) {
+#pragma unroll
+        for (int dd = 0; dd < 3; dd++)
+#pragma unroll
+          for (int vv = 0; vv < 6; vv++) eps[vv] += bw[at + vv * 24 + 3 * a + dd] * xv[a][dd];
+        __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int vv = 0; vv < 6; vv++) {
@@ -1796,9 +1713,8 @@ __device__ void avg_slab(const EngPtrs &P, int slab, int slot, const RveDev *R,
         acc[6 + vv] += s;
       }
     }
-    block_sum<12>(acc, lds);
-    if (tid == 0)
-      for (int i = 0; i < 12; i++) part[k * 12 + i] = acc[i];
+    const double sum = block_sum_lane<12>(acc, lds);
+    if (tid < 12) part[k * 12 + tid] = sum;
   }
 }
 
@@ -1809,6 +1725,18 @@ __device__ void r_slab(const EngPtrs &P, int slab, double (&lds)[RedLds<K>::size
   const int tid = threadIdx.x;
   const int slot = P.slab_rve[slab];
   RveDev *R = P.rves + slot;
+  if (R->scw > 0) {
+    // a resident RVE: from k_sweep's state to the next launch's
+    __shared__ SolveState N;
+    if (slab == R->first_slab && tid == 0) {
+      N = R->st[0];
+      sweep_end<TS, K>(P, R, N);
+      R->st[2] = N;
+      *P.ticket = 0u;  // for the next resident sweep
+    }
+    if (R->st[0].phase == PH_AVG) avg_slab<TS, K>(P, slab, slot, R, lds);
+    return;
+  }
   const SolveState *S = &R->st[1];
   const int phase = S->phase;
   if (slab == R->first_slab && tid == 0) {
@@ -1875,8 +1803,9 @@ __global__ __launch_bounds__(256) void k_step_r(EngPtrs P, SolveParams sp)
   for_slabs_with_work(
       P,
       [](int slab, const RveDev *R) {
-        const int ph = R->st[1].phase;
-        return slab == R->first_slab || ph == PH_RES || ph == PH_AVG;
+        const bool own = R->scw > 0;  // a resident RVE's residual is k_sweep_res's
+        const int ph = R->st[own ? 0 : 1].phase;
+        return slab == R->first_slab || (ph == PH_RES && !own) || ph == PH_AVG;
       },
       [&](int slab) { r_slab<TS, K>(P, slab, lds); });
 }
@@ -1981,8 +1910,15 @@ static int launch_steps(const EngPtrs &P, const SolveParams &sp, int grid, int f
         if (P.a_slab) k_step_a<TS, K, DICT><<<grid, P.SN, 0, s>>>(P, sp);
         if (P.s_big) k_step_s<TS, K><<<grid < kRGrid ? grid : kRGrid, P.SN, 0, s>>>(P);
         break;
-      case 1: k_step_b<TS, K><<<grid, P.SN, 0, s>>>(P, sp); break;
-      default: k_step_r<TS, K><<<grid < kRGrid ? grid : kRGrid, P.SN, 0, s>>>(P, sp); break;
+      case 1:  // unless every RVE is resident
+        if (P.a_lds > 0 || P.a_slab) k_step_b<TS, K><<<grid, P.SN, 0, s>>>(P, sp);
+        break;
+      default:
+        if (P.u_grid > 0) {
+          const int rc = eng_launch_sweep_res(sizeof(TS) == 8, K, P, grid, s);
+          if (rc) return rc;
+        }
+        k_step_r<TS, K><<<grid < kRGrid ? grid : kRGrid, P.SN, 0, s>>>(P, sp);
     }
   }
   MM_HIP(hipGetLastError());

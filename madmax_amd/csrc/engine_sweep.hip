@@ -22,8 +22,8 @@
 //   waiting for r.r / r.z before w = A z instead of behind it: 31 us;
 //   the planes above and below one by one: 243 multiply-adds, 27.8 to 30.7 us.
 // Whole solves (rtol 1e-10), kernels A and B and this: 128 x 30^3 tangents 187 and
-// 62 ms, 64 uneven cells 8^3 .. 32^3 50 and 13.8 ms, 24 x 20^3 in FP64 25.5 and 6.0
-// ms, one 10^3 4.7 and 0.87.
+// 60 ms, 64 uneven cells 8^3 .. 32^3 50 and 12.7 ms, 24 x 20^3 in FP64 25.5 and 5.6
+// ms, one 10^3 4.7 and 0.77.
 // Sharing the rows: 32 x 33 x 36 x 40 tangents 122 and 44 ms, 4 x 60^3 93 and 32;
 // one load case of 48^3 7.9 and 4.1 ms, of 100^3 (195 workgroups) 50 and 17, 74 us
 // an iteration by kernels A, S, B and R and 25 here.
@@ -178,20 +178,17 @@ __device__ __forceinline__ void sweep_key(const TS *Db, const X &x, TS (&w)[LP][
   }
 }
 
-// w += the nine blocks of the columns at dy, whose rows start at zr: those of the
-// node's own plane, then the planes below and above together.  The cell is the
+// w += the nine blocks of the columns at dy, of which the lane's has the rows x
+// (from the plane below the first node): those of the node's own plane, then the planes below and above together.  The cell is the
 // same mirrored in z (the phases do not vary along z), so the block below is the
 // block above with the signs of its xz, yz, zx and zy entries changed: of z above
 // and below, the sum goes with the others and the difference with these.  That
 // takes 162 multiply-adds and 18 adds per node in place of 243, two thirds of the
 // dictionary's reads, and reads a column's z once.
 template <typename TS, int LP>
-__device__ __forceinline__ void sweep_strip(const TS *zr, int ps, const TS *dict, int dy, TS (&w)[LP][3])
+__device__ __forceinline__ void sweep_rows(const TS (&x)[LP + 2][3], const TS *dict, int dy, TS (&w)[LP][3])
 {
   constexpr int blk = sweep_dict_block((int)sizeof(TS));
-  TS x[LP + 2][3];
-#pragma unroll
-  for (int l = 0; l < LP + 2; l++) lds_read3(zr + l * ps, x[l]);
   {
     const TS *Db = dict + (3 * dy + 9) * blk;
     const auto own = [&](int l, int e, int) -> const TS & { return x[l + 1][e]; };
@@ -212,6 +209,31 @@ __device__ __forceinline__ void sweep_strip(const TS *zr, int ps, const TS *dict
   sweep_key<TS, LP, 0>(Db, pair, w);
   sweep_key<TS, LP, 1>(Db, pair, w);
   sweep_key<TS, LP, 2>(Db, pair, w);
+}
+
+// The same for rows in LDS from zr.
+template <typename TS, int LP>
+__device__ __forceinline__ void sweep_strip(const TS *zr, int ps, const TS *dict, int dy, TS (&w)[LP][3])
+{
+  TS x[LP + 2][3];
+#pragma unroll
+  for (int l = 0; l < LP + 2; l++) lds_read3(zr + l * ps, x[l]);
+  sweep_rows<TS, LP>(x, dict, dy, w);
+}
+
+// The LDS dictionary of an RVE, by `lanes` lanes: the blocks of the 16 patterns
+// that repeat along z, rounded from the FP64 dictionary D (the values of the
+// solver dictionary), and an entry of zeros.
+template <typename TS>
+__device__ __forceinline__ void sweep_dict_load(TS *dict, const double *D, int lanes)
+{
+  constexpr int stride = sweep_dict_stride((int)sizeof(TS)), blk = sweep_dict_block((int)sizeof(TS));
+  for (int i = threadIdx.x; i < stride; i += lanes) dict[16 * stride + i] = (TS)0;
+  for (int i = threadIdx.x; i < 16 * 27 * 9; i += lanes) {
+    const int e = i / (27 * 9), o = i - e * (27 * 9), key = o / 9, j = o - key * 9;
+    dict[e * stride + key * blk + (j / 3) * (blk / 3) + j % 3] =
+        (TS)D[(size_t)(e * 17) * kDictEntry + key * kDictBlk + (j / 3) * 4 + j % 3];
+  }
 }
 
 // Bound on a wait in polls (half a minute or more).  A rank waits for the
@@ -674,8 +696,7 @@ extern __shared__ __attribute__((aligned(16))) double sweep_dyn[];
 // kSweepFreeRanks workgroups waiting, and the GPU has more places than the
 // queues' launches can fill with those; a larger cluster waits only before it has
 // started, and not for long: cluster_meet).
-// A sweep's end (its iteration count is the largest of the load cases') is
-// entered into the state by kernel B.
+// The residual follows (k_sweep_res), and kernel R passes the state on.
 template <typename TS, int K>
 __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp)
 {
@@ -702,7 +723,7 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
     if (!writer) return;
     if (tid == 0) N = R->st[2];
     __syncthreads();
-    finish_rve<K>(P, slot, R, N, sp, lds);
+    finish_rve<K>(P, slot, R, N, sp);
     if (tid == 0) R->st[0] = N;
     return;
   }
@@ -725,15 +746,8 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   }
   TS *dict = reinterpret_cast<TS *>(sweep_dyn);
   TS *zl = reinterpret_cast<TS *>(reinterpret_cast<unsigned char *>(sweep_dyn) + sweep_dict_bytes(tsz));
-  // the 16 blocks of patterns that repeat along z, rounded from the FP64
-  // dictionary (the values of the solver dictionary)
   const double *D = P.dict64 + (size_t)slot * kDictPat * kDictEntry;
-  for (int i = tid; i < sweep_dict_stride(tsz); i += kSweepLanes) dict[16 * sweep_dict_stride(tsz) + i] = (TS)0;
-  for (int i = tid; i < 16 * 27 * 9; i += kSweepLanes) {
-    const int e = i / (27 * 9), o = i - e * (27 * 9), key = o / 9, j = o - key * 9;
-    dict[e * sweep_dict_stride(tsz) + key * sweep_dict_block(tsz) + (j / 3) * (sweep_dict_block(tsz) / 3) + j % 3] =
-        (TS)D[(size_t)(e * 17) * kDictEntry + key * kDictBlk + (j / 3) * 4 + j % 3];
-  }
+  sweep_dict_load<TS>(dict, D, kSweepLanes);
   for (int i = tid; i < 16 * 3; i += kSweepLanes) {
     const int e = i / 3, d = i - e * 3;
     // the solver's dinv of a node of that pattern, and its reciprocal
@@ -766,6 +780,122 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   if (rk == 0 && tid == 0) R->lits[k] = n;
 }
 
+// The resident RVEs' FP64 residual (kernel R does the others'), between sweeps:
+// r = -K x64, z = dinv r, the partial sums of kernel R, and the words of the next
+// sweep zeroed.  The state is still k_sweep's (st[0]); kernel R passes it on.
+//
+// Workgroup b of an RVE takes items b * kResWaves + wave, + nslab * kResWaves, ..:
+// a strip of 62 positions of a plane's rows, kResPlanes nodes of each column and
+// one load case, with the sweep's product (sweep_rows) on rows read from memory.
+// x-neighbours come from the lanes beside, the dictionary from LDS.  Bound by
+// vector issue (180 FP64 operations per node, and 54 moves between lanes).  Kernel
+// R gathers 27 neighbours per node through L1, 81 reads in place of 13.5, and took
+// 22 us for one 10^3 cell with 6 load cases and 100 for 24 cells of 12^3 .. 30^3
+// with 7; this takes 14 and, with the boundary part twice, 82.
+constexpr int kResWaves = 4;
+constexpr int kResPlanes = 4;
+
+template <typename TS, int K>
+__global__ __launch_bounds__(64 * kResWaves) void k_sweep_res(EngPtrs P)
+{
+  __shared__ double acc[kResWaves][4 * K];
+  int slab;
+  if (!active_slab(P, slab)) return;
+  slab = scalar(slab);
+  const int slot = scalar(P.slab_rve[slab]);
+  if (slot < 0) return;
+  const RveDev *R = P.rves + slot;
+  if (scalar(R->scw) == 0 || !sweep_ran<TS, K>(P, R)) return;
+  const bool cold = scalar((R->warm || R->affine) && R->st[0].phase == PH_RES && R->st[0].sweep == 0) != 0;
+  const int tid = threadIdx.x, ln = tid & 63, wv = tid >> 6;
+  const int nx = scalar(R->nx), ny = scalar(R->ny), nz = scalar(R->nz), nxy = nx * ny;
+  const int fs = scalar(R->first_slab), nslab = scalar(R->nslab), nload = scalar(R->nload);
+  const int SN = P.SN, RS = 3 * SN, b = slab - fs;
+  const int npos = nx * (ny - 2), nstrip = (npos + kSweepStrip - 1) / kSweepStrip;
+  const int nrun = (nz - 2 + kResPlanes - 1) / kResPlanes, items = nstrip * nrun * nload;
+  if (R->scw > 1) sweep_words_zero<TS, K>(P, R, slab);
+  double *dict = sweep_dyn;
+  for (int i = tid; i < kResWaves * 4 * K; i += 64 * kResWaves) (&acc[0][0])[i] = 0.0;
+  if (b * kResWaves < items) sweep_dict_load<double>(dict, P.dict64 + (size_t)slot * kDictPat * kDictEntry, 64 * kResWaves);
+  __syncthreads();
+#pragma unroll 1
+  for (int it = scalar(b * kResWaves + wv); it < items; it += nslab * kResWaves) {
+    const int k = it % nload, u = it / nload, run = u % nrun, st = u / nrun;
+    const int zf = 1 + run * kResPlanes, cnt = min(kResPlanes, nz - 1 - zf);
+    const int pos = st * kSweepStrip + ln - 1, pc = min(max(pos, 0), npos - 1);
+    const int iy = pc / nx, ix = pc - iy * nx;  // row iy + 1 of the plane
+    const bool bx = ix == 0 || ix == nx - 1;
+    const bool on = ln >= 1 && ln <= kSweepStrip && pos < npos && !bx;
+    const int n0 = ix + (iy + 1) * nx + zf * nxy;
+    const int pat = P.npat[(long long)(fs + (n0 >> P.sn_shift)) * SN + (n0 & (SN - 1))] & 15;
+    const double *Db = dict + (on ? pat : 16) * sweep_dict_stride(8);
+    double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+    for (int pass = 0; pass <= (cold ? 1 : 0); pass++) {  // pass 1: the boundary nodes' part alone
+      double w[kResPlanes][3];
+#pragma unroll
+      for (int l = 0; l < kResPlanes; l++)
+#pragma unroll
+        for (int d = 0; d < 3; d++) w[l][d] = 0.0;
+#pragma unroll 1
+      for (int dy = 0; dy < 3; dy++) {
+        const bool column = pass == 0 || bx || iy + dy == 0 || iy + dy == ny - 1;
+        double x[kResPlanes + 2][3];
+#pragma unroll
+        for (int l = 0; l < kResPlanes + 2; l++) {
+          const int z = min(zf - 1 + l, nz - 1), m = n0 + (dy - 1) * nx + (z - zf) * nxy;
+          const double *src = P.x64 + ((long long)(fs + (m >> P.sn_shift)) * K + k) * RS + 3 * (m & (SN - 1));
+          const bool keep = column || z == 0 || z == nz - 1;
+#pragma unroll
+          for (int d = 0; d < 3; d++) x[l][d] = keep ? src[d] : 0.0;
+        }
+        sweep_rows<double, kResPlanes>(x, Db, dy, w);
+      }
+#pragma unroll
+      for (int l = 0; l < kResPlanes; l++) {
+        if (!on || l >= cnt) continue;
+        const int m = n0 + l * nxy;
+        const long long sl = fs + (m >> P.sn_shift);
+        const int row = 3 * (m & (SN - 1));
+        const TS *dinv = (const TS *)P.dinv + sl * RS + row;
+        TS *z = (TS *)P.z + (sl * K + k) * RS + row;
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+          const double r64 = -w[l][d];
+          if (pass == 0) {
+            const TS r = (TS)r64, zi = dinv[d] * r;
+            z[d] = zi;
+            v[0] = fma(r64, r64, v[0]);
+            v[1] = fma((double)r, (double)r, v[1]);
+            v[2] = fma((double)r, (double)zi, v[2]);
+          } else {
+            v[3] = fma(r64, r64, v[3]);
+          }
+        }
+      }
+    }
+    int q;
+    const double t = wave_sum4(v, q);
+    if ((ln & 15) == 0) acc[wv][q * K + k] += t;
+  }
+  __syncthreads();
+  if (tid < 4 * K) {
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < kResWaves; w++) t += acc[w][tid];
+    slab_part(P, slab)[3 * K + tid] = t;
+  }
+}
+
+template <typename TS, int K>
+static int launch_sweep_res(const EngPtrs &P, int grid, hipStream_t s)
+{
+  if (grid <= 0) return MM_ERR_ARG;
+  k_sweep_res<TS, K><<<grid, 64 * kResWaves, sweep_dict_bytes(8), s>>>(P);
+  MM_HIP(hipGetLastError());
+  return 0;
+}
+
 template <typename TS, int K>
 static int launch_sweep(const EngPtrs &P, const SolveParams &sp, hipStream_t s)
 {
@@ -796,6 +926,11 @@ static int launch_sweep(const EngPtrs &P, const SolveParams &sp, hipStream_t s)
 int eng_launch_sweep(bool fp64, int K, const EngPtrs &P, const SolveParams &sp, hipStream_t s)
 {
   MM_SWEEP_DISPATCH(fp64, K, launch_sweep, P, sp, s);
+}
+
+int eng_launch_sweep_res(bool fp64, int K, const EngPtrs &P, int grid, hipStream_t s)
+{
+  MM_SWEEP_DISPATCH(fp64, K, launch_sweep_res, P, grid, s);
 }
 
 }  // namespace mm

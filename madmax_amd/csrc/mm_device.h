@@ -39,6 +39,20 @@ __device__ __forceinline__ double halve(double a, double b)
   return __builtin_bit_cast(double, p) + __builtin_bit_cast(double, q);
 }
 
+// Sums four values over a wave (lanes 32, 16, 8, 4, 2 and 1 apart); lanes 0, 32, 16
+// and 48 return the sum of value q = 0, 1, 2 and 3.
+__device__ __forceinline__ double wave_sum4(const double (&v)[4], int &q)
+{
+  const int lane = threadIdx.x & 63;
+  double t = halve<16>(halve<32>(v[0], v[1]), halve<32>(v[2], v[3]));
+  t += dpp_move<0x108>(t);  // row_shl:8, 4, 2, 1: lane l takes lane l + 8 ... of its 16
+  t += dpp_move<0x104>(t);
+  t += dpp_move<0x102>(t);
+  t += dpp_move<0x101>(t);
+  q = (lane >> 5) + 2 * ((lane >> 4) & 1);
+  return t;
+}
+
 // Sums NV values over the block in a fixed order; returns the sum of value i in
 // thread i < NV.  lds holds 16 doubles per value (blockDim.x <= 1024); its size
 // is checked at compile time.  Each wave adds lanes 32, 16, 8, 4, 2 and 1 apart,
@@ -55,16 +69,10 @@ __device__ inline double block_sum_lane(const double (&v)[NV], double (&lds)[L])
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
 #pragma unroll
   for (int i = 0; i < NV; i += 4) {
-    const double a = halve<32>(v[i], i + 1 < NV ? v[i + 1] : v[i]);
-    const double b = i + 2 < NV ? halve<32>(v[i + 2], i + 3 < NV ? v[i + 3] : v[i + 2]) : a;
-    double t = halve<16>(a, b);
-    t += dpp_move<0x108>(t);  // row_shl:8, 4, 2, 1: lane l takes lane l + 8 ... of its 16
-    t += dpp_move<0x104>(t);
-    t += dpp_move<0x102>(t);
-    t += dpp_move<0x101>(t);
-    // lanes 0, 32, 16 and 48: values i, i + 1, i + 2 and i + 3
-    const int k = i + (lane >> 5) + 2 * ((lane >> 4) & 1);
-    if ((lane & 15) == 0 && k < NV) lds[k * 16 + wid] = t;
+    const double v4[4] = {v[i], v[i + 1 < NV ? i + 1 : i], v[i + 2 < NV ? i + 2 : i], v[i + 3 < NV ? i + 3 : i]};
+    int q;
+    const double t = wave_sum4(v4, q);
+    if ((lane & 15) == 0 && i + q < NV) lds[(i + q) * 16 + wid] = t;
     __builtin_amdgcn_sched_barrier(0);  // (NV sums at a time would take many registers)
   }
   __syncthreads();

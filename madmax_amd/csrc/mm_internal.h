@@ -292,6 +292,8 @@ int eng_launch_steps(bool fp64, int K, bool dict, const EngPtrs &P, const SolveP
                      int first, int nkern, hipStream_t s);
 // the resident sweep of the RVEs in P.units
 int eng_launch_sweep(bool fp64, int K, const EngPtrs &P, const SolveParams &sp, hipStream_t s);
+// their residual; grid covers the active slabs
+int eng_launch_sweep_res(bool fp64, int K, const EngPtrs &P, int grid, hipStream_t s);
 int eng_launch_dict(bool fp64, int n, const int *slots, const double *ke_tab, void *dict, hipStream_t s);
 int eng_launch_assemble(bool fp64, int K, const EngPtrs &P, int nblk, const int *slab_list, int mode,
                         hipStream_t s);
