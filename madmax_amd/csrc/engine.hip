@@ -73,10 +73,16 @@ struct RangeAlloc {
 };
 
 // Solver steps per launch where every RVE is solved by resident sweeps: the
-// first residual, up to three sweeps, the averages and the result.
-constexpr int kSweepSteps = 6;
+// first residual, up to two sweeps, the averages and the result (a step without
+// work is 15 us of launches, a second launch with its synchronisation 50).
+constexpr int kSweepSteps = 5;
 
 enum SlotState { SL_FREE = 0, SL_ACTIVE = 1, SL_CACHED = 2 };
+
+// Split of a resident sweep (RveDev::scw ..), cw = 0: kernels A and B.
+struct SweepTiling {
+  int cw = 0, ty = 1, lp = 0, nch = 0;
+};
 
 struct HostSlot {
   int state = SL_FREE;
@@ -86,6 +92,7 @@ struct HostSlot {
   int prev_nload = 0;
   long long first_slab = 0, nslab = 0, elem_base = 0, nelm = 0;
   int nrow = 0;
+  SweepTiling sweep;
   double t_submit = 0, t_admit = 0;
   uint64_t lru = 0;
 };
@@ -179,6 +186,7 @@ struct mm_engine {
   void *d = nullptr, *z = nullptr, *p = nullptr, *q = nullptr;
   double *part = nullptr;
   int *slab_rve = nullptr, *slab_node0 = nullptr;
+  std::vector<int2> freed;  // (first slab, slabs) released but still in slab_rve
   RveDev *rves = nullptr;
   uint8_t *elem_mat = nullptr;
   uint8_t *npat = nullptr;
@@ -599,12 +607,38 @@ extern "C" int mm_engine_submit(mm_engine *e, const mm_request *req)
   return 0;
 }
 
+// Marks the slabs released since the last call as nobody's, adjacent runs
+// together.  Solver launches never name such a slab, so this waits until slabs
+// change hands or a kernel looks at all of them.
+static int flush_freed(mm_engine *e)
+{
+  if (e->freed.empty()) return 0;
+  std::sort(e->freed.begin(), e->freed.end(), [](const int2 &a, const int2 &b) { return a.x < b.x; });
+  SlabRuns r;
+  r.n = 0;
+  for (size_t i = 0; i < e->freed.size(); i++) {
+    const int2 f = e->freed[i];
+    if (r.n > 0 && r.run[r.n - 1].x + r.run[r.n - 1].y == f.x) {
+      r.run[r.n - 1].y += f.y;
+      continue;
+    }
+    if (r.n == kSlabRuns) {
+      const int rc = eng_launch_unown(r, e->slab_rve, e->stream);
+      if (rc) return rc;
+      r.n = 0;
+    }
+    r.run[r.n++] = f;
+  }
+  e->freed.clear();
+  return eng_launch_unown(r, e->slab_rve, e->stream);
+}
+
 static void release_slot_resources(mm_engine *e, int slot)
 {
   HostSlot &h = e->slots[slot];
   e->slabs.release(h.first_slab, h.nslab);
   e->elems.release(h.elem_base, h.nelm);
-  (void)hipMemsetAsync(e->slab_rve + h.first_slab, 0xff, (size_t)h.nslab * 4, e->stream);
+  e->freed.push_back(make_int2((int)h.first_slab, (int)h.nslab));
   if (h.req.warm_key) {
     auto it = e->warm_map.find(h.req.warm_key);
     if (it != e->warm_map.end() && it->second == slot) e->warm_map.erase(it);
@@ -772,10 +806,6 @@ static int march_lds_need(const mm_engine *e, const HostSlot &h)
 // are single PCG iterations by request: sync_every_step reads the state after
 // each, profile_step_kernel times each one's kernel A.  Fixed by the RVE and the
 // engine configuration alone.
-struct SweepTiling {
-  int cw = 0, ty = 1, lp = 0, nch = 0;
-};
-
 // Enters ty shares of the rows times cz of the planes into t if they fit and cost
 // less than its `best`; cost(workgroups, time).
 template <typename Cost>
@@ -882,7 +912,7 @@ static void fill_state(const mm_engine *e, const HostSlot &h, RveDev *st, int wa
   st->mnzc = mt.mnzc;
   st->mnt = mt.mnt;
   st->mncg = mt.mncg;
-  const SweepTiling sw = sweep_tiling(e, s, h.nslab);
+  const SweepTiling &sw = h.sweep;
   st->scw = sw.cw;
   st->sty = sw.ty;
   st->slp = sw.lp;
@@ -983,7 +1013,8 @@ static int admit(mm_engine *e)
   if ((rc = ensure_device(&e->dv_slabs, &e->dcap_slabs, nsl + nsl_re + 1))) return rc;
   size_t i = 0, ik = 0, ip = 0, is = 0;
   for (int s : fresh) {
-    const HostSlot &h = e->slots[s];
+    HostSlot &h = e->slots[s];
+    h.sweep = sweep_tiling(e, h.req.rve, h.nslab);
     fill_state(e, h, &e->st_states[i], 0);
     e->st_slots[i++] = s;
     for (int m = 0; m < kNmat; m++) {
@@ -1002,15 +1033,14 @@ static int admit(mm_engine *e)
   }
   for (int s : fresh) e->out_host[s].phase = 0;
   for (int s : reused) e->out_host[s].phase = 0;
-  MM_HIP(hipMemcpyAsync(e->dv_states, e->st_states, n * sizeof(RveDev), hipMemcpyHostToDevice, e->stream));
-  MM_HIP(hipMemcpyAsync(e->dv_slots, e->st_slots, n * sizeof(int), hipMemcpyHostToDevice, e->stream));
-  if (nke)
-    MM_HIP(hipMemcpyAsync(e->dv_ke, e->st_ke, 2 * nke * sizeof(int), hipMemcpyHostToDevice, e->stream));
-  if (nph)
-    MM_HIP(hipMemcpyAsync(e->dv_phase, e->st_phase, nph * sizeof(int2), hipMemcpyHostToDevice, e->stream));
-  if (nsl + nsl_re)
-    MM_HIP(hipMemcpyAsync(e->dv_slabs, e->st_slabs, (nsl + nsl_re) * sizeof(int), hipMemcpyHostToDevice,
-                          e->stream));
+  if ((rc = flush_freed(e))) return rc;
+  CopyIn in;
+  in.add(e->dv_states, e->st_states, n * sizeof(RveDev));
+  in.add(e->dv_slots, e->st_slots, n * sizeof(int));
+  in.add(e->dv_ke, e->st_ke, 2 * nke * sizeof(int));
+  in.add(e->dv_phase, e->st_phase, nph * sizeof(int2));
+  in.add(e->dv_slabs, e->st_slabs, (nsl + nsl_re) * sizeof(int));
+  if ((rc = eng_launch_copy_in(in, e->stream))) return rc;
   EngPtrs P = e->ptrs();
   if ((rc = eng_launch_admit((int)n, e->dv_slots, e->dv_states, e->rves, e->slab_rve, e->slab_node0, e->SN,
                              e->stream)))
@@ -1069,7 +1099,7 @@ static int update_active(mm_engine *e)
   for (auto &r : runs) {
     const HostSlot &h = e->slots[r.second];
     if (half == 0 && ngroup == 2 && n[0] > 0 && 2 * n[0] >= total) half = 1;
-    const SweepTiling sw = sweep_tiling(e, h.req.rve, h.nslab);
+    const SweepTiling &sw = h.sweep;
     // clusters that need most of the CUs at once stay in one chain of launches
     const int g = sw.cw > kSweepFreeRanks ? 0 : half;
     for (long long b = 0; b < h.nslab; b++) e->st_act[g * stride + 1 + n[g]++] = (int)(r.first + b);
@@ -1086,15 +1116,13 @@ static int update_active(mm_engine *e)
       slab_mode[g] = 1;
     }
   }
+  CopyIn in;
   for (int q = 0; q < 2; q++) {
     e->st_act[q * stride] = (int)n[q];
     e->st_act[(2 + q) * stride] = (int)nt[q];
     if (q < ngroup) {
-      MM_HIP(hipMemcpyAsync(e->act_list + q * stride, e->st_act + q * stride, (size_t)(n[q] + 1) * 4,
-                            hipMemcpyHostToDevice, e->stream));
-      if (march)
-        MM_HIP(hipMemcpyAsync(e->act_list + (2 + q) * stride, e->st_act + (2 + q) * stride,
-                              (size_t)(nt[q] + 1) * 4, hipMemcpyHostToDevice, e->stream));
+      in.add(e->act_list + q * stride, e->st_act + q * stride, (size_t)(n[q] + 1) * 4);
+      if (march) in.add(e->act_list + (2 + q) * stride, e->st_act + (2 + q) * stride, (size_t)(nt[q] + 1) * 4);
     }
     // the largest RVEs first, so that the last workgroups to finish are short
     std::stable_sort(res[q].begin(), res[q].end(),
@@ -1105,9 +1133,7 @@ static int update_active(mm_engine *e)
       for (int k = 0; k < e->slots[r.second.x].req.nload; k++)
         for (int c = 0; c < r.second.y; c++) un[1 + nu++] = make_int2(r.second.x, k * kSweepUnitRanks + c);
     un[0] = make_int2((int)nu, 0);
-    if (q < ngroup)
-      MM_HIP(hipMemcpyAsync(e->units + q * e->unit_stride, un, (size_t)(nu + 1) * sizeof(int2),
-                            hipMemcpyHostToDevice, e->stream));
+    if (q < ngroup) in.add(e->units + q * e->unit_stride, un, (size_t)(nu + 1) * sizeof(int2));
     e->unit_n[q] = nu;
     e->act_n[q] = n[q];
     e->tile_n[q] = nt[q];
@@ -1115,6 +1141,8 @@ static int update_active(mm_engine *e)
     e->a_slab[q] = slab_mode[q];
     e->s_big[q] = big[q];
   }
+  const int rc = eng_launch_copy_in(in, e->stream);
+  if (rc) return rc;
   e->act_dirty = false;
   return 0;
 }
@@ -1193,7 +1221,7 @@ static int run_steps(mm_engine *e)
   const int grid0 = launch_grid(e->act_n[0]), grid1 = launch_grid(e->act_n[1]);
   if (grid0 == 0 && grid1 == 0) return 0;
   // where every RVE is resident a step is a whole sweep: kSweepSteps of them
-  // finish a solve of up to three sweeps
+  // finish a solve of up to two sweeps
   int nsteps = e->cfg.steps_per_launch;
   if (e->tile_n[0] + e->tile_n[1] == 0 && !e->a_slab[0] && !e->a_slab[1]) nsteps = std::min(nsteps, kSweepSteps);
   if (!e->cfg.use_graph) return queue_steps(e, grid0, grid1, nsteps);
@@ -1589,7 +1617,9 @@ static int time_kernel(mm_engine *e, int what, int reps, double *avg_ms, double 
   hipEvent_t a, b;
   MM_HIP(hipEventCreate(&a));
   MM_HIP(hipEventCreate(&b));
-  int rc = eng_launch_time(e->fp64, e->K, e->dict_mode, P, grid, what, e->stream);  // warm-up
+  int rc = flush_freed(e);
+  if (rc) return rc;
+  rc = eng_launch_time(e->fp64, e->K, e->dict_mode, P, grid, what, e->stream);  // warm-up
   if (rc) return rc;
   MM_HIP(hipEventRecord(a, e->stream));
   for (int i = 0; i < reps; i++) {

@@ -78,11 +78,27 @@ __global__ void k_admit(int n, const int *__restrict__ slots, const RveDev *__re
   if (i >= n) return;
   const int slot = slots[i];
   const RveDev &st = states[i];
-  if (threadIdx.x == 0) rves[slot] = st;
+  static_assert(sizeof(RveDev) % 4 == 0, "copied in words");
+  for (int w = threadIdx.x; w < (int)(sizeof(RveDev) / 4); w += blockDim.x)
+    reinterpret_cast<unsigned *>(rves + slot)[w] = reinterpret_cast<const unsigned *>(states + i)[w];
   for (int s = threadIdx.x; s < st.nslab; s += blockDim.x) {
     slab_rve[st.first_slab + s] = slot;
     slab_node0[st.first_slab + s] = s * SN;
   }
+}
+
+__global__ __launch_bounds__(256) void k_copy_in(CopyIn c)
+{
+  const size_t step = (size_t)gridDim.x * blockDim.x;
+  for (int p = 0; p < c.n; p++)
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < c.words[p]; i += step) c.dst[p][i] = c.src[p][i];
+}
+
+__global__ __launch_bounds__(256) void k_unown(SlabRuns r, int *__restrict__ slab_rve)
+{
+  const int step = gridDim.x * blockDim.x;
+  for (int p = 0; p < r.n; p++)
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < r.run[p].y; i += step) slab_rve[r.run[p].x + i] = -1;
 }
 
 // Element stiffness per (RVE, material), one wavefront each.  The derivatives
@@ -2013,6 +2029,28 @@ int eng_launch_time(bool fp64, int K, bool dict, const EngPtrs &P, int grid, int
 #define CALL_TIME(T, KK) launch_time<T, KK, false>(P, grid, what, s)
   MM_DISPATCH(fp64, K, CALL_TIME);
 #undef CALL_TIME
+}
+
+int eng_launch_copy_in(const CopyIn &c, hipStream_t s)
+{
+  size_t most = 0;
+  for (int p = 0; p < c.n; p++) most = c.words[p] > most ? c.words[p] : most;
+  if (most == 0) return 0;
+  const size_t grid = (most + 255) / 256;
+  k_copy_in<<<(unsigned)(grid < 512 ? grid : 512), 256, 0, s>>>(c);
+  MM_HIP(hipGetLastError());
+  return 0;
+}
+
+int eng_launch_unown(const SlabRuns &r, int *slab_rve, hipStream_t s)
+{
+  int most = 0;
+  for (int p = 0; p < r.n; p++) most = r.run[p].y > most ? r.run[p].y : most;
+  if (most == 0) return 0;
+  const int grid = (most + 255) / 256;
+  k_unown<<<grid < 512 ? grid : 512, 256, 0, s>>>(r, slab_rve);
+  MM_HIP(hipGetLastError());
+  return 0;
 }
 
 int eng_launch_admit(int n, const int *slots, const RveDev *states, RveDev *rves, int *slab_rve,

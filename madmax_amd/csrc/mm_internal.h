@@ -284,7 +284,32 @@ __host__ __device__ constexpr int sweep_sum_words(int cw) { return 16 * cw + 2; 
 // assembly modes
 enum AsmMode : int { ASM_FULL = 0, ASM_X_ONLY = 1, ASM_DICT = 2 };
 
+// Pieces of pinned host memory that one kernel copies to the device: a launch in
+// place of as many copies, 8 us each.  Whole 32-bit words.
+constexpr int kCopyPieces = 6;
+struct CopyIn {
+  const unsigned *src[kCopyPieces];
+  unsigned *dst[kCopyPieces];
+  size_t words[kCopyPieces];
+  int n = 0;
+  void add(void *d, const void *s, size_t bytes)
+  {
+    if (bytes == 0) return;
+    src[n] = (const unsigned *)s;
+    dst[n] = (unsigned *)d;
+    words[n++] = bytes / 4;
+  }
+};
+// Runs of slabs (first, count).
+constexpr int kSlabRuns = 32;
+struct SlabRuns {
+  int2 run[kSlabRuns];
+  int n;
+};
+
 // launchers (engine_kernels.hip)
+int eng_launch_copy_in(const CopyIn &c, hipStream_t s);
+int eng_launch_unown(const SlabRuns &r, int *slab_rve, hipStream_t s);
 int upload_slot_tables(hipStream_t s);
 bool eng_supported_rhs(int K);
 // nkern solver launches of the cycle A (0) -> B (1) -> R (2), from `first`
