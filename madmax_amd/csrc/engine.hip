@@ -819,10 +819,10 @@ static void sweep_split(const mm_rve_spec &s, int tsz, int ty, int cz, const Cos
   const long long fit = (kSweepMaxLds - sweep_dict_bytes(tsz)) / plane;  // planes
   for (long long nch = 1; nch <= L && nch * ns <= items; nch++) {
     const long long lp = (L + nch - 1) / nch;
-    if (lp > sweep_max_planes(tsz) || sweep_lds_planes((int)lp, (int)nch) > fit) continue;
+    if (lp > sweep_max_planes(tsz) || sweep_lds_planes(tsz, (int)lp, (int)nch) > fit) continue;
     // an iteration's time in planes of a strip: the longest wave's items, each
     // with its latency, or the fullest SIMD's, and the barriers and sums
-    const double S = (double)(ns * nch), u = sweep_unroll((int)lp);
+    const double S = (double)(ns * nch), u = sweep_unroll(tsz, (int)lp);
     const double time = std::max(std::ceil(S / waves) * (u + 4.0), std::ceil(S / 4.0) * (u + 1.0)) +
                         (cw > kSweepFreeRanks ? 18.0 : cw > 1 ? 12.0 : 4.0);
     const double cost = cost_of((double)cw, time);

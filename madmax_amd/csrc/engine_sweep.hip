@@ -22,11 +22,11 @@
 //   waiting for r.r / r.z before w = A z instead of behind it: 31 us;
 //   the planes above and below one by one: 243 multiply-adds, 27.8 to 30.7 us.
 // Whole solves (rtol 1e-10), kernels A and B and this: 128 x 30^3 tangents 187 and
-// 60 ms, 64 uneven cells 8^3 .. 32^3 50 and 12.7 ms, 24 x 20^3 in FP64 25.5 and 5.6
-// ms, one 10^3 4.7 and 0.77.
-// Sharing the rows: 32 x 33 x 36 x 40 tangents 122 and 44 ms, 4 x 60^3 93 and 32;
-// one load case of 48^3 7.9 and 4.1 ms, of 100^3 (195 workgroups) 50 and 17, 74 us
-// an iteration by kernels A, S, B and R and 25 here.
+// 57 ms, 64 uneven cells 8^3 .. 32^3 50 and 12 ms, 24 x 20^3 in FP64 25.5 and 5.2
+// ms, one 10^3 4.7 and 0.67.
+// Sharing the rows: 32 x 33 x 36 x 40 tangents 122 and 42 ms, 4 x 60^3 93 and 32;
+// one load case of 48^3 7.9 and 3.6 ms, of 100^3 50 and 14, 74 us
+// an iteration by kernels A, S, B and R and 20 here.
 #include <hip/hip_runtime.h>
 
 #include "engine_device.h"
@@ -518,15 +518,20 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
   constexpr int NI = kSweepItems;
   const int tid = threadIdx.x, fs = g.fs, SN = P.SN, RS = 3 * SN;
   TS p[NI][LP][3], q[NI][LP][3], dd[NI][LP][3];
-  int z0[NI], d0[NI], cnt[NI], hc[NI], wd[NI];
-  bool on[NI], edge[NI];
+  int z0[NI], d0[NI], cnt[NI], wd[NI];
+  unsigned put[NI];  // bit l: another rank reads the lane's node l; bit 31: the lane has nodes
 #pragma unroll
   for (int j = 0; j < NI; j++) {
     const SweepItem it = sweep_item(g, tid, j);
     cnt[j] = scalar(it.cnt);
-    hc[j] = scalar(it.h);
-    on[j] = it.on;
-    edge[j] = it.edge;
+    const unsigned own = (1u << it.cnt) - 1u;
+    put[j] = 0u;
+    if (it.on) {
+      put[j] = it.edge ? own : 0u;
+      if (g.zlo && it.h == 0) put[j] |= 1u;
+      if (g.zhi && it.h == g.nch - 1) put[j] |= own & ~(own >> 1);  // the last plane
+      put[j] |= 1u << 31;
+    }
     wd[j] = it.word;
     z0[j] = it.lds * 3;
     // the phases do not vary along z: one pattern per column; lanes without a
@@ -552,7 +557,7 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
     int ps = ps0;
     asm volatile("" : "+s"(ps));
 #pragma unroll
-    for (int j = 0; j < NI; j++) asm volatile("" : "+v"(z0[j]), "+v"(wd[j]));
+    for (int j = 0; j < NI; j++) asm volatile("" : "+v"(z0[j]), "+v"(wd[j]), "+v"(put[j]));
 #pragma unroll
     for (int j = 0; j < NI; j++) {
       if (j > 0 && cnt[j] == 0) continue;
@@ -623,11 +628,10 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
           v2[0] = fma((double)r, (double)r, v2[0]);
           v2[1] = fma((double)r, (double)zi, v2[1]);
         }
-        if (on[j]) {
+        if ((int)put[j] < 0) {
 #pragma unroll
           for (int d = 0; d < 3; d++) zl[z0[j] + (l + 1) * ps + d] = x[l][d];
-          if (edge[j] || (l == 0 && g.zlo && hc[j] == 0) || (l == cnt[j] - 1 && g.zhi && hc[j] == g.nch - 1))
-            put_node(X, g.ni, wd[j] + l * g.nixy, tag, x[l]);
+          if ((put[j] >> l) & 1u) put_node(X, g.ni, wd[j] + l * g.nixy, tag, x[l]);
         }
       }
     }
@@ -678,7 +682,7 @@ struct SweepRun {
   __device__ __forceinline__ int go() const
   {
     if constexpr (LP > 2)
-      if (g.lp <= LP - 2) return go<LP - 2>();
+      if (g.lp <= sweep_shorter(LP)) return go<sweep_shorter(LP)>();
     return sweep_case<TS, LP>(P, g, K, k, zl, dict, red, fail, X, rz, tgt, max_its);
   }
 };
@@ -756,7 +760,7 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
     o[0] = dg;
     o[sweep_dict_block(tsz) / 3] = (TS)1 / dg;
   }
-  const int zlen = sweep_lds_planes(g.lp, g.nch) * g.pw * 3;
+  const int zlen = sweep_lds_planes(tsz, g.lp, g.nch) * g.pw * 3;
   for (int i = tid; i < zlen; i += kSweepLanes) zl[i] = (TS)0;
   __syncthreads();
   for (int s = 0; s < g.np + 2; s++) {

@@ -242,10 +242,15 @@ constexpr unsigned long long kMeetGo = 1, kMeetOff = 2;
 constexpr int kSweepUnitRanks = 256;  // a unit is (slot, load case * this + rank)
 constexpr int kSweepMaxLds = 160 * 1024 - 2816;  // dynamic; the static part is below 2.75 KB
 __host__ __device__ constexpr int sweep_max_planes(int tsz) { return tsz == 8 ? 4 : 8; }
-// The unrolled item lengths: a sweep of lp planes per item runs the next one.
-__host__ __device__ constexpr int sweep_unroll(int lp)
+// The unrolled item lengths: 2, 5, 7 and 8 planes in FP32, 2, 3 and 4 in FP64; a
+// sweep of lp planes per item runs the next one.  A plane too many costs as much
+// as one with nodes; over cells of 8^3 .. 36^3 these four cost 2% more than all of
+// 2 .. 8, and 2, 4, 6 and 8 4%.  A fifth in the kernel makes the compiler spill in
+// the longest (30^3 cells 9% slower).
+__host__ __device__ constexpr int sweep_shorter(int lp) { return lp == 8 ? 7 : lp == 7 ? 5 : lp == 4 ? 3 : 2; }
+__host__ __device__ constexpr int sweep_unroll(int tsz, int lp)
 {
-  return lp <= 2 ? 2 : (lp + 1) / 2 * 2;
+  return lp <= 2 ? 2 : tsz == 8 ? lp : lp <= 5 ? 5 : lp <= 7 ? 7 : 8;
 }
 // Positions per wave: lanes 0 and 63 supply the x-neighbours of lanes 1 and 62.
 constexpr int kSweepStrip = 62;
@@ -255,9 +260,9 @@ __host__ __device__ constexpr int sweep_strips(int nx, int ny)
   return (sweep_positions(nx, ny) + kSweepStrip - 1) / kSweepStrip;
 }
 // LDS planes of a tile: every plane that the unrolled items read.
-__host__ __device__ constexpr int sweep_lds_planes(int lp, int nch)
+__host__ __device__ constexpr int sweep_lds_planes(int tsz, int lp, int nch)
 {
-  return (nch - 1) * lp + sweep_unroll(lp) + 2;
+  return (nch - 1) * lp + sweep_unroll(tsz, lp) + 2;
 }
 // Values per LDS plane: interior nodes, a zero column between rows, a zero row
 // before and after them and one value in front.
