@@ -6,12 +6,16 @@ six unit-strain load cases solved as a 6-RHS block by FP32 Jacobi-PCG inside
 FP64 iterative refinement, and their 6x6 tangents averaged in FP64.
 
 The JSON line also carries:
-  roofline      the solve's dominant kernel, kernel A (the PCG step's SpMV +
-                p/q update, dictionary ELL storage): the median duration of
-                its launches inside a solve of the batch (HIP events around
-                every launch, one stream, no graph), against the algorithmic
-                bytes of one launch; the stand-alone replica of its work is
-                reported beside it
+  roofline      the engine's HBM-streaming kernel, kernel A of the
+                step-by-step path (the PCG step's SpMV + p/q update,
+                dictionary ELL storage): the median duration of its launches
+                inside such a solve of the batch (profile_step_kernel: HIP
+                events around every launch, one stream, no graph), against
+                the algorithmic bytes of one launch; the stand-alone replica
+                of its work is reported beside it.  The batch that `value`
+                times is solved by whole sweeps on chip (k_sweep, bound by
+                vector issue), which move next to no HBM bytes; cells beyond
+                about 100^3 elements take the step-by-step path
   spmv          the ELL SpMV alone: dictionary storage and the full per-row
                 ELL on the batch, and the HBM-resident figures of one 100^3
                 RVE (2.0 GB FP32 ELL, 3.05 GB FP64 reference-layout ELL)
@@ -720,7 +724,8 @@ def main():
                                         "calibrated on the copy kernel); not measured in this run"
                                         if traffic else None),
                      "kernel": "k_step_a_march_dict<float,6> (kernel A: SpMV + p/q update, dictionary ELL, "
-                               "z-plane march through LDS) inside a solve of %d RVEs: median of %d launches"
+                               "z-plane march through LDS) inside a step-by-step solve of %d RVEs: median of "
+                               "%d launches (the timed batch is solved on chip by k_sweep)"
                                % (B, len(a_ms)),
                      "avg_ms": in_solve_ms, "bytes_per_launch": step_bytes,
                      "replica_ms": rep_ms, "replica_frac": step_bytes / (rep_ms * 1e-3) / 1e9 / HBM_PEAK_GBS,
