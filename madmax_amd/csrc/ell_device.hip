@@ -579,10 +579,10 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
 // ---- the same iteration with the matrix on chip ------------------------------
 // k_pcg_resident runs a whole solve in one launch, one workgroup per slab of 256
 // rows.  Each lane holds its row: the values and the LDS places of its columns
-// (two to a register) for the whole solve, x, r, z and p too.  p of every column
-// between the slab's lowest and highest lives in LDS: after an update the owners
-// publish z as tagged words, and every workgroup forms p = z + beta p for its
-// columns, the same bits as the owner.  p.q and {r.r, r.z} go round as tagged
+// (two to a register) for the whole solve, x, r, z and p too (in LDS with LIST).  p
+// of the slab's columns (LIST: those it has entries in) lives in LDS: after an update the owners publish z
+// as tagged words, and every workgroup forms p = z + beta p for its columns, the
+// same bits as the owner.  p.q and {r.r, r.z} go round as tagged
 // words too and are summed by every workgroup in the order of the other mappings
 // (group_sum_rows: slab-strided, then block_sum).  With the same row arithmetic
 // and scalar steps all mappings give the same bits.
@@ -591,8 +591,8 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
 // the two launches per iteration that it replaces were bound by the host's
 // launches for small matrices and by reading 12 bytes per entry for larger ones.
 // Elasticity systems of N^3 elements with 81 slots, us per iteration, two launches
-// against this: 2,970 rows 22.7 and 7.0, 14,739 rows 23.6 and 8.4, 46,875 rows
-// 25.0 and 11.4, 89,373 rows 32.5 and 17.1.
+// against this: 2,970 rows 22.7 and 7.0, 14,739 rows 23.6 and 8.2, 46,875 rows
+// 25.0 and 9.8, 89,373 rows 32.5 and 13.0.
 //
 // All workgroups have to run at the same time.  They are at most 384, two to a CU
 // (one, 192, where the LDS of two does not fit): 192 CUs, which leaves 64 for
@@ -602,10 +602,15 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
 // for instance beside another process's, is done again in the two-launch form.
 constexpr int kResSlots = 81;  // rows of 27 nodes' 3 dofs; five registers for two slots, 203 of 256
 constexpr int kResMaxSlabs = 384;
-constexpr int kResOneCuLds = 78 * 1024;  // up to this, two workgroups per CU
-constexpr int kResMaxLds = 156 * 1024;
+constexpr int kResOneCuLds = 69 * 1024;  // dynamic LDS up to which two workgroups fit a CU
+constexpr int kResMaxLds = 149 * 1024;
 constexpr int kResPolls = 1 << 18;  // about 0.2 s
 constexpr int kResMaxDevices = 64;
+// Spans from which a slab lists the columns it has entries in, in place of keeping
+// all: the list costs 20 us a solve and a look-up, and saves asking for columns.
+// us an iteration without and with it, spans of 867, 1,359, 2,103 and 6,219 columns:
+// 5.3 and 5.5, 6.7 and 6.6, 7.6 and 7.0, 15.9 and 11.6.
+constexpr int kResListSpan = 1536;
 
 // Sums NV values over all slabs, valid in every lane: lane 0 of each workgroup
 // has posted its own (NV doubles at sums + slab * 8).  False, in every lane, when
@@ -655,6 +660,7 @@ __device__ __forceinline__ double rounded(double v)
 
 // zw: two words per row (z of the last update), sums: 16 words per slab, all
 // zero on entry (no iteration's tag); zp[row].x is the first z, .y receives x.
+template <bool LIST>
 __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__ cols, const double *__restrict__ vals,
                                                          int nrow, int nnz, int nslab, int lds_rows,
                                                          const double *__restrict__ dinv, const double *__restrict__ x0,
@@ -663,7 +669,8 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
 {
   __shared__ double lds[48];
   __shared__ double bc[2];
-  __shared__ int s_lo, s_hi, s_fail;
+  __shared__ double s_row[LIST ? 5 : 1][256];  // x, dinv, r, z and p of the rows, where the registers are full
+  __shared__ int s_lo, s_hi, s_fail, s_wave[4];
   if (st->done) return;
   const int lane = threadIdx.x, slab = blockIdx.x;
   const long long row = (long long)slab * 256 + lane, base = (long long)slab * 256 * nnz;
@@ -675,9 +682,10 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
   }
   __syncthreads();
   // the row up to its first -1, column places two to a register; the slots
-  // after it add -0.0 * res_p[lds_rows] = -0.0, which changes no sum
+  // after it add -0.0 * res_p[nneed] = -0.0, which changes no sum
   double v[kResSlots];
   unsigned o[(kResSlots + 1) / 2];
+  unsigned short *need = reinterpret_cast<unsigned short *>(res_p + lds_rows + 1);
   const int *rc = cols + base + lane;
   const double *rv = vals + base + lane;
   int cnt = 0, lo = nrow, hi = -1;
@@ -706,14 +714,67 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
     if (lane == 0) st->pad0 = 1;
     return;
   }
+  // with LIST only the columns that the slab has entries in get a place, else all
+  // between the lowest and the highest: they are marked in bytes (neighbouring rows
+  // share columns, so that an atomic on bits would meet 64 lanes at a word), then
+  // as bits, 32 columns a word: a column's place is its rank, and need lists them.
+  // In res_p's place until p is there.
+  unsigned *bits = reinterpret_cast<unsigned *>(res_p);
+  const int nw = LIST && hi >= lo ? (hi - lo) / 32 + 1 : 0;
+  unsigned char *mark = reinterpret_cast<unsigned char *>(bits + nw);
+  unsigned short *rank = reinterpret_cast<unsigned short *>(mark + 32 * nw);
+  for (int w = lane; w < 8 * nw; w += 256) reinterpret_cast<unsigned *>(mark)[w] = 0;
+  __syncthreads();
+#pragma unroll 1
+  for (int u0 = 0; u0 < (LIST ? nnz : 0); u0 += 9) {
+    int c[9];
+#pragma unroll
+    for (int u = 0; u < 9; u++) c[u] = u0 + u < cnt ? rc[(u0 + u) * 256] - lo : -1;
+#pragma unroll
+    for (int u = 0; u < 9; u++)
+      if (c[u] >= 0) mark[c[u]] = 1;
+  }
+  __syncthreads();
+  for (int w = 2 * (lane >> 6); w < nw; w += 8) {
+    const int e = 32 * w + (lane & 63);
+    const unsigned long long b = __ballot(e < 32 * nw && mark[min(e, 32 * nw - 1)] != 0);
+    if ((lane & 63) == 0) {
+      bits[w] = (unsigned)b;
+      if (w + 1 < nw) bits[w + 1] = (unsigned)(b >> 32);
+    }
+  }
+  __syncthreads();
+  const int per = (nw + 255) / 256;
+  int mine = 0;
+  for (int w = lane * per; w < min((lane + 1) * per, nw); w++) mine += __popc(bits[w]);
+  int at = mine;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int t = __shfl_up(at, off, 64);
+    if ((lane & 63) >= off) at += t;
+  }
+  if ((lane & 63) == 63) s_wave[lane >> 6] = at;
+  __syncthreads();
+  at -= mine;
+  for (int w = 0; w < (lane >> 6); w++) at += s_wave[w];
+  const int nneed = LIST ? s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3] : max(hi - lo + 1, 0);
+  for (int w = lane * per; w < min((lane + 1) * per, nw); w++) {
+    for (unsigned b = bits[w]; b; b &= b - 1) {
+      const int e = w * 32 + __ffs(b) - 1;
+      rank[e] = (unsigned short)at;
+      need[at++] = (unsigned short)e;
+    }
+  }
+  __syncthreads();
 #pragma unroll
   for (int u0 = 0; u0 < kResSlots; u0 += 9) {
 #pragma unroll
     for (int u = u0; u < u0 + 9; u++) {
-      unsigned c = lds_rows;
+      unsigned c = nneed;
       v[u] = -0.0;
       if (u < cnt) {
         c = rc[u * 256] - lo;
+        if (LIST) c = rank[c];
         v[u] = rv[u * 256];
       }
       if (u & 1) o[u / 2] |= c << 16;
@@ -721,14 +782,21 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
     }
     __builtin_amdgcn_sched_barrier(0);
   }
+  __syncthreads();  // the tables make way for p
   int most = cnt;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) most = max(most, __shfl_xor(most, off, 64));
   most = __builtin_amdgcn_readfirstlane(most);
-  double xi = on ? x0[row] : 0.0, ri = on ? r0[row] : 0.0, zi = on ? zp[row].x : 0.0, pi = 0.0;
-  const double di = on ? dinv[row] : 0.0;
-  for (int e = lo + lane; e <= hi; e += 256) res_p[e - lo] = 0.0;
-  if (lane == 0) res_p[lds_rows] = 0.0;
+  double xi = on ? x0[row] : 0.0, di = on ? dinv[row] : 0.0, ri = on ? r0[row] : 0.0, zi = on ? zp[row].x : 0.0;
+  double pi = 0.0;
+  if constexpr (LIST) {
+    s_row[0][lane] = xi;
+    s_row[1][lane] = di;
+    s_row[2][lane] = ri;
+    s_row[3][lane] = zi;
+    s_row[4][lane] = pi;
+  }
+  for (int e = lane; e <= nneed; e += 256) res_p[e] = 0.0;
   __syncthreads();
   const double bnorm = st->bnorm, rtol = st->rtol;
   const int max_its = st->max_its;
@@ -743,12 +811,21 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
       pcg_after_update(s[0], s[1], rtol, bnorm, max_its, its, rnorm, rz, beta, done);
       if (__builtin_amdgcn_readfirstlane(done)) break;
     }
-    // p = z + beta p for the slab's columns, four per trip
-    for (int e0 = lo + lane; e0 <= hi; e0 += 4 * 256) {
+    // p = z + beta p for the slab's columns, four per lane and trip
+    for (int e0 = lane; e0 < nneed; e0 += 4 * 256) {
       double z[4];
+      int listed[4];
+      if constexpr (LIST) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) listed[i] = lo + need[min(e0 + 256 * i, nneed - 1)];
+      }
+      const auto col = [&](int i) {
+        if constexpr (LIST) return listed[i];
+        else return min(lo + e0 + 256 * i, hi);
+      };
       if (n == 0) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) z[i] = (e0 + 256 * i <= hi) ? zp[e0 + 256 * i].x : 0.0;
+        for (int i = 0; i < 4; i++) z[i] = zp[col(i)].x;
       } else {
         word_t a[4], b[4];
         int m = 0;
@@ -756,9 +833,9 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
           bool all = true;
 #pragma unroll
           for (int i = 0; i < 4; i++) {
-            const int e = min(e0 + 256 * i, hi);
-            a[i] = get_word(zw + 2LL * e);
-            b[i] = get_word(zw + 2LL * e + 1);
+            const word_t *w = zw + 2LL * col(i);
+            a[i] = get_word(w);
+            b[i] = get_word(w + 1);
           }
 #pragma unroll
           for (int i = 0; i < 4; i++)
@@ -774,9 +851,10 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
       }
 #pragma unroll
       for (int i = 0; i < 4; i++)
-        if (e0 + 256 * i <= hi) res_p[e0 + 256 * i - lo] = fma(beta, res_p[e0 + 256 * i - lo], z[i]);
+        if (e0 + 256 * i < nneed) res_p[e0 + 256 * i] = fma(beta, res_p[e0 + 256 * i], z[i]);
     }
-    pi = fma(beta, pi, zi);
+    if constexpr (LIST) s_row[4][lane] = fma(beta, s_row[4][lane], s_row[3][lane]);
+    else pi = fma(beta, pi, zi);
     __syncthreads();
     // (o is taken apart anew each time: the places would not fit the registers)
 #pragma unroll
@@ -793,14 +871,26 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
       }
     }
     const unsigned tag = (unsigned)n + 1u;
+    if constexpr (LIST) pi = s_row[4][lane];
     double s1[1] = {rounded(pi * qi)};
     block_sum<1>(s1, lds);
     if (lane == 0) put_double(sums + (long long)slab * 8, tag, s1[0]);
     if (!res_collect<1>(sums, nslab, tag, s1, lds, bc, &s_fail)) break;
     alpha = pcg_alpha(rz, s1[0]);
+    if constexpr (LIST) {
+      xi = s_row[0][lane];
+      di = s_row[1][lane];
+      ri = s_row[2][lane];
+      pi = s_row[4][lane];
+    }
     xi = fma(alpha, pi, xi);
     ri = fma(-alpha, qi, ri);
     zi = di * ri;
+    if constexpr (LIST) {
+      s_row[0][lane] = xi;
+      s_row[2][lane] = ri;
+      s_row[3][lane] = zi;
+    }
     if (on) put_double(zw + 2 * row, tag, zi);
     double s2[2] = {rounded(ri * ri), rounded(ri * zi)};  // (zero beyond the last row)
     block_sum<2>(s2, lds);
@@ -814,7 +904,7 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
     if (lane == 0) st->pad0 = 1;  // (any of them may; the host reads it after the kernel)
     return;
   }
-  if (on) zp[row].y = xi;
+  if (on) zp[row].y = LIST ? s_row[0][lane] : xi;
   if (slab == 0 && lane == 0) {
     st->its = n;
     st->rnorm = rnorm;
@@ -825,6 +915,9 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
     st->fresh = 0;
   }
 }
+
+// Its LDS for slabs spanning `rows` columns: p and a zero, and the columns' list.
+static size_t res_lds(int rows) { return (size_t)(rows + 1) * sizeof(double) + (size_t)rows * sizeof(short); }
 
 // The exchange sums of k_pcg_resident (its z words are zeroed by k_pcg_init).
 __global__ void k_res_zero(word_t *sums, int n)
@@ -1263,10 +1356,10 @@ static int pcg_run(ell_device *d, const PcgVecs &V, ell_solver *solver, const do
 {
   // the matrix on chip (k_pcg_resident) where the columns that a slab spans fit
   // the LDS and the workgroups the GPU; it was the faster at every size it takes
-  const int res_rows = d->band > 0 ? d->band : d->nrow;
+  const int span = d->band > 0 ? d->band : d->nrow, res_rows = span > 64 ? span : 64;  // (its tables want as much)
   const bool resident = may_stay && d->fused_its == 0 && d->S == 256 && d->nnz <= kResSlots &&
-                        d->device < kResMaxDevices && res_rows <= kResMaxLds / 8 &&
-                        d->nslab <= (res_rows * 8 <= kResOneCuLds ? kResMaxSlabs : kResMaxSlabs / 2);
+                        d->device < kResMaxDevices && res_lds(res_rows) <= (size_t)kResMaxLds &&
+                        d->nslab <= (res_lds(res_rows) <= (size_t)kResOneCuLds ? kResMaxSlabs : kResMaxSlabs / 2);
   const int max_its = (solver && solver->max_its > 0) ? solver->max_its : MAX_ITS;
   const double rtol = (solver && solver->min_err > 0) ? solver->min_err : MIN_ERR;
   int rc = set_state(d, V.st, max_its, rtol, 0.0);
@@ -1277,10 +1370,11 @@ static int pcg_run(ell_device *d, const PcgVecs &V, ell_solver *solver, const do
   MM_HIP(hipGetLastError());
   IterState h;
   if (resident) {
-    ResShare share(d->device, res_rows * 8 <= kResOneCuLds ? d->nslab : 2 * d->nslab);
+    ResShare share(d->device, res_lds(res_rows) <= (size_t)kResOneCuLds ? d->nslab : 2 * d->nslab);
     word_t *zw = reinterpret_cast<word_t *>(V.zpB), *sums = reinterpret_cast<word_t *>(V.q);
     k_res_zero<<<(16 * d->nslab + 255) / 256, 256, 0, d->stream>>>(sums, 16 * d->nslab);
-    k_pcg_resident<<<d->nslab, 256, (size_t)(res_rows + 1) * sizeof(double), d->stream>>>(
+    const auto solve = span > kResListSpan ? k_pcg_resident<true> : k_pcg_resident<false>;
+    solve<<<d->nslab, 256, res_lds(res_rows), d->stream>>>(
         d->cols, d->vals, d->nrow, d->nnz, d->nslab, res_rows, d->dinv, x, V.r, V.zpA, zw, sums, V.st);
     k_res_take<<<(d->nrow + 255) / 256, 256, 0, d->stream>>>(V.st, V.zpA, x, d->nrow);
     MM_HIP(hipGetLastError());
