@@ -2,9 +2,9 @@
 iteration and the CPU.
 
 Shapes are where it could go wrong: one row, one row more than a slab, rows of
-different lengths and an empty tail, the 81 slots it takes and one more, columns
-spanning a slab's LDS for two workgroups per CU, for one, and beyond it, the most
-slabs it takes and one more.  The fused kernel works on the same 256-row slabs in
+different lengths and an empty tail, the 81 slots it takes and one more, spans of
+1,536 columns and the next that list theirs, columns spanning a slab's LDS for two
+workgroups per CU, for one, and beyond it, the most slabs it takes and one more.  The fused kernel works on the same 256-row slabs in
 the same order and rounds alike, so the bits are equal; x is also held against
 numpy's residual: the solve stops at ||r|| <= 1e-10 ||b|| by the recurrence, and
 the true residual of these well-conditioned systems (diagonally dominant by a
@@ -76,6 +76,7 @@ def residual(cols, vals, b, x):
 
 @pytest.mark.parametrize("n,width,reach", [
     (1, 1, 1), (255, 5, 3), (257, 8, 200), (700, 81, 300), (700, 82, 300), (3993, 81, 500),
+    (3000, 9, 640), (3000, 9, 642), (4000, 81, 1900),
     (12000, 27, 4700), (12000, 27, 9000), (20500, 9, 20400), (384 * 256, 9, 300), (384 * 256 + 1, 9, 300),
     (192 * 256 + 1, 9, 9000),
 ])
