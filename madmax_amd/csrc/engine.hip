@@ -21,6 +21,7 @@
 
 #include "micro_api.h"
 #include "mm_internal.h"
+#include "sweep_geo.h"
 
 using namespace mm;
 
@@ -547,12 +548,17 @@ extern "C" int mm_engine_destroy(mm_engine *e)
   return 0;
 }
 
+static long long rve_slabs(const mm_rve_spec &s, int SN)
+{
+  return ((long long)(s.nex + 1) * (s.ney + 1) * (s.nez + 1) + SN - 1) / SN;
+}
+
 static void footprint(const mm_engine *e, const mm_rve_spec &s, int *nrow, long long *nslab,
                       long long *nelm)
 {
   const long long nn = (long long)(s.nex + 1) * (s.ney + 1) * (s.nez + 1);
   *nrow = (int)(3 * nn);
-  *nslab = (nn + e->SN - 1) / e->SN;
+  *nslab = rve_slabs(s, e->SN);
   *nelm = (long long)s.nex * s.ney * s.nez;
 }
 
@@ -798,14 +804,6 @@ static int march_lds_need(const mm_engine *e, const HostSlot &h)
                      : 0;
 }
 
-// Resident sweep of an RVE of nx x ny x nz nodes (RveDev::scw ..): the cheapest
-// split of the interior z-planes, and, if whole rows of planes are too many, of
-// the rows, whose shares fit the lanes' items and the LDS, cut into items of few
-// enough planes that small RVEs still occupy the lanes.  cw = 0 (kernels A and
-// B) without an interior, where nothing fits, and for the engines whose steps
-// are single PCG iterations by request: sync_every_step reads the state after
-// each, profile_step_kernel times each one's kernel A.  Fixed by the RVE and the
-// engine configuration alone.
 // Enters ty shares of the rows times cz of the planes into t if they fit and cost
 // less than its `best`; cost(workgroups, time).
 template <typename Cost>
@@ -835,11 +833,18 @@ static void sweep_split(const mm_rve_spec &s, int tsz, int ty, int cz, const Cos
   }
 }
 
-static SweepTiling sweep_tiling(const mm_engine *e, const mm_rve_spec &s, long long nslab)
+// Resident sweep of an RVE of nx x ny x nz nodes (RveDev::scw ..): the cheapest
+// split of the interior z-planes, and, if whole rows of planes are too many, of
+// the rows, whose shares fit the lanes' items and the LDS, cut into items of few
+// enough planes that small RVEs still occupy the lanes.  cw = 0 (kernels A and
+// B) without an interior and where nothing fits.  Fixed by the RVE and the engine
+// configuration alone: K load cases and rve_cap slots of tsz-byte values, slabs of
+// SN nodes.
+static SweepTiling sweep_tiling(const mm_rve_spec &s, int tsz, int K, int rve_cap, int SN)
 {
   SweepTiling t;
-  if (e->cfg.sync_every_step || e->cfg.profile_step_kernel) return t;
-  const int nix = s.nex - 1, niy = s.ney - 1, niz = s.nez - 1, tsz = (int)e->tsz;
+  const int nix = s.nex - 1, niy = s.ney - 1, niz = s.nez - 1;
+  const long long nslab = rve_slabs(s, SN);
   if (nix < 1 || niy < 1 || niz < 1 || nix > 4096 || niy > 4096) return t;
   // (past kSweepFreeRanks, workgroups are bounded by the slabs for the unit lists' sake)
   const int few = (int)std::min<long long>(kSweepFreeRanks, nslab);
@@ -849,14 +854,14 @@ static SweepTiling sweep_tiling(const mm_engine *e, const mm_rve_spec &s, long l
     for (int ty = ty0; ty <= ty1 && ty <= most && ty <= niy; ty++)
       for (int cz = 1; ty * cz <= most && cz <= niz; cz++) sweep_split(s, tsz, ty, cz, cost, best, t);
   };
-  const double room = 256.0 / ((double)e->K * e->rve_cap);
+  const double room = 256.0 / ((double)K * rve_cap);
   if (room >= 2.0) {
     // An engine of few RVEs leaves CUs idle: time counts, and, past the CUs that
     // each cluster has when all of them are active, a little of their cost.  One
     // load case, ms by kernels A and B, the cheapest split and this one: 30^3 4.7,
     // 5.8 and 3.0; 48^3 7.9, 10.1 and 4.9; 60 x 52 x 50 11.3, 12.5 and 6.5.
     search(many, 1, niy, [&](double cw, double time) { return time * std::sqrt(std::sqrt(std::max(1.0, cw / room))); });
-  } else if (e->K == 1) {
+  } else if (K == 1) {
     // Otherwise the CUs' time, but a lone cell must not lose against the launches
     // of kernels A and B, 23 us an iteration, 40 of this unit.
     search(many, 1, niy, [](double cw, double time) { return cw * time + std::max(0.0, time - 38.0) * 1e6; });
@@ -866,10 +871,82 @@ static SweepTiling sweep_tiling(const mm_engine *e, const mm_rve_spec &s, long l
     if (!t.cw) search(many, 1, niy, cus);
   }
   if (t.cw > 1) {  // the exchanged words must fit the RVE's part of d
-    const long long part = nslab * e->rows_per_slab() * (long long)tsz;
+    const long long part = nslab * 3 * SN * (long long)tsz;
     if (8LL * ((long long)nix * niy * niz * (tsz / 4) + sweep_sum_words(t.cw)) > part) t = SweepTiling();
   }
   return t;
+}
+
+// The same for an engine; none where its steps are single PCG iterations by
+// request: sync_every_step reads the state after each, profile_step_kernel times
+// each one's kernel A.
+static SweepTiling sweep_tiling(const mm_engine *e, const mm_rve_spec &s)
+{
+  if (e->cfg.sync_every_step || e->cfg.profile_step_kernel) return SweepTiling();
+  return sweep_tiling(s, (int)e->tsz, e->K, e->rve_cap, e->SN);
+}
+
+extern "C" int mm_sweep_split(int nex, int ney, int nez, int fp64, int nrhs, int max_rves, int slab_nodes, int *split)
+{
+  if (!split || nex < 1 || ney < 1 || nez < 1 || nrhs < 1 || max_rves < 1 || slab_nodes < 1) return MM_ERR_ARG;
+  mm_rve_spec s = {};
+  s.nex = nex;
+  s.ney = ney;
+  s.nez = nez;
+  const SweepTiling t = sweep_tiling(s, fp64 ? 8 : 4, nrhs, max_rves, slab_nodes);
+  split[0] = t.cw;
+  split[1] = t.ty;
+  split[2] = t.lp;
+  split[3] = t.nch;
+  return 0;
+}
+
+extern "C" int mm_sweep_check(int nex, int ney, int nez, int fp64, const int *split, int *faults)
+{
+  if (!split || !faults || nex < 2 || ney < 2 || nez < 2 || split[0] < 1 || split[1] < 1 || split[0] % split[1])
+    return MM_ERR_ARG;
+  const int tsz = fp64 ? 8 : 4, cw = split[0], lp = split[2], nch = split[3];
+  const size_t ni = (size_t)(nex - 1) * (ney - 1) * (nez - 1);
+  std::vector<uint8_t> owned(ni, 0), put(ni, 0), got(ni, 0);
+  int lds = 0;
+  for (int rk = 0; rk < cw; rk++) {
+    const SweepGeo g = sweep_geo(nex + 1, ney + 1, nez + 1, cw, split[1], lp, nch, rk);
+    for (int st = 0; st < kSweepItems * (kSweepLanes / 64); st++)
+      for (int ln = 0; ln < 64; ln++) {
+        const SweepItem it = sweep_item(g, st, ln);
+        const unsigned p = sweep_put(g, it);
+        for (int l = 0; l < it.cnt && (p >> 31); l++) {
+          owned[it.word + l * g.nixy]++;
+          put[it.word + l * g.nixy] += (p >> l) & 1u;
+        }
+      }
+    // the LDS position of interior node w in this rank's tile, -1 outside
+    const int zlen = sweep_lds_planes(tsz, lp, nch) * g.pw;
+    const auto position = [&](int w) {
+      const int z = w / g.nixy + 2 - g.zs, r = w % g.nixy / g.nix + 1 - g.ys, at = z * g.pw + 1 + r * g.rsx + w % g.nix;
+      return z < 0 || r < 0 || r > g.nr + 1 || at >= zlen ? -1 : at;
+    };
+    const SweepHalo h = sweep_halo(g);
+    for (int c = 0; c < h.n; c++) {
+      int at, dst, dat, ddst;
+      bool lo, hi;
+      sweep_place(g, h.r0, h.n1, h.n, c, at, dst, dat, ddst, lo, hi);
+      for (int up = 0; up < 2; up++) {
+        if (!(up ? hi : lo)) continue;
+        const int w = at + (up ? dat : 0), to = dst + (up ? ddst : 0);
+        if (w < 0 || (size_t)w >= ni || position(w) != to) lds++;
+        else got[w] = 1;
+      }
+    }
+  }
+  for (int i = 0; i < 4; i++) faults[i] = 0;
+  for (size_t w = 0; w < ni; w++) {
+    if (owned[w] != 1) faults[0]++;
+    if (put[w] > 1) faults[1]++;
+    if (got[w] && !put[w]) faults[2]++;
+  }
+  faults[3] = lds;
+  return 0;
 }
 
 static void fill_state(const mm_engine *e, const HostSlot &h, RveDev *st, int warm)
@@ -1014,7 +1091,7 @@ static int admit(mm_engine *e)
   size_t i = 0, ik = 0, ip = 0, is = 0;
   for (int s : fresh) {
     HostSlot &h = e->slots[s];
-    h.sweep = sweep_tiling(e, h.req.rve, h.nslab);
+    h.sweep = sweep_tiling(e, h.req.rve);
     fill_state(e, h, &e->st_states[i], 0);
     e->st_slots[i++] = s;
     for (int m = 0; m < kNmat; m++) {

@@ -32,60 +32,20 @@
 #include "engine_device.h"
 #include "mm_device.h"
 #include "mm_internal.h"
+#include "sweep_geo.h"
 
 namespace mm {
 
 namespace {
 
-// The tile of one workgroup: rank rk = rz sty + ry of the RVE's scw owns the
-// interior planes zs .. ze-1 and of each the nr interior rows from ys (counted
-// from 0).  LDS plane s holds plane zs - 1 + s; inside a plane, node (ix, iy) of
-// the tile (both counted from 0) sits at pos = 1 + (iy + 1) (nix + 1) + ix, so
-// that a zero column lies between the rows, and a row before and after them
-// holds the neighbouring tiles' or is zero.  Zeros stand for the boundary nodes,
-// whose z is zero in every correction solve.
-struct SweepGeo {
-  int nix, rsx, pw;  // interior columns per row; row and plane strides
-  int npos, nstrip;  // positions of a plane's rows with their zero column; strips of them
-  int zs, ze, np, ys, nr, rk, cw;
-  bool zlo, zhi, ylo, yhi;  // neighbouring ranks
-  int lp, nch;              // planes per item; items per column
-  int nx, nxy, nixy, ni, fs;
-};
-
 // The RVE's fields are the same in every lane but read through vector memory;
 // readfirstlane keeps them, and every address formed from them, scalar.
 __device__ __forceinline__ int scalar(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-__device__ __forceinline__ SweepGeo sweep_geo(const RveDev *R, int rk)
+__device__ __forceinline__ SweepGeo sweep_geo_of(const RveDev *R, int rk)
 {
-  SweepGeo g;
-  g.nx = scalar(R->nx);
-  const int ny = scalar(R->ny), niz = scalar(R->nz) - 2, ty = scalar(R->sty);
-  g.nix = g.nx - 2;
-  g.rsx = g.nix + 1;
-  g.rk = rk;
-  g.cw = scalar(R->scw);
-  const int cz = g.cw / ty, rz = rk / ty, ry = rk - rz * ty;
-  g.zs = 1 + rz * niz / cz;
-  g.ze = 1 + (rz + 1) * niz / cz;
-  g.np = g.ze - g.zs;
-  g.ys = ry * (ny - 2) / ty;
-  g.nr = (ry + 1) * (ny - 2) / ty - g.ys;
-  g.zlo = rz > 0;
-  g.zhi = rz + 1 < cz;
-  g.ylo = ry > 0;
-  g.yhi = ry + 1 < ty;
-  g.pw = sweep_plane(g.nx, g.nr + 2);
-  g.npos = g.rsx * g.nr;
-  g.nstrip = sweep_strips(g.nx, g.nr + 2);
-  g.nixy = g.nix * (ny - 2);
-  g.ni = g.nixy * niz;
-  g.lp = scalar(R->slp);
-  g.nch = scalar(R->snch);
-  g.nxy = g.nx * ny;
-  g.fs = scalar(R->first_slab);
-  return g;
+  return sweep_geo(scalar(R->nx), scalar(R->ny), scalar(R->nz), scalar(R->scw), scalar(R->sty), scalar(R->slp),
+                   scalar(R->snch), rk);
 }
 
 // Three consecutive values: one 96-bit LDS read in FP32.
@@ -408,42 +368,24 @@ __device__ __forceinline__ void word_node(const word_t *w, double *dst)
   for (int d = 0; d < 3; d++) dst[d] = word_double(w[2 * d], w[2 * d + 1]);
 }
 
-// The nodes beside the tile <- the words that the neighbouring ranks published
-// under `tag`: the planes below and above with the rows beside the tile, then of
-// the tile's own planes the rows before and after it.  U nodes of either side
-// per trip, all their words asked for together, again until each carries the tag.
+// The nodes beside the tile (sweep_place) <- the words that the neighbouring ranks
+// published under `tag`.  U nodes of either side per trip, all their words asked
+// for together, again until each carries the tag.
 template <typename TS>
 __device__ __forceinline__ bool get_halo(const SweepGeo &g, TS *zl, const SweepWords &X, unsigned tag)
 {
   constexpr int H = (int)(sizeof(TS) / 4), W = 3 * H, U = H == 1 ? 2 : 1;
-  const int r0 = g.ylo ? 0 : 1, n1 = (g.zlo || g.zhi) ? (g.nr + (g.ylo ? 1 : 0) + (g.yhi ? 1 : 0)) * g.nix : 0;
-  const int n = n1 + ((g.ylo || g.yhi) ? g.np * g.nix : 0);
+  const SweepHalo h = sweep_halo(g);
   const word_t none = (word_t)tag << 32;
   bool ok = true;
   int c0 = threadIdx.x;
   asm volatile("" : "+v"(c0));  // the places are formed here, not kept from one iteration to the next
-  for (; c0 < n; c0 += U * kSweepLanes) {
-    int at[U], dst[U], dat[U], ddst[U];  // the lower side's word and place, the upper side's distance from them
+  for (; c0 < h.n; c0 += U * kSweepLanes) {
+    int at[U], dst[U], dat[U], ddst[U];
     bool lo[U], hi[U];
 #pragma unroll
     for (int u = 0; u < U; u++) {
-      int c = c0 + u * kSweepLanes;
-      const bool in = c < n, plane = c < n1;
-      if (!plane) c -= n1;
-      const int r = c / g.nix, ix = c - r * g.nix;
-      if (plane) {  // row r0 + r of planes 0 and np + 1
-        at[u] = ix + g.nix * (g.ys + r0 + r - 1) + g.nixy * (g.zs - 2);
-        dst[u] = 1 + (r0 + r) * g.rsx + ix;
-        dat[u] = (g.np + 1) * g.nixy;
-        ddst[u] = (g.np + 1) * g.pw;
-      } else {  // rows 0 and nr + 1 of plane r + 1
-        at[u] = ix + g.nix * (g.ys - 1) + g.nixy * (g.zs - 1 + r);
-        dst[u] = 1 + ix + (r + 1) * g.pw;
-        dat[u] = (g.nr + 1) * g.nix;
-        ddst[u] = (g.nr + 1) * g.rsx;
-      }
-      lo[u] = in && (plane ? g.zlo : g.ylo);
-      hi[u] = in && (plane ? g.zhi : g.yhi);
+      sweep_place(g, h.r0, h.n1, h.n, c0 + u * kSweepLanes, at[u], dst[u], dat[u], ddst[u], lo[u], hi[u]);
     }
     word_t a[U][W], b[U][W];
     int m = 0;
@@ -477,29 +419,10 @@ __device__ __forceinline__ bool get_halo(const SweepGeo &g, TS *zl, const SweepW
   return ok;
 }
 
-// Item j of lane tid: the LDS position of its column in the plane below its
-// first node, that node, the planes of the wave's strip (0: none), and whether
-// the lane has a node there (if not it only supplies z to its neighbours).  Strip st of the tile is nstrip
-// strips per run of planes; lanes 1 .. 62 of its wave work.
-struct SweepItem {
-  int lds, node, cnt, h, word;  // word: the first node's among the interior nodes
-  bool on, edge;                // edge: in a row that a neighbouring rank reads
-};
-__device__ __forceinline__ SweepItem sweep_item(const SweepGeo &g, int tid, int j)
+// Item j of lane tid.
+__device__ __forceinline__ SweepItem sweep_item_of(const SweepGeo &g, int tid, int j)
 {
-  const int st = scalar((tid >> 6) + j * (kSweepLanes / 64)), ln = tid & 63;
-  const int h = st / g.nstrip, pos = (st - h * g.nstrip) * kSweepStrip + ln - 1;
-  const int iy = pos < 0 ? 0 : pos / g.rsx, ix = pos < 0 ? g.nix : pos - iy * g.rsx;
-  const int zf = g.zs + h * g.lp;
-  SweepItem it;
-  it.cnt = h < g.nch ? max(min(g.lp, g.ze - zf), 0) : 0;
-  it.on = it.cnt > 0 && ix < g.nix && pos < g.npos && ln >= 1 && ln <= kSweepStrip;
-  it.h = h;
-  it.lds = (h < g.nch ? h * g.lp : 0) * g.pw + min(pos, g.npos - 1) + g.rsx + 1;
-  it.node = it.on ? (ix + 1) + (g.ys + iy + 1) * g.nx + zf * g.nxy : 1 + g.nx + g.nxy;  // any interior one if off
-  it.word = ix + g.nix * (g.ys + iy) + g.nixy * (zf - 1);
-  it.edge = (g.ylo && iy == 0) || (g.yhi && iy == g.nr - 1);
-  return it;
+  return sweep_item(g, scalar((tid >> 6) + j * (kSweepLanes / 64)), tid & 63);
 }
 
 // The sweep of one load case on this workgroup's tile; zl holds z = dinv r of
@@ -511,27 +434,20 @@ __device__ __forceinline__ SweepItem sweep_item(const SweepGeo &g, int tid, int 
 // (sweep_strip) and the dot products are grouped differently.  Returns the
 // iterations taken.
 template <typename TS, int LP>
-__device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, int K, int k, TS *zl,
+__device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, int fs, int K, int k, TS *zl,
                                           const TS *dict, double *red, int *s_fail, const SweepWords &X, double rz,
                                           double tgt, int max_its)
 {
   constexpr int NI = kSweepItems;
-  const int tid = threadIdx.x, fs = g.fs, SN = P.SN, RS = 3 * SN;
+  const int tid = threadIdx.x, SN = P.SN, RS = 3 * SN;
   TS p[NI][LP][3], q[NI][LP][3], dd[NI][LP][3];
   int z0[NI], d0[NI], cnt[NI], wd[NI];
-  unsigned put[NI];  // bit l: another rank reads the lane's node l; bit 31: the lane has nodes
+  unsigned put[NI];  // sweep_put
 #pragma unroll
   for (int j = 0; j < NI; j++) {
-    const SweepItem it = sweep_item(g, tid, j);
+    const SweepItem it = sweep_item_of(g, tid, j);
     cnt[j] = scalar(it.cnt);
-    const unsigned own = (1u << it.cnt) - 1u;
-    put[j] = 0u;
-    if (it.on) {
-      put[j] = it.edge ? own : 0u;
-      if (g.zlo && it.h == 0) put[j] |= 1u;
-      if (g.zhi && it.h == g.nch - 1) put[j] |= own & ~(own >> 1);  // the last plane
-      put[j] |= 1u << 31;
-    }
+    put[j] = sweep_put(g, it);
     wd[j] = it.word;
     z0[j] = it.lds * 3;
     // the phases do not vary along z: one pattern per column; lanes without a
@@ -652,7 +568,7 @@ __device__ __forceinline__ int sweep_case(const EngPtrs &P, const SweepGeo &g, i
   asm volatile("" : "+v"(t2));  // the items' nodes are formed again, not kept
 #pragma unroll
   for (int j = 0; j < NI; j++) {
-    const SweepItem it = sweep_item(g, t2, j);
+    const SweepItem it = sweep_item_of(g, t2, j);
 #pragma unroll
     for (int l = 0; l < LP; l++)
       if (it.on && l < it.cnt) {
@@ -670,7 +586,7 @@ template <typename TS>
 struct SweepRun {
   const EngPtrs &P;
   const SweepGeo &g;
-  int K, k;
+  int fs, K, k;
   TS *zl;
   const TS *dict;
   double *red;
@@ -683,7 +599,7 @@ struct SweepRun {
   {
     if constexpr (LP > 2)
       if (g.lp <= sweep_shorter(LP)) return go<sweep_shorter(LP)>();
-    return sweep_case<TS, LP>(P, g, K, k, zl, dict, red, fail, X, rz, tgt, max_its);
+    return sweep_case<TS, LP>(P, g, fs, K, k, zl, dict, red, fail, X, rz, tgt, max_its);
   }
 };
 
@@ -740,8 +656,8 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   if (writer && tid == 0) R->st[0] = N;
   if (N.phase != PH_INNER || ((N.done_in >> k) & 1u)) return;
 
-  const SweepGeo g = sweep_geo(R, rk);
-  const int SN = P.SN, RS = 3 * SN, fs = g.fs, tsz = (int)sizeof(TS);
+  const SweepGeo g = sweep_geo_of(R, rk);
+  const int SN = P.SN, RS = 3 * SN, fs = scalar(R->first_slab), tsz = (int)sizeof(TS);
   const SweepWords X = sweep_words<TS>(P, scalar(R->nslab), K, fs, k, g.ni);
   if (g.cw > kSweepFreeRanks) {
     if (tid == 0) s_unit = cluster_meet(X.sum + 16 * g.cw, g.cw) ? 1 : 0;
@@ -779,7 +695,7 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   __syncthreads();
   const double rz = N.rz[k], tgt = N.bnorm_in[k];
   int n;
-  const SweepRun<TS> run{P, g, K, k, zl, dict, red, &s_fail, X, rz, tgt, sp.max_inner_its};
+  const SweepRun<TS> run{P, g, fs, K, k, zl, dict, red, &s_fail, X, rz, tgt, sp.max_inner_its};
   n = run.template go<sweep_max_planes((int)sizeof(TS))>();
   if (rk == 0 && tid == 0) R->lits[k] = n;
 }

@@ -312,6 +312,14 @@ struct SlabRuns {
   int n;
 };
 
+// The split of an RVE in an engine of that configuration as {scw, sty, slp, snch}
+// (no engine, no GPU).
+extern "C" int mm_sweep_split(int nex, int ney, int nez, int fp64, int nrhs, int max_rves, int slab_nodes, int *split);
+// Follows a split over its ranks and lanes.  faults: interior nodes not owned by one
+// item, words published twice, words read but not published, and words read from
+// outside the RVE or into another node's LDS place.
+extern "C" int mm_sweep_check(int nex, int ney, int nez, int fp64, const int *split, int *faults);
+
 // launchers (engine_kernels.hip)
 int eng_launch_copy_in(const CopyIn &c, hipStream_t s);
 int eng_launch_unown(const SlabRuns &r, int *slab_rve, hipStream_t s);
