@@ -83,6 +83,7 @@ enum SlotState { SL_FREE = 0, SL_ACTIVE = 1, SL_CACHED = 2 };
 // Split of a resident sweep (RveDev::scw ..), cw = 0: kernels A and B.
 struct SweepTiling {
   int cw = 0, ty = 1, lp = 0, nch = 0;
+  bool meet = false;
 };
 
 struct HostSlot {
@@ -166,7 +167,7 @@ int ensure_device(T **p, size_t *cap, size_t n)
 
 struct mm_engine {
   mm_engine_config cfg;
-  int SN = 128, K = 1;
+  int SN = 128, K = 1, ncu = 0;
   bool fp64 = false;
   bool dict_mode = false;  // MM_ELL_DICT: no per-row ELL arrays, dictionary + pattern bytes
   size_t tsz = 4;
@@ -414,6 +415,10 @@ extern "C" int mm_engine_create(const mm_engine_config *cfg, mm_engine **out)
   e->tsz = e->fp64 ? 8 : 4;
   e->dict_mode = (cfg->ell_storage == MM_ELL_DICT);
   e->rve_cap = cfg->max_rves > 0 ? cfg->max_rves : 4096;
+  if (hipDeviceGetAttribute(&e->ncu, hipDeviceAttributeMultiprocessorCount, cfg->device) != hipSuccess || e->ncu < 1) {
+    delete e;
+    return MM_ERR_HIP;
+  }
   e->t0 = std::chrono::steady_clock::now();
   int rc = 0;
   size_t budget = cfg->hbm_budget;
@@ -442,7 +447,7 @@ extern "C" int mm_engine_create(const mm_engine_config *cfg, mm_engine **out)
   const size_t nrows = (size_t)e->nslab_cap * e->rows_per_slab();
   const size_t slots = nrows * kW;
   // the active lists, then the resident sweep's units (a resident RVE has K *
-  // scw of them, scw at most its slabs, and past kSweepFreeRanks an eighth)
+  // scw of them, scw at most its slabs, and past sweep_free_ranks an eighth)
   const size_t act_ints = 4 * ((size_t)e->nslab_cap + 1);
   e->unit_stride = 1 + (size_t)e->K * std::min<size_t>((size_t)kSweepFreeRanks * e->rve_cap + (size_t)e->nslab_cap / 8, (size_t)e->nslab_cap);
   const size_t lists = act_ints * sizeof(int) + 2 * e->unit_stride * sizeof(int2);
@@ -839,22 +844,22 @@ static void sweep_split(const mm_rve_spec &s, int tsz, int ty, int cz, const Cos
 // enough planes that small RVEs still occupy the lanes.  cw = 0 (kernels A and
 // B) without an interior and where nothing fits.  Fixed by the RVE and the engine
 // configuration alone: K load cases and rve_cap slots of tsz-byte values, slabs of
-// SN nodes.
-static SweepTiling sweep_tiling(const mm_rve_spec &s, int tsz, int K, int rve_cap, int SN)
+// SN nodes, ncu CUs.
+static SweepTiling sweep_tiling(const mm_rve_spec &s, int tsz, int K, int rve_cap, int SN, int ncu)
 {
   SweepTiling t;
   const int nix = s.nex - 1, niy = s.ney - 1, niz = s.nez - 1;
   const long long nslab = rve_slabs(s, SN);
   if (nix < 1 || niy < 1 || niz < 1 || nix > 4096 || niy > 4096) return t;
-  // (past kSweepFreeRanks, workgroups are bounded by the slabs for the unit lists' sake)
-  const int few = (int)std::min<long long>(kSweepFreeRanks, nslab);
-  const int many = (int)std::max<long long>(few, std::min<long long>(kSweepMaxRanks, nslab / 8));
+  // (past sweep_free_ranks, workgroups are bounded by the slabs for the unit lists' sake)
+  const int few = (int)std::min<long long>(sweep_free_ranks(ncu), nslab);
+  const int many = (int)std::max<long long>(few, std::min<long long>(sweep_max_ranks(ncu), nslab / 8));
   const auto search = [&](int most, int ty0, int ty1, const auto &cost) {
     double best = 0.0;
     for (int ty = ty0; ty <= ty1 && ty <= most && ty <= niy; ty++)
       for (int cz = 1; ty * cz <= most && cz <= niz; cz++) sweep_split(s, tsz, ty, cz, cost, best, t);
   };
-  const double room = 256.0 / ((double)K * rve_cap);
+  const double room = (double)ncu / ((double)K * rve_cap);
   if (room >= 2.0) {
     // An engine of few RVEs leaves CUs idle: time counts, and, past the CUs that
     // each cluster has when all of them are active, a little of their cost.  One
@@ -874,6 +879,7 @@ static SweepTiling sweep_tiling(const mm_rve_spec &s, int tsz, int K, int rve_ca
     const long long part = nslab * 3 * SN * (long long)tsz;
     if (8LL * ((long long)nix * niy * niz * (tsz / 4) + sweep_sum_words(t.cw)) > part) t = SweepTiling();
   }
+  t.meet = t.cw > sweep_free_ranks(ncu);
   return t;
 }
 
@@ -883,21 +889,24 @@ static SweepTiling sweep_tiling(const mm_rve_spec &s, int tsz, int K, int rve_ca
 static SweepTiling sweep_tiling(const mm_engine *e, const mm_rve_spec &s)
 {
   if (e->cfg.sync_every_step || e->cfg.profile_step_kernel) return SweepTiling();
-  return sweep_tiling(s, (int)e->tsz, e->K, e->rve_cap, e->SN);
+  return sweep_tiling(s, (int)e->tsz, e->K, e->rve_cap, e->SN, e->ncu);
 }
 
-extern "C" int mm_sweep_split(int nex, int ney, int nez, int fp64, int nrhs, int max_rves, int slab_nodes, int *split)
+extern "C" int mm_sweep_split(int nex, int ney, int nez, int fp64, int nrhs, int max_rves, int slab_nodes, int ncu,
+                              int *split)
 {
-  if (!split || nex < 1 || ney < 1 || nez < 1 || nrhs < 1 || max_rves < 1 || slab_nodes < 1) return MM_ERR_ARG;
+  if (!split || nex < 1 || ney < 1 || nez < 1 || nrhs < 1 || max_rves < 1 || slab_nodes < 1 || ncu < 1)
+    return MM_ERR_ARG;
   mm_rve_spec s = {};
   s.nex = nex;
   s.ney = ney;
   s.nez = nez;
-  const SweepTiling t = sweep_tiling(s, fp64 ? 8 : 4, nrhs, max_rves, slab_nodes);
+  const SweepTiling t = sweep_tiling(s, fp64 ? 8 : 4, nrhs, max_rves, slab_nodes, ncu);
   split[0] = t.cw;
   split[1] = t.ty;
   split[2] = t.lp;
   split[3] = t.nch;
+  split[4] = t.meet;
   return 0;
 }
 
@@ -994,6 +1003,7 @@ static void fill_state(const mm_engine *e, const HostSlot &h, RveDev *st, int wa
   st->sty = sw.ty;
   st->slp = sw.lp;
   st->snch = sw.nch;
+  st->smeet = sw.meet ? 1 : 0;
   st->big = (sw.cw == 0 && h.nslab >= e->cfg.big_slabs) ? 1 : 0;
   for (int k = 0; k < h.req.nload; k++)
     for (int i = 0; i < MM_NVOI; i++) st->load[k][i] = h.req.strain[k][i];
@@ -1178,7 +1188,7 @@ static int update_active(mm_engine *e)
     if (half == 0 && ngroup == 2 && n[0] > 0 && 2 * n[0] >= total) half = 1;
     const SweepTiling &sw = h.sweep;
     // clusters that need most of the CUs at once stay in one chain of launches
-    const int g = sw.cw > kSweepFreeRanks ? 0 : half;
+    const int g = sw.meet ? 0 : half;
     for (long long b = 0; b < h.nslab; b++) e->st_act[g * stride + 1 + n[g]++] = (int)(r.first + b);
     if (sw.cw > 0) {
       res[g].push_back({h.nrow / 3, make_int2(r.second, sw.cw)});

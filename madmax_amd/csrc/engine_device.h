@@ -113,7 +113,7 @@ __device__ __forceinline__ bool sweep_ran(const EngPtrs &P, const RveDev *R)
   const SolveState *S = &R->st[0];
   if (S->phase != PH_INNER) return S->phase == PH_RES;
   const int cw = R->scw;
-  if (cw <= kSweepFreeRanks) return true;
+  if (!R->smeet) return true;
   const long long ni = (long long)(R->nx - 2) * (R->ny - 2) * (R->nz - 2);
   bool ran = true;
   for (int k = 0; k < K; k++)
@@ -135,7 +135,7 @@ __device__ void sweep_end(const EngPtrs &P, const RveDev *R, SolveState &N)
   if (phase == PH_INNER || phase == PH_RES) {
     for (int k = 0; k < K; k++) {
       const bool run = phase == PH_INNER && !((N.done_in >> k) & 1u);
-      if (cw > kSweepFreeRanks) {
+      if (R->smeet) {
         word_t *meet = sweep_words<TS>(P, R->nslab, K, R->first_slab, k, ni).sum + 16 * cw;
         const bool ran = meet[1] == kMeetGo;
         meet[0] = meet[1] = 0;

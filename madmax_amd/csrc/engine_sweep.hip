@@ -613,7 +613,7 @@ extern __shared__ __attribute__((aligned(16))) double sweep_dyn[];
 // workgroups form whole clusters but for the last one, the whole ones finish
 // without waiting for anyone else, and their places go to the missing ranks
 // (also beside other such launches: each leaves at most one cluster of at most
-// kSweepFreeRanks workgroups waiting, and the GPU has more places than the
+// sweep_free_ranks workgroups waiting, and the GPU has more places than the
 // queues' launches can fill with those; a larger cluster waits only before it has
 // started, and not for long: cluster_meet).
 // The residual follows (k_sweep_res), and kernel R passes the state on.
@@ -659,7 +659,7 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   const SweepGeo g = sweep_geo_of(R, rk);
   const int SN = P.SN, RS = 3 * SN, fs = scalar(R->first_slab), tsz = (int)sizeof(TS);
   const SweepWords X = sweep_words<TS>(P, scalar(R->nslab), K, fs, k, g.ni);
-  if (g.cw > kSweepFreeRanks) {
+  if (scalar(R->smeet)) {
     if (tid == 0) s_unit = cluster_meet(X.sum + 16 * g.cw, g.cw) ? 1 : 0;
     __syncthreads();
     if (scalar(s_unit) == 0) return;

@@ -130,6 +130,7 @@ struct RveDev {
   // items of slp planes of one column; lits[k] is the iteration count of load
   // case k in the sweep.  scw == 0: kernels A and B.
   int scw, sty, slp, snch;
+  int smeet;  // the workgroups of a load case meet before they wait for each other
   int lits[MM_MAX_RHS];
   double rr_rz[2 * MM_MAX_RHS];
   double pq[MM_MAX_RHS];
@@ -233,11 +234,13 @@ constexpr int kMarchMaxLds = 64 * 1024;
 // kernel.
 constexpr int kSweepLanes = 512;  // two waves per SIMD, 256 VGPRs each
 constexpr int kSweepItems = 2;    // items (a column times slp planes) per lane
-// Workgroups per load case.  A cluster that waits for ranks without a CU holds
-// the CUs of the others; with up to kSweepFreeRanks, four queues of waiting
-// clusters leave room for any missing rank, and larger clusters first meet.
-constexpr int kSweepFreeRanks = 16;
-constexpr int kSweepMaxRanks = 240;  // of 256 CUs
+// Workgroups per load case, of a device of ncu CUs.  A cluster that waits for ranks
+// without a CU holds the CUs of the others; with up to sweep_free_ranks, four queues
+// of waiting clusters leave room for any missing rank, and larger clusters first
+// meet (RveDev::smeet).
+constexpr int kSweepFreeRanks = 16, kSweepMaxRanks = 240;  // of the 256 CUs of a whole device
+inline int sweep_free_ranks(int ncu) { return ncu >= 256 ? kSweepFreeRanks : ncu >= 32 ? ncu / 16 : 1; }
+inline int sweep_max_ranks(int ncu) { return ncu >= 256 ? kSweepMaxRanks : ncu - (ncu + 15) / 16; }
 constexpr unsigned long long kMeetGo = 1, kMeetOff = 2;
 constexpr int kSweepUnitRanks = 256;  // a unit is (slot, load case * this + rank)
 constexpr int kSweepMaxLds = 160 * 1024 - 2816;  // dynamic; the static part is below 2.75 KB
@@ -312,9 +315,10 @@ struct SlabRuns {
   int n;
 };
 
-// The split of an RVE in an engine of that configuration as {scw, sty, slp, snch}
-// (no engine, no GPU).
-extern "C" int mm_sweep_split(int nex, int ney, int nez, int fp64, int nrhs, int max_rves, int slab_nodes, int *split);
+// The split of an RVE in an engine of that configuration on a device of ncu CUs as
+// {scw, sty, slp, snch, smeet} (no engine, no GPU).
+extern "C" int mm_sweep_split(int nex, int ney, int nez, int fp64, int nrhs, int max_rves, int slab_nodes, int ncu,
+                              int *split);
 // Follows a split over its ranks and lanes.  faults: interior nodes not owned by one
 // item, words published twice, words read but not published, and words read from
 // outside the RVE or into another node's LDS place.

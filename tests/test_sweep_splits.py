@@ -11,10 +11,15 @@ import pytest
 from madmax_amd import _lib
 
 
-def split(n, fp64, nrhs, max_rves, slab_nodes=128):
+def split(n, fp64, nrhs, max_rves, slab_nodes=128, ncu=256):
     """(ranks, shares of the rows, planes per item, items per column); 0 ranks: not swept on chip."""
-    out = (C.c_int * 4)()
-    assert _lib.lib().mm_sweep_split(*n, int(fp64), nrhs, max_rves, slab_nodes, out) == 0
+    return split_meet(n, fp64, nrhs, max_rves, slab_nodes, ncu)[:4]
+
+
+def split_meet(n, fp64, nrhs, max_rves, slab_nodes, ncu):
+    """The same and whether the ranks meet before they wait for each other."""
+    out = (C.c_int * 5)()
+    assert _lib.lib().mm_sweep_split(*n, int(fp64), nrhs, max_rves, slab_nodes, ncu, out) == 0
     return tuple(out)
 
 
@@ -63,6 +68,24 @@ def test_every_word_that_is_read_is_published():
     # every kind of split was among them
     assert kinds[True, False] > 100 and kinds[False, False] > 100 and kinds[True, True] + kinds[False, True] > 20
     assert shared > 100 and lengths >= {(False, i) for i in range(1, 9)} | {(True, i) for i in range(1, 5)}
+
+
+@pytest.mark.parametrize("ncu", [1, 8, 32, 64, 128, 256, 304])
+def test_splits_fit_the_device(ncu):
+    """A cluster never has more ranks than the device can run at once, and one that does not meet first is small
+    enough that four waiting ones leave room for a missing rank."""
+    rng, some = random.Random(ncu), 0
+    for _ in range(1500):
+        n = tuple(rng.randint(2, rng.choice([24, 60, 110])) for _ in range(3))
+        fp64, nrhs, max_rves = rng.random() < 0.5, rng.choice([1, 6, 7]), rng.choice([1, 4, 16, 64, 4096])
+        s = split_meet(n, fp64, nrhs, max_rves, 128, ncu)
+        if s[0] == 0:
+            continue
+        some += 1
+        assert s[0] <= max(1, min(ncu - 1, 240)) and faults(n, fp64, s[:4]) == (0, 0, 0, 0)
+        if s[0] > 1 and not s[4]:
+            assert s[0] <= 16 and 4 * (s[0] - 1) < ncu
+    assert some > 100
 
 
 def test_cells_without_an_interior_or_too_wide_are_not_swept():
