@@ -80,6 +80,11 @@ constexpr int kSweepSteps = 5;
 
 enum SlotState { SL_FREE = 0, SL_ACTIVE = 1, SL_CACHED = 2 };
 
+// Launches (of kSweepSteps steps or more) in a row in which no cluster of workgroups met
+// and some called their meeting off, after which those go on by kernels A and B: half a
+// second or so of other work that holds the CUs.
+constexpr int kMeetLaunches = 8;
+
 // Split of a resident sweep (RveDev::scw ..), cw = 0: kernels A and B.
 struct SweepTiling {
   int cw = 0, ty = 1, lp = 0, nch = 0;
@@ -95,6 +100,8 @@ struct HostSlot {
   long long first_slab = 0, nslab = 0, elem_base = 0, nelm = 0;
   int nrow = 0;
   SweepTiling sweep;
+  int met = 0, missed = 0;  // RveOut's, as last looked at
+  bool stepped = false;     // sweep given up for kernels A and B
   double t_submit = 0, t_admit = 0;
   uint64_t lru = 0;
 };
@@ -238,6 +245,9 @@ struct mm_engine {
   unsigned *ticket = nullptr;
   size_t unit_stride = 0;
   long long unit_n[2] = {0, 0};
+  // launches in a row without a meeting (kMeetLaunches)
+  int meet_lost = 0;
+  unsigned meet_off = 0;
   // one captured graph per set of launch shapes (grids: powers of two >= 64
   // covering each group's slabs and tiles, 0 for an empty group; kernel A's
   // LDS); the kernels read the active count from their list
@@ -304,6 +314,7 @@ struct mm_engine {
     sp.inner_rtol = cfg.inner_rtol;
     sp.max_inner_its = cfg.max_inner_its;
     sp.max_sweeps = cfg.max_sweeps;
+    sp.meet_off = meet_off;
     return sp;
   }
   double now() const
@@ -1102,6 +1113,7 @@ static int admit(mm_engine *e)
   for (int s : fresh) {
     HostSlot &h = e->slots[s];
     h.sweep = sweep_tiling(e, h.req.rve);
+    h.stepped = false;
     fill_state(e, h, &e->st_states[i], 0);
     e->st_slots[i++] = s;
     for (int m = 0; m < kNmat; m++) {
@@ -1113,13 +1125,19 @@ static int admit(mm_engine *e)
     for (long long b = 0; b < h.nslab; b++) e->st_slabs[is++] = (int)(h.first_slab + b);
   }
   for (int s : reused) {
-    const HostSlot &h = e->slots[s];
+    HostSlot &h = e->slots[s];
+    if (h.stepped) h.sweep = sweep_tiling(e, h.req.rve);
+    h.stepped = false;
     fill_state(e, h, &e->st_states[i], h.req.warm_start ? 1 : 0);
     e->st_slots[i++] = s;
     for (long long b = 0; b < h.nslab; b++) e->st_slabs[is++] = (int)(h.first_slab + b);
   }
-  for (int s : fresh) e->out_host[s].phase = 0;
-  for (int s : reused) e->out_host[s].phase = 0;
+  for (const auto *list : {&fresh, &reused})
+    for (int s : *list) {
+      RveOut &o = e->out_host[s];
+      o.phase = o.met = o.missed = 0;
+      e->slots[s].met = e->slots[s].missed = 0;
+    }
   if ((rc = flush_freed(e))) return rc;
   CopyIn in;
   in.add(e->dv_states, e->st_states, n * sizeof(RveDev));
@@ -1337,6 +1355,42 @@ static int run_steps(mm_engine *e)
   return 0;
 }
 
+// After a launch: counts it if clusters called their meeting off and none met, and
+// after kMeetLaunches of those moves the RVEs that still wait to kernels A and B.  One
+// such launch is enough until a cluster meets again.
+static int check_meetings(mm_engine *e)
+{
+  bool met = false;
+  std::vector<int> waiting;
+  for (int s = 0; s < e->rve_cap; s++) {
+    HostSlot &h = e->slots[s];
+    if (h.state != SL_ACTIVE || !h.sweep.meet) continue;
+    const volatile RveOut *o = e->out_host + s;
+    if (o->met != h.met) met = true;
+    else if (o->missed != h.missed) waiting.push_back(s);
+    h.met = o->met;
+    h.missed = o->missed;
+  }
+  if (met) e->meet_lost = 0;
+  if (met || waiting.empty() || ++e->meet_lost < kMeetLaunches) return 0;
+  for (int s : waiting) {
+    HostSlot &h = e->slots[s];
+    const int rc = eng_launch_stepped(e->rves, s, h.nslab >= e->cfg.big_slabs ? 1 : 0, e->stream);
+    if (rc) return rc;
+    h.sweep = SweepTiling();
+    h.stepped = true;
+  }
+  e->act_dirty = true;
+  return 0;
+}
+
+extern "C" int mm_engine_set_meet_off(mm_engine *e, unsigned mask)
+{
+  if (!e || e->nsteps > 0) return MM_ERR_ARG;
+  e->meet_off = mask;
+  return 0;
+}
+
 static void retire(mm_engine *e)
 {
   for (int s = 0; s < e->rve_cap; s++) {
@@ -1394,6 +1448,7 @@ extern "C" int mm_engine_step(mm_engine *e)
   }
   e->prof_pending = 0;
   e->nsteps++;
+  if ((rc = check_meetings(e))) return e->last_error = rc;
   retire(e);
   return 0;
 }

@@ -125,9 +125,10 @@ __device__ __forceinline__ bool sweep_ran(const EngPtrs &P, const RveDev *R)
 // A resident RVE's state between launches, by one lane, after the residual (if
 // any).  The end of a sweep: its iteration count is the largest of the load cases'
 // (as inner_check counts).  Load cases whose cluster did not meet are left for the
-// next launch.
+// next launch; the host counts those without a meeting and puts the RVE on kernels
+// A and B after a few.
 template <typename TS, int K>
-__device__ void sweep_end(const EngPtrs &P, const RveDev *R, SolveState &N)
+__device__ void sweep_end(const EngPtrs &P, int slot, RveDev *R, SolveState &N)
 {
   const int cw = R->scw, phase = N.phase;
   const long long ni = (long long)(R->nx - 2) * (R->ny - 2) * (R->nz - 2);
@@ -141,11 +142,19 @@ __device__ void sweep_end(const EngPtrs &P, const RveDev *R, SolveState &N)
         meet[0] = meet[1] = 0;
         if (run && !ran) {
           left = true;
+          R->missed += 1;
           continue;
         }
-        if (run) N.done_in |= 1u << k;
+        if (run) {
+          N.done_in |= 1u << k;
+          R->met += 1;
+        }
       }
       if (run) N.its = max(N.its, R->lits[k]);
+    }
+    if (R->smeet && phase == PH_INNER) {
+      P.out[slot].met = R->met;
+      P.out[slot].missed = R->missed;
     }
   }
   if (phase == PH_INNER && !left) {
@@ -173,7 +182,7 @@ __device__ void start_sweep(SolveState &N, const double (&s4)[4 * K], const RveD
     N.rnorm[k] = rn;
     if (N.sweep == 0) N.r0[k] = need_cold ? sqrt(s4[3 * K + k]) : rn;
     const bool conv = (k >= R->nload) || N.r0[k] == 0.0 || rn <= sp.rtol * N.r0[k] ||
-                      rn < sp.abs_tol || N.sweep >= sp.max_sweeps;
+                      rn < sp.abs_tol || N.sweep >= sp.max_sweeps + R->again;
     if (conv) done_out |= 1u << k;
     // absolute target of this sweep: inner_rtol of the sweep's right-hand
     // side, but no tighter than what the outer tolerance still needs
@@ -279,7 +288,7 @@ __device__ void finish_rve(const EngPtrs &P, int slot, const RveDev *R, SolveSta
   }
   o->residual_rel = rel;
   o->its_total = N.its_total;
-  o->sweeps = N.sweep;
+  o->sweeps = N.sweep - R->idle;
   o->status = ok ? MM_OK : MM_NOT_CONVERGED;
   N.status = o->status;
   N.phase = PH_DONE;

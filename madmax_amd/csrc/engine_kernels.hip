@@ -101,6 +101,23 @@ __global__ __launch_bounds__(256) void k_unown(SlabRuns r, int *__restrict__ sla
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < r.run[p].y; i += step) slab_rve[r.run[p].x + i] = -1;
 }
 
+// Ends the sweep of a resident RVE as it stands (x has the load cases that ran) and
+// leaves the RVE to kernels A and B, from a new residual.  The sweep counts, so that r0
+// stays that of the first one, but not against max_sweeps, nor in the result if no load
+// case ran.
+__global__ void k_stepped(RveDev *R, int big)
+{
+  SolveState N = R->st[2];
+  N.its_total += N.its;
+  N.sweep += 1;
+  N.phase = PH_RES;
+  for (int c = 0; c < 3; c++) R->st[c] = N;
+  R->again += 1;
+  if (N.done_in == N.done_out) R->idle += 1;
+  R->scw = R->sty = R->slp = R->snch = R->smeet = 0;
+  R->big = big;
+}
+
 // Element stiffness per (RVE, material), one wavefront each.  The derivatives
 // at the 8 gauss points are built in LDS from the hex8 tables of
 // src/fem.c:309-405 with dN/dx_d = ds * 2 / h_d; C is the isotropic tangent in
@@ -1746,7 +1763,7 @@ __device__ void r_slab(const EngPtrs &P, int slab, double (&lds)[RedLds<K>::size
     __shared__ SolveState N;
     if (slab == R->first_slab && tid == 0) {
       N = R->st[0];
-      sweep_end<TS, K>(P, R, N);
+      sweep_end<TS, K>(P, slot, R, N);
       R->st[2] = N;
       *P.ticket = 0u;  // for the next resident sweep
     }
@@ -2049,6 +2066,13 @@ int eng_launch_unown(const SlabRuns &r, int *slab_rve, hipStream_t s)
   if (most == 0) return 0;
   const int grid = (most + 255) / 256;
   k_unown<<<grid < 512 ? grid : 512, 256, 0, s>>>(r, slab_rve);
+  MM_HIP(hipGetLastError());
+  return 0;
+}
+
+int eng_launch_stepped(RveDev *rves, int slot, int big, hipStream_t s)
+{
+  k_stepped<<<1, 1, 0, s>>>(rves + slot, big);
   MM_HIP(hipGetLastError());
   return 0;
 }

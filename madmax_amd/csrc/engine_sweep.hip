@@ -320,10 +320,15 @@ __device__ __forceinline__ bool cluster_sum(double (&v)[NV], const word_t *sum, 
 // case all leave and the sweep is tried again by the next launch.  The wait
 // covers the clusters before it in this launch that still run; it differs from
 // one attempt to the next, so that two clusters on different streams that keep
-// each other from the CUs do not go on doing so.  Run by one lane.
+// each other from the CUs do not go on doing so.  Run by one lane.  off: call it off
+// at once.
 constexpr int kMeetPolls = 1 << 14;  // some 10 ms, plus as much at random
-__device__ __forceinline__ bool cluster_meet(word_t *meet, int cw)
+__device__ __forceinline__ bool cluster_meet(word_t *meet, int cw, bool off)
 {
+  if (off) {
+    __hip_atomic_store(&meet[1], (word_t)kMeetOff, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return false;
+  }
   const word_t n = __hip_atomic_fetch_add(&meet[0], (word_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   word_t none = 0;
   if (n + 1 == (word_t)cw)
@@ -660,7 +665,7 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   const int SN = P.SN, RS = 3 * SN, fs = scalar(R->first_slab), tsz = (int)sizeof(TS);
   const SweepWords X = sweep_words<TS>(P, scalar(R->nslab), K, fs, k, g.ni);
   if (scalar(R->smeet)) {
-    if (tid == 0) s_unit = cluster_meet(X.sum + 16 * g.cw, g.cw) ? 1 : 0;
+    if (tid == 0) s_unit = cluster_meet(X.sum + 16 * g.cw, g.cw, ((sp.meet_off >> k) & 1u) != 0) ? 1 : 0;
     __syncthreads();
     if (scalar(s_unit) == 0) return;
   }

@@ -131,6 +131,9 @@ struct RveDev {
   // case k in the sweep.  scw == 0: kernels A and B.
   int scw, sty, slp, snch;
   int smeet;  // the workgroups of a load case meet before they wait for each other
+  // load cases whose workgroups met and did not since admission, and sweeps that
+  // ended (k_stepped) without an update of some load cases and of all
+  int met, missed, again, idle;
   int lits[MM_MAX_RHS];
   double rr_rz[2 * MM_MAX_RHS];
   double pq[MM_MAX_RHS];
@@ -148,6 +151,7 @@ struct RveDev {
 struct RveOut {
   int phase;   // mirrors RveDev::phase once the RVE is finished
   int status, its_total, sweeps;
+  int met, missed;  // RveDev's
   double residual_rel;
   double stress[MM_MAX_RHS][MM_NVOI];
   double strain[MM_MAX_RHS][MM_NVOI];
@@ -158,6 +162,7 @@ struct SolveParams {
   int nrhs, slab_nodes;
   double rtol, abs_tol, inner_rtol;
   int max_inner_its, max_sweeps;
+  unsigned meet_off;  // load cases whose workgroups are not to meet (mm_engine_set_meet_off)
 };
 
 // Device pointers of the engine arena handed to every solver kernel.
@@ -319,6 +324,9 @@ struct SlabRuns {
 // {scw, sty, slp, snch, smeet} (no engine, no GPU).
 extern "C" int mm_sweep_split(int nex, int ney, int nez, int fp64, int nrhs, int max_rves, int slab_nodes, int ncu,
                               int *split);
+// Before an engine's first step: the load cases of `mask` (bit k: case k) never meet, as
+// if other work kept the CUs.  For tests.
+extern "C" int mm_engine_set_meet_off(mm_engine *e, unsigned mask);
 // Follows a split over its ranks and lanes.  faults: interior nodes not owned by one
 // item, words published twice, words read but not published, and words read from
 // outside the RVE or into another node's LDS place.
@@ -327,6 +335,8 @@ extern "C" int mm_sweep_check(int nex, int ney, int nez, int fp64, const int *sp
 // launchers (engine_kernels.hip)
 int eng_launch_copy_in(const CopyIn &c, hipStream_t s);
 int eng_launch_unown(const SlabRuns &r, int *slab_rve, hipStream_t s);
+// a resident RVE whose sweep waits for a meeting, to kernels A and B
+int eng_launch_stepped(RveDev *rves, int slot, int big, hipStream_t s);
 int upload_slot_tables(hipStream_t s);
 bool eng_supported_rhs(int K);
 // nkern solver launches of the cycle A (0) -> B (1) -> R (2), from `first`
