@@ -1477,10 +1477,14 @@ extern "C" int mm_engine_drain(mm_engine *e)
   if (!e) return MM_ERR_ARG;
   long long stall = 0;
   size_t last_q = (size_t)-1;
-  // every RVE finishes within max_sweeps * (max_inner_its + 3) PCG steps;
-  // a drain that makes no progress for longer than that reports an error
-  const long long limit =
-      (long long)e->cfg.max_sweeps * (e->cfg.max_inner_its + 4) / e->cfg.steps_per_launch + 64;
+  // every RVE finishes within max_sweeps * (max_inner_its + 3) PCG steps, of which a
+  // launch has steps_per_launch, or max_sweeps + 3 whole sweeps, of which it has
+  // kSweepSteps at most; a drain that makes no progress for longer than that, and for
+  // the launches that may pass without a meeting, reports an error
+  const long long steps = e->cfg.steps_per_launch, sweeps = std::min<long long>(steps, kSweepSteps);
+  const long long limit = std::max((long long)e->cfg.max_sweeps * (e->cfg.max_inner_its + 4) / steps,
+                                   ((long long)e->cfg.max_sweeps + 3) / sweeps) +
+                          kMeetLaunches + 64;
   long long idle = 0, done0 = e->completed;
   while (has_work(e)) {
     int rc = mm_engine_step(e);
