@@ -17,10 +17,10 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-#include <condition_variable>
 #include <mutex>
 
 #include "ell.h"
+#include "fair_share.h"
 #include "fe.h"
 #include "mm_device.h"
 #include "mm_internal.h"
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
 // (one, 192, where the LDS of two does not fit): 192 CUs, which leaves 64 for
 // kernels of other streams that wait for workgroups of their own, as the engine's
 // sweeps do (at most 15 CUs each).  Solves of one process share the 192 CUs
-// (ResShare).  Every wait is bounded all the same, and a solve whose wait ran out,
+// (FairShare).  Every wait is bounded all the same, and a solve whose wait ran out,
 // for instance beside another process's, is done again in the two-launch form.
 constexpr int kResSlots = 81;  // rows of 27 nodes' 3 dofs; five registers for two slots, 203 of 256
 constexpr int kResMaxSlabs = 384;
@@ -1311,41 +1311,12 @@ extern "C" int ell_device_solve_jacobi(ell_device *d, ell_solver *solver, const 
   return 0;
 }
 
-// The part of a device that resident solves of this process hold together, in
-// halves of a CU; a solve waits here until its workgroups fit beside the others.
-class ResShare {
- public:
-  ResShare(int device, int halves) : g_(gate(device)), halves_(halves)
-  {
-    std::unique_lock<std::mutex> lk(g_.mu);
-    g_.cv.wait(lk, [&] { return g_.used + halves_ <= kResMaxSlabs; });
-    g_.used += halves_;
-  }
-  ~ResShare()
-  {
-    {
-      std::lock_guard<std::mutex> lk(g_.mu);
-      g_.used -= halves_;
-    }
-    g_.cv.notify_all();
-  }
-  ResShare(const ResShare &) = delete;
-  ResShare &operator=(const ResShare &) = delete;
-
- private:
-  struct Gate {
-    std::mutex mu;
-    std::condition_variable cv;
-    int used = 0;
-  };
-  static Gate &gate(int device)
-  {
-    static Gate g[kResMaxDevices];
-    return g[device];
-  }
-  Gate &g_;
-  const int halves_;
-};
+// What resident solves of this process hold together of a device, in halves of a CU.
+static ShareGate &res_gate(int device)
+{
+  static ShareGate g[kResMaxDevices];
+  return g[device];
+}
 
 // Jacobi-PCG on the device mirror with b and x (initial guess in, solution
 // out) in device memory and the work vectors V; the host polls the
@@ -1370,16 +1341,19 @@ static int pcg_run(ell_device *d, const PcgVecs &V, ell_solver *solver, const do
   MM_HIP(hipGetLastError());
   IterState h;
   if (resident) {
-    ResShare share(d->device, res_lds(res_rows) <= (size_t)kResOneCuLds ? d->nslab : 2 * d->nslab);
-    word_t *zw = reinterpret_cast<word_t *>(V.zpB), *sums = reinterpret_cast<word_t *>(V.q);
-    k_res_zero<<<(16 * d->nslab + 255) / 256, 256, 0, d->stream>>>(sums, 16 * d->nslab);
-    const auto solve = span > kResListSpan ? k_pcg_resident<true> : k_pcg_resident<false>;
-    solve<<<d->nslab, 256, res_lds(res_rows), d->stream>>>(
-        d->cols, d->vals, d->nrow, d->nnz, d->nslab, res_rows, d->dinv, x, V.r, V.zpA, zw, sums, V.st);
-    k_res_take<<<(d->nrow + 255) / 256, 256, 0, d->stream>>>(V.st, V.zpA, x, d->nrow);
-    MM_HIP(hipGetLastError());
-    rc = get_state(d, V.st, &h);
-    if (rc) return rc;
+    {
+      FairShare share(res_gate(d->device), res_lds(res_rows) <= (size_t)kResOneCuLds ? d->nslab : 2 * d->nslab,
+                      kResMaxSlabs);
+      word_t *zw = reinterpret_cast<word_t *>(V.zpB), *sums = reinterpret_cast<word_t *>(V.q);
+      k_res_zero<<<(16 * d->nslab + 255) / 256, 256, 0, d->stream>>>(sums, 16 * d->nslab);
+      const auto solve = span > kResListSpan ? k_pcg_resident<true> : k_pcg_resident<false>;
+      solve<<<d->nslab, 256, res_lds(res_rows), d->stream>>>(d->cols, d->vals, d->nrow, d->nnz, d->nslab, res_rows,
+                                                             d->dinv, x, V.r, V.zpA, zw, sums, V.st);
+      k_res_take<<<(d->nrow + 255) / 256, 256, 0, d->stream>>>(V.st, V.zpA, x, d->nrow);
+      MM_HIP(hipGetLastError());
+      rc = get_state(d, V.st, &h);
+      if (rc) return rc;
+    }
     if (h.pad0) return pcg_run(d, V, solver, b, x, false);  // a wait ran out: x is as it was
   } else {
     rc = get_state(d, V.st, &h);
