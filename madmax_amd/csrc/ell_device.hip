@@ -594,14 +594,18 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
 // against this: 2,970 rows 22.7 and 7.0, 14,739 rows 23.6 and 8.2, 46,875 rows
 // 25.0 and 9.8, 89,373 rows 32.5 and 13.0.
 //
-// All workgroups have to run at the same time.  They are at most 384, two to a CU
-// (one, 192, where the LDS of two does not fit): 192 CUs, which leaves 64 for
-// kernels of other streams that wait for workgroups of their own, as the engine's
-// sweeps do (at most 15 CUs each).  Solves of one process share the 192 CUs
-// (FairShare).  Every wait is bounded all the same, and a solve whose wait ran out,
-// for instance beside another process's, is done again in the two-launch form.
+// All workgroups have to run at the same time.  They are at most three quarters of what
+// the CUs take, two to a CU (one where the LDS of two does not fit): 384 or 192 of 256
+// CUs, which leaves a quarter for kernels of other streams that wait for workgroups of
+// their own, as the engine's sweeps do (at most 15 CUs each).  Solves of one process
+// share that (FairShare).  Beside other work they may still not find their CUs, for
+// instance beside another process's solves: they meet before their first exchange, and
+// a solve that did not meet, some 10 ms later, is done in the two-launch form, as are
+// the mirror's next ones (1, 3, 7, .. 63 of them until one meets again).  After the
+// meeting all of them run; the waits are bounded all the same.
 constexpr int kResSlots = 81;  // rows of 27 nodes' 3 dofs; five registers for two slots, 203 of 256
-constexpr int kResMaxSlabs = 384;
+constexpr int kResRest = 63;  // most solves in two launches between attempts
+inline int res_cus(int ncu) { return ncu - ncu / 4; }
 constexpr int kResOneCuLds = 69 * 1024;  // dynamic LDS up to which two workgroups fit a CU
 constexpr int kResMaxLds = 149 * 1024;
 constexpr int kResPolls = 1 << 18;  // about 0.2 s
@@ -659,18 +663,19 @@ __device__ __forceinline__ double rounded(double v)
 }
 
 // zw: two words per row (z of the last update), sums: 16 words per slab, all
-// zero on entry (no iteration's tag); zp[row].x is the first z, .y receives x.
+// zero on entry (no iteration's tag; two words of the first slab's are for the
+// meeting); zp[row].x is the first z, .y receives x.  stay_away: call the meeting off.
 template <bool LIST>
 __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__ cols, const double *__restrict__ vals,
                                                          int nrow, int nnz, int nslab, int lds_rows,
                                                          const double *__restrict__ dinv, const double *__restrict__ x0,
                                                          const double *__restrict__ r0, double2 *__restrict__ zp,
-                                                         word_t *zw, word_t *sums, IterState *st)
+                                                         word_t *zw, word_t *sums, IterState *st, int stay_away)
 {
   __shared__ double lds[48];
   __shared__ double bc[2];
   __shared__ double s_row[LIST ? 5 : 1][256];  // x, dinv, r, z and p of the rows, where the registers are full
-  __shared__ int s_lo, s_hi, s_fail, s_wave[4];
+  __shared__ int s_lo, s_hi, s_fail, s_place, s_wave[4];
   if (st->done) return;
   const int lane = threadIdx.x, slab = blockIdx.x;
   const long long row = (long long)slab * 256 + lane, base = (long long)slab * 256 * nnz;
@@ -711,8 +716,15 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
   lo = __builtin_amdgcn_readfirstlane(s_lo);
   hi = __builtin_amdgcn_readfirstlane(s_hi);
   if (hi - lo >= lds_rows) {  // (the host sized the LDS by the widest slab)
-    if (lane == 0) st->pad0 = 1;
+    if (lane == 0) {
+      meet_off(sums + 6);
+      st->pad0 = 1;
+    }
     return;
+  }
+  if (lane == 0) {
+    if (stay_away) meet_off(sums + 6);
+    s_place = meet_arrive(sums + 6, nslab);
   }
   // with LIST only the columns that the slab has entries in get a place, else all
   // between the lowest and the highest: they are marked in bytes (neighbouring rows
@@ -797,7 +809,12 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
     s_row[4][lane] = pi;
   }
   for (int e = lane; e <= nneed; e += 256) res_p[e] = 0.0;
+  if (lane == 0 && !meet_wait(sums + 6, s_place)) s_fail = 1;
   __syncthreads();
+  if (__builtin_amdgcn_readfirstlane(s_fail)) {
+    if (lane == 0) st->pad0 = 1;
+    return;
+  }
   const double bnorm = st->bnorm, rtol = st->rtol;
   const int max_its = st->max_its;
   double rz = st->rz, beta = 0.0, alpha = 0.0, rnorm = st->rnorm;
@@ -1059,6 +1076,10 @@ struct ell_device_ {
   unsigned *bar;
   char *stage;     // row-major entries on their way in (null until the first upload)
   int band;        // most columns that a slab's rows span (0: not known)
+  int ncu;         // CUs of the device
+  // k_pcg_resident: solves to do otherwise before the next attempt, and how many that
+  // was last time; solves that stayed, and that were given up; tests: never meet
+  int res_rest, res_rested, res_stayed, res_left, res_away;
   int fused_its;   // 0: two launches per PCG iteration; n > 0: k_pcg_fused, n iterations per launch
   int fused_grid;  // co-resident workgroups of k_pcg_fused (set with fused_its)
   hipStream_t stream;
@@ -1145,7 +1166,8 @@ extern "C" int ell_device_create(const ell_matrix *m, int slab_rows, ell_device 
   d->nnz = m->nnz;
   d->S = S;
   d->nslab = (m->nrow + S - 1) / S;
-  if (hipGetDevice(&d->device) != hipSuccess) {
+  if (hipGetDevice(&d->device) != hipSuccess ||
+      hipDeviceGetAttribute(&d->ncu, hipDeviceAttributeMultiprocessorCount, d->device) != hipSuccess) {
     free(d);
     return MM_ERR_HIP;
   }
@@ -1328,9 +1350,13 @@ static int pcg_run(ell_device *d, const PcgVecs &V, ell_solver *solver, const do
   // the matrix on chip (k_pcg_resident) where the columns that a slab spans fit
   // the LDS and the workgroups the GPU; it was the faster at every size it takes
   const int span = d->band > 0 ? d->band : d->nrow, res_rows = span > 64 ? span : 64;  // (its tables want as much)
-  const bool resident = may_stay && d->fused_its == 0 && d->S == 256 && d->nnz <= kResSlots &&
-                        d->device < kResMaxDevices && res_lds(res_rows) <= (size_t)kResMaxLds &&
-                        d->nslab <= (res_lds(res_rows) <= (size_t)kResOneCuLds ? kResMaxSlabs : kResMaxSlabs / 2);
+  const bool pairs = res_lds(res_rows) <= (size_t)kResOneCuLds;  // two workgroups to a CU
+  bool resident = may_stay && d->fused_its == 0 && d->S == 256 && d->nnz <= kResSlots && d->device < kResMaxDevices &&
+                  res_lds(res_rows) <= (size_t)kResMaxLds && d->nslab <= (pairs ? 2 : 1) * res_cus(d->ncu);
+  if (resident && d->res_rest > 0) {
+    d->res_rest--;
+    resident = false;
+  }
   const int max_its = (solver && solver->max_its > 0) ? solver->max_its : MAX_ITS;
   const double rtol = (solver && solver->min_err > 0) ? solver->min_err : MIN_ERR;
   int rc = set_state(d, V.st, max_its, rtol, 0.0);
@@ -1342,19 +1368,24 @@ static int pcg_run(ell_device *d, const PcgVecs &V, ell_solver *solver, const do
   IterState h;
   if (resident) {
     {
-      FairShare share(res_gate(d->device), res_lds(res_rows) <= (size_t)kResOneCuLds ? d->nslab : 2 * d->nslab,
-                      kResMaxSlabs);
+      FairShare share(res_gate(d->device), pairs ? d->nslab : 2 * d->nslab, 2 * res_cus(d->ncu));
       word_t *zw = reinterpret_cast<word_t *>(V.zpB), *sums = reinterpret_cast<word_t *>(V.q);
       k_res_zero<<<(16 * d->nslab + 255) / 256, 256, 0, d->stream>>>(sums, 16 * d->nslab);
       const auto solve = span > kResListSpan ? k_pcg_resident<true> : k_pcg_resident<false>;
       solve<<<d->nslab, 256, res_lds(res_rows), d->stream>>>(d->cols, d->vals, d->nrow, d->nnz, d->nslab, res_rows,
-                                                             d->dinv, x, V.r, V.zpA, zw, sums, V.st);
+                                                             d->dinv, x, V.r, V.zpA, zw, sums, V.st, d->res_away);
       k_res_take<<<(d->nrow + 255) / 256, 256, 0, d->stream>>>(V.st, V.zpA, x, d->nrow);
       MM_HIP(hipGetLastError());
       rc = get_state(d, V.st, &h);
       if (rc) return rc;
     }
-    if (h.pad0) return pcg_run(d, V, solver, b, x, false);  // a wait ran out: x is as it was
+    if (h.pad0) {  // no meeting, or a wait that ran out: x is as it was
+      d->res_left++;
+      d->res_rest = d->res_rested = d->res_rested < kResRest ? 2 * d->res_rested + 1 : kResRest;
+      return pcg_run(d, V, solver, b, x, false);
+    }
+    d->res_stayed++;
+    d->res_rested = 0;
   } else {
     rc = get_state(d, V.st, &h);
     if (rc) return rc;
@@ -1462,7 +1493,8 @@ int mm::ell_device_alloc(int nrow, int nnz, int S, ell_device **out)
   d->nnz = nnz;
   d->S = S;
   d->nslab = (nrow + S - 1) / S;
-  if (hipGetDevice(&d->device) != hipSuccess) {
+  if (hipGetDevice(&d->device) != hipSuccess ||
+      hipDeviceGetAttribute(&d->ncu, hipDeviceAttributeMultiprocessorCount, d->device) != hipSuccess) {
     free(d);
     return MM_ERR_HIP;
   }
@@ -1522,6 +1554,22 @@ int mm::ell_device_pcg_device(ell_device *d, ell_solver *solver, const double *b
   if (d->nrow == 0) return 0;
   const PcgVecs V{d->r, d->zpA, d->zpB, d->q, d->part, d->st, d->bar};
   return pcg_run(d, V, solver, b, x);
+}
+
+extern "C" int ell_device_pcg_counts(const ell_device *d, int *counts)
+{
+  if (!d || !counts) return MM_ERR_ARG;
+  counts[0] = d->res_stayed;
+  counts[1] = d->res_left;
+  counts[2] = d->res_rest;
+  return 0;
+}
+
+extern "C" int ell_device_set_stay_away(ell_device *d, int on)
+{
+  if (!d) return MM_ERR_ARG;
+  d->res_away = on ? 1 : 0;
+  return 0;
 }
 
 // ---- the same solve without any allocation ----------------------------------

@@ -315,38 +315,6 @@ __device__ __forceinline__ bool cluster_sum(double (&v)[NV], const word_t *sum, 
   return cluster_collect<NV>(v, sum, cw, tag);
 }
 
-// A cluster of many ranks meets before its first exchange: the last to arrive
-// lets it go; the first calls it off when ranks stay away for long, in which
-// case all leave and the sweep is tried again by the next launch.  The wait
-// covers the clusters before it in this launch that still run; it differs from
-// one attempt to the next, so that two clusters on different streams that keep
-// each other from the CUs do not go on doing so.  Run by one lane.  off: call it off
-// at once.
-constexpr int kMeetPolls = 1 << 14;  // some 10 ms, plus as much at random
-__device__ __forceinline__ bool cluster_meet(word_t *meet, int cw, bool off)
-{
-  if (off) {
-    __hip_atomic_store(&meet[1], (word_t)kMeetOff, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return false;
-  }
-  const word_t n = __hip_atomic_fetch_add(&meet[0], (word_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  word_t none = 0;
-  if (n + 1 == (word_t)cw)
-    __hip_atomic_compare_exchange_strong(&meet[1], &none, kMeetGo, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-  const int most = n == 0 ? kMeetPolls + (int)(clock64() & (kMeetPolls - 1)) : 4 * kMeetPolls;
-  for (int i = 0;; i++) {
-    const word_t m = get_word(&meet[1]);
-    if (m != 0) return m == kMeetGo;
-    if (i >= most) {
-      none = 0;
-      __hip_atomic_compare_exchange_strong(&meet[1], &none, kMeetOff, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __builtin_amdgcn_s_sleep(8);
-  }
-}
-
 // Publishes a node's three rows as the words of interior node at.
 __device__ __forceinline__ void put_node(const SweepWords &X, int ni, int at, unsigned tag, const float (&x)[3])
 {
@@ -665,7 +633,11 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   const int SN = P.SN, RS = 3 * SN, fs = scalar(R->first_slab), tsz = (int)sizeof(TS);
   const SweepWords X = sweep_words<TS>(P, scalar(R->nslab), K, fs, k, g.ni);
   if (scalar(R->smeet)) {
-    if (tid == 0) s_unit = cluster_meet(X.sum + 16 * g.cw, g.cw, ((sp.meet_off >> k) & 1u) != 0) ? 1 : 0;
+    if (tid == 0) {
+      word_t *meet = X.sum + 16 * g.cw;
+      if ((sp.meet_off >> k) & 1u) meet_off(meet);
+      s_unit = meet_wait(meet, meet_arrive(meet, g.cw)) ? 1 : 0;
+    }
     __syncthreads();
     if (scalar(s_unit) == 0) return;
   }

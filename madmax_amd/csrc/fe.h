@@ -80,6 +80,11 @@ int ell_device_alloc(int nrow, int nnz, int S, ell_device **out);
 void ell_device_arrays(ell_device *d, int **cols, double **vals, double **dinv, int *S, hipStream_t *s);
 // States that the rows of a slab span at most `band` columns.
 void ell_device_set_band(ell_device *d, long long band);
+// PCG solves of a mirror with the matrix on chip: done, given up and done in two
+// launches, and to be done in two launches before the next attempt.
+extern "C" int ell_device_pcg_counts(const ell_device *d, int *counts);
+// The mirror's on-chip solves do not meet, as if other work kept the CUs.  For tests.
+extern "C" int ell_device_set_stay_away(ell_device *d, int on);
 int ell_device_pcg_device(ell_device *d, ell_solver *solver, const double *b, double *x);
 
 }  // namespace mm

@@ -200,4 +200,37 @@ __device__ __forceinline__ double word_double(word_t lo, word_t hi)
   return __builtin_bit_cast(double, (hi << 32) | (lo & 0xffffffffull));
 }
 
+// Workgroups that are to wait for each other meet first, at two words that are zero
+// before: the last to arrive lets them go; the first calls it off when some stay away
+// for long, in which case all leave, also those that come later.  Its wait covers
+// kernels before this one that still run; it differs from one attempt to the next, so
+// that two groups on different streams that keep each other from the CUs do not go on
+// doing so.  Run by one lane of each workgroup.
+constexpr word_t kMeetGo = 1, kMeetOff = 2;
+constexpr int kMeetPolls = 1 << 14;  // some 10 ms, plus as much at random
+__device__ __forceinline__ void meet_set(word_t *meet, word_t to)
+{
+  word_t none = 0;
+  __hip_atomic_compare_exchange_strong(&meet[1], &none, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void meet_off(word_t *meet) { meet_set(meet, kMeetOff); }
+// Returns the place among those that arrived (0: the first).
+__device__ __forceinline__ int meet_arrive(word_t *meet, int count)
+{
+  const int n = (int)__hip_atomic_fetch_add(&meet[0], (word_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (n + 1 == count) meet_set(meet, kMeetGo);
+  return n;
+}
+__device__ __forceinline__ bool meet_wait(word_t *meet, int place)
+{
+  const int most = place == 0 ? kMeetPolls + (int)(clock64() & (kMeetPolls - 1)) : 4 * kMeetPolls;
+  for (int i = 0;; i++) {
+    const word_t m = get_word(&meet[1]);
+    if (m != 0) return m == kMeetGo;
+    if (i >= most) meet_off(meet);
+    __builtin_amdgcn_s_sleep(8);
+  }
+}
+
 }  // namespace mm

@@ -246,7 +246,6 @@ constexpr int kSweepItems = 2;    // items (a column times slp planes) per lane
 constexpr int kSweepFreeRanks = 16, kSweepMaxRanks = 240;  // of the 256 CUs of a whole device
 inline int sweep_free_ranks(int ncu) { return ncu >= 256 ? kSweepFreeRanks : ncu >= 32 ? ncu / 16 : 1; }
 inline int sweep_max_ranks(int ncu) { return ncu >= 256 ? kSweepMaxRanks : ncu - (ncu + 15) / 16; }
-constexpr unsigned long long kMeetGo = 1, kMeetOff = 2;
 constexpr int kSweepUnitRanks = 256;  // a unit is (slot, load case * this + rank)
 constexpr int kSweepMaxLds = 160 * 1024 - 2816;  // dynamic; the static part is below 2.75 KB
 __host__ __device__ constexpr int sweep_max_planes(int tsz) { return tsz == 8 ? 4 : 8; }
