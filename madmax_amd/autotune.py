@@ -2,13 +2,16 @@
 workgroup), the z-run length of the plane-march step kernel, and the
 per-sweep FP32 PCG tolerance of the mixed-precision path.
 
-The slab shape and the run length change only how fast the kernels run, so
-each candidate is judged by the PCG step kernel's own duration on a resident
-sample batch (HIP events, mm_engine_time_step), which is stable where a whole
-small solve is not.  Longer runs mean fewer, longer workgroups: faster for a
-large batch, slower to finish for a few RVEs at a time, so a serving engine
-keeps the engine default.  The sweep tolerance changes the iteration and sweep counts, so its
-candidates are judged by the best of two whole solves of the sample.  Every
+The slab shape and the run length change only how fast the kernels run.  The run
+length is judged by the PCG step kernel's own duration on a resident sample
+batch (HIP events, mm_engine_time_step), which is stable where a whole small
+solve is not.  Longer runs mean fewer, longer workgroups: faster for a large
+batch, slower to finish for a few RVEs at a time, so a serving engine keeps the
+engine default.  The slab shape is judged by the same duration where every RVE
+of the sample is stepped by that kernel (beyond about 100^3 elements).  RVEs
+that are swept on chip do not run it; of them the shape cuts the residuals and
+averages, and it is judged by the best of two whole solves of the sample.  So is
+the sweep tolerance, which changes the iteration and sweep counts.  Every
 candidate must converge to the outer FP64 tolerance, so the choice only
 trades speed.  Results are cached as JSON keyed by device, RVE size, load
 cases and precision.
@@ -53,7 +56,8 @@ def _solve_time(specs, slab_nodes, inner_rtol, rtol, nrhs, precision, budget, ma
         ok = all(r["status"] == 0 for r in res)
         its = max(r["pcg_its"] for r in res)
         step_ms, _ = eng.time_step(reps=20)
-    return dict(seconds=dt, ok=ok, its=its, step_ms=step_ms)
+        swept = any(eng.swept(s) for s in specs)
+    return dict(seconds=dt, ok=ok, its=its, step_ms=step_ms, swept=swept)
 
 
 def tune(specs, nrhs=6, precision=_lib.MM_PREC_MIXED, rtol=1e-9, budget=None, use_cache=True,
@@ -61,7 +65,7 @@ def tune(specs, nrhs=6, precision=_lib.MM_PREC_MIXED, rtol=1e-9, budget=None, us
     """Returns {"slab_nodes", "march_planes", "inner_rtol", "trials": [...]} for this
     workload."""
     n = specs[0].nex
-    key = "%s|n%d|k%d|p%d|b%d|r%g|m" % (os.environ.get("HIP_VISIBLE_DEVICES", "0"), n, nrhs,
+    key = "%s|n%d|k%d|p%d|b%d|r%g|s" % (os.environ.get("HIP_VISIBLE_DEVICES", "0"), n, nrhs,
                                        precision, len(specs), rtol)
     path = _cache_path()
     cache = {}
@@ -84,7 +88,8 @@ def tune(specs, nrhs=6, precision=_lib.MM_PREC_MIXED, rtol=1e-9, budget=None, us
         if log:
             log("tune slab_nodes=%d: step kernel %.3f ms, solve %.3f s, %d its"
                 % (sn, r["step_ms"], r["seconds"], r["its"]))
-        if r["ok"] and (best is None or r["step_ms"] < best["step_ms"]):
+        what = "seconds" if r["swept"] else "step_ms"
+        if r["ok"] and (best is None or r[what] < best[what]):
             best = r
     sn = best["slab_nodes"] if best else 128
     if best is not None:

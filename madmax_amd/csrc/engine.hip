@@ -921,6 +921,11 @@ extern "C" int mm_sweep_split(int nex, int ney, int nez, int fp64, int nrhs, int
   return 0;
 }
 
+extern "C" int mm_engine_swept(const mm_engine *e, const mm_rve_spec *spec)
+{
+  return e && spec && spec_valid(*spec) ? sweep_tiling(e, *spec).cw : 0;
+}
+
 extern "C" int mm_sweep_check(int nex, int ney, int nez, int fp64, const int *split, int *faults)
 {
   if (!split || !faults || nex < 2 || ney < 2 || nez < 2 || split[0] < 1 || split[1] < 1 || split[0] % split[1])

@@ -326,6 +326,8 @@ extern "C" int mm_sweep_split(int nex, int ney, int nez, int fp64, int nrhs, int
 // Before an engine's first step: the load cases of `mask` (bit k: case k) never meet, as
 // if other work kept the CUs.  For tests.
 extern "C" int mm_engine_set_meet_off(mm_engine *e, unsigned mask);
+// Workgroups per load case of such an RVE in this engine, 0: kernels A and B.
+extern "C" int mm_engine_swept(const mm_engine *e, const mm_rve_spec *spec);
 // Follows a split over its ranks and lanes.  faults: interior nodes not owned by one
 // item, words published twice, words read but not published, and words read from
 // outside the RVE or into another node's LDS place.

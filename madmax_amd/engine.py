@@ -216,6 +216,10 @@ class Engine:
         check(lib().mm_engine_download_x(self.h, key, load, _dp(x)), "download_x")
         return x
 
+    def swept(self, spec):
+        """Whether the engine solves such an RVE by on-chip sweeps (not by the step kernels)."""
+        return lib().mm_engine_swept(self.h, C.byref(spec)) > 0
+
     def time_spmv(self, reps=20):
         ms, by = C.c_double(), C.c_double()
         check(lib().mm_engine_time_spmv(self.h, reps, C.byref(ms), C.byref(by)), "time_spmv")
