@@ -177,11 +177,20 @@ def ell_api_spmv(mm, spec, reps=20, pcg_its=(60, 260)):
         mm._lib.check(L.ell_device_time_mvp(h, reps, C.byref(ms)), "ell_device_time_mvp")
         if pcg_its:
             pcg = {"bytes_per_iteration": rows * PCG_ROW_BYTES}
-            # per-step kernels: two launches per iteration up to 1024 slabs of
-            # 256 rows (every workgroup sums the partials), four beyond
-            pcg["per_step_launches_per_iteration"] = 2 if -(-rows // 256) <= 1024 else 4
             for name, f in (("per_step", 0), ("fused_1", 1), ("fused_32", 32), ("fused_all", 1 << 30)):
                 t = pcg_ms_per_iteration(mm, h, rows, f, *pcg_its)
+                counts = (C.c_int * 3)()
+                mm._lib.check(L.ell_device_pcg_counts(h, counts), "ell_device_pcg_counts")
+                if f == 0 and counts[0] > 0 and counts[1] == 0:
+                    # one launch per solve with the matrix on chip, where an
+                    # iteration reads none of bytes_per_iteration from memory
+                    pcg["on_chip"] = dict(ms_per_it=t)
+                    log("fp64 pcg (on chip), %d rows: %.4f ms/iteration" % (rows, t))
+                    continue
+                if f == 0:
+                    # per-step kernels: two launches per iteration up to 1024 slabs of
+                    # 256 rows (every workgroup sums the partials), four beyond
+                    pcg["per_step_launches_per_iteration"] = 2 if -(-rows // 256) <= 1024 else 4
                 pcg[name] = dict(ms_per_it=t, gbs=rows * PCG_ROW_BYTES / (t * 1e-3) / 1e9)
                 log("fp64 pcg (%s), %d rows: %.4f ms/iteration -> %.0f GB/s"
                     % (name, rows, t, pcg[name]["gbs"]))
