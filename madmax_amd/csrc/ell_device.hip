@@ -339,11 +339,14 @@ __device__ __forceinline__ void pcg_update_row(long long row, double alpha, cons
 // First the update's r.r / r.z (part[.][1..2]) give the iteration count, the
 // convergence test and beta (nothing to sum right after the start); then
 // q = A p (pcg_q_row) with partial p.q (part[.][0]).  The row's first slots are
-// asked for before the scalars are formed.
+// asked for before the scalars are formed.  Without AHEAD four waves per SIMD, though
+// the registers would allow six: 3,090,903 rows 618 us with six and 607 with four.
 template <int U, bool AHEAD>
-__global__ __launch_bounds__(AHEAD ? 256 : 1024) void k_pcg_spmv(const int *__restrict__ cols, const double *__restrict__ vals, int nrow, int nnz, int S,
-                           int nslab, double2 *__restrict__ zpA, double2 *__restrict__ zpB, double *__restrict__ q,
-                           double *__restrict__ part, const IterState *st_in, IterState *st_out, int self_sum)
+__global__ __launch_bounds__(AHEAD ? 256 : 1024)
+__attribute__((amdgpu_waves_per_eu(AHEAD ? 2 : 4, AHEAD ? 8 : 4)))
+void k_pcg_spmv(const int *__restrict__ cols, const double *__restrict__ vals, int nrow, int nnz, int S, int nslab,
+                double2 *__restrict__ zpA, double2 *__restrict__ zpB, double *__restrict__ q,
+                double *__restrict__ part, const IterState *st_in, IterState *st_out, int self_sum)
 {
   __shared__ double lds[48];
   __shared__ IterState N;
@@ -376,8 +379,10 @@ __global__ __launch_bounds__(AHEAD ? 256 : 1024) void k_pcg_spmv(const int *__re
 
 // alpha from the p.q partials; x += alpha p, r -= alpha q, z = dinv r
 // (pcg_update_row); partials r.r, r.z (part[.][1..2]).  The row's vectors are
-// asked for before the scalars are formed, both buffers' p because the state
-// says which is the new one.
+// asked for before the scalars are formed, where that takes the sums (self_sum) both
+// buffers' p because the state says which is the new one.  Past that, where memory
+// bounds the kernel, both cost more than they hide: 3,090,903 rows 48.3 us with both,
+// 44.0 with one.
 __global__ void k_pcg_update(int nrow, int S, int nslab, const double *__restrict__ dinv,
                              double2 *__restrict__ zpA, double2 *__restrict__ zpB, const double *__restrict__ q,
                              double *__restrict__ x, double *__restrict__ r, double *__restrict__ part,
@@ -392,8 +397,10 @@ __global__ void k_pcg_update(int nrow, int S, int nslab, const double *__restric
   double pA = 0.0, pB = 0.0;
   if (on) {
     pcg_row_load(row, dinv, q, x, r, w);
-    pA = zpA[row].y;
-    pB = zpB[row].y;
+    if (self_sum) {
+      pA = zpA[row].y;
+      pB = zpB[row].y;
+    }
   }
   if (lane == 0) N = *st_in;
   __syncthreads();
@@ -408,8 +415,9 @@ __global__ void k_pcg_update(int nrow, int S, int nslab, const double *__restric
   }
   if (blockIdx.x == 0 && lane == 0) *st_out = N;
   if (N.done) return;
-  w.p = N.pbuf ? pB : pA;                // the pairs whose p k_pcg_spmv wrote
-  double2 *zp = N.pbuf ? zpB : zpA;
+  double2 *zp = N.pbuf ? zpB : zpA;  // the pairs whose p k_pcg_spmv wrote
+  w.p = N.pbuf ? pB : pA;
+  if (!self_sum && on) w.p = zp[row].y;
   double v[2] = {0.0, 0.0};
   if (on) pcg_update_row(row, N.alpha, w, zp, x, r, v);
   block_sum<2>(v, lds);
