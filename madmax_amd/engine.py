@@ -93,6 +93,11 @@ def result_dicts(buf, n, nload):
     return out
 
 
+def result_dict(r, nload):
+    """One Result as such a dict."""
+    return result_dicts((Result * 1)(r), 1, lambda rid: nload)[0]
+
+
 class Engine:
     """Batched / serving RVE engine (mm_engine_*)."""
 
