@@ -18,6 +18,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <pthread.h>
 
 #include "ell.h"
 #include "fair_share.h"
@@ -1082,7 +1083,8 @@ struct ell_device_ {
   double2 *zpA, *zpB;  // PCG {z, p} pairs
   IterState *st;
   unsigned *bar;
-  char *stage;     // row-major entries on their way in (null until the first upload)
+  char *stage;     // row-major entries on their way in or out (null until the first)
+  pthread_mutex_t stage_mu;  // of downloads, which may overlap
   int band;        // most columns that a slab's rows span (0: not known)
   int ncu;         // CUs of the device
   // k_pcg_resident: solves to do otherwise before the next attempt, and how many that
@@ -1119,6 +1121,8 @@ static int stage_slabs(const ell_device *d)
   return most < 1 ? 1 : most < (size_t)d->nslab ? (int)most : d->nslab;
 }
 
+static size_t stage_bytes(const ell_device *d) { return (size_t)stage_slabs(d) * d->S * d->nnz * 12 + 8; }
+
 static dim3 place_grid(const ell_device *d, int slabs)
 {
   const int strips = (d->nnz + kPlaceSlots - 1) / kPlaceSlots;
@@ -1137,7 +1141,7 @@ static int upload(ell_device *d, const ell_matrix *m)
   }
   const int cs = stage_slabs(d);
   const size_t chunk = (size_t)cs * d->S * d->nnz;
-  if (!d->stage) MM_HIP(hipMalloc((void **)&d->stage, chunk * 12 + 8));
+  if (!d->stage) MM_HIP(hipMalloc((void **)&d->stage, stage_bytes(d)));
   double *sv = reinterpret_cast<double *>(d->stage);
   int *sc = reinterpret_cast<int *>(sv + chunk), *band = sc + chunk;
   k_zero_int<<<1, 64, 0, d->stream>>>(band, 1);
@@ -1169,6 +1173,7 @@ extern "C" int ell_device_create(const ell_matrix *m, int slab_rows, ell_device 
   if (check_cols(m)) return 1;
   ell_device *d = (ell_device *)calloc(1, sizeof(ell_device));
   if (!d) return 2;
+  pthread_mutex_init(&d->stage_mu, nullptr);
   d->nrow = m->nrow;
   d->ncol = m->ncol;
   d->nnz = m->nnz;
@@ -1225,17 +1230,20 @@ extern "C" int ell_device_update(ell_device *d, const ell_matrix *m)
   return upload(d, m);
 }
 
+// (Through the mirror's stage: memory allocated and freed by each call would make it
+// wait for all streams of the device, 39 ms beside an engine at work in place of 2.)
 extern "C" int ell_device_download(const ell_device *d, int *cols, double *vals)
 {
   if (!d || !cols || !vals) return 1;
   if (d->nrow == 0 || d->nnz == 0) return 0;
+  ell_device *m = const_cast<ell_device *>(d);
+  pthread_mutex_lock(&m->stage_mu);
+  hipError_t e = hipSuccess;
+  if (!m->stage) e = hipMalloc((void **)&m->stage, stage_bytes(d));
   const int cs = stage_slabs(d);
   const size_t chunk = (size_t)cs * d->S * d->nnz;
-  char *stage = nullptr;  // of this call: downloads of one mirror may overlap
-  MM_HIP(hipMalloc((void **)&stage, chunk * 12));
-  double *sv = reinterpret_cast<double *>(stage);
+  double *sv = reinterpret_cast<double *>(m->stage);
   int *sc = reinterpret_cast<int *>(sv + chunk);
-  hipError_t e = hipSuccess;
   for (int s = 0; s < d->nslab && e == hipSuccess; s += cs) {
     const int slabs = d->nslab - s < cs ? d->nslab - s : cs;
     const size_t r0 = (size_t)s * d->S, left = (size_t)d->nrow - r0;
@@ -1249,7 +1257,7 @@ extern "C" int ell_device_download(const ell_device *d, int *cols, double *vals)
     if (e == hipSuccess) e = hipMemcpyAsync(vals + at, sv, n * sizeof(double), hipMemcpyDeviceToHost, d->stream);
   }
   if (e == hipSuccess) e = hipStreamSynchronize(d->stream);
-  (void)hipFree(stage);
+  pthread_mutex_unlock(&m->stage_mu);
   MM_HIP(e);
   return 0;
 }
@@ -1497,6 +1505,7 @@ int mm::ell_device_alloc(int nrow, int nnz, int S, ell_device **out)
   if (!out || nrow < 0 || nnz < 1 || S % 64 != 0 || S < 64 || S > 1024) return MM_ERR_ARG;
   ell_device *d = (ell_device *)calloc(1, sizeof(ell_device));
   if (!d) return MM_ERR_ALLOC;
+  pthread_mutex_init(&d->stage_mu, nullptr);
   d->nrow = d->ncol = nrow;
   d->nnz = nnz;
   d->S = S;
