@@ -109,7 +109,8 @@ int ell_device_destroy(ell_device *d);
 /* How ell_device_solve_pcg (and the _noalloc variant) runs its iterations on
  * this mirror.  0 (the default): small matrices with slabs of 256 rows (up to
  * 384 slabs of at most 81 slots, the columns that one slab spans within the LDS)
- * in one launch per solve with the matrix on chip; others in two launches per
+ * in one launch per solve with the matrix on chip, unless other work keeps the
+ * CUs (then, and for some solves after, as the others); others in two launches per
  * iteration, q = A p and the vector update, each of whose workgroups first sums
  * the other's slab partials itself.  n > 0: one cooperative persistent kernel that runs up to
  * n whole iterations per launch, its workgroups meeting at two grid barriers

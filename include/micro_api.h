@@ -184,7 +184,9 @@ typedef struct {
   int device;
   size_t hbm_budget;     /* bytes for the RVE arena (0 = 80% of free memory) */
   int max_rves;          /* resident RVE slots (0 = 4096); on-chip sweeps of an
-                            engine of few slots spread over more of the GPU */
+                            engine of few slots spread over more of the GPU: one
+                            30^3 tangent takes 4.7 ms with 4096 slots and 2.7
+                            with 8, a batch that fills the GPU takes longer */
   int slab_nodes;        /* nodes per ELL slab = lanes per workgroup: 64, 128 or 256
                             (0 = 128); a slab holds 3 * slab_nodes rows */
   int nrhs;              /* load cases per RVE, 1..MM_MAX_RHS */
@@ -194,10 +196,11 @@ typedef struct {
   double inner_rtol;     /* per-sweep PCG target */
   int max_inner_its;
   int max_sweeps;
-  int steps_per_launch;  /* PCG iterations per launch / graph replay (whole
-                            sweeps, at most six, while every RVE being solved
-                            is small enough to be swept on chip: up to about
-                            100^3 elements in FP32 and 85^3 in FP64) */
+  int steps_per_launch;  /* PCG iterations per launch / graph replay.  While every
+                            RVE being solved is small enough to be swept on chip
+                            (up to about 100^3 elements in FP32 and 85^3 in FP64):
+                            whole steps, at most five: the first residual, up to
+                            two sweeps, the averages and the result */
   int use_graph;         /* capture the steps in a hipGraph */
   int sync_every_step;   /* plain path: host reads the state after every PCG
                             iteration (no on-chip sweeps) */

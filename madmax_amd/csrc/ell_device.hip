@@ -599,9 +599,10 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
 // Bound by the two exchanges of an iteration and the columns' z between them;
 // the two launches per iteration that it replaces were bound by the host's
 // launches for small matrices and by reading 12 bytes per entry for larger ones.
-// Elasticity systems of N^3 elements with 81 slots, us per iteration, two launches
-// against this: 2,970 rows 22.7 and 7.0, 14,739 rows 23.6 and 8.2, 46,875 rows
-// 25.0 and 9.8, 89,373 rows 32.5 and 13.0.
+// Elasticity systems of N^3 elements with 81 slots, time of a solve by its iterations
+// (81 .. 241), us, two launches against this: 2,970 rows 22.7 and 7.4, 14,739 rows 23.6
+// and 8.2, 46,875 rows 25.0 and 9.6, 89,373 rows 32.5 and 13.0 (11.7 each beside what
+// a solve takes once).
 //
 // All workgroups have to run at the same time.  They are at most three quarters of what
 // the CUs take, two to a CU (one where the LDS of two does not fit): 384 or 192 of 256
@@ -613,6 +614,7 @@ __global__ __launch_bounds__(kFusedLanes) void k_pcg_fused(
 // the mirror's next ones (1, 3, 7, .. 63 of them until one meets again).  After the
 // meeting all of them run; the waits are bounded all the same.
 constexpr int kResSlots = 81;  // rows of 27 nodes' 3 dofs; five registers for two slots, 203 of 256
+                              // (20 to 28 of the others spill, outside the product)
 constexpr int kResRest = 63;  // most solves in two launches between attempts
 inline int res_cus(int ncu) { return ncu - ncu / 4; }
 constexpr int kResOneCuLds = 69 * 1024;  // dynamic LDS up to which two workgroups fit a CU

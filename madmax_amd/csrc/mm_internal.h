@@ -191,7 +191,7 @@ struct EngPtrs {
   int a_slab;    // march on: some RVEs (mcpp == 0) need k_step_a as well
   int s_big;     // the group holds an RVE with big != 0: kernel S runs after A
   const int2 *units;  // [0].x: resident-sweep workgroups, [1..]: (slot, load case * 256 + rank)
-  unsigned *ticket;   // next unit to take; kernel B zeroes it (resident RVEs' first slabs)
+  unsigned *ticket;   // next unit to take; kernel R zeroes it (resident RVEs' first slabs)
   int u_grid, u_lds;  // launch of the resident sweep (0: none in the group)
 };
 
