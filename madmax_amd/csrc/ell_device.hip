@@ -820,7 +820,7 @@ __global__ __launch_bounds__(256, 2) void k_pcg_resident(const int *__restrict__
     s_row[4][lane] = pi;
   }
   for (int e = lane; e <= nneed; e += 256) res_p[e] = 0.0;
-  if (lane == 0 && !meet_wait(sums + 6, s_place)) s_fail = 1;
+  if (lane == 0 && !meet_wait(sums + 6, s_place, kMeetPolls)) s_fail = 1;
   __syncthreads();
   if (__builtin_amdgcn_readfirstlane(s_fail)) {
     if (lane == 0) st->pad0 = 1;

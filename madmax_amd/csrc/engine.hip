@@ -80,15 +80,16 @@ constexpr int kSweepSteps = 5;
 
 enum SlotState { SL_FREE = 0, SL_ACTIVE = 1, SL_CACHED = 2 };
 
-// Launches (of kSweepSteps steps or more) in a row in which no cluster of workgroups met
-// and some called their meeting off, after which those go on by kernels A and B: half a
-// second or so of other work that holds the CUs.
-constexpr int kMeetLaunches = 8;
+// Launches in a row, and their time in seconds, in which no cluster of workgroups met and
+// some called their meeting off, after which those go on by kernels A and B; and how many
+// cells do from the start, at most, before a cluster is tried again.
+constexpr int kMeetLaunches = 8, kMeetRest = 63;
+constexpr double kMeetSeconds = 0.5;
 
 // Split of a resident sweep (RveDev::scw ..), cw = 0: kernels A and B.
 struct SweepTiling {
   int cw = 0, ty = 1, lp = 0, nch = 0;
-  bool meet = false;
+  int meet = 0;
 };
 
 struct HostSlot {
@@ -245,8 +246,10 @@ struct mm_engine {
   unsigned *ticket = nullptr;
   size_t unit_stride = 0;
   long long unit_n[2] = {0, 0};
-  // launches in a row without a meeting (kMeetLaunches)
-  int meet_lost = 0;
+  // launches in a row without a meeting and when the first of them began, cells to step
+  // before the next cluster, and how many those were last time
+  int meet_lost = 0, meet_rest = 0, meet_rested = 0;
+  double meet_since = 0, t_step = 0;
   unsigned meet_off = 0;
   // one captured graph per set of launch shapes (grids: powers of two >= 64
   // covering each group's slabs and tiles, 0 for an empty group; kernel A's
@@ -890,7 +893,7 @@ static SweepTiling sweep_tiling(const mm_rve_spec &s, int tsz, int K, int rve_ca
     const long long part = nslab * 3 * SN * (long long)tsz;
     if (8LL * ((long long)nix * niy * niz * (tsz / 4) + sweep_sum_words(t.cw)) > part) t = SweepTiling();
   }
-  t.meet = t.cw > sweep_free_ranks(ncu);
+  t.meet = t.cw > sweep_free_ranks(ncu) ? kSweepMeetLarge : t.cw > 1 ? kSweepMeetFew : 0;
   return t;
 }
 
@@ -974,6 +977,16 @@ extern "C" int mm_sweep_check(int nex, int ney, int nez, int fp64, const int *sp
   return 0;
 }
 
+// The split of an RVE that is admitted.
+static void set_sweep(mm_engine *e, HostSlot &h)
+{
+  h.sweep = sweep_tiling(e, h.req.rve);
+  h.stepped = h.sweep.meet && e->meet_rest > 0;
+  if (!h.stepped) return;
+  e->meet_rest--;
+  h.sweep = SweepTiling();
+}
+
 static void fill_state(const mm_engine *e, const HostSlot &h, RveDev *st, int warm)
 {
   memset(st, 0, sizeof(*st));
@@ -1019,7 +1032,7 @@ static void fill_state(const mm_engine *e, const HostSlot &h, RveDev *st, int wa
   st->sty = sw.ty;
   st->slp = sw.lp;
   st->snch = sw.nch;
-  st->smeet = sw.meet ? 1 : 0;
+  st->smeet = sw.meet;
   st->big = (sw.cw == 0 && h.nslab >= e->cfg.big_slabs) ? 1 : 0;
   for (int k = 0; k < h.req.nload; k++)
     for (int i = 0; i < MM_NVOI; i++) st->load[k][i] = h.req.strain[k][i];
@@ -1117,8 +1130,7 @@ static int admit(mm_engine *e)
   size_t i = 0, ik = 0, ip = 0, is = 0;
   for (int s : fresh) {
     HostSlot &h = e->slots[s];
-    h.sweep = sweep_tiling(e, h.req.rve);
-    h.stepped = false;
+    set_sweep(e, h);
     fill_state(e, h, &e->st_states[i], 0);
     e->st_slots[i++] = s;
     for (int m = 0; m < kNmat; m++) {
@@ -1131,8 +1143,7 @@ static int admit(mm_engine *e)
   }
   for (int s : reused) {
     HostSlot &h = e->slots[s];
-    if (h.stepped) h.sweep = sweep_tiling(e, h.req.rve);
-    h.stepped = false;
+    if (h.stepped) set_sweep(e, h);
     fill_state(e, h, &e->st_states[i], h.req.warm_start ? 1 : 0);
     e->st_slots[i++] = s;
     for (long long b = 0; b < h.nslab; b++) e->st_slabs[is++] = (int)(h.first_slab + b);
@@ -1211,7 +1222,7 @@ static int update_active(mm_engine *e)
     if (half == 0 && ngroup == 2 && n[0] > 0 && 2 * n[0] >= total) half = 1;
     const SweepTiling &sw = h.sweep;
     // clusters that need most of the CUs at once stay in one chain of launches
-    const int g = sw.meet ? 0 : half;
+    const int g = sw.meet == kSweepMeetLarge ? 0 : half;
     for (long long b = 0; b < h.nslab; b++) e->st_act[g * stride + 1 + n[g]++] = (int)(r.first + b);
     if (sw.cw > 0) {
       res[g].push_back({h.nrow / 3, make_int2(r.second, sw.cw)});
@@ -1361,8 +1372,9 @@ static int run_steps(mm_engine *e)
 }
 
 // After a launch: counts it if clusters called their meeting off and none met, and
-// after kMeetLaunches of those moves the RVEs that still wait to kernels A and B.  One
-// such launch is enough until a cluster meets again.
+// after kMeetLaunches or kMeetSeconds of those moves the RVEs that still wait to kernels
+// A and B, and the next 1, 3, 7, .. 63 cells with them.  After those one lost launch is
+// enough, until a cluster meets again.
 static int check_meetings(mm_engine *e)
 {
   bool met = false;
@@ -1376,8 +1388,12 @@ static int check_meetings(mm_engine *e)
     h.met = o->met;
     h.missed = o->missed;
   }
-  if (met) e->meet_lost = 0;
-  if (met || waiting.empty() || ++e->meet_lost < kMeetLaunches) return 0;
+  if (met) e->meet_lost = e->meet_rest = e->meet_rested = 0;
+  if (met || waiting.empty()) return 0;
+  if (e->meet_lost++ == 0) e->meet_since = e->t_step;
+  if (e->meet_lost < kMeetLaunches && e->now() - e->meet_since < kMeetSeconds) return 0;
+  e->meet_lost = kMeetLaunches;
+  e->meet_rest = e->meet_rested = std::min(2 * e->meet_rested + 1, kMeetRest);
   for (int s : waiting) {
     HostSlot &h = e->slots[s];
     const int rc = eng_launch_stepped(e->rves, s, h.nslab >= e->cfg.big_slabs ? 1 : 0, e->stream);
@@ -1439,6 +1455,7 @@ extern "C" int mm_engine_step(mm_engine *e)
   if (!e) return MM_ERR_ARG;
   std::lock_guard<std::mutex> lk(e->step_mu);
   MM_HIP(hipSetDevice(e->cfg.device));
+  e->t_step = e->now();
   int rc = admit(e);
   if (rc) return e->last_error = rc;
   if (e->n_active > 0) {

@@ -105,6 +105,38 @@ __device__ void sweep_words_zero(const EngPtrs &P, const RveDev *R, int slab)
   }
 }
 
+// The words of the meetings: load case k's are two, k times `step` on from the first.
+struct MeetWords {
+  word_t *w;
+  long long step;
+};
+template <typename TS, int K>
+__device__ __forceinline__ MeetWords sweep_meeting(const EngPtrs &P, const RveDev *R)
+{
+  const long long ni = (long long)(R->nx - 2) * (R->ny - 2) * (R->nz - 2);
+  return {sweep_words<TS>(P, R->nslab, K, R->first_slab, 0, ni).sum + 16 * R->scw,
+          (long long)R->nslab * 3 * P.SN * (int)sizeof(TS) / 8};
+}
+// Which load cases' workgroups met in the launch (bit k); and parts them again.
+template <typename TS, int K>
+__device__ __forceinline__ unsigned sweep_met(const EngPtrs &P, const RveDev *R)
+{
+  const MeetWords m = sweep_meeting<TS, K>(P, R);
+  word_t w[K];
+  unsigned met = 0;
+#pragma unroll
+  for (int k = 0; k < K; k++) w[k] = m.w[k * m.step + 1];
+#pragma unroll
+  for (int k = 0; k < K; k++) met |= (w[k] == kMeetGo ? 1u : 0u) << k;
+  return met;
+}
+template <typename TS, int K>
+__device__ __forceinline__ void sweep_part(const EngPtrs &P, const RveDev *R)
+{
+  const MeetWords m = sweep_meeting<TS, K>(P, R);
+  for (int k = 0; k < K; k++) m.w[k * m.step] = m.w[k * m.step + 1] = 0;
+}
+
 // Whether a resident RVE's state st[0] is ready for the residual: it wants its
 // first one, or the sweep has run for every load case that needed it.
 template <typename TS, int K>
@@ -112,14 +144,7 @@ __device__ __forceinline__ bool sweep_ran(const EngPtrs &P, const RveDev *R)
 {
   const SolveState *S = &R->st[0];
   if (S->phase != PH_INNER) return S->phase == PH_RES;
-  const int cw = R->scw;
-  if (!R->smeet) return true;
-  const long long ni = (long long)(R->nx - 2) * (R->ny - 2) * (R->nz - 2);
-  bool ran = true;
-  for (int k = 0; k < K; k++)
-    if (!((S->done_in >> k) & 1u))
-      ran = ran && sweep_words<TS>(P, R->nslab, K, R->first_slab, k, ni).sum[16 * cw + 1] == kMeetGo;
-  return ran;
+  return !R->smeet || (~(S->done_in | sweep_met<TS, K>(P, R)) & ((1u << K) - 1u)) == 0;
 }
 
 // A resident RVE's state between launches, by one lane, after the residual (if
@@ -130,33 +155,24 @@ __device__ __forceinline__ bool sweep_ran(const EngPtrs &P, const RveDev *R)
 template <typename TS, int K>
 __device__ void sweep_end(const EngPtrs &P, int slot, RveDev *R, SolveState &N)
 {
-  const int cw = R->scw, phase = N.phase;
-  const long long ni = (long long)(R->nx - 2) * (R->ny - 2) * (R->nz - 2);
+  const int phase = N.phase, meets = R->smeet;
   bool left = false;
-  if (phase == PH_INNER || phase == PH_RES) {
+  if (phase == PH_INNER) {
+    unsigned ran = ~0u;
+    if (meets) ran = sweep_met<TS, K>(P, R);
     for (int k = 0; k < K; k++) {
-      const bool run = phase == PH_INNER && !((N.done_in >> k) & 1u);
-      if (R->smeet) {
-        word_t *meet = sweep_words<TS>(P, R->nslab, K, R->first_slab, k, ni).sum + 16 * cw;
-        const bool ran = meet[1] == kMeetGo;
-        meet[0] = meet[1] = 0;
-        if (run && !ran) {
-          left = true;
-          R->missed += 1;
-          continue;
-        }
-        if (run) {
-          N.done_in |= 1u << k;
-          R->met += 1;
-        }
-      }
-      if (run) N.its = max(N.its, R->lits[k]);
+      if ((N.done_in >> k) & 1u) continue;
+      if ((ran >> k) & 1u) N.its = max(N.its, R->lits[k]);
+      else left = true;
     }
-    if (R->smeet && phase == PH_INNER) {
-      P.out[slot].met = R->met;
-      P.out[slot].missed = R->missed;
+    if (meets) {
+      const unsigned run = ~N.done_in & ((1u << K) - 1u);
+      P.out[slot].met = R->met += __popc(run & ran);
+      P.out[slot].missed = R->missed += __popc(run & ~ran);
+      N.done_in |= ran;
     }
   }
+  if (meets && (phase == PH_INNER || phase == PH_RES)) sweep_part<TS, K>(P, R);
   if (phase == PH_INNER && !left) {
     N.its_total += N.its;
     N.sweep += 1;

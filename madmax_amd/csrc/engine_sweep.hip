@@ -587,8 +587,8 @@ extern __shared__ __attribute__((aligned(16))) double sweep_dyn[];
 // without waiting for anyone else, and their places go to the missing ranks
 // (also beside other such launches: each leaves at most one cluster of at most
 // sweep_free_ranks workgroups waiting, and the GPU has more places than the
-// queues' launches can fill with those; a larger cluster waits only before it has
-// started, and not for long: cluster_meet).
+// queues' launches can fill with those).  A cluster waits only before it has
+// started (meet_wait), a larger one not for long.
 // The residual follows (k_sweep_res), and kernel R passes the state on.
 template <typename TS, int K>
 __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp)
@@ -632,11 +632,12 @@ __global__ __launch_bounds__(kSweepLanes) void k_sweep(EngPtrs P, SolveParams sp
   const SweepGeo g = sweep_geo_of(R, rk);
   const int SN = P.SN, RS = 3 * SN, fs = scalar(R->first_slab), tsz = (int)sizeof(TS);
   const SweepWords X = sweep_words<TS>(P, scalar(R->nslab), K, fs, k, g.ni);
-  if (scalar(R->smeet)) {
+  const int meets = scalar(R->smeet);
+  if (meets) {
     if (tid == 0) {
       word_t *meet = X.sum + 16 * g.cw;
       if ((sp.meet_off >> k) & 1u) meet_off(meet);
-      s_unit = meet_wait(meet, meet_arrive(meet, g.cw)) ? 1 : 0;
+      s_unit = meet_wait(meet, meet_arrive(meet, g.cw), meets == kSweepMeetLarge ? kMeetPolls : kMeetPatience) ? 1 : 0;
     }
     __syncthreads();
     if (scalar(s_unit) == 0) return;

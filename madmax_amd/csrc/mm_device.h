@@ -207,7 +207,8 @@ __device__ __forceinline__ double word_double(word_t lo, word_t hi)
 // that two groups on different streams that keep each other from the CUs do not go on
 // doing so.  Run by one lane of each workgroup.
 constexpr word_t kMeetGo = 1, kMeetOff = 2;
-constexpr int kMeetPolls = 1 << 14;  // some 10 ms, plus as much at random
+constexpr int kMeetPolls = 1 << 14;     // some 10 ms, plus as much at random
+constexpr int kMeetPatience = 1 << 18;  // some 0.2 s, for groups that leave the others room
 __device__ __forceinline__ void meet_set(word_t *meet, word_t to)
 {
   word_t none = 0;
@@ -222,9 +223,9 @@ __device__ __forceinline__ int meet_arrive(word_t *meet, int count)
   if (n + 1 == count) meet_set(meet, kMeetGo);
   return n;
 }
-__device__ __forceinline__ bool meet_wait(word_t *meet, int place)
+__device__ __forceinline__ bool meet_wait(word_t *meet, int place, int polls)
 {
-  const int most = place == 0 ? kMeetPolls + (int)(clock64() & (kMeetPolls - 1)) : 4 * kMeetPolls;
+  const int most = place == 0 ? polls + (int)(clock64() & (polls - 1)) : 4 * polls;
   for (int i = 0;; i++) {
     const word_t m = get_word(&meet[1]);
     if (m != 0) return m == kMeetGo;

@@ -130,7 +130,7 @@ struct RveDev {
   // items of slp planes of one column; lits[k] is the iteration count of load
   // case k in the sweep.  scw == 0: kernels A and B.
   int scw, sty, slp, snch;
-  int smeet;  // the workgroups of a load case meet before they wait for each other
+  int smeet;  // scw > 1: kSweepMeetFew or kSweepMeetLarge
   // load cases whose workgroups met and did not since admission, and sweeps that
   // ended (k_stepped) without an update of some load cases and of all
   int met, missed, again, idle;
@@ -239,10 +239,12 @@ constexpr int kMarchMaxLds = 64 * 1024;
 // kernel.
 constexpr int kSweepLanes = 512;  // two waves per SIMD, 256 VGPRs each
 constexpr int kSweepItems = 2;    // items (a column times slp planes) per lane
-// Workgroups per load case, of a device of ncu CUs.  A cluster that waits for ranks
-// without a CU holds the CUs of the others; with up to sweep_free_ranks, four queues
-// of waiting clusters leave room for any missing rank, and larger clusters first
-// meet (RveDev::smeet).
+// Workgroups per load case, of a device of ncu CUs.  The ranks of a cluster meet before
+// they wait for each other (RveDev::smeet): other work, or a mask of CUs, may leave
+// fewer than they need.  A cluster that waits for ranks without a CU holds the CUs of
+// the others; with up to sweep_free_ranks, four queues of waiting clusters leave room
+// for any missing rank, and they have patience.  Larger ones do not.
+constexpr int kSweepMeetFew = 1, kSweepMeetLarge = 2;
 constexpr int kSweepFreeRanks = 16, kSweepMaxRanks = 240;  // of the 256 CUs of a whole device
 inline int sweep_free_ranks(int ncu) { return ncu >= 256 ? kSweepFreeRanks : ncu >= 32 ? ncu / 16 : 1; }
 inline int sweep_max_ranks(int ncu) { return ncu >= 256 ? kSweepMaxRanks : ncu - (ncu + 15) / 16; }

@@ -44,12 +44,13 @@ def _solve(eng, specs, loads, mode, **kw):
 
 @pytest.mark.parametrize("guess", [MM_GUESS_AFFINE, MM_GUESS_ZERO])
 @pytest.mark.parametrize("precision", [MM_PREC_MIXED, MM_PREC_FP64])
-def test_no_meeting_one_load_case(precision, guess):
-    """Alone, then beside a cell of few workgroups (swept on chip in the launches that step the other), the first one
-    again from its kept displacements, and with the kept slot on chip again."""
-    n = (36, 34, 33)
-    assert split_meet(n, precision == MM_PREC_FP64, 1, 4, 128, 256)[4] == 1
-    big, small = rve_spec(n, [(0.45, 0.55, 0.3)]), rve_spec((12, 11, 9), [(0.5, 0.5, 0.3)])
+@pytest.mark.parametrize("n,meet", [((36, 34, 33), 2), ((24, 24, 24), 1)])
+def test_no_meeting_one_load_case(n, meet, precision, guess):
+    """Alone, then, stepped from the start, beside a cell of one workgroup (swept on chip in the launches that step the
+    other), and the first one again from its kept displacements, when its cluster is tried again."""
+    fp64 = precision == MM_PREC_FP64
+    assert split_meet(n, fp64, 1, 4, 128, 256)[4] == meet and split_meet((5, 5, 5), fp64, 1, 4, 128, 256)[0] == 1
+    big, small = rve_spec(n, [(0.45, 0.55, 0.3)]), rve_spec((5, 5, 5), [(0.5, 0.5, 0.3)])
     ref = []
     with Engine(nrhs=1, sync_every_step=True, **_kw(precision, initial_guess=guess)) as eng:
         ref += _solve(eng, [big, small], [EPS], MM_TANGENT_NONE, warm_key=1)
@@ -68,10 +69,10 @@ def test_no_meeting_one_load_case(precision, guess):
 
 
 @pytest.mark.parametrize("mask", [0b000101, 0b111110, 0b111111])
-def test_some_load_cases_do_not_meet(mask):
+@pytest.mark.parametrize("n,meet", [((50, 47, 45), 2), ((24, 24, 24), 1)])
+def test_some_load_cases_do_not_meet(n, meet, mask):
     """The displacements of the load cases that ran are kept, in one and in two stream groups."""
-    n = (50, 47, 45)
-    assert split_meet(n, False, 6, 4, 128, 256)[4] == 1
+    assert split_meet(n, False, 6, 4, 128, 256)[4] == meet
     spec = rve_spec(n, [(0.45, 0.55, 0.3)])
     with Engine(nrhs=6, sync_every_step=True, **_kw(MM_PREC_MIXED)) as eng:
         s = _solve(eng, [spec], unit_loads(), MM_TANGENT_UNIT)[0]

@@ -17,7 +17,7 @@ def split(n, fp64, nrhs, max_rves, slab_nodes=128, ncu=256):
 
 
 def split_meet(n, fp64, nrhs, max_rves, slab_nodes, ncu):
-    """The same and whether the ranks meet before they wait for each other."""
+    """The same and how the ranks meet before they wait for each other: 1 with patience, 2 without, 0 not (one)."""
     out = (C.c_int * 5)()
     assert _lib.lib().mm_sweep_split(*n, int(fp64), nrhs, max_rves, slab_nodes, ncu, out) == 0
     return tuple(out)
@@ -72,8 +72,8 @@ def test_every_word_that_is_read_is_published():
 
 @pytest.mark.parametrize("ncu", [1, 8, 32, 64, 128, 256, 304])
 def test_splits_fit_the_device(ncu):
-    """A cluster never has more ranks than the device can run at once, and one that does not meet first is small
-    enough that four waiting ones leave room for a missing rank."""
+    """A cluster never has more ranks than the device can run at once, all but single workgroups meet first, and one
+    that waits with patience is small enough that four of them leave room for a missing rank."""
     rng, some = random.Random(ncu), 0
     for _ in range(1500):
         n = tuple(rng.randint(2, rng.choice([24, 60, 110])) for _ in range(3))
@@ -83,7 +83,8 @@ def test_splits_fit_the_device(ncu):
             continue
         some += 1
         assert s[0] <= max(1, min(ncu - 1, 240)) and faults(n, fp64, s[:4]) == (0, 0, 0, 0)
-        if s[0] > 1 and not s[4]:
+        assert (s[4] > 0) == (s[0] > 1)
+        if s[4] == 1:
             assert s[0] <= 16 and 4 * (s[0] - 1) < ncu
     assert some > 100
 
