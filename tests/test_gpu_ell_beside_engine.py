@@ -3,7 +3,9 @@ engine's launches, which take some 40 ms each here.  Downloads of one mirror on 
 threads do not disturb each other.
 
 The bar of 10 ms lies between the two: without a wait for the engine a download takes
-some 2 ms, the time until a running sweep leaves a CU."""
+some 2 ms, the time until a running sweep leaves a CU.  Streams share the process's four
+hardware queues in turn, and one that shares the engine's waits for it whatever it does:
+of six mirrors, made one after the other, at least two do not."""
 import ctypes as C
 import threading
 import time
@@ -25,10 +27,11 @@ def _download(h, shape):
 
 def test_download_beside_an_engine_at_work():
     cols, vals = matrix(3000, 3000, 81, 1)
-    m, h, rc = create(cols, vals, 3000, 0)
-    assert rc == 0
-    specs, stop, times = [configs.c2_spec(1, i) for i in range(128)], threading.Event(), []
+    specs, stop, medians = [configs.c2_spec(1, i) for i in range(128)], threading.Event(), []
     with Engine(nrhs=6, hbm_budget=8 << 30, max_rves=136, rtol=1e-9) as eng:
+        mirrors = [create(cols, vals, 3000, 0) for _ in range(6)]
+        assert all(rc == 0 for _, _, rc in mirrors)
+
         def work():
             while not stop.is_set():
                 for i, s in enumerate(specs):
@@ -40,18 +43,22 @@ def test_download_beside_an_engine_at_work():
         th.start()
         try:
             time.sleep(0.3)
-            for _ in range(21):
-                t = time.perf_counter()
-                got = _download(h, cols.shape)
-                times.append(time.perf_counter() - t)
-                assert np.array_equal(got[0], cols) and np.array_equal(got[1], vals)
-                time.sleep(0.005)
+            for _, h, _ in mirrors:
+                times = []
+                for _ in range(11):
+                    t = time.perf_counter()
+                    got = _download(h, cols.shape)
+                    times.append(time.perf_counter() - t)
+                    assert np.array_equal(got[0], cols) and np.array_equal(got[1], vals)
+                    time.sleep(0.005)
+                medians.append(np.median(times))
         finally:
             stop.set()
             th.join()
-    _lib.lib().ell_device_destroy(h)
-    print("download: median %.2f ms, longest %.2f" % (1e3 * np.median(times), 1e3 * max(times)))
-    assert np.median(times) < 0.010
+    for _, h, _ in mirrors:
+        _lib.lib().ell_device_destroy(h)
+    print("download, medians:", ", ".join("%.2f ms" % (1e3 * t) for t in medians))
+    assert sorted(medians)[1] < 0.010
 
 
 def test_downloads_on_several_threads():

@@ -102,3 +102,13 @@ def test_cells_of_the_sweep_tests_are_swept(n):
     for fp64 in (False, True):
         for max_rves in (32, 64):
             assert split(n, fp64, 6, max_rves)[0] > 0
+
+
+@pytest.mark.parametrize("fp64,n,max_rves,large", [
+    (False, (24, 22, 20), 4, False), (False, (44, 41, 39), 200, False), (False, (60, 52, 50), 4, True),
+    (False, (82, 80, 78), 2, True), (True, (30, 28, 26), 2, False), (True, (50, 47, 45), 200, True),
+    (False, (72, 70, 68), 3, True), (False, (100, 100, 100), 9, True)])
+def test_cells_of_the_one_load_case_tests_are_swept(fp64, n, max_rves, large):
+    """And those that are to be split over large clusters are."""
+    s = split_meet(n, fp64, 1, max_rves, 128, 256)
+    assert s[0] > 1 and s[4] == (2 if large else 1)
